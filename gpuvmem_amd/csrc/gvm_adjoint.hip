@@ -1,4 +1,8 @@
-// DChi2 adjoint on gfx950 MFMA.
+// DChi2 adjoint on gfx950: the choice of its form, and the forms on the MFMA
+// units and the VALU.  Where it applies the adjoint runs by gridding and FFT
+// (gvm_adjoint_fft.hip, 50 to 150 times faster at the workloads' sizes and closer
+// to FP64); the GEMM below takes observations of few rows on a large image and
+// w terms too large for that form's planes.
 //
 // Reference: DChi2 (src/functions.cu:3698-3791) evaluates, for every pixel
 // inside the mask,
@@ -152,19 +156,6 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 constexpr int kGemmThreads = 512;
-constexpr int kPScale = 15;  // max |P| = 2^15 < 65504 (FP16 max)
-constexpr int kPScaleLimit = 100;
-
-// Exponent of the power-of-two scale of P for a slice whose largest |c| is
-// cm: 2^e cm <= 2^kPScale.  Clamped to [-kPScaleLimit, kPScaleLimit] so that
-// the scale and its inverse stay finite and normal in FP32 for any cm (an
-// unclamped exponent overflows for cm below about 2^-113, and 0 * inf would
-// turn the zero amplitudes of off-grid samples into NaN); 0 when cm is 0.
-__device__ __forceinline__ int p_scale_exponent(float cm) {
-  if (!(cm > 0.0f)) return 0;
-  const int e = kPScale - (int)ceilf(log2f(cm));
-  return min(max(e, -kPScaleLimit), kPScaleLimit);
-}
 constexpr int kHalfKV = kKV / 2;
 
 // One workgroup (8 waves, 2 per SIMD) owns a 256x256 tile of G for one
@@ -678,10 +669,37 @@ gvm_status build_splits(gvm_ctx* ctx, int mode, int ntiles, long n) {
 
 }  // namespace
 
-gvm_status rebuild_splits(gvm_ctx* ctx) {
-  const int N = ctx->g.N;
+// Fewer rows than this over all slices: the GEMM is the faster one.  The
+// gridded form's time is that of its FFTs, the GEMM's falls with the rows:
+// one evaluation at 2048^2 takes 226 / 163 us (gridded / GEMM) at 30 rows, 248
+// / 270 at 840, 264 / 307 at 5,700; at 4096^2 881 / 631, 1005 / 820, 1160 / 1332;
+// at 1024^2 and below the gridded form is faster from 30 rows on (73 / 80).
+static long min_gridded_rows(int N) { return N < 2048 ? 0 : (long)N * N / 8192; }
+
+// Decides how the adjoint of the current form runs and sizes its workspace:
+// the GEMM forms by gridding and FFT (gvm_adjoint_fft.hip) where that applies,
+// else in ranges of visibilities; the direct form one range per slice.
+static gvm_status split_work(gvm_ctx* ctx) {
+  const int N = ctx->g.N, mode = ctx->adjoint_mode;
+  ctx->adj_gridded = false;
+  long rows = 0;
+  for (const Slice& s : ctx->slices) rows += s.nvis;
+  if (mode != GVM_ADJOINT_DIRECT && rows >= min_gridded_rows(N)) {
+    bool ok = false;
+    gvm_status st = build_grid_plan(ctx, &ok);
+    if (st) return st;
+    if (ok) {
+      ctx->adj_gridded = true;
+      ctx->split_mode = mode;
+      return GVM_OK;
+    }
+  }
   const int tiles_x = (N + kTile - 1) / kTile;
-  gvm_status st = build_splits(ctx, ctx->adjoint_mode, tiles_x * tiles_x, (long)N * N);
+  return build_splits(ctx, mode, tiles_x * tiles_x, (long)N * N);
+}
+
+gvm_status rebuild_splits(gvm_ctx* ctx) {
+  gvm_status st = split_work(ctx);
   if (st) return st;
   ctx->epoch++;
   return GVM_OK;
@@ -700,11 +718,11 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
     GVM_REQUIRE(!ctx->capturing,
                 "gvm_dchi2: the workspace is sized by the first gvm_dchi2; run one before "
                 "capturing");
-    gvm_status st = build_splits(ctx, mode, ntiles, n);
+    gvm_status st = split_work(ctx);
     if (st) return st;
     ctx->epoch++;
   }
-  if (mode != GVM_ADJOINT_DIRECT) {
+  if (mode != GVM_ADJOINT_DIRECT && !ctx->adj_gridded) {
     long vmax = 0;
     for (const Slice& s : ctx->slices) vmax = std::max(vmax, s.nvis);
     const unsigned nbp = (unsigned)std::min<long>(2048, std::max<long>(1, (vmax + 255) / 256));
@@ -722,7 +740,10 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
     pair = (ctx->tev_head + ctx->tev_pending) % gvm_ctx::kTimingPairs;
     GVM_HIP_TRY(hipEventRecord(ctx->tev[2 * pair], ctx->stream));
   }
-  if (mode == GVM_ADJOINT_DIRECT) {
+  if (ctx->adj_gridded) {
+    gvm_status st = adjoint_grid(ctx, I, result, flag_opt, normalize);
+    if (st) return st;
+  } else if (mode == GVM_ADJOINT_DIRECT) {
     const double dxr = g.deltax * 3.14159265358979323846 / 180.0;
     const double dyr = g.deltay * 3.14159265358979323846 / 180.0;
     for (int si = 0; si < nsl; si++) {
@@ -752,6 +773,7 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
     GVM_HIP_TRY(hipEventRecord(ctx->tev[2 * pair + 1], ctx->stream));
     ctx->tev_pending++;
   }
+  if (ctx->adj_gridded) return GVM_OK;  // its last kernel is the epilogue
   hipLaunchKernelGGL(adjoint_epilogue_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
                      ctx->stream, ctx->adj_part, ctx->slice_p0, ctx->slice_tab, nsl, n, ctx->cmax,
                      mode == GVM_ADJOINT_DIRECT ? 0 : 1, ctx->noise, g.noise_cut, g.fg_scale,

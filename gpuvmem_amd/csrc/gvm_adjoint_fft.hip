@@ -1,0 +1,1146 @@
+// DChi2 adjoint by gridding and FFT on gfx950.
+//
+// The adjoint's sums G(i,j) = Re sum_v c_v e^{i phi_v(i,j)}, c_v = w_v
+// conj(Vr_v), phi = 2 pi (x_j u_v + y_i v_v + (z_ij - 1) w_v)
+// (src/functions.cu:3698-3791) are a non-uniform discrete Fourier transform.
+// Here it is evaluated as one: every visibility is spread onto a uv grid
+// oversampled twice with a narrow kernel, the grid is transformed with FFTs
+// and the image is divided by the kernel's transform (the method of Dutt and
+// Rokhlin, SIAM J. Sci. Comput. 14 (1993) 1368; a kernel exp(-polynomial) in the
+// manner of the "exponential of semicircle" of Barnett, Magland and af
+// Klinteberg, SIAM J. Sci. Comput. 41 (2019) C479).  The work falls from 4 N^2 Nvis flop (the GEMM of
+// gvm_adjoint.hip) to about 81 K grid updates per visibility and K FFTs of
+// (2N)^2; all arithmetic is FP32 or better, and the approximation (9 taps at
+// twice oversampling, 2.3e-8) is under FP32 rounding.
+//
+// w term.  With t = w / W in [-1, 1] and zeta = 2 pi W (z - 1), the
+// Jacobi-Anger expansion e^{i zeta t} = J_0(zeta) + 2 sum_k i^k J_k(zeta)
+// T_k(t) turns the w phase into K planes: plane k grids i^k c T_k(t) and is
+// weighted by J_k(zeta) per pixel.  K is the smallest count whose truncation
+// 2 (|zeta|/2)^K / K! over the pixels on the mask is below kPlaneTol.  (The
+// pixel coordinate is the exact z - 1, not the per-axis split of the GEMM.)
+//
+// Real output.  Only Re is wanted, so a visibility with u beyond the grid's
+// Nyquist column is folded to the conjugate point, only columns X = 0 .. N of
+// the 2N x 2N grid exist, and the second transform is complex-to-real.
+//
+// Steps of one evaluation:
+//  1. spread_kernel   one wave per work item (at most `chunk` visibilities of
+//                     one 8 x 8 tile of the grid, sorted at set-up): the
+//                     item's 16 x 16 subgrid of every plane as a product on
+//                     the FP32 MFMA units, sum_v ky_v(row) [kx_v(col) c_v T_k];
+//  2. merge_kernel    subgrids of tiles with several items, summed in FP64;
+//  3. cols_kernel     gathers the (up to four) subgrids that overlap each grid
+//                     cell and transforms the columns (2N points);
+//  4. rows_kernel     per image row: complex-to-real transforms of the K
+//                     planes, their combination, the kernel correction,
+//                     -fg PB, the chain rule (the GEMM form's epilogue).
+// Every sum has a fixed order, so results are reproducible bit for bit.
+#include <hip/hip_runtime.h>
+
+#include <rocprim/device/device_radix_sort.hpp>
+#include <rocprim/device/device_scan.hpp>
+
+#include <algorithm>
+#include <cmath>
+#include <utility>
+#include <vector>
+
+#include "gvm_fft.h"
+#include "gvm_internal.h"
+
+namespace gvm {
+
+namespace {
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr double kPi = 3.14159265358979323846;
+constexpr int kTaps = 9;                 // kernel width in cells of the 2N grid
+constexpr double kPlaneTol = 5e-8;       // truncation of the w expansion
+constexpr int kMaxPlanes = 32;
+constexpr int kPlaneGroup = 8;           // planes one spread launch accumulates
+constexpr int kSub = 512;                // floats of a 16 x 16 complex subgrid
+constexpr long kGroupRows = 1L << 27;    // rows sorted together at set-up
+constexpr size_t kBatchBytes = 512u << 20;  // workspace one batch of slices aims at
+
+// The spreading kernel: 2^-P(v), v = (d / 4.5)^2, 0 beyond 4.5 cells.  P's
+// coefficients minimise the aliased part of the kernel's transform over the
+// pixels kept (least squares over |offset| <= N / 2 and the first six images
+// of the band): 2.3e-8 rms, 3.9e-8 at most, where the exponential of semicircle
+// of the same width (beta 20.7) has 1.3e-8 and 5.0e-8 but takes a square root
+// and a reciprocal more per value.
+constexpr float kInvHalf = (float)(2.0 / kTaps);
+constexpr double kLog2e = 1.44269504088896340736;
+constexpr float kP1 = (float)(10.596313090281376 * kLog2e);
+constexpr float kP2 = (float)(2.670875389609385 * kLog2e);
+constexpr float kP3 = (float)(1.278424264908622 * kLog2e);
+constexpr float kP4 = (float)(0.7525254439992803 * kLog2e);
+constexpr float kP5 = (float)(0.31046272601257235 * kLog2e);
+constexpr float kP6 = (float)(0.4732201062869989 * kLog2e);
+__device__ __forceinline__ float spread_value(float d) {
+  const float u = d * kInvHalf, v = u * u;
+  float p = fmaf(v, kP6, kP5);
+  p = fmaf(v, p, kP4);
+  p = fmaf(v, p, kP3);
+  p = fmaf(v, p, kP2);
+  p = fmaf(v, p, kP1);
+  const float e = __builtin_amdgcn_exp2f(-(v * p));
+  return v <= 1.0f ? e : 0.0f;
+}
+
+int blocks_for(long n) { return (int)std::max(1L, std::min<long>((n + 255) / 256, 8192)); }
+
+// ---------------------------------------------------------------------------
+// set-up: visibilities of a group of slices sorted by (slice, tile)
+// ---------------------------------------------------------------------------
+
+// Position of a visibility on the oversampled half grid.
+struct GridPos {
+  int bx, by;     // nearest cell, bx in [0, N], by in [0, 2N)
+  double dx, dy;  // offset from it, in [-1/2, 1/2]
+  bool conj;      // folded: the conjugate point
+};
+
+__device__ __forceinline__ GridPos grid_pos(float4 p, int N) {
+  // turns per pixel, exact (gvm_add_visibilities splits them into two floats)
+  const double a = (double)p.x + (double)p.y;
+  double b = (double)p.z + (double)p.w;
+  const double L = 2.0 * N;
+  GridPos g;
+  const double X = (a - floor(a)) * L;
+  double bx = rint(X);
+  g.dx = X - bx;
+  g.conj = bx > (double)N;
+  if (g.conj) {
+    bx = L - bx;
+    g.dx = -g.dx;
+    b = -b;
+  }
+  const double Y = (b - floor(b)) * L;
+  const double by = rint(Y);
+  g.dy = Y - by;
+  g.bx = (int)bx;
+  g.by = (int)by & (2 * N - 1);
+  return g;
+}
+
+// max |w| over rows with a weight, as float bits; an infinite or NaN w counts
+// with any weight (it makes the sums NaN) and is larger than any number
+__global__ __launch_bounds__(256) void wmax_kernel(const SliceDev* __restrict__ tab,
+                                                   unsigned int* __restrict__ out) {
+  const SliceDev& sd = tab[blockIdx.y];
+  unsigned int m = 0u;
+  for (long v = blockIdx.x * 256L + threadIdx.x; v < sd.nvis; v += (long)gridDim.x * 256) {
+    const unsigned int b = __float_as_uint(ldg(sd.wcoord + v)) & 0x7fffffffu;
+    if (ldg(sd.weight + v) != 0.0f || b >= 0x7f800000u) m = max(m, b);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned int)__shfl_xor((int)m, o, 64));
+  if ((threadIdx.x & 63) == 0 && m) atomicMax(out, m);
+}
+
+// keys of the rows of slice s0 + blockIdx.y; off[] are the slices' first rows
+// within the group
+__global__ __launch_bounds__(256) void plan_keys_kernel(const SliceDev* __restrict__ tab, int s0,
+                                                        const unsigned int* __restrict__ off, int N,
+                                                        unsigned int* __restrict__ keys,
+                                                        unsigned int* __restrict__ ids) {
+  const SliceDev& sd = tab[s0 + blockIdx.y];
+  const unsigned int ntiles = (unsigned int)(N / 8 + 1) * (N / 4);
+  const unsigned int o = off[blockIdx.y];
+  for (long v = blockIdx.x * 256L + threadIdx.x; v < sd.nvis; v += (long)gridDim.x * 256) {
+    const GridPos g = grid_pos(ldg(sd.phs + v), N);
+    keys[o + v] = blockIdx.y * ntiles + (unsigned int)(g.bx >> 3) * (N / 4) + (g.by >> 3);
+    ids[o + v] = o + (unsigned int)v;
+  }
+}
+
+// Sorted records: (dx, dy, w, weight) and (row of its slice, cell within the
+// tile and fold), and the phase-centre rotation when the image is not centred
+// on it.
+__global__ __launch_bounds__(256) void plan_records_kernel(
+    const SliceDev* __restrict__ tab, int s0, const unsigned int* __restrict__ off, int N, long n,
+    const unsigned int* __restrict__ keys, const unsigned int* __restrict__ ids,
+    int shift_x, int shift_y, float4* __restrict__ rec, uint2* __restrict__ meta,
+    float2* __restrict__ rot) {
+  const unsigned int ntiles = (unsigned int)(N / 8 + 1) * (N / 4);
+  for (long p = blockIdx.x * 256L + threadIdx.x; p < n; p += (long)gridDim.x * 256) {
+    const unsigned int s = keys[p] / ntiles;
+    const SliceDev& sd = tab[s0 + s];
+    const unsigned int v = ids[p] - off[s];
+    const float4 ph = ldg(sd.phs + v);
+    const GridPos g = grid_pos(ph, N);
+    const float w = ldg(sd.wcoord + v);
+    rec[p] = make_float4((float)g.dx, (float)g.dy, g.conj ? -w : w, ldg(sd.weight + v));
+    meta[p] = make_uint2(v, (unsigned int)(g.bx & 7) | (g.by & 7) << 3 | (g.conj ? 64u : 0u));
+    if (rot) {
+      double r = ((double)ph.x + (double)ph.y) * shift_x + ((double)ph.z + (double)ph.w) * shift_y;
+      r -= rint(r);
+      double sn, cs;
+      sincospi(2.0 * r, &sn, &cs);
+      rot[p] = make_float2((float)cs, (float)sn);
+    }
+  }
+}
+
+// start[k] = the first sorted row with key >= k, k in [0, nkeys]
+__global__ __launch_bounds__(256) void tile_starts_kernel(const unsigned int* __restrict__ keys,
+                                                          long n, long nkeys,
+                                                          unsigned int* __restrict__ start) {
+  for (long k = blockIdx.x * 256L + threadIdx.x; k <= nkeys; k += (long)gridDim.x * 256) {
+    long lo = 0, hi = n;
+    while (lo < hi) {
+      const long m = (lo + hi) >> 1;
+      if ((long)keys[m] < k)
+        lo = m + 1;
+      else
+        hi = m;
+    }
+    start[k] = (unsigned int)lo;
+  }
+}
+
+// items per tile, and whether it has several (0 past the last tile)
+__global__ __launch_bounds__(256) void item_counts_kernel(const unsigned int* __restrict__ start,
+                                                          long nkeys, int chunk,
+                                                          unsigned int* __restrict__ cnt,
+                                                          unsigned int* __restrict__ several) {
+  for (long k = blockIdx.x * 256L + threadIdx.x; k <= nkeys; k += (long)gridDim.x * 256) {
+    const unsigned int c =
+        k < nkeys ? (start[k + 1] - start[k] + (unsigned int)chunk - 1) / (unsigned int)chunk : 0u;
+    cnt[k] = c;
+    several[k] = c > 1 ? 1u : 0u;
+  }
+}
+
+// Items of tile k at [islot[k], islot[k + 1]): (first row, rows, slice, 0);
+// islot[k] becomes tile_slot[k] (-1 for a tile without rows); merge mslot[k]
+// is tile k's when it has several items.
+__global__ __launch_bounds__(256) void items_kernel(const unsigned int* __restrict__ start,
+                                                    const unsigned int* __restrict__ islot,
+                                                    const unsigned int* __restrict__ mslot,
+                                                    long nkeys, int chunk, long row0,
+                                                    unsigned int ntiles, int s0,
+                                                    unsigned int item0, unsigned int merge0,
+                                                    long4* __restrict__ items,
+                                                    int2* __restrict__ merges,
+                                                    int* __restrict__ tile_slot) {
+  for (long k = blockIdx.x * 256L + threadIdx.x; k < nkeys; k += (long)gridDim.x * 256) {
+    const unsigned int a = islot[k], e = islot[k + 1];
+    tile_slot[k] = e > a ? (int)a : -1;
+    if (e > a + 1) merges[mslot[k] - merge0] = make_int2((int)a, (int)(e - a));
+    const long first = start[k], last = start[k + 1];
+    for (unsigned int i = a; i < e; i++) {
+      const long b = first + (long)(i - a) * chunk;
+      long4 it;
+      it.x = row0 + b;
+      it.y = min((long)chunk, last - b);
+      it.z = s0 + (long)(k / ntiles);
+      it.w = 0;
+      items[i - item0] = it;
+    }
+  }
+}
+
+// the slices' first items and merges
+__global__ void pick_kernel(const unsigned int* __restrict__ islot,
+                            const unsigned int* __restrict__ mslot, unsigned int ntiles, int nsl,
+                            uint2* __restrict__ out) {
+  for (int s = threadIdx.x; s <= nsl; s += blockDim.x)
+    out[s] = make_uint2(islot[(long)s * ntiles], mslot[(long)s * ntiles]);
+}
+
+// ---------------------------------------------------------------------------
+// 1. spreading
+// ---------------------------------------------------------------------------
+// One wave per item.  64 rows at a time: each lane loads one row, forms c
+// (scaled as the GEMM form scales it, by a power of two undone at the end) and
+// leaves it in LDS; then four rows per step, lane l evaluates the kernel of
+// row l / 16 at grid row and column l % 16, and the planes' products go to
+// v_mfma_f32_16x16x4_f32 (A: ky, B: kx c T_k; real and imaginary parts).
+// Per step and wave 2 NP MFMAs of 32 cycles against about 50 VALU
+// instructions: at NP = 4 the MFMA pipe bounds it, 64 cycles per visibility,
+// 54 us of the chip for 1.76 M visibilities at 2 GHz.
+template <int NP>
+__global__ __launch_bounds__(256) void spread_kernel(
+    const long4* __restrict__ items, int nitems, const float4* __restrict__ rec,
+    const uint2* __restrict__ meta, const float2* __restrict__ rot,
+    const SliceDev* __restrict__ tab, const unsigned int* __restrict__ cmaxs, double inv_w, int k0,
+    int nplanes, float* __restrict__ part) {
+  __shared__ float4 sa[4][64];  // (dx, dy, c)
+  __shared__ float2 sb[4][64];  // the row's cell within the subgrid
+  __shared__ float st[4][64][(NP + 3) / 4 * 4];  // T_k0 .. of each row
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int item = blockIdx.x * 4 + wave;
+  if (item >= nitems) return;
+  const long4 it = items[item];
+  const float2* __restrict__ vr = tab[it.z].vr;
+  const float scale = ldexpf(1.0f, p_scale_exponent(__uint_as_float(cmaxs[it.z])));
+  const float q = (float)(lane & 15);
+  // 64 rows accumulate in the MFMAs, the item's (at most eight) sums of 64 in a
+  // second FP32 sum: one long FP32 sum would round more than the whole
+  // transform does
+  f32x4_t tre[NP], tim[NP];
+#pragma unroll
+  for (int k = 0; k < NP; k++) tre[k] = tim[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // the next 64 rows are loaded (their residuals too: a dependent gather)
+  // while these are spread
+  const int rows = (int)it.y;
+  auto load_row = [&](int i, float4* r, uint2* m) {
+    const long p = it.x + min(i, rows - 1);
+    *r = rec[p];
+    *m = meta[p];
+  };
+  float4 r, rn;
+  uint2 m, mn;
+  load_row(lane, &r, &m);
+  float2 v = ldg(vr + m.x);
+  load_row(64 + lane, &rn, &mn);
+  for (int b = 0; b < rows; b += 64) {
+    const int cnt = min(64, rows - b);
+    f32x4_t re[NP], im[NP];
+#pragma unroll
+    for (int k = 0; k < NP; k++) re[k] = im[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    float2 c = make_float2(4.f, 4.f);
+    double t = 0.0;
+    if (lane < cnt) {
+      float cr = r.w * v.x, ci = -(r.w * v.y);
+      if (rot) {
+        const float2 e = rot[it.x + b + lane];
+        const float x = cr * e.x - ci * e.y;
+        ci = cr * e.y + ci * e.x;
+        cr = x;
+      }
+      if (m.y & 64u) ci = -ci;
+      a = make_float4(r.x, r.y, cr * scale, ci * scale);
+      c = make_float2((float)(4 + (m.y & 7u)), (float)(4 + ((m.y >> 3) & 7u)));
+      t = fmin(1.0, fmax(-1.0, (double)r.z * inv_w));  // rows without weight may lie beyond W
+    }
+    if (b + 64 < rows) {
+      r = rn;
+      m = mn;
+      v = ldg(vr + m.x);
+      load_row(b + 128 + lane, &rn, &mn);
+    }
+    __builtin_amdgcn_wave_barrier();
+    sa[wave][lane] = a;
+    sb[wave][lane] = c;
+    double ta = 1.0, tb = t;
+    for (int k = 0; k < k0; k++) {
+      const double tn = 2.0 * t * tb - ta;
+      ta = tb;
+      tb = tn;
+    }
+#pragma unroll
+    for (int k = 0; k < NP; k++) {
+      st[wave][lane][k] = (float)ta;
+      const double tn = 2.0 * t * tb - ta;
+      ta = tb;
+      tb = tn;
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int s = 0; s < cnt; s += 4) {
+      const int j = s + (lane >> 4);
+      const float4 va = sa[wave][j];
+      const float2 vb = sb[wave][j];
+      const float kx = spread_value((q - vb.x) - va.x);
+      const float ky = spread_value((q - vb.y) - va.y);
+      const float ux = kx * va.z, ui = kx * va.w;
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        // even planes grid c T_k, odd ones -i c T_k
+        const float tk = st[wave][j][k];
+        const float br = (k & 1) ? ui * tk : ux * tk;
+        const float bi = (k & 1) ? -(ux * tk) : ui * tk;
+        re[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky, br, re[k], 0, 0, 0);
+        im[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky, bi, im[k], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NP; k++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        tre[k][e] += re[k][e];
+        tim[k][e] += im[k][e];
+      }
+  }
+  // subgrid layout: [plane][column half][16 rows][8 columns] complex
+  const int col = lane & 15, row = 4 * (lane >> 4);
+#pragma unroll
+  for (int k = 0; k < NP; k++) {
+    if (k0 + k >= nplanes) break;
+    float2* o = (float2*)(part + ((long)item * nplanes + k0 + k) * kSub) + (col >> 3) * 128 +
+                (col & 7);
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[(row + e) * 8] = make_float2(tre[k][e], tim[k][e]);
+  }
+}
+
+// 2. The items of a tile with several, summed into its first one, in item
+// order, in FP64.
+__global__ __launch_bounds__(256) void merge_kernel(const int2* __restrict__ merges, int slot0,
+                                                    int nplanes, float* __restrict__ part) {
+  const int2 mg = merges[blockIdx.x];  // (first item, items)
+  const int cnt = mg.y;
+  const long stride = (long)nplanes * kSub;
+  float* p = part + (long)(mg.x - slot0) * stride + blockIdx.y * 256 + threadIdx.x;
+  double s = 0.0;
+  int i = 0;
+  for (; i + 16 <= cnt; i += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = p[(long)(i + u) * stride];
+#pragma unroll
+    for (int u = 0; u < 16; u++) s += (double)v[u];
+  }
+  for (; i < cnt; i++) s += (double)p[(long)i * stride];
+  *p = (float)s;
+}
+
+// ---------------------------------------------------------------------------
+// 3. columns
+// ---------------------------------------------------------------------------
+// Tile column X_t covers columns 8 X_t - 4 .. 8 X_t + 11, so grid column X
+// lies in the left half of tile column (X + 4) / 8 and in the right half of
+// the one before; likewise tile rows and Y, which wraps at 2N.  A cell is the
+// sum of up to four subgrids.
+
+// Four of the columns beyond an end of the half grid (X < 0 or X > N), folded:
+// minus the conjugate cell (mx, -Y).
+__device__ __forceinline__ float2 folded_cell(const float2* __restrict__ part,
+                                              const int* __restrict__ slot, int slot0, int N,
+                                              int nplanes, int plane, int mx, int Y) {
+  const int nty = N / 4, tx = (mx + 4) >> 3;
+  const int My = -Y & (2 * N - 1);
+  const int ty = ((My + 4) >> 3) & (nty - 1), c = (mx + 4) & 7, r = (My + 4) & 7;
+  float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int tc = tx - (u >> 1);
+    if (tc < 0 || tc > N / 8) continue;
+    const int i = slot[tc * nty + ((ty - (u & 1)) & (nty - 1))];
+    if (i < 0) continue;
+    const float2 v = part[((long)(i - slot0) * nplanes + plane) * (kSub / 2) + (u >> 1) * 128 +
+                          (r + (u & 1) * 8) * 8 + c];
+    s.x += v.x;
+    s.y -= v.y;
+  }
+  return s;
+}
+
+// H[slice][plane][image row][X], X in [0, N], rows of `pitch` values: BC
+// columns (a divisor of four, so they share their two tile columns) of one
+// plane per block.  The tiles' slots are staged in LDS and two columns are
+// loaded at a time, so that a thread keeps sixteen loads in flight: a gather
+// through slots in memory waited twice per cell and took 97 us at 1024^2.
+template <int N, int BC, int T>
+__global__ __launch_bounds__(T) void grid_cols_kernel(const float2* __restrict__ part,
+                                                      const int* __restrict__ tile_slot, int slot0,
+                                                      int nplanes, const float2* __restrict__ tw,
+                                                      int pitch, float2* __restrict__ Hbuf) {
+  constexpr int L = 2 * N, NTY = N / 4, CP = BC / 2;
+  __shared__ float2 lds[BC * L];
+  __shared__ int ss[2][NTY];
+  // consecutive column blocks, which write the same lines of H, on one XCD
+  const int per = gridDim.x / 8;
+  const int X0 = ((blockIdx.x % 8) * per + blockIdx.x / 8) * BC;
+  if (X0 > N) return;
+  const int plane = blockIdx.y, sl = blockIdx.z;
+  const int* slot = tile_slot + (long)sl * (N / 8 + 1) * NTY;
+  const int tx = (X0 + 4) >> 3;
+  // a block without any row's subgrid needs no transform
+  int any = X0 <= 4 || X0 + BC - 1 >= N - 4;
+  for (int y = threadIdx.x; y < 2 * NTY; y += T) {
+    const int h = y / NTY, t = tx - h;
+    const int s = t >= 0 && t <= N / 8 ? slot[t * NTY + y % NTY] : -1;
+    // (the smallest valid index where there is none: loaded, not used)
+    ss[h][y % NTY] = s < 0 ? -1 : s - slot0;
+    any |= s >= 0;
+  }
+  any = __syncthreads_or(any);
+  float2* H = Hbuf + ((long)sl * nplanes + plane) * (long)N * pitch;
+  if (any) {
+    const float4* p4 = (const float4*)part;
+    const long per_item = (long)nplanes * (kSub / 4), at_plane = (long)plane * (kSub / 4);
+    const int c0 = (X0 + 4) & 7;
+    constexpr int U = 4, IT = CP * L / T;
+    static_assert(IT * T == CP * L && IT % U == 0, "whole rounds");
+    for (int i0 = 0; i0 < IT; i0 += U) {
+      float4 v[U][4];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int idx = threadIdx.x + (i0 + u) * T;
+        const int t = idx % CP, Y = idx / CP;
+        const int ty = ((Y + 4) >> 3) & (NTY - 1), r = (Y + 4) & 7;
+        const int c = (c0 >> 1) + t;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int s = ss[q >> 1][(ty - (q & 1)) & (NTY - 1)];
+          v[u][q] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (s >= 0)
+            v[u][q] = p4[s * per_item + at_plane + (q >> 1) * 64 + (r + (q & 1) * 8) * 4 + c];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int idx = threadIdx.x + (i0 + u) * T;
+        float4 s;
+        s.x = (v[u][0].x + v[u][1].x) + (v[u][2].x + v[u][3].x);
+        s.y = (v[u][0].y + v[u][1].y) + (v[u][2].y + v[u][3].y);
+        s.z = (v[u][0].z + v[u][1].z) + (v[u][2].z + v[u][3].z);
+        s.w = (v[u][0].w + v[u][1].w) + (v[u][2].w + v[u][3].w);
+        ((float4*)lds)[idx] = s;
+      }
+    }
+    __syncthreads();
+    // cells beyond either end are the conjugates of cells inside
+    if (X0 <= 4 || X0 + BC - 1 >= N - 4) {
+      for (int idx = threadIdx.x; idx < BC * L; idx += T) {
+        const int X = X0 + idx % BC, Y = idx / BC;
+        const int mx = X >= 1 && X <= 4 ? -X : X >= N - 4 && X < N ? L - X : 0;
+        if (mx == 0) continue;
+        const float2 m = folded_cell(part, slot, slot0, N, nplanes, plane, mx, Y);
+        lds[idx].x += m.x;
+        lds[idx].y += m.y;
+      }
+      __syncthreads();
+    }
+    fft_lds<L, BC, true, T>(lds, tw);
+  }
+  // image row i is frequency row i - N / 2 (mod 2N)
+  for (int idx = threadIdx.x; idx < CP * N; idx += T) {
+    const int t = idx % CP, i = idx / CP, X = X0 + 2 * t;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (any) v = ((const float4*)lds)[((i - N / 2) & (L - 1)) * CP + t];
+    if (X <= N) *(float4*)(H + (long)i * pitch + X) = v;  // (column N + 1 is padding)
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 4. rows
+// ---------------------------------------------------------------------------
+struct RowsArgs {
+  const float2* H;
+  int pitch, nplanes, terms;
+  const float2* tw;   // e^{2 pi i k / N}
+  const float2* tw2;  // e^{2 pi i k / 2N}
+  const double* corr; // 1 / the kernel's transform per axis offset
+  const double* wcoef;
+  const SliceDev* tab;
+  int s0, nsl;        // slices [s0, s0 + nsl); H holds these
+  const unsigned int* cmaxs;
+  const float* noise;
+  float noise_cut, fg_scale, threshold;
+  const float* gcf;
+  int normalize, flag_opt;
+  double wz;          // 2 pi W
+  double dx, dy;      // radians per pixel
+  int x0, y0;         // phase centre
+  const float* I;
+  float* result;
+  float* each;        // per-slice d, or none (one slice: straight to result)
+};
+
+// One slice's contribution d at pixel k to the running gradient r: the chain
+// rule of DChi2_total_I_nu_0 / DChi2_total_alpha (src/functions.cu:4000-4024,
+// 3968-3998), in float.
+__device__ __forceinline__ float chain_rule(float r, float d, float nudiv, float i0, float alpha,
+                                            const RowsArgs& a) {
+  const float dI = powf(nudiv, alpha);
+  if ((a.flag_opt & 1) == 0) return r + d * dI;
+  if (i0 > a.threshold) return r + d * (i0 * dI * a.fg_scale * logf(nudiv));
+  return r;
+}
+
+// Weight of a plane at a pixel, over zeta^k: its power series in zeta^2.
+__device__ __forceinline__ double plane_series(const double* __restrict__ c, int terms,
+                                               double zeta2) {
+  double s = c[terms - 1];
+  for (int m = terms - 2; m >= 0; m--) s = fma(s, zeta2, c[m]);
+  return s;
+}
+
+// One block per image row; B planes are transformed together.  The transform
+// of 2N real values from N + 1 complex ones runs as one complex transform of N
+// points (even outputs in the real part, odd ones in the imaginary part).
+template <int N, int B, int T>
+__global__ __launch_bounds__(T) void grid_rows_kernel(RowsArgs a) {
+  __shared__ float2 lds[B * N];
+  constexpr int PP = (N / 2 + T - 1) / T;  // column pairs per thread
+  const int i = blockIdx.x;
+  const long n = (long)N * N;
+  const float* noise = a.noise + (long)i * N;
+  bool on[PP][2];
+  bool some = false;
+#pragma unroll
+  for (int u = 0; u < PP; u++) {
+    const int cp = threadIdx.x + u * T;
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      on[u][e] = cp < N / 2 && noise[2 * cp + e] < a.noise_cut;
+      some |= on[u][e];
+    }
+  }
+  if (!__syncthreads_or(some)) return;
+  double zeta[PP][2];
+#pragma unroll
+  for (int u = 0; u < PP; u++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      const int j = 2 * ((int)threadIdx.x + u * T) + e;
+      const double x = (j - a.x0) * a.dx, y = (i - a.y0) * a.dy;
+      const double r2 = x * x + y * y;
+      zeta[u][e] = a.wz * (-r2 / (1.0 + sqrt(fmax(0.0, 1.0 - r2))));
+    }
+  const int s = blockIdx.y;
+  double g[PP][2], zk[PP][2];
+#pragma unroll
+  for (int u = 0; u < PP; u++) {
+    g[u][0] = g[u][1] = 0.0;
+    zk[u][0] = zk[u][1] = 1.0;  // zeta^k
+  }
+  for (int k0 = 0; k0 < a.nplanes; k0 += B) {
+    __syncthreads();  // the previous group's outputs have been read
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      const int k = k0 + b;
+      const float2* h = a.H + (((long)s * a.nplanes + min(k, a.nplanes - 1)) * N + i) * a.pitch;
+#pragma unroll 4
+      for (int X = threadIdx.x; X < N; X += T) {
+        float2 f = h[X], m = h[N - X];
+        if (X == 0) {
+          f = make_float2(f.x, 0.f);
+          m = make_float2(m.x, 0.f);
+        } else {
+          f = make_float2(0.5f * f.x, 0.5f * f.y);
+          m = make_float2(0.5f * m.x, -0.5f * m.y);
+        }
+        const float2 d = cmul(make_float2(f.x - m.x, f.y - m.y), a.tw2[X]);
+        lds[b * N + X] = k < a.nplanes ? make_float2((f.x + m.x) - d.y, (f.y + m.y) + d.x)
+                                       : make_float2(0.f, 0.f);
+      }
+    }
+    __syncthreads();
+    fft_lds<N, B, false, T>(lds, a.tw);
+#pragma unroll
+    for (int u = 0; u < PP; u++) {
+      const int cp = threadIdx.x + u * T;
+      if (cp < N / 2 && (on[u][0] || on[u][1])) {
+        const int j = (cp - N / 4) & (N - 1);
+        for (int b = 0; b < B && k0 + b < a.nplanes; b++) {
+          const float2 z = lds[b * N + j];
+          const double* c = a.wcoef + (k0 + b) * a.terms;
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const double zt = zeta[u][e];
+            g[u][e] += (double)(e ? z.y : z.x) * zk[u][e] * plane_series(c, a.terms, zt * zt);
+            zk[u][e] *= zt;
+          }
+        }
+      }
+    }
+  }
+  const SliceDev& sd = a.tab[a.s0 + s];
+  const double inv_scale = ldexp(1.0, -p_scale_exponent(__uint_as_float(a.cmaxs[a.s0 + s])));
+  const double inv_nvis = a.normalize ? 1.0 / (double)sd.nvis : 1.0;
+  float* out = a.each ? a.each + (long)s * n : a.result + (a.flag_opt & 1) * n;
+#pragma unroll
+  for (int u = 0; u < PP; u++)
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+      if (!on[u][e]) continue;
+      const int j = 2 * ((int)threadIdx.x + u * T) + e;
+      const long k = (long)i * N + j;
+      const double gv = g[u][e] * (a.corr[i] * a.corr[j]);
+      float sc = a.fg_scale * sd.pb[k];
+      if (a.gcf) sc = sc * a.gcf[k];
+      const float d = (float)(-(gv * inv_scale) * (double)sc * inv_nvis);
+      out[k] = a.each ? d : chain_rule(out[k], d, sd.nudiv, a.I[k], a.I[n + k], a);
+    }
+}
+
+// Several slices: their d's into the result, one slice after the other as
+// the reference's per-channel launches do (src/functions.cu:4456-4558).
+__global__ __launch_bounds__(256) void chain_kernel(RowsArgs a, int N) {
+  const long n = (long)N * N;
+  for (long k = blockIdx.x * 256L + threadIdx.x; k < n; k += (long)gridDim.x * 256) {
+    if (!(a.noise[k] < a.noise_cut)) continue;
+    const float i0 = a.I[k], alpha = a.I[n + k];
+    float* out = a.result + (a.flag_opt & 1) * n + k;
+    float r = *out;
+    for (int s = 0; s < a.nsl; s++)
+      r = chain_rule(r, a.each[(long)s * n + k], a.tab[a.s0 + s].nudiv, i0, alpha, a);
+    *out = r;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+
+// 1 / integral of the kernel times cos(2 pi x d / 2N), for pixel offsets from
+// the image centre: Gauss-Legendre over the (even) kernel's half width, with
+// the constants as the device evaluates them.
+std::vector<double> kernel_correction(int N) {
+  constexpr int Q = 64;
+  double x[Q], w[Q];
+  for (int q = 0; q < Q; q++) {
+    double t = std::cos(kPi * (q + 0.75) / (Q + 0.5)), d = 1.0;
+    for (int it = 0; it < 100; it++) {
+      double p0 = 1.0, p1 = t;
+      for (int k = 2; k <= Q; k++) {
+        const double p2 = ((2 * k - 1) * t * p1 - (k - 1) * p0) / k;
+        p0 = p1;
+        p1 = p2;
+      }
+      d = Q * (t * p1 - p0) / (t * t - 1.0);
+      const double s = p1 / d;
+      t -= s;
+      if (std::fabs(s) < 1e-15) break;
+    }
+    x[q] = t;
+    w[q] = 2.0 / ((1.0 - t * t) * d * d);
+  }
+  const double half = 0.5 * kTaps;
+  double pos[Q], val[Q];
+  for (int q = 0; q < Q; q++) {
+    pos[q] = 0.5 * half * (x[q] + 1.0);
+    const double u = pos[q] * (double)kInvHalf, v = u * u;
+    const double p =
+        v * (kP1 + v * (kP2 + v * (kP3 + v * (kP4 + v * (kP5 + v * (double)kP6)))));
+    val[q] = half * w[q] * std::exp2(-p);
+  }
+  std::vector<double> c(N);
+  for (int o = 0; o <= N / 2; o++) {
+    double s = 0.0;
+    for (int q = 0; q < Q; q++) s += val[q] * std::cos(kPi * o * pos[q] / N);
+    if (o < N / 2) c[N / 2 + o] = 1.0 / s;
+    c[N / 2 - o] = 1.0 / s;
+  }
+  return c;
+}
+
+template <typename T>
+bool device_array(T** p, size_t count) {
+  *p = nullptr;
+  if (hipMalloc((void**)p, sizeof(T) * std::max<size_t>(count, 1)) == hipSuccess) return true;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return false;
+}
+
+int row_pitch(int N) { return N + 8; }
+
+}  // namespace
+
+void free_grid_plan(GridPlan& g) {
+  (void)hipFree(g.rec);
+  (void)hipFree(g.meta);
+  (void)hipFree(g.rot);
+  (void)hipFree(g.items);
+  (void)hipFree(g.merges);
+  (void)hipFree(g.tile_slot);
+  (void)hipFree(g.tw2);
+  (void)hipFree(g.corr);
+  (void)hipFree(g.wcoef);
+  (void)hipFree(g.ws);
+  g = GridPlan{};
+}
+
+namespace {
+
+// Scratch of the plan's set-up, freed when it ends.
+struct PlanScratch {
+  unsigned int *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr, *start = nullptr,
+               *cnt = nullptr, *islot = nullptr, *several = nullptr, *mslot = nullptr,
+               *off = nullptr, *small = nullptr;
+  uint2* pick = nullptr;
+  void* tmp = nullptr;
+  size_t tmp_bytes = 0;
+  ~PlanScratch() {
+    for (void* p : {(void*)k0, (void*)k1, (void*)v0, (void*)v1, (void*)start, (void*)cnt,
+                    (void*)islot, (void*)several, (void*)mslot, (void*)off, (void*)small,
+                    (void*)pick, tmp})
+      (void)hipFree(p);
+  }
+  bool temp(size_t bytes) {
+    if (bytes <= tmp_bytes) return true;
+    (void)hipFree(tmp);
+    tmp_bytes = 0;
+    if (!device_array((char**)&tmp, bytes)) return false;
+    tmp_bytes = bytes;
+    return true;
+  }
+};
+
+}  // namespace
+
+// Sorts every slice's visibilities by tile and lays out the work items and
+// the workspace.  *ok = false (and GVM_OK) when this form does not apply: too
+// many w planes, or not enough memory; the GEMM form then takes the call.
+gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
+  *ok = false;
+  GridPlan& g = ctx->gplan;
+  if (g.built) {
+    *ok = g.usable;
+    return GVM_OK;
+  }
+  GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  free_grid_plan(g);
+  g.built = true;
+  const int N = ctx->g.N, nsl = (int)ctx->slices.size();
+  const unsigned int ntiles = (unsigned int)(N / 8 + 1) * (N / 4);
+  hipStream_t st = ctx->stream;
+  auto give_up = [&]() {
+    free_grid_plan(g);
+    g.built = true;
+    return GVM_OK;
+  };
+
+  PlanScratch sc;
+  if (!device_array(&sc.small, 1)) return give_up();
+  // W and the planes it needs
+  const unsigned int zero = 0u;
+  GVM_HIP_TRY(hipMemcpyAsync(sc.small, &zero, sizeof zero, hipMemcpyHostToDevice, st));
+  long vmax = 0, total = 0;
+  for (const Slice& s : ctx->slices) {
+    vmax = std::max(vmax, s.nvis);
+    total += s.nvis;
+  }
+  hipLaunchKernelGGL(wmax_kernel, dim3((unsigned)std::min<long>(256, (vmax + 255) / 256), nsl),
+                     dim3(256), 0, st, ctx->slice_tab, sc.small);
+  GVM_CHECK_LAUNCH();
+  unsigned int wbits = 0;
+  GVM_HIP_TRY(hipMemcpyAsync(&wbits, sc.small, sizeof wbits, hipMemcpyDeviceToHost, st));
+  GVM_HIP_TRY(hipStreamSynchronize(st));
+  if (wbits >= 0x7f800000u) return give_up();  // an infinite or NaN w
+  float W;
+  static_assert(sizeof W == sizeof wbits, "float bits");
+  __builtin_memcpy(&W, &wbits, sizeof W);
+  const double zmax = 2.0 * kPi * (double)W * ctx->mask_fmax;
+  int K = 1;
+  for (double e = zmax; e > kPlaneTol; e *= 0.5 * zmax / K) {  // 2 (zmax / 2)^K / K!
+    K++;
+    if (K > kMaxPlanes) return give_up();
+  }
+  g.planes = K;
+  g.wz = 2.0 * kPi * (double)W;
+  // terms of the J_k series until they fall below 1e-11 of the first
+  g.terms = 2;
+  for (double t = 0.25 * zmax * zmax; t > 1e-11; g.terms++)
+    t *= 0.25 * zmax * zmax / ((double)g.terms * g.terms);
+  g.inv_w = W > 0.0f ? 1.0 / (double)W : 0.0;
+
+  // items of at most `chunk` rows: long enough to amortise a subgrid's
+  // stores, short enough that a small observation fills the chip
+  g.chunk = (int)std::min(512L, std::max(64L, (total / 4096 + 63) / 64 * 64));
+  const int shift_x = N / 2 - (int)ctx->g.x0_phs, shift_y = N / 2 - (int)ctx->g.y0_phs;
+  const bool shifted = shift_x != 0 || shift_y != 0;
+  if (!device_array(&g.rec, (size_t)total) || !device_array(&g.meta, (size_t)total) ||
+      !device_array(&g.tile_slot, (size_t)nsl * ntiles) ||
+      (shifted && !device_array(&g.rot, (size_t)total)))
+    return give_up();
+
+  std::vector<std::pair<long4*, int2*>> parts;  // a group's items and merges
+  std::vector<std::pair<long, long>> counts;
+  struct PartsFree {
+    decltype(parts)& v;
+    ~PartsFree() {
+      for (auto& p : v) {
+        (void)hipFree(p.first);
+        (void)hipFree(p.second);
+      }
+    }
+  } parts_free{parts};
+  g.slice_slot.assign(nsl + 1, 0);
+  g.slice_merge.assign(nsl + 1, 0);
+  long row0 = 0, nitems = 0, nmerges = 0;
+  for (int s0 = 0; s0 < nsl;) {
+    int s1 = s0;
+    long n = 0;
+    while (s1 < nsl && (s1 == s0 || n + ctx->slices[s1].nvis <= kGroupRows) &&
+           (unsigned long)(s1 - s0 + 1) * ntiles < 0x7fffffffUL)
+      n += ctx->slices[s1++].nvis;
+    const int ns = s1 - s0;
+    const long nkeys = (long)ns * ntiles;
+    PlanScratch gs;
+    std::vector<unsigned int> off(ns);
+    unsigned int first = 0;
+    for (int s = 0; s < ns; s++) {
+      off[s] = first;
+      first += (unsigned int)ctx->slices[s0 + s].nvis;
+    }
+    if (!device_array(&gs.k0, n) || !device_array(&gs.k1, n) || !device_array(&gs.v0, n) ||
+        !device_array(&gs.v1, n) || !device_array(&gs.start, nkeys + 1) ||
+        !device_array(&gs.cnt, nkeys + 1) || !device_array(&gs.islot, nkeys + 1) ||
+        !device_array(&gs.several, nkeys + 1) || !device_array(&gs.mslot, nkeys + 1) ||
+        !device_array(&gs.off, ns) || !device_array(&gs.pick, ns + 1))
+      return give_up();
+    GVM_HIP_TRY(hipMemcpyAsync(gs.off, off.data(), sizeof(unsigned int) * ns,
+                               hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(plan_keys_kernel, dim3((unsigned)std::min<long>(1024, (vmax + 255) / 256), ns),
+                       dim3(256), 0, st, ctx->slice_tab, s0, gs.off, N, gs.k0, gs.v0);
+    GVM_CHECK_LAUNCH();
+    int bits = 1;
+    while (bits < 32 && (nkeys >> bits) != 0) bits++;
+    rocprim::double_buffer<unsigned int> kb(gs.k0, gs.k1), vb(gs.v0, gs.v1);
+    size_t bytes = 0;
+    GVM_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits, st));
+    if (!gs.temp(bytes)) return give_up();
+    GVM_HIP_TRY(rocprim::radix_sort_pairs(gs.tmp, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits, st));
+    hipLaunchKernelGGL(plan_records_kernel, dim3(blocks_for(n)), dim3(256), 0, st, ctx->slice_tab,
+                       s0, gs.off, N, n, kb.current(), vb.current(), shift_x, shift_y,
+                       g.rec + row0, g.meta + row0, shifted ? g.rot + row0 : nullptr);
+    GVM_CHECK_LAUNCH();
+    hipLaunchKernelGGL(tile_starts_kernel, dim3(blocks_for(nkeys + 1)), dim3(256), 0, st,
+                       kb.current(), n, nkeys, gs.start);
+    GVM_CHECK_LAUNCH();
+    hipLaunchKernelGGL(item_counts_kernel, dim3(blocks_for(nkeys + 1)), dim3(256), 0, st, gs.start,
+                       nkeys, g.chunk, gs.cnt, gs.several);
+    GVM_CHECK_LAUNCH();
+    GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, gs.cnt, gs.islot, (unsigned int)nitems,
+                                        (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
+    if (!gs.temp(bytes)) return give_up();
+    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, bytes, gs.cnt, gs.islot, (unsigned int)nitems,
+                                        (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
+    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, bytes, gs.several, gs.mslot, (unsigned int)nmerges,
+                                        (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
+    hipLaunchKernelGGL(pick_kernel, dim3(1), dim3(256), 0, st, gs.islot, gs.mslot, ntiles, ns,
+                       gs.pick);
+    GVM_CHECK_LAUNCH();
+    std::vector<uint2> pick(ns + 1);
+    GVM_HIP_TRY(hipMemcpyAsync(pick.data(), gs.pick, sizeof(uint2) * (ns + 1),
+                               hipMemcpyDeviceToHost, st));
+    GVM_HIP_TRY(hipStreamSynchronize(st));
+    for (int s = 0; s <= ns; s++) {
+      g.slice_slot[s0 + s] = (long)pick[s].x;
+      g.slice_merge[s0 + s] = (long)pick[s].y;
+    }
+    const long ni = (long)pick[ns].x - nitems, nm = (long)pick[ns].y - nmerges;
+    std::pair<long4*, int2*> part{nullptr, nullptr};
+    const bool got = device_array(&part.first, (size_t)ni) && device_array(&part.second, (size_t)nm);
+    parts.push_back(part);
+    counts.push_back({ni, nm});
+    if (!got) return give_up();
+    hipLaunchKernelGGL(items_kernel, dim3(blocks_for(nkeys)), dim3(256), 0, st, gs.start, gs.islot,
+                       gs.mslot, nkeys, g.chunk, row0, ntiles, s0, (unsigned int)nitems,
+                       (unsigned int)nmerges, part.first, part.second,
+                       g.tile_slot + (long)s0 * ntiles);
+    GVM_CHECK_LAUNCH();
+    GVM_HIP_TRY(hipStreamSynchronize(st));  // the group's scratch is freed
+    nitems += ni;
+    nmerges += nm;
+    if (nitems > 0x7fffffffL) return give_up();
+    row0 += n;
+    s0 = s1;
+  }
+  if (parts.size() == 1) {
+    g.items = parts[0].first;
+    g.merges = parts[0].second;
+    parts.clear();
+  } else {
+    if (!device_array(&g.items, (size_t)nitems) || !device_array(&g.merges, (size_t)nmerges))
+      return give_up();
+    long o = 0, om = 0;
+    for (size_t k = 0; k < parts.size(); k++) {
+      GVM_HIP_TRY(hipMemcpyAsync(g.items + o, parts[k].first, sizeof(long4) * counts[k].first,
+                                 hipMemcpyDeviceToDevice, st));
+      GVM_HIP_TRY(hipMemcpyAsync(g.merges + om, parts[k].second, sizeof(int2) * counts[k].second,
+                                 hipMemcpyDeviceToDevice, st));
+      o += counts[k].first;
+      om += counts[k].second;
+    }
+    GVM_HIP_TRY(hipStreamSynchronize(st));
+  }
+
+  // batches of slices that share the workspace
+  const size_t per_item = sizeof(float) * kSub * (size_t)K;
+  const size_t per_slice = sizeof(float2) * (size_t)K * N * row_pitch(N);
+  size_t free_b = 0, total_b = 0;
+  GVM_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+  const size_t budget = std::min<size_t>(32UL << 30, (free_b + sizeof(float) * ctx->adj_part_elems) / 2);
+  g.batch0.clear();
+  size_t need_part = 0, need_slices = 0;
+  for (int s = 0; s < nsl;) {
+    g.batch0.push_back(s);
+    size_t b = 0;
+    int e = s;
+    while (e < nsl) {
+      const size_t add = per_item * (size_t)(g.slice_slot[e + 1] - g.slice_slot[e]) + per_slice;
+      if (e > s && b + add > kBatchBytes) break;
+      b += add;
+      e++;
+    }
+    // subgrids; after them, with several slices, their N x N images
+    need_part = std::max({need_part, per_item * (size_t)(g.slice_slot[e] - g.slice_slot[s]),
+                          sizeof(float) * (size_t)N * N * (size_t)(e - s > 1 ? e - s : 0)});
+    need_slices = std::max(need_slices, (size_t)(e - s));
+    s = e;
+  }
+  g.batch0.push_back(nsl);
+  g.part_bytes = (need_part + 255) / 256 * 256;
+  const size_t bytes = g.part_bytes + per_slice * need_slices;
+  if (bytes > budget) return give_up();
+  if (!device_array((char**)&g.ws, bytes)) return give_up();
+
+  std::vector<float2> tw2(2 * (size_t)N);
+  for (int k = 0; k < 2 * N; k++) {
+    const double t = (double)k / (2 * N);
+    tw2[k] = make_float2((float)std::cos(2.0 * kPi * t), (float)std::sin(2.0 * kPi * t));
+  }
+  const std::vector<double> corr = kernel_correction(N);
+  // J_0, then 2 (+-) J_k (the planes hold c T_k for even k, -i c T_k for odd):
+  // J_k(zeta) = zeta^k / (2^k k!) sum_m (-1)^m (zeta / 2)^2m k! / (m! (m + k)!)
+  std::vector<double> wc((size_t)K * g.terms);
+  double lead = 1.0;
+  for (int k = 0; k < K; k++) {
+    if (k > 0) lead *= 0.5 / k;
+    const int odd = (k & 1) ? ((k + 1) >> 1) & 1 : (k >> 1) & 1;
+    double c = k == 0 ? 1.0 : odd ? -2.0 * lead : 2.0 * lead;
+    for (int m = 0; m < g.terms; m++) {
+      wc[(size_t)k * g.terms + m] = c;
+      c *= -0.25 / ((m + 1.0) * (m + 1.0 + k));
+    }
+  }
+  if (!device_array(&g.tw2, tw2.size()) || !device_array(&g.corr, corr.size()) ||
+      !device_array(&g.wcoef, wc.size()))
+    return give_up();
+  GVM_HIP_TRY(hipMemcpy(g.wcoef, wc.data(), sizeof(double) * wc.size(), hipMemcpyHostToDevice));
+  GVM_HIP_TRY(hipMemcpy(g.tw2, tw2.data(), sizeof(float2) * tw2.size(), hipMemcpyHostToDevice));
+  GVM_HIP_TRY(hipMemcpy(g.corr, corr.data(), sizeof(double) * corr.size(), hipMemcpyHostToDevice));
+  g.usable = true;
+  *ok = true;
+  return GVM_OK;
+}
+
+namespace {
+
+template <int NP>
+void launch_spread(gvm_ctx* ctx, long slot0, int nitems, int k0, float* part) {
+  const GridPlan& g = ctx->gplan;
+  hipLaunchKernelGGL((spread_kernel<NP>), dim3((nitems + 3) / 4), dim3(256), 0, ctx->stream,
+                     g.items + slot0, nitems, g.rec, g.meta, g.rot, ctx->slice_tab, ctx->cmax,
+                     g.inv_w, k0, g.planes, part);
+}
+
+template <int N>
+void launch_cols(gvm_ctx* ctx, int s0, int ns, const float* part, float2* H) {
+  // four columns per block (64 KB of LDS at 2N = 2048, two blocks per CU), two
+  // where four would need 256 KB
+  constexpr int BC = N <= 2048 ? 4 : 2;
+  constexpr int T = N <= 128 ? 64 : N >= 1024 ? 512 : N / 2;
+  const GridPlan& g = ctx->gplan;
+  const int nb = (N + BC) / BC;  // columns 0 .. N
+  hipLaunchKernelGGL((grid_cols_kernel<N, BC, T>), dim3((nb + 7) / 8 * 8, g.planes, ns), dim3(T), 0,
+                     ctx->stream, (const float2*)part,
+                     g.tile_slot + (long)s0 * (N / 8 + 1) * (N / 4), (int)g.slice_slot[s0],
+                     g.planes, g.tw2, row_pitch(N), H);
+}
+
+template <int N, int B>
+void launch_rows(gvm_ctx* ctx, const RowsArgs& a) {
+  constexpr int T = N / 4 < 64 ? 64 : N / 4 > 512 ? 512 : N / 4;
+  hipLaunchKernelGGL((grid_rows_kernel<N, B, T>), dim3(N, a.nsl), dim3(T), 0, ctx->stream, a);
+}
+
+template <int N>
+gvm_status run_batch(gvm_ctx* ctx, int s0, int s1, const float* I, float* result, int flag_opt,
+                     int normalize) {
+  const GridPlan& g = ctx->gplan;
+  const int K = g.planes;
+  const long slot0 = g.slice_slot[s0];
+  const int nitems = (int)(g.slice_slot[s1] - slot0);
+  float* part = (float*)g.ws;
+  float2* H = (float2*)(g.ws + g.part_bytes);
+  for (int k0 = 0; k0 < K; k0 += kPlaneGroup) {
+    const int np = std::min(kPlaneGroup, K - k0);
+    switch (np) {
+      case 1: launch_spread<1>(ctx, slot0, nitems, k0, part); break;
+      case 2: launch_spread<2>(ctx, slot0, nitems, k0, part); break;
+      case 3: launch_spread<3>(ctx, slot0, nitems, k0, part); break;
+      case 4: launch_spread<4>(ctx, slot0, nitems, k0, part); break;
+      case 5: launch_spread<5>(ctx, slot0, nitems, k0, part); break;
+      case 6: launch_spread<6>(ctx, slot0, nitems, k0, part); break;
+      case 7: launch_spread<7>(ctx, slot0, nitems, k0, part); break;
+      default: launch_spread<8>(ctx, slot0, nitems, k0, part); break;
+    }
+    GVM_CHECK_LAUNCH();
+  }
+  const int nmerges = (int)(g.slice_merge[s1] - g.slice_merge[s0]);
+  if (nmerges > 0) {
+    hipLaunchKernelGGL(merge_kernel, dim3(nmerges, K * kSub / 256), dim3(256), 0, ctx->stream,
+                       g.merges + g.slice_merge[s0], (int)slot0, K, part);
+    GVM_CHECK_LAUNCH();
+  }
+  launch_cols<N>(ctx, s0, s1 - s0, part, H);
+  GVM_CHECK_LAUNCH();
+  RowsArgs a{};
+  a.H = H;
+  a.pitch = row_pitch(N);
+  a.nplanes = K;
+  a.terms = g.terms;
+  a.tw = ctx->twiddle;
+  a.tw2 = g.tw2;
+  a.corr = g.corr;
+  a.wcoef = g.wcoef;
+  a.tab = ctx->slice_tab;
+  a.s0 = s0;
+  a.nsl = s1 - s0;
+  a.cmaxs = ctx->cmax;
+  a.noise = ctx->noise;
+  a.noise_cut = ctx->g.noise_cut;
+  a.fg_scale = ctx->g.fg_scale;
+  a.threshold = ctx->g.threshold;
+  a.gcf = ctx->gcf;
+  a.normalize = normalize;
+  a.flag_opt = flag_opt;
+  a.wz = g.wz;
+  a.dx = ctx->g.deltax * kPi / 180.0;
+  a.dy = ctx->g.deltay * kPi / 180.0;
+  a.x0 = (int)ctx->g.x0_phs;
+  a.y0 = (int)ctx->g.y0_phs;
+  a.I = I;
+  a.result = result;
+  // the subgrids have been read when the rows run: their memory takes the
+  // slices' d's
+  a.each = a.nsl > 1 ? part : nullptr;
+  // planes per transform: as few groups of at most four as K needs
+  const int groups = (K + 3) / 4, B = (K + groups - 1) / groups;
+  if (B <= 2)
+    launch_rows<N, 2>(ctx, a);
+  else if (B == 3)
+    launch_rows<N, 3>(ctx, a);
+  else
+    launch_rows<N, 4>(ctx, a);
+  GVM_CHECK_LAUNCH();
+  if (a.each) {
+    hipLaunchKernelGGL(chain_kernel, dim3(blocks_for((long)N * N)), dim3(256), 0, ctx->stream, a, N);
+    GVM_CHECK_LAUNCH();
+  }
+  return GVM_OK;
+}
+
+}  // namespace
+
+gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize) {
+  const GridPlan& g = ctx->gplan;
+  for (size_t b = 0; b + 1 < g.batch0.size(); b++) {
+    const int s0 = g.batch0[b], s1 = g.batch0[b + 1];
+    gvm_status st = GVM_ERR_ARG;
+    switch (ctx->g.N) {
+      case 64: st = run_batch<64>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 128: st = run_batch<128>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 256: st = run_batch<256>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 512: st = run_batch<512>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 1024: st = run_batch<1024>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 2048: st = run_batch<2048>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 4096: st = run_batch<4096>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+    }
+    if (st) return st;
+  }
+  return GVM_OK;
+}
+
+}  // namespace gvm

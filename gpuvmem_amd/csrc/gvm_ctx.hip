@@ -196,6 +196,7 @@ gvm_status register_slice(gvm_ctx* ctx, Slice& s) {
   }
   ctx->slices.push_back(s);
   ctx->split_mode = -1;
+  free_grid_plan(ctx->gplan);
   ctx->have_residuals = false;
   ctx->epoch++;
   return GVM_OK;
@@ -306,6 +307,7 @@ extern "C" gvm_status gvm_destroy(gvm_ctx* ctx) {
   (void)hipFree(ctx->dscalars);
   (void)hipFree(ctx->cmax);
   (void)hipFree(ctx->adj_part);
+  free_grid_plan(ctx->gplan);
   (void)hipFree(ctx->slice_tab);
   (void)hipFree(ctx->split_tab);
   (void)hipFree(ctx->slice_p0);
@@ -369,6 +371,28 @@ static gvm_status create_impl(const gvm_geometry* g, const float* noise_host, gv
     }
     ctx->adj_px_gemm = gemm_px;
     ctx->adj_px_direct = direct_px;
+  }
+  // the farthest pixel on the mask from the phase centre (a row's farthest is
+  // its first or last on the mask)
+  {
+    const long wpr = N / 32;
+    double r2max = 0.0;
+    for (int r = 0; r < N; r++) {
+      long first = -1, last = -1;
+      for (long w = 0; w < wpr; w++) {
+        const unsigned int b = bits[(size_t)(r * wpr + w)];
+        if (!b) continue;
+        if (first < 0) first = 32 * w + __builtin_ctz(b);
+        last = 32 * w + 31 - __builtin_clz(b);
+      }
+      if (first < 0) continue;
+      const double y = (r - (int)g->y0_phs) * g->deltay * kRad;
+      for (long c : {first, last}) {
+        const double x = (c - (int)g->x0_phs) * g->deltax * kRad;
+        r2max = std::max(r2max, x * x + y * y);
+      }
+    }
+    ctx->mask_fmax = r2max / (1.0 + std::sqrt(std::max(0.0, 1.0 - r2max)));
   }
   if ((st = dev_alloc(&ctx->grid, n))) return st;
   ctx->grid_slices = 1;

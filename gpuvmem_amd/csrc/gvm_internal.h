@@ -68,6 +68,33 @@ struct SliceDev {
   float pad;
 };
 
+// The gridded adjoint's plan (gvm_adjoint_fft.hip): every slice's visibilities
+// sorted by grid tile, the work items, and the workspace.  Built by the first
+// gvm_dchi2 after the slices changed.
+struct GridPlan {
+  bool built = false;   // decided for the current slices
+  bool usable = false;  // this form applies to them
+  int planes = 0;       // w planes
+  int terms = 0;        // terms of the plane weights' series
+  int chunk = 0;        // rows per work item at most
+  double wz = 0.0;      // 2 pi max |w|
+  double inv_w = 0.0;   // 1 / max |w| (0 without w)
+  float4* rec = nullptr;     // sorted rows: (dx, dy, w, weight)
+  uint2* meta = nullptr;     // (row of its slice, cell within the tile and fold)
+  float2* rot = nullptr;     // phase-centre rotation, or none
+  long4* items = nullptr;    // (first row, rows, slice, 0)
+  int2* merges = nullptr;    // tiles with several items: (first, count)
+  int* tile_slot = nullptr;  // [slice][tile]: first item, or -1
+  float2* tw2 = nullptr;     // e^{2 pi i k / 2N}
+  double* corr = nullptr;    // kernel correction per axis
+  double* wcoef = nullptr;   // [plane][term] of the plane weights
+  char* ws = nullptr;        // subgrids, then the transformed columns
+  size_t part_bytes = 0;     // of the subgrids
+  std::vector<long> slice_slot;  // slice s owns items [slice_slot[s], slice_slot[s + 1])
+  std::vector<long> slice_merge;  // and merges [slice_merge[s], slice_merge[s + 1])
+  std::vector<int> batch0;       // slices that share the workspace: [batch0[b], batch0[b + 1])
+};
+
 constexpr int kReduceBlocks = 1024;
 constexpr int kReduceThreads = 256;
 constexpr int kMaxSlots = 4096;  // slices per context (and reduction slots)
@@ -110,7 +137,10 @@ struct gvm_ctx {
   int* slice_p0 = nullptr;      // kMaxSlots + 1 entries
   int split_cap = 0;
   int nsplit_total = 0;
-  int split_mode = -1;          // adjoint mode the table was built for (-1: stale)
+  int split_mode = -1;          // adjoint mode the work split was decided for (-1: stale)
+  bool adj_gridded = false;     // that split: the gridded form, else the GEMM's ranges
+  double mask_fmax = 0.0;       // max |sqrt(1 - r^2) - 1| over the pixels on the mask
+  gvm::GridPlan gplan;
   int adjoint_mode = GVM_ADJOINT_BF16X3;
   long split_vis = 6144;        // target visibilities per adjoint range (K tile), default_split_vis
   int fft_mode = 0;             // FFT batching: 0 automatic, 1 wide, 2 narrow
@@ -153,6 +183,11 @@ gvm_status forward_chi2(gvm_ctx* ctx, float* I, int flag_opt, int normalize,
                         double* out);
 gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt,
                    int normalize);
+// The gridded form of the adjoint: its plan (*ok = false when it does not
+// apply) and its launches; free_grid_plan frees and clears a plan.
+gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok);
+gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize);
+void free_grid_plan(GridPlan& g);
 // Rebuilds the adjoint's range table and workspace for the current form.
 gvm_status rebuild_splits(gvm_ctx* ctx);
 // Block-partial reduction helpers: reduce `nblocks` partials of slot s into
@@ -218,6 +253,20 @@ __device__ __forceinline__ void stg(float2* p, float2 v) {
   w.x = v.x;
   w.y = v.y;
   *(__attribute__((address_space(1))) gf2_t*)p = w;
+}
+
+constexpr int kPScale = 15;  // max |P| = 2^15 < 65504 (FP16 max)
+constexpr int kPScaleLimit = 100;
+
+// Exponent of the power-of-two scale of P for a slice whose largest |c| is
+// cm: 2^e cm <= 2^kPScale.  Clamped to [-kPScaleLimit, kPScaleLimit] so that
+// the scale and its inverse stay finite and normal in FP32 for any cm (an
+// unclamped exponent overflows for cm below about 2^-113, and 0 * inf would
+// turn the zero amplitudes of off-grid samples into NaN); 0 when cm is 0.
+__device__ __forceinline__ int p_scale_exponent(float cm) {
+  if (!(cm > 0.0f)) return 0;
+  const int e = kPScale - (int)ceilf(log2f(cm));
+  return min(max(e, -kPScaleLimit), kPScaleLimit);
 }
 
 // |r|^2 of a residual with each operation rounded (no multiply-add

@@ -46,7 +46,11 @@ typedef int gvm_status;
 #define GVM_BEAM_AIRYDISK 0
 #define GVM_BEAM_GAUSSIAN 1
 
-/* Adjoint (DChi2) evaluation forms. */
+/* Adjoint (DChi2) evaluation forms.  The first three evaluate the sums by
+ * gridding and FFT in FP32 (FP32 MFMA spreading, FP64 combination) where that
+ * applies, with the same result for each; where it does not (few rows on a
+ * large image, w terms of more than about two turns, no memory for its
+ * workspace) they are a GEMM with the operands named here. */
 #define GVM_ADJOINT_F32 0      /* separable complex GEMM, FP32 MFMA            */
 #define GVM_ADJOINT_F16X3 1    /* FP16 hi/lo split, 3 MFMA products, FP32 acc  */
 #define GVM_ADJOINT_BF16X3 2   /* BF16 hi/lo split, 3 MFMA products, FP32 acc  */
@@ -468,14 +472,15 @@ gvm_status gvm_device_info(char* name, int name_len, int* cu_count,
                            int* clock_khz);
 
 /* ---- timing of the adjoint (for measurement) ---------------------------- */
-/* Average duration in ms of the adjoint GEMM kernel over the gvm_dchi2 calls
- * since the last reset, measured with HIP events on the context's stream. */
+/* Average duration in ms of the adjoint's kernels (the GEMM without its
+ * epilogue, or the gridded form's launches) over the gvm_dchi2 calls since the
+ * last reset, measured with HIP events on the context's stream. */
 gvm_status gvm_timing_reset(gvm_ctx* ctx);
 gvm_status gvm_timing_adjoint_ms(gvm_ctx* ctx, double* avg_ms, long* count);
 
 /* ---- adjoint K tile: the visibility-range length ------------------------ */
-/* No counterpart in the reference.  Each workgroup of the split-precision
- * adjoint accumulates one 256 x 256 output tile over a range of about
+/* No counterpart in the reference.  It has no effect while the adjoint runs by
+ * gridding and FFT.  Each workgroup of the split-precision adjoint accumulates one 256 x 256 output tile over a range of about
  * `split_vis` visibilities in FP32 (the ranges are summed in FP64): shorter
  * ranges keep the FP32 accumulation short, longer ones write fewer partial
  * tiles.  Default 6144, and 3072 for images of 2048^2 and larger (where
@@ -490,7 +495,7 @@ gvm_status gvm_set_fft_mode(gvm_ctx* ctx, int mode);
 gvm_status gvm_get_split_vis(const gvm_ctx* ctx, long* split_vis);
 /* No counterpart in the reference (whose DChi2 computes the pixels on the
  * mask, noise < noise_cut): the pixels whose sums the adjoint of the current
- * form computes.  The split-precision GEMM computes the 128 x 64 sub-tiles of
+ * form computes when it runs as a GEMM or as the direct sum.  The split-precision GEMM computes the 128 x 64 sub-tiles of
  * its workgroup tiles that hold a pixel on the mask and skips the others; the
  * direct form, its blocks of 256 consecutive pixels that hold one.  The work
  * of one adjoint launch is 4 x pixels x visibilities flop. */
