@@ -314,6 +314,7 @@ extern "C" gvm_status gvm_destroy(gvm_ctx* ctx) {
   if (ctx->hscalars) (void)hipHostFree(ctx->hscalars);
   if (ctx->dvalues) (void)hipHostFree(ctx->dvalues);
   (void)hipFree(ctx->nn_part);
+  (void)hipFree(ctx->setup_ws);
   for (hipEvent_t& e : ctx->tev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

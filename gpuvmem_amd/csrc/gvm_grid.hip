@@ -7,17 +7,24 @@
 // Both the gridder and the weighting schemes accumulate per-cell sums in
 // float.  The reference adds rows to a cell one at a time in row order (with
 // one OpenMP thread), so a parallel float sum would not reproduce its
-// rounding.  Here every (row, tap) pair becomes a (cell, entry) key pair;
-// a stable radix sort groups the pairs by cell while keeping the row order
-// inside each cell, and one thread per cell then adds that cell's entries in
-// sequence.  The result is the reference's single-thread sum, bit for bit,
-// and does not depend on scheduling.
+// rounding.  Here rows are sorted by where they fall (a stable radix sort keeps
+// their order) and each cell's owner adds its rows in sequence.  The result is
+// the reference's single-thread sum, bit for bit, and does not depend on
+// scheduling.
+//
+// Gridder: rows are sorted by 8 x 8 tile of cells, once for every tile that
+// their taps reach (at most four tiles for kernels up to 9 x 9), and a wave
+// owns a tile, one cell per lane.  Sorting every (row, tap) pair instead, 173 M
+// pairs for 1.76 M rows and 7 x 7 taps, took 12 ms and 5 GB of scratch memory
+// allocated and freed on each call, 107 - 137 ms in all.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
+#include <rocprim/iterator/transform_iterator.hpp>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <string>
 #include <vector>
 
 #include "gvm_internal.h"
@@ -34,33 +41,46 @@ int blocks_for(long n) {
   return (int)std::max(1L, std::min<long>((n + kThreads - 1) / kThreads, 65536));
 }
 
-// Device allocation released when it goes out of scope (set-up paths only).
-struct DevMem {
-  void* p = nullptr;
-  DevMem() = default;
-  DevMem(const DevMem&) = delete;
-  DevMem& operator=(const DevMem&) = delete;
-  ~DevMem() {
-    if (p) (void)hipFree(p);
+// Scratch of one call, cut from the context's set-up workspace: sizes are
+// added up first, then reserve() and take() in the same order.
+constexpr size_t kKeepScratch = 1UL << 30;  // a larger workspace is given back
+
+struct Scratch {
+  gvm_ctx* ctx;
+  size_t need = 0, at = 0;
+  explicit Scratch(gvm_ctx* c) : ctx(c) {}
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  ~Scratch() {
+    if (ctx->setup_bytes > kKeepScratch) {
+      (void)hipFree(ctx->setup_ws);
+      ctx->setup_ws = nullptr;
+      ctx->setup_bytes = 0;
+    }
+  }
+  static size_t round(size_t bytes) { return (bytes + 255) / 256 * 256; }
+  void add(size_t bytes) { need += round(bytes); }
+  gvm_status reserve(const char* what) {
+    if (need <= ctx->setup_bytes) return GVM_OK;
+    (void)hipFree(ctx->setup_ws);
+    ctx->setup_ws = nullptr;
+    ctx->setup_bytes = 0;
+    if (hipMalloc((void**)&ctx->setup_ws, need) != hipSuccess) {
+      (void)hipGetLastError();
+      ctx->setup_ws = nullptr;
+      set_error(std::string(what) + ": out of device memory");
+      return GVM_ERR_OOM;
+    }
+    ctx->setup_bytes = need;
+    return GVM_OK;
   }
   template <class T>
-  T* as() const {
-    return static_cast<T*>(p);
+  T* take(size_t count) {
+    T* p = (T*)(ctx->setup_ws + at);
+    at += round(sizeof(T) * count);
+    return p;
   }
 };
-
-gvm_status dev_alloc(DevMem& m, size_t bytes, const char* what) {
-  if (m.p) {
-    (void)hipFree(m.p);
-    m.p = nullptr;
-  }
-  if (hipMalloc(&m.p, std::max<size_t>(bytes, 16)) != hipSuccess) {
-    m.p = nullptr;
-    set_error(std::string(what) + ": out of device memory");
-    return GVM_ERR_OOM;
-  }
-  return GVM_OK;
-}
 
 // Number of bits a radix sort needs for keys in [0, sentinel].
 int key_bits(uint32_t sentinel) {
@@ -69,51 +89,42 @@ int key_bits(uint32_t sentinel) {
   return b;
 }
 
-// Sorted (cell key, entry) pairs of one pass, with the buffers reused across
-// slices.  After sort(), keys()/ids() are the sorted arrays.
-struct CellSort {
-  DevMem k0, k1, v0, v1, tmp;
+// Stable sort of up to `cap` (key, id) pairs.
+struct PairSort {
+  uint32_t *k[2] = {}, *v[2] = {};
+  char* tmp = nullptr;
   size_t cap = 0, tmp_bytes = 0;
   rocprim::double_buffer<uint32_t> kb, vb;
 
-  gvm_status reserve(long n, const char* what) {
-    if ((size_t)n <= cap) return GVM_OK;
-    gvm_status st;
-    if ((st = dev_alloc(k0, sizeof(uint32_t) * n, what)) ||
-        (st = dev_alloc(k1, sizeof(uint32_t) * n, what)) ||
-        (st = dev_alloc(v0, sizeof(uint32_t) * n, what)) ||
-        (st = dev_alloc(v1, sizeof(uint32_t) * n, what)))
-      return st;
-    cap = (size_t)n;
-    rocprim::double_buffer<uint32_t> k(k0.as<uint32_t>(), k1.as<uint32_t>());
-    rocprim::double_buffer<uint32_t> v(v0.as<uint32_t>(), v1.as<uint32_t>());
+  // room for a sort of n pairs (call it for every n that will be sorted)
+  gvm_status size(size_t n, int bits, const char* what) {
+    rocprim::double_buffer<uint32_t> a((uint32_t*)nullptr, (uint32_t*)nullptr), b = a;
     size_t bytes = 0;
-    if (rocprim::radix_sort_pairs(nullptr, bytes, k, v, (size_t)n, 0u, 32u) != hipSuccess) {
+    if (rocprim::radix_sort_pairs(nullptr, bytes, a, b, n, 0u, (unsigned)bits) != hipSuccess) {
       set_error(std::string(what) + ": radix sort sizing failed");
       return GVM_ERR_HIP;
     }
-    tmp_bytes = bytes;
-    return dev_alloc(tmp, bytes, what);
+    cap = std::max(cap, n);
+    tmp_bytes = std::max(tmp_bytes, bytes);
+    return GVM_OK;
   }
-  uint32_t* in_keys() const { return k0.as<uint32_t>(); }
-  uint32_t* in_ids() const { return v0.as<uint32_t>(); }
-  gvm_status sort(long n, int bits, const char* what) {
-    kb = rocprim::double_buffer<uint32_t>(k0.as<uint32_t>(), k1.as<uint32_t>());
-    vb = rocprim::double_buffer<uint32_t>(v0.as<uint32_t>(), v1.as<uint32_t>());
-    size_t bytes = 0;
-    if (rocprim::radix_sort_pairs(nullptr, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits) !=
-        hipSuccess) {
-      set_error(std::string(what) + ": radix sort sizing failed");
-      return GVM_ERR_HIP;
+  void add(Scratch& sc) const {
+    for (int i = 0; i < 4; i++) sc.add(sizeof(uint32_t) * cap);
+    sc.add(tmp_bytes);
+  }
+  void take(Scratch& sc) {
+    for (int i = 0; i < 2; i++) {
+      k[i] = sc.take<uint32_t>(cap);
+      v[i] = sc.take<uint32_t>(cap);
     }
-    if (bytes > tmp_bytes) {
-      gvm_status st = dev_alloc(tmp, bytes, what);
-      if (st) return st;
-      tmp_bytes = bytes;
-    }
-    bytes = tmp_bytes;
-    if (rocprim::radix_sort_pairs(tmp.p, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits) !=
-        hipSuccess) {
+    tmp = sc.take<char>(tmp_bytes);
+  }
+  // sorts k[0] / v[0]; keys() / ids() are the sorted arrays
+  gvm_status sort(size_t n, int bits, const char* what) {
+    kb = rocprim::double_buffer<uint32_t>(k[0], k[1]);
+    vb = rocprim::double_buffer<uint32_t>(v[0], v[1]);
+    size_t bytes = tmp_bytes;
+    if (rocprim::radix_sort_pairs(tmp, bytes, kb, vb, n, 0u, (unsigned)bits) != hipSuccess) {
       set_error(std::string(what) + ": radix sort failed");
       return GVM_ERR_HIP;
     }
@@ -125,161 +136,235 @@ struct CellSort {
 
 // ---- convolutional gridding -----------------------------------------------
 
+constexpr int kGTile = 8;           // edge of a tile of cells
+constexpr int kLdsTaps = 1024;      // taps staged in LDS; larger kernels read memory
+
 struct GridGeom {
   double deltau, deltav;  // 1 / (M dx), 1 / (N dy), radians (dx < 0: deltau < 0)
   double cj, ck;          // floor(N / 2), floor(M / 2)
   double lambda;          // float wavelength of the slice, promoted
   int M, N;
-  int km, kn;             // kernel rows / columns
+  int kn;                 // kernel columns
   int supx, supy;         // supports
-  int nx, taps;           // 2 supx + 1, (2 supy + 1) nx
-  uint32_t off;           // key of entries that land off the grid (sorts last)
+  int wx, wy;             // columns and rows of taps a row of data reaches
+  int tx, ty;             // tiles they can span
+  int ntx, nty;           // tiles of the grid
 };
 
-// One (row, tap) entry per thread: its cell key, or g.off.  Entry e is row
-// z = e / taps (z >= nvis: the Hermitian twin of row z - nvis) and tap
-// t = e % taps; keys are written in entry order, so a stable sort keeps the
-// rows of a cell in row order (do_gridding, src/functions.cu:1424-1480).
+// A record of every row and its Hermitian twin (row z >= nvis is the twin of
+// z - nvis): w, w Vo.x, w Vo.y and the first cell reached (16 bits each); and one
+// (tile, row) entry per tile that the row's taps can span, in row order: the
+// tile's index, or ntx nty for none.
+// (do_gridding, src/functions.cu:1424-1480)
 __global__ __launch_bounds__(kThreads) void grid_keys_kernel(const double* __restrict__ uvw,
+                                                             const float* __restrict__ weight,
+                                                             const float2* __restrict__ vo,
                                                              long nvis, GridGeom g,
+                                                             float4* __restrict__ rec,
                                                              uint32_t* __restrict__ keys,
                                                              uint32_t* __restrict__ ids) {
 #pragma clang fp contract(off)
-  const long n = 2 * nvis * g.taps;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n;
-       e += (long)gridDim.x * blockDim.x) {
-    const long z = e / g.taps;
-    const int t = (int)(e % g.taps);
-    const long vi = z < nvis ? z : z - nvis;
-    double u = uvw[3 * vi], v = uvw[3 * vi + 1];
-    if (z >= nvis) {
-      u = -u;
-      v = -v;
-    }
-    u = u / g.lambda;  // metres_to_lambda (src/MSFITSIO.cu:41-45)
-    v = v / g.lambda;
-    const double jf = u / g.deltau + g.cj + 0.5;
-    const double kf = v / g.deltav + g.ck + 0.5;
-    uint32_t key = g.off;
-    if (fabs(jf) < 1073741824.0 && fabs(kf) < 1073741824.0) {
-      const int j = (int)jf, k = (int)kf;  // C truncation, as int(j_fp)
-      const int ki = t / g.nx, kj = t % g.nx;
-      const int sj = j + kj - g.supx, sk = k + ki - g.supy;
-      if (sk >= 0 && sk < g.M && sj >= 0 && sj < g.N && ki < g.km && kj < g.kn)
-        key = (uint32_t)((long)g.N * sk + sj);
-    }
-    keys[e] = key;
-    ids[e] = (uint32_t)e;
-  }
-}
-
-// Run starts: flag[i] = 1 where a run of equal keys begins (the run of
-// off-grid entries included, so every run ends where the next begins).
-__global__ __launch_bounds__(kThreads) void run_heads_kernel(const uint32_t* __restrict__ keys,
-                                                             long n, int* __restrict__ flag) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x)
-    flag[i] = (i == 0 || keys[i - 1] != keys[i]) ? 1 : 0;
-}
-
-// starts[rank[i]] = i at run starts, and starts[number of runs] = n.
-__global__ __launch_bounds__(kThreads) void run_starts_kernel(const int* __restrict__ flag,
-                                                              const int* __restrict__ rank,
-                                                              long n, int* __restrict__ starts) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    if (flag[i]) starts[rank[i]] = (int)i;
-    if (i == n - 1) starts[rank[i] + flag[i]] = (int)n;
-  }
-}
-
-// One wave per cell (run r of the sorted entries): the float sums of
-// do_gridding in entry order, then the normalisation
-// (src/functions.cu:1424-1559).  The 64 lanes load a chunk of the run's
-// entries and form the products w k, w k^2, w Vo.x k, w Vo.y k in parallel;
-// lane 0 then adds them in entry order, so the rounding is the reference's
-// single-thread sum.  Writes, at index r, whether the cell is kept
-// (weight > 0) and its values.
-__global__ __launch_bounds__(64) void grid_cells_kernel(
-    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ ids,
-    const int* __restrict__ starts, long nvis, GridGeom g, const float* __restrict__ taps,
-    const float* __restrict__ weight, const float2* __restrict__ vo, int* __restrict__ keep,
-    float2* __restrict__ cell_vo, float* __restrict__ cell_w) {
-#pragma clang fp contract(off)
-  __shared__ float prod[4][64];
-  const int r = blockIdx.x;
-  const int s = starts[r], e = starts[r + 1];
-  const int lane = threadIdx.x;
-  if (keys[s] == g.off) {
-    if (lane == 0) keep[r] = 0;
-    return;
-  }
-  float ws = 0.f, aux = 0.f, re = 0.f, im = 0.f;
-  for (int c = s; c < e; c += 64) {
-    const int p = c + lane;
-    if (p < e) {
-      const uint32_t id = ids[p];
-      const long z = id / g.taps;
-      const int t = (int)(id % g.taps);
-      const long vi = z < nvis ? z : z - nvis;
+  const int T = g.tx * g.ty;
+  for (long vi = blockIdx.x * (long)blockDim.x + threadIdx.x; vi < nvis;
+       vi += (long)gridDim.x * blockDim.x) {
+    for (int twin = 0; twin < 2; twin++) {
+      double u = uvw[3 * vi], v = uvw[3 * vi + 1];
+      if (twin) {
+        u = -u;
+        v = -v;
+      }
+      u = u / g.lambda;  // metres_to_lambda (src/MSFITSIO.cu:41-45)
+      v = v / g.lambda;
+      const double jf = u / g.deltau + g.cj + 0.5;
+      const double kf = v / g.deltav + g.ck + 0.5;
+      const long z = vi + (twin ? nvis : 0);
+      int j = 0, k = 0;
+      const bool ok = fabs(jf) < 1073741824.0 && fabs(kf) < 1073741824.0;
+      if (ok) {
+        j = (int)jf - g.supx;  // C truncation, as int(j_fp); the first cell reached
+        k = (int)kf - g.supy;
+      }
+      // (a row that reaches a tile starts within 255 cells of the grid)
       const float w = weight[vi];
-      float2 v = vo[vi];
-      if (z >= nvis) v.y = -v.y;
-      const float kv = taps[g.kn * (t / g.nx) + (t % g.nx)];
-      const float kv2 = kv * kv;
-      prod[0][lane] = w * kv;
-      prod[1][lane] = w * kv2;
-      prod[2][lane] = w * v.x * kv;
-      prod[3][lane] = w * v.y * kv;
-    }
-    __syncthreads();
-    if (lane == 0) {
-      const int cnt = min(64, e - c);
-      for (int j = 0; j < cnt; j++) {
-        ws = ws + prod[0][j];
-        aux = aux + prod[1][j];
-        re = re + prod[2][j];
-        im = im + prod[3][j];
+      const float2 d = vo[vi];
+      const int jc = min(max(j, -32768), 32767), kc = min(max(k, -32768), 32767);
+      rec[z] = make_float4(w, w * d.x, w * (twin ? -d.y : d.y),
+                           __int_as_float((jc & 0xffff) | kc << 16));
+      const int ca = j >> 3, cb = (j + g.wx - 1) >> 3, ra = k >> 3, rb = (k + g.wy - 1) >> 3;
+      for (int t = 0; t < T; t++) {
+        const int c = ca + t % g.tx, r = ra + t / g.tx;
+        const bool in = ok && c <= cb && r <= rb && c >= 0 && r >= 0 && c < g.ntx && r < g.nty;
+        keys[z * T + t] = (uint32_t)(in ? r * g.ntx + c : g.ntx * g.nty);
+        ids[z * T + t] = (uint32_t)z;
       }
     }
-    __syncthreads();
-  }
-  if (lane == 0) {
-    float weff = 0.f;
-    float2 out = make_float2(0.f, 0.f);
-    if (aux != 0.0f && ws != 0.0f) {
-      weff = ws * ws / aux;
-      out = make_float2(re / ws, im / ws);
-    }
-    keep[r] = weff > 0.0f ? 1 : 0;
-    cell_vo[r] = out;
-    cell_w[r] = weff;
   }
 }
 
-// Kept cells to rows at the cell centre, in row-major cell order
-// (src/functions.cu:1527-1539, 1587-1607): uvw in metres, w = 0.  One
-// thread per run.
-__global__ __launch_bounds__(kThreads) void grid_emit_kernel(
-    const uint32_t* __restrict__ keys, const int* __restrict__ starts,
-    const int* __restrict__ keep, const int* __restrict__ pos, long nruns, GridGeom g,
-    const float2* __restrict__ cell_vo, const float* __restrict__ cell_w, long capacity,
-    double* __restrict__ uvw_out, float2* __restrict__ vo_out, float* __restrict__ w_out) {
+// start[k] = the first sorted entry with key >= k, k in [0, nkeys]
+__global__ __launch_bounds__(kThreads) void tile_first_kernel(const uint32_t* __restrict__ keys,
+                                                              long n, int nkeys,
+                                                              uint32_t* __restrict__ start) {
+  for (int k = blockIdx.x * kThreads + threadIdx.x; k <= nkeys; k += gridDim.x * kThreads) {
+    long lo = 0, hi = n;
+    while (lo < hi) {
+      const long m = (lo + hi) >> 1;
+      if (keys[m] < (uint32_t)k)
+        lo = m + 1;
+      else
+        hi = m;
+    }
+    start[k] = (uint32_t)lo;
+  }
+}
+
+// One block per tile, one wave per quadrant (4 x 4 cells), 16 lanes for each of
+// the four float sums of do_gridding: a lane adds one sum of one cell over the
+// rows in order; then the normalisation (src/functions.cu:1424-1559).  256 rows
+// at a time are staged in LDS; each wave keeps, in order, those that reach its
+// quadrant (half of a tile's for 7 x 7 taps) and every lane goes through them.
+// 1.6 ms for 1.76 M rows and 7 x 7 taps on 1024^2, set by the fullest tiles' chains
+// (29,000 rows).  Before: one wave per tile, a lane per cell with its four sums,
+// 3.9 ms; a branch per row instead of the selection, 2.8 ms; each wave gathering
+// the rows' values itself, 2.2 ms.
+typedef short short2_t __attribute__((ext_vector_type(2)));
+typedef short short8_t __attribute__((ext_vector_type(8)));
+
+template <bool LDS_TAPS>
+__global__ __launch_bounds__(kThreads) void grid_tiles_kernel(
+    const uint32_t* __restrict__ ids, const uint32_t* __restrict__ start, GridGeom g,
+    const float* __restrict__ taps, const float4* __restrict__ rec, float2* __restrict__ cell_vo,
+    float* __restrict__ cell_w) {
 #pragma clang fp contract(off)
-  for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < nruns;
+  __shared__ float lt[2][LDS_TAPS ? kLdsTaps : 1];  // k and k^2
+  __shared__ float4 stage[kThreads];                // the block's next rows
+  __shared__ __align__(16) float val[4][4][68];     // w, w, w Vo.x, w Vo.y of each row
+  __shared__ __align__(16) short2_t rel[4][68];     // the first cell it reaches
+  if constexpr (LDS_TAPS) {
+    for (int t = threadIdx.x; t < g.wx * g.wy; t += kThreads) {
+      const float k = taps[g.kn * (t / g.wx) + t % g.wx];
+      lt[0][t] = k;
+      lt[1][t] = k * k;
+    }
+  }
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, sum = lane >> 4;
+  const int tile = blockIdx.x;
+  // the quadrant's first cell, and this lane's
+  const int c0 = tile % g.ntx * kGTile + (wave & 1) * 4, r0 = tile / g.ntx * kGTile + (wave >> 1) * 4;
+  const short2_t cell = {(short)(lane & 3), (short)((lane >> 2) & 3)};
+  const short2_t size = {(short)g.wx, (short)g.wy}, origin = {(short)c0, (short)r0};
+  const float* tap = lt[sum == 1 ? 1 : 0];
+  const long s = start[tile], e = start[tile + 1];
+  float acc = 0.f;
+  // a record is a gather behind its id: ids are loaded two rounds ahead,
+  // records one, so that a round waits for neither
+  float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+  uint32_t z = 0;
+  auto fetch = [&](long p) {
+    if (p < e) r = rec[z];
+    z = p + kThreads < e ? ids[p + kThreads] : 0;
+  };
+  if (s + threadIdx.x < e) z = ids[s + threadIdx.x];
+  fetch(s + threadIdx.x);
+  for (long c = s; c < e; c += kThreads) {
+    __syncthreads();  // the round before has been read (and the taps are there)
+    stage[threadIdx.x] = r;
+    __syncthreads();
+    fetch(c + kThreads + threadIdx.x);
+    const int rows = (int)min((long)kThreads, e - c);
+    for (int o = 0; o < rows; o += 64) {
+      const float4 q0 = stage[o + lane];
+      const short2_t first = __builtin_bit_cast(short2_t, q0.w) - origin;
+      const bool in = o + lane < rows && first.x < 4 && first.y < 4 && first.x + g.wx > 0 &&
+                      first.y + g.wy > 0;
+      const unsigned long long m = __ballot(in);
+      const int cnt = __popcll(m), at = __popcll(m & ((1ull << lane) - 1));
+      __builtin_amdgcn_wave_barrier();
+      if (in) {
+        val[wave][0][at] = val[wave][1][at] = q0.x;
+        val[wave][2][at] = q0.y;
+        val[wave][3][at] = q0.z;
+        rel[wave][at] = first;
+      }
+      // rounds of four rows: the last is filled with rows that reach nothing
+      if (lane < 4) rel[wave][cnt + lane] = short2_t{16384, 16384};
+      __builtin_amdgcn_wave_barrier();
+      for (int j = 0; j < cnt; j += 4) {
+        const short8_t r4 = *(const short8_t*)&rel[wave][j];
+        const float4 q4 = *(const float4*)&val[wave][sum][j];
+        const float q[4] = {q4.x, q4.y, q4.z, q4.w};
+        // every load first, then the sums in row order by selection: a branch per
+        // row waited for two dependent LDS reads each time (2.8 ms)
+        bool hit[4];
+        float k[4];
+  #pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const short2_t d = cell - short2_t{r4[2 * u], r4[2 * u + 1]};
+          const short2_t past = d - size;
+          // 0 <= d < size in both: d not negative, d - size negative
+          const unsigned int out = __builtin_bit_cast(unsigned int, d) |
+                                   ~__builtin_bit_cast(unsigned int, past);
+          hit[u] = (out & 0x80008000u) == 0u;
+          const unsigned int pitch = LDS_TAPS ? (unsigned int)g.wx : (unsigned int)g.kn;
+          unsigned int at = __umul24((unsigned int)(unsigned short)d.y, pitch) +
+                            (unsigned int)(unsigned short)d.x;
+          at = hit[u] ? at : 0u;
+          if constexpr (LDS_TAPS) {
+            k[u] = tap[at];
+          } else {
+            k[u] = taps[at];
+            if (sum == 1) k[u] = k[u] * k[u];
+          }
+        }
+  #pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const float t = acc + q[u] * k[u];
+          acc = hit[u] ? t : acc;
+        }
+      }
+    }
+  }
+  // lane l < 16 takes its cell's four sums
+  const float ws = acc, aux = __shfl(acc, (lane & 15) + 16, 64), re = __shfl(acc, (lane & 15) + 32, 64),
+              im = __shfl(acc, (lane & 15) + 48, 64);
+  if (lane >= 16) return;
+  const int cx = c0 + cell.x, cy = r0 + cell.y;
+  float weff = 0.f;
+  float2 out = make_float2(0.f, 0.f);
+  if (aux != 0.0f && ws != 0.0f) {
+    weff = ws * ws / aux;
+    out = make_float2(re / ws, im / ws);
+  }
+  cell_vo[(long)g.N * cy + cx] = out;
+  cell_w[(long)g.N * cy + cx] = weff;
+}
+
+struct IsKept {
+  __device__ __host__ int operator()(float w) const { return w > 0.0f ? 1 : 0; }
+};
+
+// Kept cells (weight > 0) to rows at the cell centre, in row-major cell order
+// (src/functions.cu:1527-1539, 1587-1607): uvw in metres, w = 0.
+__global__ __launch_bounds__(kThreads) void grid_emit_kernel(
+    const int* __restrict__ pos, GridGeom g, const float2* __restrict__ cell_vo,
+    const float* __restrict__ cell_w, long capacity, double* __restrict__ uvw_out,
+    float2* __restrict__ vo_out, float* __restrict__ w_out) {
+#pragma clang fp contract(off)
+  const long n = (long)g.M * g.N;
+  for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < n;
        r += (long)gridDim.x * blockDim.x) {
-    if (!keep[r]) continue;
+    const float w = cell_w[r];
+    if (!(w > 0.0f)) continue;
     const long o = pos[r];
     if (o >= capacity) continue;
-    const uint32_t key = keys[starts[r]];
-    const int gj = (int)(key % (uint32_t)g.N), gk = (int)(key / (uint32_t)g.N);
+    const int gj = (int)(r % g.N), gk = (int)(r / g.N);
     const double ul = ((double)gj - g.cj) * g.deltau;
     const double vl = ((double)gk - g.ck) * g.deltav;
     uvw_out[3 * o] = ul * g.lambda;
     uvw_out[3 * o + 1] = vl * g.lambda;
     uvw_out[3 * o + 2] = 0.0;
     vo_out[o] = cell_vo[r];
-    w_out[o] = cell_w[r];
+    w_out[o] = w;
   }
 }
 
@@ -335,19 +420,74 @@ __global__ __launch_bounds__(kThreads) void weight_keys_kernel(const double* __r
   }
 }
 
-// Per cell: grid[cell] = (cumulative ? grid[cell] : 0) + the cell's weights
-// added in row order.
-__global__ __launch_bounds__(kThreads) void weight_cells_kernel(
-    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ ids, long n, uint32_t off,
-    const float* __restrict__ weight, int cumulative, float* __restrict__ grid) {
-#pragma clang fp contract(off)
+// sorted[p] = weight[ids[p]]
+__global__ __launch_bounds__(kThreads) void weight_gather_kernel(const uint32_t* __restrict__ ids,
+                                                                 const float* __restrict__ weight,
+                                                                 long n,
+                                                                 float* __restrict__ sorted) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n;
-       i += (long)gridDim.x * blockDim.x) {
-    const uint32_t key = keys[i];
-    if (key == off || (i > 0 && keys[i - 1] == key)) continue;
-    float s = cumulative ? grid[key] : 0.0f;
-    for (long p = i; p < n && keys[p] == key; p++) s = s + weight[ids[p]];
-    grid[key] = s;
+       i += (long)gridDim.x * blockDim.x)
+    sorted[i] = weight[ids[i]];
+}
+
+// Per cell: grid[cell] = (cumulative ? grid[cell] : 0) + the cell's weights
+// added in row order.  The weights are gathered into sorted order first; a
+// thread adds a short run of rows itself, a long one is added by its wave, 64
+// rows a load: one dependent gather per added row took 463 us for 1.76 M rows,
+// one thread's batches of eight 218 us, set by the fullest cell.
+__global__ __launch_bounds__(kThreads) void weight_cells_kernel(
+    const uint32_t* __restrict__ keys, const float* __restrict__ sorted, long n, uint32_t off,
+    int cumulative, float* __restrict__ grid) {
+#pragma clang fp contract(off)
+  constexpr int kShort = 16;
+  const int lane = threadIdx.x & 63;
+  const long step = (long)gridDim.x * blockDim.x;
+  for (long i0 = blockIdx.x * (long)blockDim.x + threadIdx.x - lane; i0 < n; i0 += step) {
+    const long i = i0 + lane;
+    const uint32_t key = i < n ? keys[i] : off;
+    const bool head = key != off && (i == 0 || keys[i - 1] != key);
+    float s = 0.0f;
+    bool more = false;
+    if (head) {
+      s = cumulative ? grid[key] : 0.0f;
+      uint32_t k[kShort];
+      float w[kShort];
+#pragma unroll
+      for (int u = 0; u < kShort; u++) {
+        const long q = min(i + u, n - 1);
+        k[u] = i + u < n ? keys[q] : off;
+        w[u] = sorted[q];
+      }
+      more = true;
+#pragma unroll
+      for (int u = 0; u < kShort; u++) {
+        more = more && k[u] == key;
+        if (more) s = s + w[u];
+      }
+      if (!more) grid[key] = s;
+    }
+    for (unsigned long long m = __ballot(more); m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t lk = (uint32_t)__builtin_amdgcn_readlane((int)key, l);
+      float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), l));
+      long p = i0 + l + kShort;
+      auto at = [&](long q, float* w) {
+        const bool ok = q < n && keys[min(q, n - 1)] == lk;
+        *w = sorted[min(q, n - 1)];
+        return __popcll(__ballot(ok));  // a run is contiguous
+      };
+      float w, wn;
+      int cnt = at(p + lane, &w);
+      while (cnt > 0) {
+        const int next = at(p + 64 + lane, &wn);
+        for (int j = 0; j < cnt; j++)
+          t = t + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+        p += 64;
+        cnt = cnt < 64 ? 0 : next;
+        w = wn;
+      }
+      if (lane == 0) grid[lk] = t;
+    }
   }
 }
 
@@ -442,19 +582,6 @@ gvm_status launch_ok(const char* what) {
   return GVM_OK;
 }
 
-// FP64 sum of the block partials, in block order.
-gvm_status read_partials(const double* part, int nb, double* out, const char* what) {
-  std::vector<double> h(nb);
-  if (hipMemcpy(h.data(), part, sizeof(double) * nb, hipMemcpyDeviceToHost) != hipSuccess) {
-    set_error(std::string(what) + ": partial sums copy failed");
-    return GVM_ERR_HIP;
-  }
-  double s = 0.0;
-  for (int b = 0; b < nb; b++) s += h[b];
-  *out = s;
-  return GVM_OK;
-}
-
 }  // namespace
 }  // namespace gvm
 
@@ -486,80 +613,82 @@ extern "C" gvm_status gvm_grid_visibilities_dev(gvm_ctx* ctx, const gvm_ckernel*
   g.cj = std::floor(geo.N / 2.0);
   g.ck = std::floor(geo.M / 2.0);
   g.lambda = (double)(2.99792458E8f / freq);
-  g.km = kernel->m;
   g.kn = kernel->n;
   g.supx = kernel->support_x;
   g.supy = kernel->support_y;
-  g.nx = 2 * g.supx + 1;
-  g.taps = g.nx * (2 * g.supy + 1);
-  g.off = (uint32_t)((long)geo.M * geo.N);
+  const int nx = 2 * g.supx + 1, ny = 2 * g.supy + 1;
+  g.wx = std::min(nx, kernel->n);
+  g.wy = std::min(ny, kernel->m);
+  g.tx = (g.wx + kGTile - 2) / kGTile + 1;
+  g.ty = (g.wy + kGTile - 2) / kGTile + 1;
+  g.ntx = geo.N / kGTile;
+  g.nty = geo.M / kGTile;
   *nout = 0;
-  GVM_REQUIRE(nvis >= 0 && nvis <= (((1L << 31) - 1) / (2L * g.taps)),
+  GVM_REQUIRE(nvis >= 0 && nvis <= (((1L << 31) - 1) / (2L * nx * ny)),
               "gvm_grid_visibilities_dev: rows x taps exceed 2^31 entries");
   if (nvis == 0) return GVM_OK;
-  const long n = 2 * nvis * g.taps;
+  const long n = 2 * nvis * g.tx * g.ty, cells = (long)geo.M * geo.N;
+  const int ntiles = g.ntx * g.nty, bits = key_bits((uint32_t)ntiles);
   GVM_HIP_TRY(hipSetDevice(ctx->device));
 
   gvm_status st;
-  DevMem taps_d, flag, rank, starts, keep, pos, cvo, cw;
-  CellSort cs;
-  if ((st = dev_alloc(taps_d, sizeof(float) * g.km * g.kn, what)) ||
-      (st = cs.reserve(n, what)) || (st = dev_alloc(flag, sizeof(int) * n, what)) ||
-      (st = dev_alloc(rank, sizeof(int) * n, what)) ||
-      (st = dev_alloc(starts, sizeof(int) * (n + 1), what)))
-    return st;
-  GVM_HIP_TRY(hipMemcpy(taps_d.p, kernel->taps, sizeof(float) * g.km * g.kn,
-                        hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(grid_keys_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, nullptr, uvw_m_dev,
-                     nvis, g, cs.in_keys(), cs.in_ids());
-  if ((st = launch_ok(what)) || (st = cs.sort(n, key_bits(g.off), what))) return st;
-  // the runs of equal keys (cells, then the off-grid run): start of each
-  hipLaunchKernelGGL(run_heads_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, nullptr, cs.keys(),
-                     n, flag.as<int>());
+  Scratch sc(ctx);
+  PairSort ps;
+  if ((st = ps.size((size_t)n, bits, what))) return st;
+  ps.add(sc);
+  size_t scan_bytes = 0;
+  const auto kept = [](const float* w) { return rocprim::make_transform_iterator(w, IsKept()); };
+  GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, scan_bytes, kept(nullptr), (int*)nullptr, 0,
+                                      (size_t)cells, rocprim::plus<int>()));
+  const size_t ntaps = (size_t)kernel->m * kernel->n;
+  sc.add(sizeof(float) * ntaps);
+  sc.add(sizeof(float4) * 2 * nvis);
+  sc.add(sizeof(uint32_t) * (ntiles + 1));
+  sc.add(scan_bytes);
+  sc.add(sizeof(int) * cells);
+  sc.add(sizeof(float2) * cells);
+  sc.add(sizeof(float) * cells);
+  if ((st = sc.reserve(what))) return st;
+  ps.take(sc);
+  float* taps_d = sc.take<float>(ntaps);
+  float4* rec = sc.take<float4>(2 * nvis);
+  uint32_t* start = sc.take<uint32_t>(ntiles + 1);
+  char* stmp = sc.take<char>(scan_bytes);
+  int* pos = sc.take<int>(cells);
+  float2* cvo = sc.take<float2>(cells);
+  float* cw = sc.take<float>(cells);
+  GVM_HIP_TRY(hipMemcpy(taps_d, kernel->taps, sizeof(float) * ntaps, hipMemcpyHostToDevice));
+  const float2* vo = reinterpret_cast<const float2*>(vo_dev);
+  hipLaunchKernelGGL(grid_keys_kernel, dim3(blocks_for(nvis)), dim3(kThreads), 0, nullptr,
+                     uvw_m_dev, weight_dev, vo, nvis, g, rec, ps.k[0], ps.v[0]);
+  if ((st = launch_ok(what)) || (st = ps.sort((size_t)n, bits, what))) return st;
+  hipLaunchKernelGGL(tile_first_kernel, dim3(blocks_for(ntiles + 1)), dim3(kThreads), 0, nullptr,
+                     ps.keys(), n, ntiles, start);
   if ((st = launch_ok(what))) return st;
-  size_t sbytes = 0;
-  GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, sbytes, flag.as<int>(), rank.as<int>(), 0,
-                                      (size_t)n, rocprim::plus<int>()));
-  DevMem stmp;
-  if ((st = dev_alloc(stmp, sbytes, what))) return st;
-  GVM_HIP_TRY(rocprim::exclusive_scan(stmp.p, sbytes, flag.as<int>(), rank.as<int>(), 0,
-                                      (size_t)n, rocprim::plus<int>()));
-  int last[2] = {0, 0};
-  GVM_HIP_TRY(hipMemcpy(&last[0], rank.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost));
-  GVM_HIP_TRY(hipMemcpy(&last[1], flag.as<int>() + n - 1, sizeof(int), hipMemcpyDeviceToHost));
-  const long nruns = (long)last[0] + last[1];
-  hipLaunchKernelGGL(run_starts_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, nullptr,
-                     flag.as<int>(), rank.as<int>(), n, starts.as<int>());
-  if ((st = launch_ok(what)) || (st = dev_alloc(keep, sizeof(int) * nruns, what)) ||
-      (st = dev_alloc(pos, sizeof(int) * nruns, what)) ||
-      (st = dev_alloc(cvo, sizeof(float2) * nruns, what)) ||
-      (st = dev_alloc(cw, sizeof(float) * nruns, what)))
-    return st;
-  hipLaunchKernelGGL(grid_cells_kernel, dim3((unsigned)nruns), dim3(64), 0, nullptr, cs.keys(),
-                     cs.ids(), starts.as<int>(), nvis, g, taps_d.as<float>(), weight_dev,
-                     reinterpret_cast<const float2*>(vo_dev), keep.as<int>(), cvo.as<float2>(),
-                     cw.as<float>());
+  const dim3 tiles(ntiles);
+  if (g.wx * g.wy <= kLdsTaps)
+    hipLaunchKernelGGL((grid_tiles_kernel<true>), tiles, dim3(kThreads), 0, nullptr, ps.ids(), start,
+                       g, taps_d, rec, cvo, cw);
+  else
+    hipLaunchKernelGGL((grid_tiles_kernel<false>), tiles, dim3(kThreads), 0, nullptr, ps.ids(),
+                       start, g, taps_d, rec, cvo, cw);
   if ((st = launch_ok(what))) return st;
-  // exclusive prefix sum of the keep flags: output row of each kept cell
-  size_t kbytes = 0;
-  GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, kbytes, keep.as<int>(), pos.as<int>(), 0,
-                                      (size_t)nruns, rocprim::plus<int>()));
-  if (kbytes > sbytes && (st = dev_alloc(stmp, kbytes, what))) return st;
-  kbytes = std::max(kbytes, sbytes);
-  GVM_HIP_TRY(rocprim::exclusive_scan(stmp.p, kbytes, keep.as<int>(), pos.as<int>(), 0,
-                                      (size_t)nruns, rocprim::plus<int>()));
-  GVM_HIP_TRY(hipMemcpy(&last[0], pos.as<int>() + nruns - 1, sizeof(int), hipMemcpyDeviceToHost));
-  GVM_HIP_TRY(hipMemcpy(&last[1], keep.as<int>() + nruns - 1, sizeof(int), hipMemcpyDeviceToHost));
-  const long count = (long)last[0] + last[1];
+  // output row of each kept cell
+  GVM_HIP_TRY(rocprim::exclusive_scan(stmp, scan_bytes, kept(cw), pos, 0, (size_t)cells,
+                                      rocprim::plus<int>()));
+  int last = 0;
+  float last_w = 0.f;
+  GVM_HIP_TRY(hipMemcpy(&last, pos + cells - 1, sizeof(int), hipMemcpyDeviceToHost));
+  GVM_HIP_TRY(hipMemcpy(&last_w, cw + cells - 1, sizeof(float), hipMemcpyDeviceToHost));
+  const long count = (long)last + IsKept()(last_w);
   if (count > capacity) {
     set_error("gvm_grid_visibilities_dev: " + std::to_string(count) +
               " gridded rows exceed the output capacity " + std::to_string(capacity));
     return GVM_ERR_ARG;
   }
-  hipLaunchKernelGGL(grid_emit_kernel, dim3(blocks_for(nruns)), dim3(kThreads), 0, nullptr,
-                     cs.keys(), starts.as<int>(), keep.as<int>(), pos.as<int>(), nruns, g,
-                     cvo.as<float2>(), cw.as<float>(), capacity, uvw_out_dev,
-                     reinterpret_cast<float2*>(vo_out_dev), weight_out_dev);
+  hipLaunchKernelGGL(grid_emit_kernel, dim3(blocks_for(cells)), dim3(kThreads), 0, nullptr, pos, g,
+                     cvo, cw, capacity, uvw_out_dev, reinterpret_cast<float2*>(vo_out_dev),
+                     weight_out_dev);
   if ((st = launch_ok(what))) return st;
   GVM_HIP_TRY(hipDeviceSynchronize());
   *nout = count;
@@ -575,21 +704,27 @@ extern "C" gvm_status gvm_add_visibilities_gridded_dev(gvm_ctx* ctx, const gvm_c
   static const char* what = "gvm_add_visibilities_gridded_dev";
   GVM_REQUIRE(ctx, "gvm_add_visibilities_gridded_dev: null context");
   GVM_HIP_TRY(hipSetDevice(ctx->device));
-  const long cap = (long)ctx->g.M * ctx->g.N;
-  DevMem u, v, w;
-  gvm_status st;
-  if ((st = dev_alloc(u, sizeof(double) * 3 * cap, what)) ||
-      (st = dev_alloc(v, sizeof(float) * 2 * cap, what)) ||
-      (st = dev_alloc(w, sizeof(float) * cap, what)))
-    return st;
+  const size_t cap = (size_t)ctx->g.M * ctx->g.N;
+  // the gridded rows: uvw, Vo, weight (the gridder's scratch is the context's)
+  struct Rows {
+    char* p = nullptr;
+    ~Rows() { (void)hipFree(p); }
+  } rows;
+  if (hipMalloc((void**)&rows.p, cap * (3 * sizeof(double) + 3 * sizeof(float))) != hipSuccess) {
+    (void)hipGetLastError();
+    rows.p = nullptr;
+    set_error(std::string(what) + ": out of device memory");
+    return GVM_ERR_OOM;
+  }
+  double* u = (double*)rows.p;
+  float *v = (float*)(u + 3 * cap), *w = v + 2 * cap;
   long count = 0;
-  st = gvm_grid_visibilities_dev(ctx, kernel, freq, nvis, uvw_m_dev, vo_dev, weight_dev,
-                                 u.as<double>(), v.as<float>(), w.as<float>(), cap, &count);
+  gvm_status st = gvm_grid_visibilities_dev(ctx, kernel, freq, nvis, uvw_m_dev, vo_dev, weight_dev,
+                                            u, v, w, (long)cap, &count);
   if (st) return st;
   GVM_REQUIRE(count > 0, "gvm_add_visibilities_gridded_dev: no visibility falls on the grid");
   if (ngridded) *ngridded = count;
-  return gvm_add_visibilities_dev(ctx, freq, count, u.as<double>(), v.as<float>(), w.as<float>(),
-                                  slice_out);
+  return gvm_add_visibilities_dev(ctx, freq, count, u, v, w, slice_out);
 }
 
 extern "C" gvm_status gvm_set_gcf(gvm_ctx* ctx, const float* gcf_host) {
@@ -659,42 +794,67 @@ extern "C" gvm_status gvm_weighting_apply_dev(gvm_ctx* ctx, int scheme, float ro
   const bool gridded = scheme == GVM_WEIGHTING_UNIFORM || scheme == GVM_WEIGHTING_BRIGGS;
   const int bits = key_bits(g.off);
   gvm_status st;
-  CellSort cs;
-  DevMem grid, part;
-  const size_t gbytes = sizeof(float) * (size_t)geo.M * geo.N;
-  if (gridded && ((st = cs.reserve(nmax, what)) || (st = dev_alloc(grid, gbytes, what)) ||
-                  (st = dev_alloc(part, sizeof(double) * kSumBlocks, what))))
-    return st;
+  const size_t cells = (size_t)geo.M * geo.N, gbytes = sizeof(float) * cells;
+  Scratch sc(ctx);
+  PairSort ps;
+  float *grid = nullptr, *sorted = nullptr;
+  double* part = nullptr;  // per slice: kSumBlocks partials of sum w, then of sum G^2
+  if (gridded) {
+    for (int s = 0; s < nsl; s++)
+      if (nvis[s] > 0 && (st = ps.size((size_t)nvis[s], bits, what))) return st;
+    ps.add(sc);
+    sc.add(gbytes);
+    sc.add(sizeof(float) * nmax);
+    if (scheme == GVM_WEIGHTING_BRIGGS) sc.add(sizeof(double) * 2 * kSumBlocks * nsl);
+    if ((st = sc.reserve(what))) return st;
+    ps.take(sc);
+    grid = sc.take<float>(cells);
+    sorted = sc.take<float>(nmax);
+    if (scheme == GVM_WEIGHTING_BRIGGS) part = sc.take<double>(2 * (size_t)kSumBlocks * nsl);
+  }
+  // the cell sums of slice s (added to the grid's when cumulative)
+  auto cell_sums = [&](int s, int cumulative) -> gvm_status {
+    g.lambda = (double)(2.99792458E8f / freq[s]);
+    hipLaunchKernelGGL(weight_keys_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0, nullptr,
+                       uvw_m_dev[s], nvis[s], g, ps.k[0], ps.v[0]);
+    gvm_status r;
+    if ((r = launch_ok(what)) || (r = ps.sort((size_t)nvis[s], bits, what))) return r;
+    hipLaunchKernelGGL(weight_gather_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0, nullptr,
+                       ps.ids(), weight_dev[s], nvis[s], sorted);
+    hipLaunchKernelGGL(weight_cells_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0, nullptr,
+                       ps.keys(), sorted, nvis[s], g.off, cumulative, grid);
+    return launch_ok(what);
+  };
 
   float f2 = 0.0f;
   if (scheme == GVM_WEIGHTING_BRIGGS) {
     // Pass 1 (src/briggsweightingscheme.cu:44-105): the sum of the weights,
     // and per slice the sum of G^2 over the right half of a grid that is not
     // cleared between slices (the reference clears it only after the pass).
-    double sum_w = 0.0, sum_g2 = 0.0;
-    GVM_HIP_TRY(hipMemset(grid.p, 0, gbytes));
+    GVM_HIP_TRY(hipMemsetAsync(grid, 0, gbytes, nullptr));
+    const int nbg = std::min(kSumBlocks, blocks_for((long)geo.M * (geo.N - geo.N / 2)));
     for (int s = 0; s < nsl; s++) {
       if (nvis[s] == 0) continue;
-      g.lambda = (double)(2.99792458E8f / freq[s]);
-      const int nb = std::min(kSumBlocks, blocks_for(nvis[s]));
-      double ps = 0.0;
-      hipLaunchKernelGGL(weight_sum_kernel, dim3(nb), dim3(kThreads), 0, nullptr, weight_dev[s],
-                         nvis[s], part.as<double>());
-      if ((st = launch_ok(what)) || (st = read_partials(part.as<double>(), nb, &ps, what)))
-        return st;
-      sum_w += ps;
-      hipLaunchKernelGGL(weight_keys_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0,
-                         nullptr, uvw_m_dev[s], nvis[s], g, cs.in_keys(), cs.in_ids());
-      if ((st = launch_ok(what)) || (st = cs.sort(nvis[s], bits, what))) return st;
-      hipLaunchKernelGGL(weight_cells_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0,
-                         nullptr, cs.keys(), cs.ids(), nvis[s], g.off, weight_dev[s], 1,
-                         grid.as<float>());
-      const int nbg = std::min(kSumBlocks, blocks_for((long)geo.M * (geo.N - geo.N / 2)));
-      hipLaunchKernelGGL(grid_sq_sum_kernel, dim3(nbg), dim3(kThreads), 0, nullptr,
-                         grid.as<float>(), geo.M, geo.N, part.as<double>());
-      if ((st = launch_ok(what)) || (st = read_partials(part.as<double>(), nbg, &ps, what)))
-        return st;
-      sum_g2 += ps;
+      double* p = part + 2 * (size_t)kSumBlocks * s;
+      hipLaunchKernelGGL(weight_sum_kernel, dim3(std::min(kSumBlocks, blocks_for(nvis[s]))),
+                         dim3(kThreads), 0, nullptr, weight_dev[s], nvis[s], p);
+      if ((st = launch_ok(what)) || (st = cell_sums(s, 1))) return st;
+      hipLaunchKernelGGL(grid_sq_sum_kernel, dim3(nbg), dim3(kThreads), 0, nullptr, grid, geo.M,
+                         geo.N, p + kSumBlocks);
+      if ((st = launch_ok(what))) return st;
+    }
+    // the FP64 sums of the block partials, in block order, slice after slice
+    std::vector<double> h(2 * (size_t)kSumBlocks * nsl);
+    GVM_HIP_TRY(hipMemcpy(h.data(), part, sizeof(double) * h.size(), hipMemcpyDeviceToHost));
+    double sum_w = 0.0, sum_g2 = 0.0;
+    for (int s = 0; s < nsl; s++) {
+      if (nvis[s] == 0) continue;
+      const double* p = h.data() + 2 * (size_t)kSumBlocks * s;
+      double a = 0.0, b = 0.0;
+      for (int k = 0; k < std::min(kSumBlocks, blocks_for(nvis[s])); k++) a += p[k];
+      for (int k = 0; k < nbg; k++) b += p[kSumBlocks + k];
+      sum_w += a;
+      sum_g2 += b;
     }
     GVM_REQUIRE(sum_w != 0.0, "gvm_weighting_apply_dev: the sum of the weights is zero");
     const float average_weights = (float)sum_g2 / (float)sum_w;
@@ -702,23 +862,17 @@ extern "C" gvm_status gvm_weighting_apply_dev(gvm_ctx* ctx, int scheme, float ro
     f2 = f * f / average_weights;
   }
 
-  // Pass 2: per slice, the slice's own weight grid, then the row update.
+  // Pass 2: per slice, the slice's own weight grid, then the row update.  (With
+  // one slice Briggs' first pass has left that grid.)
   for (int s = 0; s < nsl; s++) {
     if (nvis[s] == 0) continue;
     g.lambda = (double)(2.99792458E8f / freq[s]);
-    if (gridded) {
-      GVM_HIP_TRY(hipMemset(grid.p, 0, gbytes));
-      hipLaunchKernelGGL(weight_keys_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0,
-                         nullptr, uvw_m_dev[s], nvis[s], g, cs.in_keys(), cs.in_ids());
-      if ((st = launch_ok(what)) || (st = cs.sort(nvis[s], bits, what))) return st;
-      hipLaunchKernelGGL(weight_cells_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0,
-                         nullptr, cs.keys(), cs.ids(), nvis[s], g.off, weight_dev[s], 0,
-                         grid.as<float>());
-      if ((st = launch_ok(what))) return st;
+    if (gridded && !(scheme == GVM_WEIGHTING_BRIGGS && nsl == 1)) {
+      GVM_HIP_TRY(hipMemsetAsync(grid, 0, gbytes, nullptr));
+      if ((st = cell_sums(s, 0))) return st;
     }
     hipLaunchKernelGGL(weight_apply_kernel, dim3(blocks_for(nvis[s])), dim3(kThreads), 0, nullptr,
-                       scheme, uvw_m_dev[s], nvis[s], g,
-                       gridded ? grid.as<float>() : nullptr, f2, tc, weight_dev[s]);
+                       scheme, uvw_m_dev[s], nvis[s], g, grid, f2, tc, weight_dev[s]);
     if ((st = launch_ok(what))) return st;
   }
   GVM_HIP_TRY(hipDeviceSynchronize());

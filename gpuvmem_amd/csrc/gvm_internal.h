@@ -150,6 +150,9 @@ struct gvm_ctx {
   // epoch changes whenever recorded device pointers or launches go stale
   bool capturing = false;
   long epoch = 0;
+  // set-up workspace: scratch of the gridder and the weighting schemes
+  char* setup_ws = nullptr;
+  size_t setup_bytes = 0;
   // network workspace: the weight-gradient partials of a convolution
   float* nn_part = nullptr;
   size_t nn_part_elems = 0;
