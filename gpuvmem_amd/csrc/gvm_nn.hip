@@ -2,10 +2,10 @@
 // optional ReLU, 2x2 average pooling, nearest 2x upsampling into a channel
 // block, channel copies, the MSE loss and Adam, forward and backward.
 //
-// Convolutions are implicit GEMMs on the FP32 MFMA units (forward, input
-// gradient, and weight gradient in pixel ranges whose partials are summed in
-// FP64 in a fixed order); bias gradients and the loss are FP64 fixed-order
-// reductions, so training is reproducible bit for bit.  Layouts are NCHW.
+// Convolutions run on the FP32 MFMA units (forward, input gradient, and weight
+// gradient in pixel ranges whose partials are summed in FP64 in a fixed order);
+// bias gradients and the loss are FP64 fixed-order reductions, so training is
+// reproducible bit for bit.  Layouts are NCHW.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,220 +26,346 @@ __device__ __forceinline__ float wload(const unsigned short* w, long i) {
   return __uint_as_float((unsigned int)w[i] << 16);
 }
 
-__device__ __forceinline__ float relu_grad(const float* out, const float* dout, long i, int relu) {
-  const float g = dout[i];
-  return relu ? (out[i] > 0.0f ? g : 0.0f) : g;
-}
-
 // ---------------------------------------------------------------------------
-// Convolutions as implicit GEMMs on the FP32 MFMA units
-// (v_mfma_f32_32x32x2_f32: FP32 products, FP32 accumulation).
+// Convolutions on the FP32 MFMA units (v_mfma_f32_32x32x2_f32: FP32 products,
+// FP32 accumulation).  tap (ky, kx) shifts a pixel by (ky - K/2, kx - K/2), zero
+// outside the image; g is the output gradient masked by the ReLU of the forward
+// output.
 //
 //   forward      out[co][q]   = sum_{ci,tap} w[co][ci][tap] in[ci][q + tap]
-//                M = Co, N = pixels (b, y, x), K = Ci K K
 //   input grad   din[ci][q]   = sum_{co,tap} w[co][ci][tap] g[co][q - tap]
-//                M = Ci, N = pixels, K = Co K K
-//   weight grad  dw[co][ci,tap] = sum_q g[co][q] in[ci][q + tap]
-//                M = Co, N = Ci K K, K = pixels, split in ranges of
-//                kWgradPixels whose FP32 partials are summed in FP64 in a
-//                fixed order (bitwise reproducible)
+//   weight grad  dw[co][ci][tap] = sum_q g[co][q] in[ci][q + tap]
 //
-// tap (ky, kx) shifts a pixel by (ky - K/2, kx - K/2), zero outside the
-// image; g is the output gradient masked by the ReLU of the forward output.
-// A workgroup (4 waves) computes a 64 x 64 tile of M x N, each wave a 32 x
-// 32 block; K advances in chunks of 16 staged in LDS (k-major, so the MFMA
-// operand reads of a wave are consecutive), the next chunk's values loaded
-// into registers while the current one is multiplied.
+// The instruction takes 64 cycles for a 32 x 32 block and two values of K, so a
+// kernel that keeps its index arithmetic out of the loop runs at its rate (154
+// TFLOP/s measured): pixels are tiled in the image's plane, a tile with its halo
+// is staged in LDS once per chunk of channels and read at nine shifts, and the
+// addresses of a thread's loads are computed once per block.  (An im2col loop
+// that formed every element's coordinates as it loaded it ran at 26 TFLOP/s.)
 // ---------------------------------------------------------------------------
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-enum { CONV_FWD = 0, CONV_BWD_DATA = 1, CONV_BWD_WEIGHT = 2 };
-constexpr int kCTile = 64;
-constexpr int kCK = 16;
-constexpr int kWgradPixels = 8192;
+enum { CONV_FWD = 0, CONV_BWD_DATA = 1 };
+
+// A plane pitch (floats) of at least n whose multiples by 0 and 1 put two rows
+// of 32 consecutive reads on different LDS banks (64 of 4 bytes).
+constexpr int plane_pitch(int n) { return (n - 32 + 63) / 64 * 64 + 32; }
 
 template <class WT>
 struct ConvArgs {
-  const float* in;    // [B][Ci][H][W]
+  const float* in;    // forward: [B][Ci][H][W]; input grad: dout [B][Co][H][W]
+  const float* mask;  // input grad: the forward output (ReLU mask), or NULL
   const WT* w;        // [Co][Ci][K][K]
   const float* bias;  // [Co] (forward)
-  const float* out;   // forward output (ReLU mask), or NULL
-  const float* dout;  // [B][Co][H][W] gradient at the activated output
-  float* dst;         // out (forward), din (input grad) or the weight-grad partials
-  int B, Ci, Co, H, W, relu;
+  float* dst;         // [B][M][H][W]
+  int B, M, C;        // output and input channels of this product
+  int H, W, relu;
+  int tiles_x, tiles_y;
 };
 
-template <int K, class WT>
-__device__ __forceinline__ float conv_in_at(const ConvArgs<WT>& a, int ci, int q, int tap) {
-  // in[b][ci][y + ky - P][x + kx - P] for pixel q = (b, y, x), 0 outside
-  constexpr int P = K / 2;
+// One block of 4 waves: MT output channels x a TH x TW tile of pixels; input
+// channels in chunks of CK, the next chunk's values loaded into registers while
+// this one is multiplied.  K runs over (channel, tap), tap fastest, two values
+// per MFMA: the products and their order are an im2col GEMM's, so the sums do
+// not depend on the tiling.  LDS: the tile's planes, and the weights [K][MT].
+// The two halves of a wave read K values 2 s and 2 s + 1, whose places in the
+// planes differ by a step that repeats every two channels: a lane keeps those
+// addresses, and the rest of a read's address is an immediate.
+template <int MODE, int KS, int MT, int TH, int TW, int CK, class WT>
+__global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
+  constexpr int KK = KS * KS, P = KS / 2, PH = TH + KS - 1, PW = TW + KS - 1;
+  constexpr int PLANE = plane_pitch(PH * PW), MTP = MT == 32 ? 32 : 96;
+  constexpr int NBT = TH * TW / 32, WN = NBT < 4 ? NBT : 4, WM = 4 / WN;
+  constexpr int NB = NBT / WN, MB = MT / 32 / WM;
+  static_assert(NB * WN == NBT && MB * WM * 32 == MT, "four waves share the tile");
+  constexpr int NI = (CK * PH * PW + 255) / 256;   // input values per thread
+  constexpr int CP = 256 / MT, NW = CK / CP;       // weights: channels per thread
+  static_assert(NW * CP == CK, "whole channels per thread");
+  __shared__ float li[CK * PLANE];
+  __shared__ float lw[KK * CK * MTP];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
+  const int wn = wave % WN, wm = wave / WN;
   const int HW = a.H * a.W;
-  const int b = q / HW, p = q - b * HW;
-  const int yy = p / a.W + tap / K - P, xx = p % a.W + tap % K - P;
-  if (yy < 0 || yy >= a.H || xx < 0 || xx >= a.W) return 0.0f;
-  return a.in[((long)b * a.Ci + ci) * HW + (long)yy * a.W + xx];
-}
-
-template <class WT>
-__device__ __forceinline__ float conv_g_at(const ConvArgs<WT>& a, int co, int q) {
-  // the masked output gradient at pixel q = (b, y, x) of output channel co
-  const int HW = a.H * a.W;
-  const int b = q / HW, p = q - b * HW;
-  const long i = ((long)b * a.Co + co) * HW + p;
-  return relu_grad(a.out, a.dout, i, a.relu);
-}
-
-template <int MODE, int K, class WT>
-__device__ __forceinline__ float conv_a(const ConvArgs<WT>& a, int m, int k, int M, int Kd) {
-  if (m >= M || k >= Kd) return 0.0f;
-  constexpr int KK = K * K;
-  if constexpr (MODE == CONV_FWD) return wload(a.w, (long)m * Kd + k);
-  if constexpr (MODE == CONV_BWD_DATA) {
-    const int co = k / KK, tap = k - co * KK;  // w[co][ci = m][tap]
-    return wload(a.w, ((long)co * a.Ci + m) * KK + tap);
-  }
-  return conv_g_at(a, m, k);  // weight grad: g[co = m][pixel k]
-}
-
-template <int MODE, int K, class WT>
-__device__ __forceinline__ float conv_b(const ConvArgs<WT>& a, int k, int n, int Kd, int Nd) {
-  if (k >= Kd || n >= Nd) return 0.0f;
-  constexpr int KK = K * K;
-  if constexpr (MODE == CONV_FWD) {
-    const int ci = k / KK;
-    return conv_in_at<K>(a, ci, n, k - ci * KK);
-  }
-  if constexpr (MODE == CONV_BWD_DATA) {
-    // g[co][q - tap] with k = (co, tap)
-    constexpr int P = K / 2;
-    const int co = k / KK, tap = k - co * KK;
-    const int HW = a.H * a.W;
-    const int b = n / HW, p = n - b * HW;
-    const int yy = p / a.W - (tap / K - P), xx = p % a.W - (tap % K - P);
-    if (yy < 0 || yy >= a.H || xx < 0 || xx >= a.W) return 0.0f;
-    return relu_grad(a.out, a.dout, ((long)b * a.Co + co) * HW + (long)yy * a.W + xx, a.relu);
-  }
-  const int ci = n / KK;  // weight grad: in[ci][pixel k + tap], n = (ci, tap)
-  return conv_in_at<K>(a, ci, k, n - ci * KK);
-}
-
-template <int MODE, int K, class WT>
-__global__ __launch_bounds__(256) void conv_mfma_kernel(ConvArgs<WT> a) {
-  constexpr int KK = K * K;
-  const int HW = a.H * a.W;
-  const int npix = a.B * HW;
-  int M, Nd, Kd, kbeg;
-  if constexpr (MODE == CONV_FWD) {
-    M = a.Co; Nd = npix; Kd = a.Ci * KK; kbeg = 0;
-  } else if constexpr (MODE == CONV_BWD_DATA) {
-    M = a.Ci; Nd = npix; Kd = a.Co * KK; kbeg = 0;
-  } else {
-    M = a.Co; Nd = a.Ci * KK; kbeg = blockIdx.z * kWgradPixels;
-    Kd = min(npix, kbeg + kWgradPixels);
-  }
-  __shared__ float As[kCK][kCTile + 4];
-  __shared__ float Bs[kCK][kCTile + 4];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int m0 = blockIdx.y * kCTile, n0 = blockIdx.x * kCTile;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  // loader coordinates: 4 A and 4 B values per thread per chunk.  The
-  // weight grad reads along pixels (its K) for both operands, the others
-  // along k for A and along pixels (N) for B.
-  float ra[4], rb[4];
-  auto load = [&](int k0) {
+  const int tile = blockIdx.x, m0 = blockIdx.y * MT;
+  const int tx = tile % a.tiles_x, ty = tile / a.tiles_x % a.tiles_y, b = tile / a.tiles_x / a.tiles_y;
+  const int x0 = tx * TW, y0 = ty * TH;
+  // this thread's input values: offset within a plane (-1: zero), plane, LDS place
+  int off[NI];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int e = t + 256 * j;
-      const int am = e / kCK, ak = e % kCK;
-      ra[j] = conv_a<MODE, K>(a, m0 + am, k0 + ak, M, Kd);
-      int bk, bn;
-      if constexpr (MODE == CONV_BWD_WEIGHT) {
-        bk = e % kCK;
-        bn = e / kCK;
-      } else {
-        bk = e / kCTile;
-        bn = e % kCTile;
+  for (int j = 0; j < NI; j++) {
+    const int e = t + 256 * j, r = e % (PH * PW);
+    const int y = y0 + r / PW - P, x = x0 + r % PW - P;
+    off[j] = e < CK * PH * PW && y >= 0 && y < a.H && x >= 0 && x < a.W ? y * a.W + x : -1;
+  }
+  const long in0 = (long)b * a.C * HW;
+  const int wco = t % MT, wc = t / MT;
+  float ri[NI], rw[NW * KK];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      const int c = c0 + (t + 256 * j) / (PH * PW);
+      ri[j] = 0.0f;
+      if (off[j] >= 0 && c < a.C) {
+        const long i = in0 + (long)c * HW + off[j];
+        if constexpr (MODE == CONV_FWD)
+          ri[j] = a.in[i];
+        else
+          ri[j] = !a.mask || a.mask[i] > 0.0f ? a.in[i] : 0.0f;
       }
-      rb[j] = conv_b<MODE, K>(a, k0 + bk, n0 + bn, Kd, Nd);
+    }
+#pragma unroll
+    for (int q = 0; q < NW; q++) {
+      const int c = c0 + wc + q * CP, m = m0 + wco;
+      const bool ok = m < a.M && c < a.C;
+      // forward: w[m][c][tap]; input grad: w[c][m][tap]
+      const long i = MODE == CONV_FWD ? ((long)m * a.C + c) * KK : ((long)c * a.M + m) * KK;
+#pragma unroll
+      for (int k = 0; k < KK; k++) rw[q * KK + k] = ok ? wload(a.w, i + k) : 0.0f;
     }
   };
   auto store = [&]() {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < NI; j++) {
       const int e = t + 256 * j;
-      As[e % kCK][e / kCK] = ra[j];
-      if constexpr (MODE == CONV_BWD_WEIGHT)
-        Bs[e % kCK][e / kCK] = rb[j];
-      else
-        Bs[e / kCTile][e % kCTile] = rb[j];
+      if (e < CK * PH * PW) li[e / (PH * PW) * PLANE + e % (PH * PW)] = ri[j];
     }
-  };
-  f32x16_t acc;
 #pragma unroll
-  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
-  const int lr = lane & 31, lh = lane >> 5;
-  load(kbeg);
-  for (int k0 = kbeg; k0 < Kd; k0 += kCK) {
-    __syncthreads();  // the previous chunk's reads are done
+    for (int q = 0; q < NW; q++)
+#pragma unroll
+      for (int k = 0; k < KK; k++) lw[((wc + q * CP) * KK + k) * MTP + wco] = rw[q * KK + k];
+  };
+  f32x16_t acc[MB][NB];
+#pragma unroll
+  for (int m = 0; m < MB; m++)
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[m][n][e] = 0.0f;
+  // places of the K values of two channels, less those of the pixel block:
+  // tap (ky, kx) reads the pixel shifted by +tap (forward) or -tap (input grad)
+  const float* pb[KK];
+  {
+    const int p = wn * NB * 32 + lr;
+#pragma unroll
+    for (int j = 0; j < KK; j++) {
+      int place[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int k = 2 * j + h, c = k / KK, tap = MODE == CONV_FWD ? k % KK : KK - 1 - k % KK;
+        place[h] = c * PLANE + tap / KS * PW + tap % KS;
+      }
+      pb[j] = li + p / TW * PW + p % TW + (lh ? place[1] : place[0]);
+    }
+  }
+  constexpr int NSTEP = TW == 32 ? PW : 32 / TW * PW;  // from a pixel block to the next
+  const float* pa = lw + lh * MTP + wm * MB * 32 + lr;
+  load(0);
+  for (int c0 = 0; c0 < a.C; c0 += CK) {
+    __syncthreads();  // the chunk before has been read
     store();
     __syncthreads();
-    if (k0 + kCK < Kd) load(k0 + kCK);
+    if (c0 + CK < a.C) load(c0 + CK);
 #pragma unroll
-    for (int s = 0; s < kCK / 2; s++)
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[2 * s + lh][wm + lr], Bs[2 * s + lh][wn + lr],
-                                                 acc, 0, 0, 0);
+    for (int c = 0; c < CK / 2; c++)
+#pragma unroll
+      for (int j = 0; j < KK; j++) {
+        float va[MB], vb[NB];
+#pragma unroll
+        for (int m = 0; m < MB; m++) va[m] = pa[(2 * KK * c + 2 * j) * MTP + m * 32];
+#pragma unroll
+        for (int n = 0; n < NB; n++) vb[n] = pb[j][2 * c * PLANE + n * NSTEP];
+#pragma unroll
+        for (int m = 0; m < MB; m++)
+#pragma unroll
+          for (int n = 0; n < NB; n++)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[m], vb[n], acc[m][n], 0, 0, 0);
+      }
   }
   // 32 x 32 accumulator layout: lane l, register e -> row 8 (e / 4) + 4 (l / 32)
-  // + e % 4 of the wave's block, column l % 32
+  // + e % 4, column l % 32
 #pragma unroll
-  for (int e = 0; e < 16; e++) {
-    const int m = m0 + wm + 8 * (e >> 2) + 4 * lh + (e & 3);
-    const int n = n0 + wn + lr;
-    if (m >= M || n >= Nd) continue;
-    if constexpr (MODE == CONV_BWD_WEIGHT) {
-      a.dst[((long)blockIdx.z * M + m) * Nd + n] = acc[e];
-    } else {
-      const int b = n / HW, p = n - b * HW;
-      float v = acc[e];
-      if constexpr (MODE == CONV_FWD) {
-        v = v + a.bias[m];
-        if (a.relu) v = fmaxf(v, 0.0f);
+  for (int n = 0; n < NB; n++) {
+    const int p = (wn * NB + n) * 32 + lr, y = y0 + p / TW, x = x0 + p % TW;
+    if (y >= a.H || x >= a.W) continue;
+#pragma unroll
+    for (int m = 0; m < MB; m++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int co = m0 + (wm * MB + m) * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
+        if (co >= a.M) continue;
+        float v = acc[m][n][e];
+        if constexpr (MODE == CONV_FWD) {
+          v = v + a.bias[co];
+          if (a.relu) v = fmaxf(v, 0.0f);
+        }
+        a.dst[((long)b * a.M + co) * HW + y * a.W + x] = v;
       }
-      a.dst[((long)b * M + m) * HW + p] = v;
+  }
+}
+
+// ---- weight gradient ----
+struct WgradArgs {
+  const float* in;    // [B][Ci][H][W]
+  const float* out;   // forward output (ReLU mask), or NULL
+  const float* dout;  // [B][Co][H][W]
+  float* part;        // [partial][Co][Ci][K][K]
+  double* bpart;      // [partial][Co]
+  int B, Ci, Co, H, W;
+  int tiles_x, tiles_y, ntiles, per;  // tiles of pixels; tiles per block
+};
+
+constexpr int kWgradW = 16;  // pixel columns of a tile
+
+// A wave owns 32 output x 32 input channels of every tap (nine 32 x 32 blocks)
+// and adds tiles of SH x 16 pixels: K = pixels, A = g[co][q], B = in[ci][q + tap]
+// read from the staged planes.  WM x WN waves cover channels, WK waves take
+// different tiles and leave a partial each; the partials are summed in FP64 in a
+// fixed order.  Channel pitches are twice an odd number, so that the 32 channels
+// and the two pixels of an MFMA operand fall on 64 different banks.  The blocks of
+// the first input channels also leave the bias gradient's partials (FP64).
+template <int KS, int WM, int WN, int WK, int SH>
+__global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
+  constexpr int KK = KS * KS, P = KS / 2, PW = kWgradW + KS - 1, PH = SH + KS - 1;
+  constexpr int Q = SH * kWgradW, GP = Q + 2, IP = (PH * PW + 3) / 4 * 4 + 2;
+  static_assert(WM * WN * WK == 4, "four waves");
+  constexpr int NG = WM * 32 * Q * WK / 256, NIN = (WN * 32 * PH * PW * WK + 255) / 256;
+  __shared__ float lg[WK][WM * 32 * GP];
+  __shared__ float li[WK][WN * 32 * IP];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
+  const int wk = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
+  const int HW = a.H * a.W;
+  const int co0 = blockIdx.y * WM * 32, ci0 = blockIdx.x * WN * 32;
+  const int first = blockIdx.z * a.per, last = min(a.ntiles, first + a.per);
+  static_assert(NG % WK == 0 && NIN * 256 == WN * 32 * PH * PW * WK && NIN % WK == 0,
+                "a thread's j-th value belongs to one tile for every thread");
+  float rg[NG], ri[NIN];
+  // origins of the tiles being loaded (one per WK), and the j-th value of each
+  // operand; the values are loaded between the MFMAs of the tiles before
+  int tx[WK], ty[WK], tb[WK];
+  bool on[WK];
+  auto origins = [&](int tile0) {
+#pragma unroll
+    for (int k = 0; k < WK; k++) {
+      const int tile = min(tile0 + k, a.ntiles - 1);
+      on[k] = tile0 + k < last;
+      tx[k] = tile % a.tiles_x * kWgradW;
+      ty[k] = tile / a.tiles_x % a.tiles_y * SH;
+      tb[k] = tile / a.tiles_x / a.tiles_y;
+    }
+  };
+  auto load_g = [&](int j) {
+    const int k = j / (NG / WK), e = t + 256 * (j % (NG / WK)), q = e % Q, co = co0 + e / Q;
+    const int x = tx[k] + q % kWgradW, y = ty[k] + q / kWgradW;
+    rg[j] = 0.0f;
+    if (on[k] && co < a.Co && x < a.W && y < a.H) {
+      const long i = ((long)tb[k] * a.Co + co) * HW + y * a.W + x;
+      rg[j] = !a.out || a.out[i] > 0.0f ? a.dout[i] : 0.0f;
+    }
+  };
+  auto load_in = [&](int j) {
+    const int k = j / (NIN / WK), e = t + 256 * (j % (NIN / WK)), r = e % (PH * PW);
+    const int ci = ci0 + e / (PH * PW);
+    const int x = tx[k] + r % PW - P, y = ty[k] + r / PW - P;
+    ri[j] = 0.0f;
+    if (on[k] && ci < a.Ci && x >= 0 && x < a.W && y >= 0 && y < a.H)
+      ri[j] = a.in[((long)tb[k] * a.Ci + ci) * HW + y * a.W + x];
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int j = 0; j < NG; j++) {
+      const int e = t + 256 * (j % (NG / WK));
+      lg[j / (NG / WK)][e / Q * GP + e % Q] = rg[j];
+    }
+#pragma unroll
+    for (int j = 0; j < NIN; j++) {
+      const int e = t + 256 * (j % (NIN / WK));
+      li[j / (NIN / WK)][e / (PH * PW) * IP + e % (PH * PW)] = ri[j];
+    }
+  };
+  f32x16_t acc[KK];
+#pragma unroll
+  for (int k = 0; k < KK; k++)
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[k][e] = 0.0f;
+  // bias: thread t sums part of the g values of channel t / TPC
+  constexpr int TPC = 256 / (WM * 32);
+  double bsum = 0.0;
+  const float* pa = &lg[wk][(wm * 32 + lr) * GP + lh];
+  const float* pb = &li[wk][(wn * 32 + lr) * IP + lh];
+  if (first < last) {
+    origins(first);
+#pragma unroll
+    for (int j = 0; j < NG; j++) load_g(j);
+#pragma unroll
+    for (int j = 0; j < NIN; j++) load_in(j);
+  }
+  for (int tile = first; tile < last; tile += WK) {
+    __syncthreads();
+    store();
+    __syncthreads();
+    if (blockIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < WK; k++)
+        for (int q = t % TPC; q < Q; q += TPC) bsum += (double)lg[k][t / TPC * GP + q];
+    }
+    origins(tile + WK);  // (past the end: nothing is loaded)
+    constexpr int STEPS = Q / 2, LG = (NG + STEPS - 1) / STEPS, LI = (NIN + STEPS - 1) / STEPS;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+      const int q = 2 * s;
+      const float va = pa[q];
+#pragma unroll
+      for (int k = 0; k < KK; k++) {
+        const float vb = pb[(q / kWgradW + k / KS) * PW + q % kWgradW + k % KS];
+        acc[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, vb, acc[k], 0, 0, 0);
+      }
+#pragma unroll
+      for (int j = s * LG; j < (s + 1) * LG && j < NG; j++) load_g(j);
+#pragma unroll
+      for (int j = s * LI; j < (s + 1) * LI && j < NIN; j++) load_in(j);
     }
   }
+  float* dst = a.part + (long)(blockIdx.z * WK + wk) * a.Co * a.Ci * KK;
+  const int ci = ci0 + wn * 32 + lr;
+#pragma unroll
+  for (int e = 0; e < 16; e++) {
+    const int co = co0 + wm * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
+    if (co >= a.Co || ci >= a.Ci) continue;
+#pragma unroll
+    for (int k = 0; k < KK; k++) dst[((long)co * a.Ci + ci) * KK + k] = acc[k][e];
+  }
+  if (blockIdx.x == 0) {
+#pragma unroll
+    for (int o = TPC / 2; o > 0; o >>= 1) bsum += __shfl_down(bsum, o, TPC);
+    const int co = co0 + t / TPC;
+    if (t % TPC == 0 && co < a.Co) a.bpart[(long)blockIdx.z * a.Co + co] = bsum;
+  }
 }
 
-// dw = the FP64 sum of the weight-grad partials over the pixel ranges, in
-// range order.
-__global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restrict__ part, int nsplit,
-                                                          long n, float* __restrict__ dw) {
-  for (long i = blockIdx.x * (long)kT + threadIdx.x; i < n; i += (long)gridDim.x * kT) {
+// dw = the FP64 sum of the weight-grad partials, dbias that of the bias
+// partials, in order.
+__global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restrict__ part, int npart,
+                                                          long n, float* __restrict__ dw,
+                                                          const double* __restrict__ bpart,
+                                                          int nbpart, int Co,
+                                                          float* __restrict__ dbias) {
+  for (long i = blockIdx.x * (long)kT + threadIdx.x; i < n + Co; i += (long)gridDim.x * kT) {
     double s = 0.0;
-    for (int r = 0; r < nsplit; r++) s += (double)part[(long)r * n + i];
-    dw[i] = (float)s;
+    if (i < n) {
+      int r = 0;
+      for (; r + 8 <= npart; r += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = part[(long)(r + u) * n + i];
+#pragma unroll
+        for (int u = 0; u < 8; u++) s += (double)v[u];
+      }
+      for (; r < npart; r++) s += (double)part[(long)r * n + i];
+      dw[i] = (float)s;
+    } else {
+      for (int r = 0; r < nbpart; r++) s += bpart[(long)r * Co + (i - n)];
+      dbias[i - n] = (float)s;
+    }
   }
-}
-
-// One workgroup per output channel: dbias[co] = sum g[b][co][:, :].
-__global__ __launch_bounds__(kT) void conv_bwd_bias_kernel(const float* __restrict__ out,
-                                                           const float* __restrict__ dout,
-                                                           float* __restrict__ dbias, int B,
-                                                           int Co, long HW, int relu) {
-  __shared__ double red[kT];
-  const int co = blockIdx.x;
-  double acc = 0.0;
-  const long n = (long)B * HW;
-  for (long i = threadIdx.x; i < n; i += kT) {
-    const long b = i / HW, p = i % HW;
-    acc += (double)relu_grad(out, dout, (b * Co + co) * HW + p, relu);
-  }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int h = kT / 2; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) dbias[co] = (float)red[0];
 }
 
 __global__ __launch_bounds__(kT) void pool_fwd_kernel(const float* __restrict__ in,
@@ -397,6 +523,29 @@ using namespace gvm;
 
 namespace {
 
+template <int MODE, int KS, int MT, int TH, int TW, int CK, class WT>
+void launch_tile(gvm_ctx* ctx, ConvArgs<WT> a) {
+  a.tiles_x = (a.W + TW - 1) / TW;
+  a.tiles_y = (a.H + TH - 1) / TH;
+  const dim3 grid((unsigned)((long)a.tiles_x * a.tiles_y * a.B), (unsigned)((a.M + MT - 1) / MT));
+  hipLaunchKernelGGL((conv_tile_kernel<MODE, KS, MT, TH, TW, CK, WT>), grid, dim3(256), 0,
+                     ctx->stream, a);
+}
+
+// The tile: 8 x 32 pixels and 64 channels (32 where there are no more) when that
+// fills the chip, else 8 x 8 pixels and 64 channels.
+template <int MODE, int KS, class WT>
+void conv_tile(gvm_ctx* ctx, const ConvArgs<WT>& a) {
+  constexpr int CK = KS == 3 ? 8 : 32;
+  const long wide = (long)((a.W + 31) / 32) * ((a.H + 7) / 8) * a.B;
+  if (a.M <= 32)
+    launch_tile<MODE, KS, 32, 8, 32, CK, WT>(ctx, a);
+  else if (wide * ((a.M + 63) / 64) >= 512)
+    launch_tile<MODE, KS, 64, 8, 32, CK, WT>(ctx, a);
+  else
+    launch_tile<MODE, KS, 64, 8, 8, CK, WT>(ctx, a);
+}
+
 template <class WT>
 gvm_status conv_fwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const float* bias,
                            float* out, int B, int Ci, int Co, int H, int W, int K, int relu) {
@@ -406,14 +555,53 @@ gvm_status conv_fwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   GVM_REQUIRE((long)B * H * W < (1L << 31) && (long)Ci * K * K < (1L << 24) &&
                   (long)Co * K * K < (1L << 24),
               "gvm_nn_conv_fwd: sizes beyond the kernels' 32-bit indices");
-  const ConvArgs<WT> a{in, w, bias, nullptr, nullptr, out, B, Ci, Co, H, W, relu};
-  const dim3 grid((unsigned)((B * H * W + kCTile - 1) / kCTile),
-                  (unsigned)((Co + kCTile - 1) / kCTile));
+  const ConvArgs<WT> a{in, nullptr, w, bias, out, B, Co, Ci, H, W, relu, 0, 0};
   if (K == 3)
-    hipLaunchKernelGGL((conv_mfma_kernel<CONV_FWD, 3, WT>), grid, dim3(256), 0, ctx->stream, a);
+    conv_tile<CONV_FWD, 3>(ctx, a);
   else
-    hipLaunchKernelGGL((conv_mfma_kernel<CONV_FWD, 1, WT>), grid, dim3(256), 0, ctx->stream, a);
+    conv_tile<CONV_FWD, 1>(ctx, a);
   return launched("gvm_nn_conv_fwd");
+}
+
+// The weight gradient's launch: how many waves cover channels, and how many
+// partials a sum over the pixels is cut into.
+struct WgradPlan {
+  int wm, wn, wk, sh, tiles_x, tiles_y, ntiles, per, nsplit;
+};
+
+WgradPlan wgrad_plan(int B, int Ci, int Co, int H, int W) {
+  WgradPlan p{};
+  p.wm = Co > 32 ? 2 : 1;
+  p.wn = Ci > 32 ? 2 : 1;
+  p.wk = 4 / (p.wm * p.wn);
+  p.sh = p.wk == 1 ? 4 : 2;
+  p.tiles_x = (W + kWgradW - 1) / kWgradW;
+  p.tiles_y = (H + p.sh - 1) / p.sh;
+  p.ntiles = B * p.tiles_x * p.tiles_y;
+  // about two rounds of one block per CU, partials of at most 8192 pixels (the FP32 sums
+  // stay short), at least four rounds of tiles per block
+  const long blocks = (long)((Co + 32 * p.wm - 1) / (32 * p.wm)) * ((Ci + 32 * p.wn - 1) / (32 * p.wn));
+  const long most = std::max(1L, (long)p.ntiles / (4 * p.wk));
+  const long fill = std::min(most, std::max(1L, 512 / blocks));
+  const long pixels = ((long)p.ntiles * p.sh * kWgradW + 8192L * p.wk - 1) / (8192L * p.wk);
+  const long want = std::max(fill, pixels);
+  p.per = (int)(((p.ntiles + want - 1) / want + p.wk - 1) / p.wk * p.wk);
+  p.nsplit = (p.ntiles + p.per - 1) / p.per;
+  return p;
+}
+
+template <int KS>
+void launch_wgrad(gvm_ctx* ctx, const WgradPlan& p, const WgradArgs& a) {
+  const dim3 grid((unsigned)((a.Ci + 32 * p.wn - 1) / (32 * p.wn)),
+                  (unsigned)((a.Co + 32 * p.wm - 1) / (32 * p.wm)), (unsigned)p.nsplit);
+  if (p.wm == 2 && p.wn == 2)
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 2, 2, 1, 4>), grid, dim3(256), 0, ctx->stream, a);
+  else if (p.wm == 2)
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 2, 1, 2, 2>), grid, dim3(256), 0, ctx->stream, a);
+  else if (p.wn == 2)
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 1, 2, 2, 2>), grid, dim3(256), 0, ctx->stream, a);
+  else
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 1, 1, 4, 2>), grid, dim3(256), 0, ctx->stream, a);
 }
 
 template <class WT>
@@ -428,23 +616,21 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   GVM_REQUIRE((long)B * H * W < (1L << 31) && (long)Ci * K * K < (1L << 24) &&
                   (long)Co * K * K < (1L << 24),
               "gvm_nn_conv_bwd: sizes beyond the kernels' 32-bit indices");
-  const int npix = B * H * W;
+  const float* mask = relu ? out : nullptr;
   if (din) {
-    const ConvArgs<WT> a{in, w, nullptr, out, dout, din, B, Ci, Co, H, W, relu};
-    const dim3 grid((unsigned)((npix + kCTile - 1) / kCTile),
-                    (unsigned)((Ci + kCTile - 1) / kCTile));
+    const ConvArgs<WT> a{dout, mask, w, nullptr, din, B, Ci, Co, H, W, 0, 0, 0};
     if (K == 3)
-      hipLaunchKernelGGL((conv_mfma_kernel<CONV_BWD_DATA, 3, WT>), grid, dim3(256), 0, ctx->stream,
-                         a);
+      conv_tile<CONV_BWD_DATA, 3>(ctx, a);
     else
-      hipLaunchKernelGGL((conv_mfma_kernel<CONV_BWD_DATA, 1, WT>), grid, dim3(256), 0, ctx->stream,
-                         a);
+      conv_tile<CONV_BWD_DATA, 1>(ctx, a);
   }
-  // weight gradient: FP32 partials per range of kWgradPixels pixels in the
-  // context's network workspace, then their FP64 sum in range order
-  const int nsplit = (npix + kWgradPixels - 1) / kWgradPixels;
+  // weight and bias gradients: partials in the context's network workspace (the
+  // bias's first, in FP64), then their FP64 sums
+  const WgradPlan p = wgrad_plan(B, Ci, Co, H, W);
   const long nw = (long)Co * Ci * K * K;
-  const size_t need = (size_t)nsplit * nw;
+  const int npart = p.nsplit * p.wk;
+  const size_t bias_elems = 2 * (size_t)p.nsplit * Co;
+  const size_t need = bias_elems + (size_t)npart * nw;
   if (need > ctx->nn_part_elems) {
     GVM_REQUIRE(!ctx->capturing, "gvm_nn_conv_bwd: the workspace would grow under capture");
     GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -454,21 +640,14 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     GVM_HIP_TRY(hipMalloc((void**)&ctx->nn_part, sizeof(float) * need));
     ctx->nn_part_elems = need;
   }
-  {
-    const ConvArgs<WT> a{in, w, nullptr, out, dout, ctx->nn_part, B, Ci, Co, H, W, relu};
-    const dim3 grid((unsigned)((Ci * K * K + kCTile - 1) / kCTile),
-                    (unsigned)((Co + kCTile - 1) / kCTile), (unsigned)nsplit);
-    if (K == 3)
-      hipLaunchKernelGGL((conv_mfma_kernel<CONV_BWD_WEIGHT, 3, WT>), grid, dim3(256), 0,
-                         ctx->stream, a);
-    else
-      hipLaunchKernelGGL((conv_mfma_kernel<CONV_BWD_WEIGHT, 1, WT>), grid, dim3(256), 0,
-                         ctx->stream, a);
-    hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblocks(nw)), dim3(kT), 0, ctx->stream,
-                       ctx->nn_part, nsplit, nw, dw);
-  }
-  hipLaunchKernelGGL(conv_bwd_bias_kernel, dim3(Co), dim3(kT), 0, ctx->stream, out, dout, dbias, B,
-                     Co, (long)H * W, relu);
+  const WgradArgs a{in,  mask, dout, ctx->nn_part + bias_elems, (double*)ctx->nn_part, B, Ci, Co, H,
+                    W,   p.tiles_x, p.tiles_y, p.ntiles, p.per};
+  if (K == 3)
+    launch_wgrad<3>(ctx, p, a);
+  else
+    launch_wgrad<1>(ctx, p, a);
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblocks(nw + Co)), dim3(kT), 0, ctx->stream, a.part,
+                     npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
   return launched("gvm_nn_conv_bwd");
 }
 
