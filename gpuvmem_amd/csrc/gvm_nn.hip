@@ -46,10 +46,6 @@ __device__ __forceinline__ float wload(const unsigned short* w, long i) {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 enum { CONV_FWD = 0, CONV_BWD_DATA = 1 };
 
-// A plane pitch (floats) of at least n whose multiples by 0 and 1 put two rows
-// of 32 consecutive reads on different LDS banks (64 of 4 bytes).
-constexpr int plane_pitch(int n) { return (n - 32 + 63) / 64 * 64 + 32; }
-
 template <class WT>
 struct ConvArgs {
   const float* in;    // forward: [B][Ci][H][W]; input grad: dout [B][Co][H][W]
@@ -73,13 +69,17 @@ struct ConvArgs {
 template <int MODE, int KS, int MT, int TH, int TW, int CK, class WT>
 __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
   constexpr int KK = KS * KS, P = KS / 2, PH = TH + KS - 1, PW = TW + KS - 1;
-  constexpr int PLANE = plane_pitch(PH * PW), MTP = MT == 32 ? 32 : 96;
+  // a row's pitch in LDS: 32 pixels in rows of 8 on 32 banks
+  constexpr int PP = TW == 8 ? 24 : PW;
+  constexpr int PLANE = PH * PP, MTP = MT + 4;
   constexpr int NBT = TH * TW / 32, WN = NBT < 4 ? NBT : 4, WM = 4 / WN;
   constexpr int NB = NBT / WN, MB = MT / 32 / WM;
   static_assert(NB * WN == NBT && MB * WM * 32 == MT, "four waves share the tile");
   constexpr int NI = (CK * PH * PW + 255) / 256;   // input values per thread
-  constexpr int CP = 256 / MT, NW = CK / CP;       // weights: channels per thread
-  static_assert(NW * CP == CK, "whole channels per thread");
+  // weights: forward, 8 threads take a row (an output channel), whose chunk lies
+  // together in memory; input grad, MT threads a channel, whose rows do
+  constexpr int CP = 256 / MT, NW = CK / CP, KR = CK * KK / 8;
+  static_assert(NW * CP == CK && KR * 8 == CK * KK, "whole channels and rows");
   __shared__ float li[CK * PLANE];
   __shared__ float lw[KK * CK * MTP];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
@@ -97,41 +97,54 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
     off[j] = e < CK * PH * PW && y >= 0 && y < a.H && x >= 0 && x < a.W ? y * a.W + x : -1;
   }
   const long in0 = (long)b * a.C * HW;
-  const int wco = t % MT, wc = t / MT;
-  float ri[NI], rw[NW * KK];
-  auto load = [&](int c0) {
-#pragma unroll
-    for (int j = 0; j < NI; j++) {
+  const int wr = MODE == CONV_FWD ? t & 7 : t % MT, wq = MODE == CONV_FWD ? t >> 3 : t / MT;
+  float ri[NI], rm[NI], rw[NW * KK];
+  // Addresses out of range read element 0 and become zero when they are stored:
+  // no branch keeps the loads of a chunk apart.
+  auto load = [&](int c0, int j) {  // the j-th of a thread's NI + NW * KK values
+    if (j < NI) {
       const int c = c0 + (t + 256 * j) / (PH * PW);
-      ri[j] = 0.0f;
-      if (off[j] >= 0 && c < a.C) {
-        const long i = in0 + (long)c * HW + off[j];
-        if constexpr (MODE == CONV_FWD)
-          ri[j] = a.in[i];
-        else
-          ri[j] = !a.mask || a.mask[i] > 0.0f ? a.in[i] : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < NW; q++) {
-      const int c = c0 + wc + q * CP, m = m0 + wco;
-      const bool ok = m < a.M && c < a.C;
-      // forward: w[m][c][tap]; input grad: w[c][m][tap]
-      const long i = MODE == CONV_FWD ? ((long)m * a.C + c) * KK : ((long)c * a.M + m) * KK;
-#pragma unroll
-      for (int k = 0; k < KK; k++) rw[q * KK + k] = ok ? wload(a.w, i + k) : 0.0f;
+      const long i = off[j] >= 0 && c < a.C ? in0 + (long)c * HW + off[j] : 0;
+      ri[j] = a.in[i];
+      if (MODE == CONV_BWD_DATA && a.mask) rm[j] = a.mask[i];
+    } else if (MODE == CONV_FWD) {  // w[m][c][tap]
+      const int q = (j - NI) / KR, k = (j - NI) % KR, m = m0 + wq + 32 * q;
+      const bool ok = m < a.M && wr + 8 * k < (a.C - c0) * KK;
+      rw[j - NI] = wload(a.w, ok ? ((long)m * a.C + c0) * KK + wr + 8 * k : 0);
+    } else {  // w[c][m][tap]
+      const int q = (j - NI) / KK, k = (j - NI) % KK, c = c0 + wq + q * CP;
+      const bool ok = c < a.C && wr + MT * k < (a.M - m0) * KK;
+      rw[j - NI] = wload(a.w, ok ? ((long)c * a.M + m0) * KK + wr + MT * k : 0);
     }
   };
-  auto store = [&]() {
+  auto store = [&](int c0) {
 #pragma unroll
     for (int j = 0; j < NI; j++) {
       const int e = t + 256 * j;
-      if (e < CK * PH * PW) li[e / (PH * PW) * PLANE + e % (PH * PW)] = ri[j];
+      const bool ok = off[j] >= 0 && c0 + e / (PH * PW) < a.C &&
+                      (MODE == CONV_FWD || !a.mask || rm[j] > 0.0f);
+      if (e < CK * PH * PW)
+        li[e / (PH * PW) * PLANE + e % (PH * PW) / PW * PP + e % PW] = ok ? ri[j] : 0.0f;
     }
+    if constexpr (MODE == CONV_FWD) {
+      const int left = (a.C - c0) * KK;
 #pragma unroll
-    for (int q = 0; q < NW; q++)
+      for (int q = 0; q < MT / 32; q++)
 #pragma unroll
-      for (int k = 0; k < KK; k++) lw[((wc + q * CP) * KK + k) * MTP + wco] = rw[q * KK + k];
+        for (int k = 0; k < KR; k++)
+          lw[(wr + 8 * k) * MTP + wq + 32 * q] =
+              m0 + wq + 32 * q < a.M && wr + 8 * k < left ? rw[q * KR + k] : 0.0f;
+    } else {
+      const int left = (a.M - m0) * KK;
+#pragma unroll
+      for (int q = 0; q < NW; q++)
+#pragma unroll
+        for (int k = 0; k < KK; k++) {
+          const int r = wr + MT * k;
+          lw[((wq + q * CP) * KK + r % KK) * MTP + r / KK] =
+              c0 + wq + q * CP < a.C && r < left ? rw[q * KK + k] : 0.0f;
+        }
+    }
   };
   f32x16_t acc[MB][NB];
 #pragma unroll
@@ -151,34 +164,50 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
 #pragma unroll
       for (int h = 0; h < 2; h++) {
         const int k = 2 * j + h, c = k / KK, tap = MODE == CONV_FWD ? k % KK : KK - 1 - k % KK;
-        place[h] = c * PLANE + tap / KS * PW + tap % KS;
+        place[h] = c * PLANE + tap / KS * PP + tap % KS;
       }
-      pb[j] = li + p / TW * PW + p % TW + (lh ? place[1] : place[0]);
+      pb[j] = li + p / TW * PP + p % TW + (lh ? place[1] : place[0]);
     }
   }
-  constexpr int NSTEP = TW == 32 ? PW : 32 / TW * PW;  // from a pixel block to the next
+  constexpr int NSTEP = TW == 32 ? PP : 32 / TW * PP;  // from a pixel block to the next
   const float* pa = lw + lh * MTP + wm * MB * 32 + lr;
-  load(0);
+  constexpr int STEPS = CK / 2 * KK, NL = NI + NW * KK, LS = (NL + STEPS - 1) / STEPS;
+#pragma unroll
+  for (int j = 0; j < NL; j++) load(0, j);
   for (int c0 = 0; c0 < a.C; c0 += CK) {
     __syncthreads();  // the chunk before has been read
-    store();
+    store(c0);
     __syncthreads();
-    if (c0 + CK < a.C) load(c0 + CK);
+    // the operands of a step are read, and the next chunk's values loaded, while
+    // the step before is multiplied (left to itself the compiler reads operands
+    // right before their use and waits); past the end all loads read element 0
+    float va[2][MB], vb[2][NB];
+    auto read = [&](int i, int at) {
+      const int c = i / KK, j = i % KK;
 #pragma unroll
-    for (int c = 0; c < CK / 2; c++)
+      for (int m = 0; m < MB; m++) va[at][m] = pa[(2 * KK * c + 2 * j) * MTP + m * 32];
 #pragma unroll
-      for (int j = 0; j < KK; j++) {
-        float va[MB], vb[NB];
+      for (int n = 0; n < NB; n++) vb[at][n] = pb[j][2 * c * PLANE + n * NSTEP];
+    };
+    read(0, 0);
 #pragma unroll
-        for (int m = 0; m < MB; m++) va[m] = pa[(2 * KK * c + 2 * j) * MTP + m * 32];
+    for (int i = 0; i < STEPS; i++) {
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int n = 0; n < NB; n++) vb[n] = pb[j][2 * c * PLANE + n * NSTEP];
+      for (int m = 0; m < MB; m++)
 #pragma unroll
-        for (int m = 0; m < MB; m++)
+        for (int n = 0; n < NB; n++) {
+          acc[m][n] =
+              __builtin_amdgcn_mfma_f32_32x32x2f32(va[i & 1][m], vb[i & 1][n], acc[m][n], 0, 0, 0);
+          if (m + n == 0) {
+            if (i + 1 < STEPS) read(i + 1, (i + 1) & 1);
 #pragma unroll
-          for (int n = 0; n < NB; n++)
-            acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[m], vb[n], acc[m][n], 0, 0, 0);
-      }
+            for (int j = 0; j < LS; j++)
+              if (i * LS + j < NL) load(c0 + CK, i * LS + j);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+    }
   }
   // 32 x 32 accumulator layout: lane l, register e -> row 8 (e / 4) + 4 (l / 32)
   // + e % 4, column l % 32
@@ -225,9 +254,13 @@ constexpr int kWgradW = 16;  // pixel columns of a tile
 template <int KS, int WM, int WN, int WK, int SH>
 __global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
   constexpr int KK = KS * KS, P = KS / 2, PW = kWgradW + KS - 1, PH = SH + KS - 1;
-  constexpr int Q = SH * kWgradW, GP = Q + 2, IP = (PH * PW + 3) / 4 * 4 + 2;
+  constexpr int Q = SH * kWgradW, GP = Q + 1, IP = PH * PW | 1;
   static_assert(WM * WN * WK == 4, "four waves");
-  constexpr int NG = WM * 32 * Q * WK / 256, NIN = (WN * 32 * PH * PW * WK + 255) / 256;
+  // A thread keeps its pixel and takes every CG-th (CI-th) channel of it: a load's
+  // address is the tile's plus a constant.
+  constexpr int CG = 256 / Q, CI = 256 / (PH * PW);
+  constexpr int NG1 = WM * 32 / CG, NI1 = (WN * 32 + CI - 1) / CI, NG = NG1 * WK, NIN = NI1 * WK;
+  static_assert(CG * Q == 256 && NG1 * CG == WM * 32, "whole channels per thread");
   __shared__ float lg[WK][WM * 32 * GP];
   __shared__ float li[WK][WN * 32 * IP];
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
@@ -235,50 +268,48 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
   const int HW = a.H * a.W;
   const int co0 = blockIdx.y * WM * 32, ci0 = blockIdx.x * WN * 32;
   const int first = blockIdx.z * a.per, last = min(a.ntiles, first + a.per);
-  static_assert(NG % WK == 0 && NIN * 256 == WN * 32 * PH * PW * WK && NIN % WK == 0,
-                "a thread's j-th value belongs to one tile for every thread");
-  float rg[NG], ri[NIN];
-  // origins of the tiles being loaded (one per WK), and the j-th value of each
-  // operand; the values are loaded between the MFMAs of the tiles before
-  int tx[WK], ty[WK], tb[WK];
-  bool on[WK];
+  const int gq = t % Q, gc = t / Q, ir = t % (PH * PW), ic = t / (PH * PW);
+  float rg[NG], rm[NG], ri[NIN];
+  // this thread's first addresses in the tiles being loaded (one per WK), and
+  // whether its pixel lies inside; the loads go between the MFMAs of the tiles
+  // before.  An address out of range reads element 0 and becomes zero when stored.
+  long ig[WK], ii[WK];
+  bool og[WK], oi[WK];
   auto origins = [&](int tile0) {
 #pragma unroll
     for (int k = 0; k < WK; k++) {
       const int tile = min(tile0 + k, a.ntiles - 1);
-      on[k] = tile0 + k < last;
-      tx[k] = tile % a.tiles_x * kWgradW;
-      ty[k] = tile / a.tiles_x % a.tiles_y * SH;
-      tb[k] = tile / a.tiles_x / a.tiles_y;
+      const int tx = tile % a.tiles_x * kWgradW, ty = tile / a.tiles_x % a.tiles_y * SH;
+      const long tb = tile / a.tiles_x / a.tiles_y;
+      const int gx = tx + gq % kWgradW, gy = ty + gq / kWgradW;
+      const int ix = tx + ir % PW - P, iy = ty + ir / PW - P;
+      og[k] = tile0 + k < last && gx < a.W && gy < a.H;
+      oi[k] = tile0 + k < last && ic < CI && ix >= 0 && ix < a.W && iy >= 0 && iy < a.H;
+      ig[k] = (tb * a.Co + co0 + gc) * HW + gy * a.W + gx;
+      ii[k] = (tb * a.Ci + ci0 + ic) * HW + iy * a.W + ix;
     }
   };
   auto load_g = [&](int j) {
-    const int k = j / (NG / WK), e = t + 256 * (j % (NG / WK)), q = e % Q, co = co0 + e / Q;
-    const int x = tx[k] + q % kWgradW, y = ty[k] + q / kWgradW;
-    rg[j] = 0.0f;
-    if (on[k] && co < a.Co && x < a.W && y < a.H) {
-      const long i = ((long)tb[k] * a.Co + co) * HW + y * a.W + x;
-      rg[j] = !a.out || a.out[i] > 0.0f ? a.dout[i] : 0.0f;
-    }
+    const int k = j / NG1, c = j % NG1 * CG;
+    const long i = og[k] && co0 + gc + c < a.Co ? ig[k] + (long)c * HW : 0;
+    rg[j] = a.dout[i];
+    if (a.out) rm[j] = a.out[i];
   };
   auto load_in = [&](int j) {
-    const int k = j / (NIN / WK), e = t + 256 * (j % (NIN / WK)), r = e % (PH * PW);
-    const int ci = ci0 + e / (PH * PW);
-    const int x = tx[k] + r % PW - P, y = ty[k] + r / PW - P;
-    ri[j] = 0.0f;
-    if (on[k] && ci < a.Ci && x >= 0 && x < a.W && y >= 0 && y < a.H)
-      ri[j] = a.in[((long)tb[k] * a.Ci + ci) * HW + y * a.W + x];
+    const int k = j / NI1, c = j % NI1 * CI;
+    ri[j] = a.in[oi[k] && ci0 + ic + c < a.Ci ? ii[k] + (long)c * HW : 0];
   };
   auto store = [&]() {
 #pragma unroll
     for (int j = 0; j < NG; j++) {
-      const int e = t + 256 * (j % (NG / WK));
-      lg[j / (NG / WK)][e / Q * GP + e % Q] = rg[j];
+      const int k = j / NG1, c = gc + j % NG1 * CG;
+      lg[k][c * GP + gq] = og[k] && co0 + c < a.Co && (!a.out || rm[j] > 0.0f) ? rg[j] : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < NIN; j++) {
-      const int e = t + 256 * (j % (NIN / WK));
-      li[j / (NIN / WK)][e / (PH * PW) * IP + e % (PH * PW)] = ri[j];
+      const int k = j / NI1, c = ic + j % NI1 * CI;
+      if (ic < CI && c < WN * 32)
+        li[k][c * IP + ir] = oi[k] && ci0 + c < a.Ci ? ri[j] : 0.0f;
     }
   };
   f32x16_t acc[KK];
@@ -309,20 +340,29 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
     }
     origins(tile + WK);  // (past the end: nothing is loaded)
     constexpr int STEPS = Q / 2, LG = (NG + STEPS - 1) / STEPS, LI = (NIN + STEPS - 1) / STEPS;
-#pragma unroll
-    for (int s = 0; s < STEPS; s++) {
+    // between two MFMAs: a value of the step after, and loads of the tiles after
+    float va[2], vb[2][KK];
+    auto read = [&](int s, int k) {
       const int q = 2 * s;
-      const float va = pa[q];
+      if (k == 0) va[s & 1] = pa[q];
+      vb[s & 1][k] = pb[(q / kWgradW + k / KS) * PW + q % kWgradW + k % KS];
+    };
+#pragma unroll
+    for (int k = 0; k < KK; k++) read(0, k);
+#pragma unroll
+    for (int s = 0; s < STEPS; s++)
 #pragma unroll
       for (int k = 0; k < KK; k++) {
-        const float vb = pb[(q / kWgradW + k / KS) * PW + q % kWgradW + k % KS];
-        acc[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, vb, acc[k], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[s & 1], vb[s & 1][k], acc[k], 0, 0, 0);
+        if (s + 1 < STEPS) read(s + 1, k);
+#pragma unroll
+        for (int q = k; q < LG + LI; q += KK) {
+          if (q < LG && s * LG + q < NG) load_g(s * LG + q);
+          if (q >= LG && s * LI + q - LG < NIN) load_in(s * LI + q - LG);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-      for (int j = s * LG; j < (s + 1) * LG && j < NG; j++) load_g(j);
-#pragma unroll
-      for (int j = s * LI; j < (s + 1) * LI && j < NIN; j++) load_in(j);
-    }
   }
   float* dst = a.part + (long)(blockIdx.z * WK + wk) * a.Co * a.Ci * KK;
   const int ci = ci0 + wn * 32 + lr;
@@ -341,31 +381,47 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
   }
 }
 
-// dw = the FP64 sum of the weight-grad partials, dbias that of the bias
-// partials, in order.
+// dw = the FP64 sum of the weight-grad partials, dbias that of the bias partials,
+// in a fixed order: SEG threads take a run of an element's partials each, and their
+// sums are added in order.  (One thread per element leaves most of the chip idle
+// where there are many partials of few weights: 9216 weights of 2048 partials took
+// 152 us.)
+template <int SEG>
 __global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restrict__ part, int npart,
                                                           long n, float* __restrict__ dw,
                                                           const double* __restrict__ bpart,
                                                           int nbpart, int Co,
                                                           float* __restrict__ dbias) {
-  for (long i = blockIdx.x * (long)kT + threadIdx.x; i < n + Co; i += (long)gridDim.x * kT) {
-    double s = 0.0;
-    if (i < n) {
-      int r = 0;
-      for (; r + 8 <= npart; r += 8) {
-        float v[8];
+  constexpr int E = kT / SEG;  // elements of a block
+  __shared__ double seg[SEG][E];
+  const int e = threadIdx.x % E, sg = threadIdx.x / E;
+  const long i = (long)blockIdx.x * E + e;
+  double s = 0.0;
+  if (i < n) {
+    const int per = (npart + SEG - 1) / SEG, last = min(npart, (sg + 1) * per);
+    int r = sg * per;
+    for (; r + 8 <= last; r += 8) {
+      float v[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = part[(long)(r + u) * n + i];
+      for (int u = 0; u < 8; u++) v[u] = part[(long)(r + u) * n + i];
 #pragma unroll
-        for (int u = 0; u < 8; u++) s += (double)v[u];
-      }
-      for (; r < npart; r++) s += (double)part[(long)r * n + i];
-      dw[i] = (float)s;
-    } else {
-      for (int r = 0; r < nbpart; r++) s += bpart[(long)r * Co + (i - n)];
-      dbias[i - n] = (float)s;
+      for (int u = 0; u < 8; u++) s += (double)v[u];
     }
+    for (; r < last; r++) s += (double)part[(long)r * n + i];
+  } else if (i < n + Co) {
+    const int per = (nbpart + SEG - 1) / SEG, last = min(nbpart, (sg + 1) * per);
+    for (int r = sg * per; r < last; r++) s += bpart[(long)r * Co + (i - n)];
   }
+  if constexpr (SEG > 1) {
+    seg[sg][e] = s;
+    __syncthreads();
+    if (sg) return;
+    for (int q = 1; q < SEG; q++) s += seg[q][e];
+  }
+  if (i < n)
+    dw[i] = (float)s;
+  else if (i < n + Co)
+    dbias[i - n] = (float)s;
 }
 
 __global__ __launch_bounds__(kT) void pool_fwd_kernel(const float* __restrict__ in,
@@ -571,8 +627,9 @@ struct WgradPlan {
 
 WgradPlan wgrad_plan(int B, int Ci, int Co, int H, int W) {
   WgradPlan p{};
-  p.wm = Co > 32 ? 2 : 1;
-  p.wn = Ci > 32 ? 2 : 1;
+  const int nco = (Co + 31) / 32, nci = (Ci + 31) / 32;
+  p.wm = nco % 2 == 0 || nco > 4 ? 2 : 1;
+  p.wn = nci % 2 == 0 || nci > 4 ? 2 : 1;
   p.wk = 4 / (p.wm * p.wn);
   p.sh = p.wk == 1 ? 4 : 2;
   p.tiles_x = (W + kWgradW - 1) / kWgradW;
@@ -646,8 +703,12 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     launch_wgrad<3>(ctx, p, a);
   else
     launch_wgrad<1>(ctx, p, a);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblocks(nw + Co)), dim3(kT), 0, ctx->stream, a.part,
-                     npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
+  if (npart >= 32)
+    hipLaunchKernelGGL(wgrad_reduce_kernel<8>, dim3((unsigned)((nw + Co + kT / 8 - 1) / (kT / 8))),
+                       dim3(kT), 0, ctx->stream, a.part, npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
+  else
+    hipLaunchKernelGGL(wgrad_reduce_kernel<1>, dim3((unsigned)((nw + Co + kT - 1) / kT)), dim3(kT), 0,
+                       ctx->stream, a.part, npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
   return launched("gvm_nn_conv_bwd");
 }
 
