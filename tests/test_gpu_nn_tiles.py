@@ -1,0 +1,121 @@
+"""The network kernels where their tiles end: channels and pixels that are no
+multiple of a tile, each shape of tile and of weight-gradient block, FP32 and
+BF16 weights, against the same layers in FP64."""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from gpuvmem_amd import native
+from gpuvmem_amd.device import Context, DeviceBuffer
+from gpuvmem_amd.problem import small_problem
+
+pytestmark = pytest.mark.gpu
+EPS = 2.0 ** -24
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(small_problem(npix=64, n_antennas=5, seed=41), add_data=False)
+    yield c
+    c.close()
+
+
+def _dev(t):
+    return DeviceBuffer.from_array(np.ascontiguousarray(t.numpy(), np.float32))
+
+
+def _get(buf, shape):
+    n = int(np.prod(shape))
+    return torch.from_numpy(buf.download(np.float32)[:n].reshape(shape).astype(np.float64))
+
+
+def _within(got, ref, size, n):
+    """A sum of n FP32 products is off by at most n units of rounding of the sum of
+    their magnitudes; two more for the bias and the result."""
+    assert torch.isfinite(got).all()
+    assert ((got - ref).abs() <= (n + 2) * EPS * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("B,Ci,Co,H,W,K,relu,bf16", [
+    (1, 9, 33, 9, 35, 3, True, False),     # 8 x 8 tiles forward; 32 + 64 channel blocks
+    (2, 40, 20, 11, 17, 3, True, True),
+    (1, 64, 40, 9, 33, 3, False, True),    # pairs of both channels
+    (1, 161, 5, 8, 16, 3, True, True),     # more than four groups of input channels
+    (1, 1, 1, 1, 1, 3, False, False),
+    (2, 3, 65, 126, 510, 3, True, True),   # 8 x 32 tiles of 64 channels, forward
+    (2, 65, 3, 126, 510, 3, True, False),  # and for the input gradient
+    (1, 33, 5, 9, 33, 1, True, True),
+    (2, 5, 70, 8, 31, 1, False, False),
+    (2, 3, 65, 126, 510, 1, True, True),
+])
+def test_convolutions_at_the_edges_of_tiles(ctx, B, Ci, Co, H, W, K, relu, bf16):
+    print(f"case: conv {B} {Ci}->{Co} {H}x{W} K={K} relu={relu} bf16={bf16}", flush=True)
+    g = torch.Generator().manual_seed(Ci * 1000 + Co)
+    x = torch.randn(B, Ci, H, W, generator=g)
+    w = torch.randn(Co, Ci, K, K, generator=g) * 0.3
+    if bf16:
+        w = w.bfloat16().float()
+    b = torch.randn(Co, generator=g)
+    dy = torch.randn(B, Co, H, W, generator=g)
+    dx, dw, db, ddy = _dev(x), _dev(w), _dev(b), _dev(dy)
+    if bf16:
+        full, dw = dw, DeviceBuffer(2 * w.numel())
+        native.check(ctx.lib.gvm_nn_to_bf16(ctx.ctx, full.ptr, dw.ptr, w.numel()), "to_bf16")
+    fwd = ctx.lib.gvm_nn_conv_fwd_bf16 if bf16 else ctx.lib.gvm_nn_conv_fwd
+    bwd = ctx.lib.gvm_nn_conv_bwd_bf16 if bf16 else ctx.lib.gvm_nn_conv_bwd
+    out = ctx.zeros(dy.numel())
+    native.check(fwd(ctx.ctx, dx.ptr, dw.ptr, db.ptr, out.ptr, B, Ci, Co, H, W, K, int(relu)), "fwd")
+    din, dwg, dbg = ctx.zeros(x.numel()), ctx.zeros(w.numel()), ctx.zeros(Co)
+    native.check(bwd(ctx.ctx, dx.ptr, dw.ptr, out.ptr if relu else None, ddy.ptr, din.ptr, dwg.ptr,
+                     dbg.ptr, B, Ci, Co, H, W, K, int(relu)), "bwd")
+    ctx.sync()
+    x, w, b, dy = (t.double() for t in (x, w, b, dy))
+    y = _get(out, dy.shape)
+    ref = F.conv2d(x, w, b, padding=K // 2)
+    size = F.conv2d(x.abs(), w.abs(), b.abs(), padding=K // 2)
+    _within(y, ref.clamp(min=0.0) if relu else ref, size, Ci * K * K)
+    if relu:
+        dy = dy * (y > 0.0)
+    back = torch.nn.grad
+    _within(_get(din, x.shape), back.conv2d_input(x.shape, w, dy, padding=K // 2),
+            back.conv2d_input(x.shape, w.abs(), dy.abs(), padding=K // 2), Co * K * K)
+    # FP32 sums of at most 8192 pixels, then FP64
+    n = min(B * H * W, 8192)
+    _within(_get(dwg, w.shape), back.conv2d_weight(x, w.shape, dy, padding=K // 2),
+            back.conv2d_weight(x.abs(), w.shape, dy.abs(), padding=K // 2), n)
+    _within(_get(dbg, b.shape), dy.sum((0, 2, 3)), dy.abs().sum((0, 2, 3)), 1)
+
+
+@pytest.mark.parametrize("H,W,shift", [(2, 2, 0), (6, 4, 0), (34, 66, 0), (18, 20, 1), (2, 1028, 3)])
+def test_plane_kernels_at_every_alignment(ctx, H, W, shift):
+    """Wide and narrow accesses: rows of 2 mod 4 pixels, pointers `shift` floats
+    past the alignment of an allocation."""
+    print(f"case: planes {H}x{W} shift={shift}", flush=True)
+    B, Cc, Cd, lib = 2, 3, 5, ctx.lib
+    x = torch.randn(B, Cc, H, W, generator=torch.Generator().manual_seed(H * W))
+    src = DeviceBuffer.from_array(np.concatenate([np.zeros(shift, np.float32), x.numpy().ravel()]))
+    h, w = H // 2, W // 2
+
+    def run(fn, shape, *args):
+        buf = ctx.zeros(shift + int(np.prod(shape)) + 4)
+        native.check(fn(ctx.ctx, src.ptr + 4 * shift, buf.ptr + 4 * shift, *args), "plane")
+        ctx.sync()
+        n = int(np.prod(shape))
+        a = buf.download(np.float32)
+        assert not a[:shift].any() and not a[shift + n:].any()
+        return torch.from_numpy(a[shift:shift + n].reshape(shape).copy())
+
+    got = run(lib.gvm_nn_pool_fwd, (B, Cc, h, w), B, Cc, H, W)
+    assert torch.allclose(got, F.avg_pool2d(x, 2), rtol=0, atol=4 * EPS * float(x.abs().max()))
+    got = run(lib.gvm_nn_up_fwd, (B, Cd, 2 * H, 2 * W), B, Cc, Cd, 1, H, W)
+    up = x.repeat_interleave(2, 2).repeat_interleave(2, 3)
+    assert torch.equal(got[:, 1:4], up) and not got[:, 0].any() and not got[:, 4].any()
+    # x as the gradient of a pooled 2H x 2W image, and of one upsampled from h x w
+    got = run(lib.gvm_nn_pool_bwd, (B, Cc, 2 * H, 2 * W), B, Cc, 2 * H, 2 * W)
+    assert torch.equal(got, 0.25 * up)
+    got = run(lib.gvm_nn_up_bwd, (B, 2, h, w), B, 2, Cc, 1, h, w)
+    assert torch.allclose(got, 4.0 * F.avg_pool2d(x[:, 1:], 2), rtol=0,
+                          atol=16 * EPS * float(x.abs().max()))
+    got = run(lib.gvm_nn_copy_channels, (B, Cd, H, W), B, 2, Cc, 1, Cd, 2, H * W)
+    assert torch.equal(got[:, 2:4], x[:, 1:]) and not got[:, :2].any() and not got[:, 4].any()
