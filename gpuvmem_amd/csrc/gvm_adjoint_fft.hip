@@ -59,6 +59,7 @@ constexpr double kPi = 3.14159265358979323846;
 constexpr int kTaps = 9;                 // kernel width in cells of the 2N grid
 constexpr double kPlaneTol = 5e-8;       // truncation of the w expansion
 constexpr int kMaxPlanes = 32;
+constexpr int kMaxTerms = 40;            // of a plane weight's series (32 planes need 31)
 constexpr int kPlaneGroup = 8;           // planes one spread launch accumulates
 constexpr int kSub = 512;                // floats of a 16 x 16 complex subgrid
 constexpr long kGroupRows = 1L << 27;    // rows sorted together at set-up
@@ -214,8 +215,11 @@ __global__ __launch_bounds__(256) void item_counts_kernel(const unsigned int* __
   }
 }
 
-// Items of tile k at [islot[k], islot[k + 1]): (first row, rows, slice, 0);
-// islot[k] becomes tile_slot[k] (-1 for a tile without rows); merge mslot[k]
+// Items of tile k at [islot[k], islot[k + 1]): (first row, rows, slice, .); .w of
+// item i of a slice is the item to take i-th: those of half a chunk or
+// more first, so that short ones fill the launch's end (which of two comes first
+// does not matter).  full[], rest[]: how many of a slice have been placed.  islot[k]
+// becomes tile_slot[k] (-1 for a tile without rows); merge mslot[k]
 // is tile k's when it has several items.
 __global__ __launch_bounds__(256) void items_kernel(const unsigned int* __restrict__ start,
                                                     const unsigned int* __restrict__ islot,
@@ -223,6 +227,8 @@ __global__ __launch_bounds__(256) void items_kernel(const unsigned int* __restri
                                                     long nkeys, int chunk, long row0,
                                                     unsigned int ntiles, int s0,
                                                     unsigned int item0, unsigned int merge0,
+                                                    unsigned int* __restrict__ full,
+                                                    unsigned int* __restrict__ rest,
                                                     long4* __restrict__ items,
                                                     int2* __restrict__ merges,
                                                     int* __restrict__ tile_slot) {
@@ -236,9 +242,15 @@ __global__ __launch_bounds__(256) void items_kernel(const unsigned int* __restri
       long4 it;
       it.x = row0 + b;
       it.y = min((long)chunk, last - b);
-      it.z = s0 + (long)(k / ntiles);
-      it.w = 0;
-      items[i - item0] = it;
+      const unsigned int s = (unsigned int)(k / ntiles);
+      it.z = s0 + (long)s;
+      long4* o = items + (i - item0);
+      o->x = it.x;
+      o->y = it.y;
+      o->z = it.z;
+      const unsigned int at = it.y >= chunk / 2 ? islot[(long)s * ntiles] + atomicAdd(full + s, 1u)
+                                                : islot[(long)(s + 1) * ntiles] - 1 - atomicAdd(rest + s, 1u);
+      items[at - item0].w = (long)i;
     }
   }
 }
@@ -263,17 +275,15 @@ __global__ void pick_kernel(const unsigned int* __restrict__ islot,
 // instructions: at NP = 4 the MFMA pipe bounds it, 64 cycles per visibility,
 // 54 us of the chip for 1.76 M visibilities at 2 GHz.
 template <int NP>
-__global__ __launch_bounds__(256) void spread_kernel(
-    const long4* __restrict__ items, int nitems, const float4* __restrict__ rec,
+__global__ __launch_bounds__(64) void spread_kernel(
+    const long4* __restrict__ items, long slot0, const float4* __restrict__ rec,
     const uint2* __restrict__ meta, const float2* __restrict__ rot,
     const SliceDev* __restrict__ tab, const unsigned int* __restrict__ cmaxs, double inv_w, int k0,
     int nplanes, float* __restrict__ part) {
-  __shared__ float4 sa[4][64];  // (dx, dy, c)
-  __shared__ float2 sb[4][64];  // the row's cell within the subgrid
-  __shared__ float st[4][64][(NP + 3) / 4 * 4];  // T_k0 .. of each row
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int item = blockIdx.x * 4 + wave;
-  if (item >= nitems) return;
+  __shared__ float4 sa[64];  // (dx, dy, c)
+  __shared__ float2 sb[64];  // the row's cell within the subgrid
+  __shared__ float st[64][(NP + 3) / 4 * 4];  // T_k0 .. of each row
+  const int lane = threadIdx.x, item = (int)(items[blockIdx.x].w - slot0);
   const long4 it = items[item];
   const float2* __restrict__ vr = tab[it.z].vr;
   const float scale = ldexpf(1.0f, p_scale_exponent(__uint_as_float(cmaxs[it.z])));
@@ -325,8 +335,8 @@ __global__ __launch_bounds__(256) void spread_kernel(
       load_row(b + 128 + lane, &rn, &mn);
     }
     __builtin_amdgcn_wave_barrier();
-    sa[wave][lane] = a;
-    sb[wave][lane] = c;
+    sa[lane] = a;
+    sb[lane] = c;
     double ta = 1.0, tb = t;
     for (int k = 0; k < k0; k++) {
       const double tn = 2.0 * t * tb - ta;
@@ -335,27 +345,59 @@ __global__ __launch_bounds__(256) void spread_kernel(
     }
 #pragma unroll
     for (int k = 0; k < NP; k++) {
-      st[wave][lane][k] = (float)ta;
+      st[lane][k] = (float)ta;
       const double tn = 2.0 * t * tb - ta;
       ta = tb;
       tb = tn;
     }
     __builtin_amdgcn_wave_barrier();
-    for (int s = 0; s < cnt; s += 4) {
-      const int j = s + (lane >> 4);
-      const float4 va = sa[wave][j];
-      const float2 vb = sb[wave][j];
+    // eight rows per turn: while four are multiplied the operands of the next four
+    // are formed, from LDS values read a step before that (rows past cnt are zero)
+    float4 va;
+    float2 vb;
+    float vt[NP], ky[2], br[2][NP], bi[2][NP];
+    auto fetch = [&](int s) {
+      const int j = (s & 63) + (lane >> 4);
+      va = sa[j];
+      vb = sb[j];
+#pragma unroll
+      for (int k = 0; k < NP; k++) vt[k] = st[j][k];
+    };
+    auto operands = [&](int h) {
       const float kx = spread_value((q - vb.x) - va.x);
-      const float ky = spread_value((q - vb.y) - va.y);
+      ky[h] = spread_value((q - vb.y) - va.y);
       const float ux = kx * va.z, ui = kx * va.w;
 #pragma unroll
       for (int k = 0; k < NP; k++) {
         // even planes grid c T_k, odd ones -i c T_k
-        const float tk = st[wave][j][k];
-        const float br = (k & 1) ? ui * tk : ux * tk;
-        const float bi = (k & 1) ? -(ux * tk) : ui * tk;
-        re[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky, br, re[k], 0, 0, 0);
-        im[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky, bi, im[k], 0, 0, 0);
+        br[h][k] = (k & 1) ? ui * vt[k] : ux * vt[k];
+        bi[h][k] = (k & 1) ? -(ux * vt[k]) : ui * vt[k];
+      }
+    };
+    auto multiply = [&](int h) {
+#pragma unroll
+      for (int k = 0; k < NP; k++) {
+        re[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky[h], br[h][k], re[k], 0, 0, 0);
+        im[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ky[h], bi[h][k], im[k], 0, 0, 0);
+      }
+    };
+    fetch(0);
+    operands(0);
+    fetch(4);
+    for (int s = 0; s < cnt; s += 8) {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(h);
+        operands(1 - h);
+        fetch(s + 4 * h + 8);
+#pragma unroll
+        for (int k = 0; k < 2 * NP; k++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);            // MFMA
+          __builtin_amdgcn_sched_group_barrier(0x002, 40 / (2 * NP) + 2, 0);  // VALU
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // LDS reads
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
@@ -408,10 +450,12 @@ __global__ __launch_bounds__(256) void merge_kernel(const int2* __restrict__ mer
 // sum of up to four subgrids.
 
 // Four of the columns beyond an end of the half grid (X < 0 or X > N), folded:
-// minus the conjugate cell (mx, -Y).
+// minus the conjugate cell (mx, -Y).  ss: the slots of tile columns txb and txb - 1,
+// which hold these cells too.
+template <int N>
 __device__ __forceinline__ float2 folded_cell(const float2* __restrict__ part,
-                                              const int* __restrict__ slot, int slot0, int N,
-                                              int nplanes, int plane, int mx, int Y) {
+                                              const int (*ss)[N / 4], int txb, int nplanes,
+                                              int plane, int mx, int Y) {
   const int nty = N / 4, tx = (mx + 4) >> 3;
   const int My = -Y & (2 * N - 1);
   const int ty = ((My + 4) >> 3) & (nty - 1), c = (mx + 4) & 7, r = (My + 4) & 7;
@@ -419,10 +463,10 @@ __device__ __forceinline__ float2 folded_cell(const float2* __restrict__ part,
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int tc = tx - (u >> 1);
-    if (tc < 0 || tc > N / 8) continue;
-    const int i = slot[tc * nty + ((ty - (u & 1)) & (nty - 1))];
+    if (tc < 0 || tc > N / 8 || tc > txb || tc < txb - 1) continue;
+    const int i = ss[txb - tc][(ty - (u & 1)) & (nty - 1)];
     if (i < 0) continue;
-    const float2 v = part[((long)(i - slot0) * nplanes + plane) * (kSub / 2) + (u >> 1) * 128 +
+    const float2 v = part[((long)i * nplanes + plane) * (kSub / 2) + (u >> 1) * 128 +
                           (r + (u & 1) * 8) * 8 + c];
     s.x += v.x;
     s.y -= v.y;
@@ -443,15 +487,16 @@ __global__ __launch_bounds__(T) void grid_cols_kernel(const float2* __restrict__
   constexpr int L = 2 * N, NTY = N / 4, CP = BC / 2;
   __shared__ float2 lds[BC * L];
   __shared__ int ss[2][NTY];
-  // consecutive column blocks, which write the same lines of H, on one XCD
-  const int per = gridDim.x / 8;
-  const int X0 = ((blockIdx.x % 8) * per + blockIdx.x / 8) * BC;
-  if (X0 > N) return;
+  // consecutive column blocks, which write the same lines of H, on one XCD; column
+  // N by itself (33 blocks on every XCD for 257 would take a third round)
+  constexpr int PER = N / BC / 8;
+  const int X0 = blockIdx.x < N / BC ? ((blockIdx.x % 8) * PER + blockIdx.x / 8) * BC : N;
   const int plane = blockIdx.y, sl = blockIdx.z;
   const int* slot = tile_slot + (long)sl * (N / 8 + 1) * NTY;
   const int tx = (X0 + 4) >> 3;
   // a block without any row's subgrid needs no transform
-  int any = X0 <= 4 || X0 + BC - 1 >= N - 4;
+  // (cells beyond either end of the half grid lie in the same two tile columns)
+  int any = 0;
   for (int y = threadIdx.x; y < 2 * NTY; y += T) {
     const int h = y / NTY, t = tx - h;
     const int s = t >= 0 && t <= N / 8 ? slot[t * NTY + y % NTY] : -1;
@@ -501,7 +546,7 @@ __global__ __launch_bounds__(T) void grid_cols_kernel(const float2* __restrict__
         const int X = X0 + idx % BC, Y = idx / BC;
         const int mx = X >= 1 && X <= 4 ? -X : X >= N - 4 && X < N ? L - X : 0;
         if (mx == 0) continue;
-        const float2 m = folded_cell(part, slot, slot0, N, nplanes, plane, mx, Y);
+        const float2 m = folded_cell<N>(part, ss, tx, nplanes, plane, mx, Y);
         lds[idx].x += m.x;
         lds[idx].y += m.y;
       }
@@ -554,20 +599,17 @@ __device__ __forceinline__ float chain_rule(float r, float d, float nudiv, float
   return r;
 }
 
-// Weight of a plane at a pixel, over zeta^k: its power series in zeta^2.
-__device__ __forceinline__ double plane_series(const double* __restrict__ c, int terms,
-                                               double zeta2) {
-  double s = c[terms - 1];
-  for (int m = terms - 2; m >= 0; m--) s = fma(s, zeta2, c[m]);
-  return s;
-}
-
 // One block per image row; B planes are transformed together.  The transform
 // of 2N real values from N + 1 complex ones runs as one complex transform of N
-// points (even outputs in the real part, odd ones in the imaginary part).
+// points (even outputs in the real part, odd ones in the imaginary part), whose
+// inputs X and N - X need the same two values.  A plane's weight at a pixel is
+// zeta^k times a power series in zeta^2; the series' coefficients are read from
+// LDS, once for all of a thread's pixels (from memory, per pixel, they were two
+// thirds of the kernel's loads and took 310 us at 2048^2 with 6 planes).
 template <int N, int B, int T>
-__global__ __launch_bounds__(T) void grid_rows_kernel(RowsArgs a) {
+__global__ __launch_bounds__(T, 4) void grid_rows_kernel(RowsArgs a) {
   __shared__ float2 lds[B * N];
+  __shared__ double sc[B * kMaxTerms];
   constexpr int PP = (N / 2 + T - 1) / T;  // column pairs per thread
   const int i = blockIdx.x;
   const long n = (long)N * N;
@@ -595,11 +637,13 @@ __global__ __launch_bounds__(T) void grid_rows_kernel(RowsArgs a) {
       zeta[u][e] = a.wz * (-r2 / (1.0 + sqrt(fmax(0.0, 1.0 - r2))));
     }
   const int s = blockIdx.y;
-  double g[PP][2], zk[PP][2];
+  double g[PP][2], zk[PP][2], z2[PP][2];
 #pragma unroll
   for (int u = 0; u < PP; u++) {
     g[u][0] = g[u][1] = 0.0;
     zk[u][0] = zk[u][1] = 1.0;  // zeta^k
+    z2[u][0] = zeta[u][0] * zeta[u][0];
+    z2[u][1] = zeta[u][1] * zeta[u][1];
   }
   for (int k0 = 0; k0 < a.nplanes; k0 += B) {
     __syncthreads();  // the previous group's outputs have been read
@@ -607,37 +651,53 @@ __global__ __launch_bounds__(T) void grid_rows_kernel(RowsArgs a) {
     for (int b = 0; b < B; b++) {
       const int k = k0 + b;
       const float2* h = a.H + (((long)s * a.nplanes + min(k, a.nplanes - 1)) * N + i) * a.pitch;
-#pragma unroll 4
-      for (int X = threadIdx.x; X < N; X += T) {
+#pragma unroll
+      for (int u = 0; u < PP; u++) {
+        const int X = threadIdx.x + u * T;
+        if (X >= N / 2) break;
         float2 f = h[X], m = h[N - X];
+        float2 z, y;  // inputs X and N - X; for X = 0: inputs 0 and N / 2
         if (X == 0) {
-          f = make_float2(f.x, 0.f);
-          m = make_float2(m.x, 0.f);
+          const float2 c = h[N / 2];
+          z = make_float2(f.x + m.x, f.x - m.x);
+          y = make_float2(c.x, -c.y);
         } else {
           f = make_float2(0.5f * f.x, 0.5f * f.y);
           m = make_float2(0.5f * m.x, -0.5f * m.y);
+          const float2 d = cmul(make_float2(f.x - m.x, f.y - m.y), a.tw2[X]);
+          const float2 e = make_float2(f.x + m.x, f.y + m.y);
+          z = make_float2(e.x - d.y, e.y + d.x);
+          y = make_float2(e.x + d.y, d.x - e.y);
         }
-        const float2 d = cmul(make_float2(f.x - m.x, f.y - m.y), a.tw2[X]);
-        lds[b * N + X] = k < a.nplanes ? make_float2((f.x + m.x) - d.y, (f.y + m.y) + d.x)
-                                       : make_float2(0.f, 0.f);
+        const bool in = k < a.nplanes;
+        lds[b * N + X] = in ? z : make_float2(0.f, 0.f);
+        lds[b * N + (X ? N - X : N / 2)] = in ? y : make_float2(0.f, 0.f);
       }
     }
+    for (int c = threadIdx.x; c < B * a.terms; c += T)
+      sc[c] = k0 * a.terms + c < a.nplanes * a.terms ? a.wcoef[k0 * a.terms + c] : 0.0;
     __syncthreads();
     fft_lds<N, B, false, T>(lds, a.tw);
+    for (int b = 0; b < B && k0 + b < a.nplanes; b++) {
+      const double* c = sc + b * a.terms;
+      double w[PP][2];
 #pragma unroll
-    for (int u = 0; u < PP; u++) {
-      const int cp = threadIdx.x + u * T;
-      if (cp < N / 2 && (on[u][0] || on[u][1])) {
-        const int j = (cp - N / 4) & (N - 1);
-        for (int b = 0; b < B && k0 + b < a.nplanes; b++) {
-          const float2 z = lds[b * N + j];
-          const double* c = a.wcoef + (k0 + b) * a.terms;
+      for (int u = 0; u < PP; u++) w[u][0] = w[u][1] = c[a.terms - 1];
+      for (int m = a.terms - 2; m >= 0; m--) {
+        const double cm = c[m];
 #pragma unroll
-          for (int e = 0; e < 2; e++) {
-            const double zt = zeta[u][e];
-            g[u][e] += (double)(e ? z.y : z.x) * zk[u][e] * plane_series(c, a.terms, zt * zt);
-            zk[u][e] *= zt;
-          }
+        for (int u = 0; u < PP; u++)
+#pragma unroll
+          for (int e = 0; e < 2; e++) w[u][e] = fma(w[u][e], z2[u][e], cm);
+      }
+#pragma unroll
+      for (int u = 0; u < PP; u++) {
+        const int cp = threadIdx.x + u * T;
+        const float2 z = lds[b * N + ((cp - N / 4) & (N - 1))];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          g[u][e] += (double)(e ? z.y : z.x) * zk[u][e] * w[u][e];
+          zk[u][e] *= zeta[u][e];
         }
       }
     }
@@ -755,13 +815,13 @@ namespace {
 struct PlanScratch {
   unsigned int *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr, *start = nullptr,
                *cnt = nullptr, *islot = nullptr, *several = nullptr, *mslot = nullptr,
-               *off = nullptr, *small = nullptr;
+               *off = nullptr, *small = nullptr, *placed = nullptr;
   uint2* pick = nullptr;
   void* tmp = nullptr;
   size_t tmp_bytes = 0;
   ~PlanScratch() {
     for (void* p : {(void*)k0, (void*)k1, (void*)v0, (void*)v1, (void*)start, (void*)cnt,
-                    (void*)islot, (void*)several, (void*)mslot, (void*)off, (void*)small,
+                    (void*)islot, (void*)several, (void*)mslot, (void*)off, (void*)small, (void*)placed,
                     (void*)pick, tmp})
       (void)hipFree(p);
   }
@@ -831,6 +891,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   g.terms = 2;
   for (double t = 0.25 * zmax * zmax; t > 1e-11; g.terms++)
     t *= 0.25 * zmax * zmax / ((double)g.terms * g.terms);
+  if (g.terms > kMaxTerms) return give_up();
   g.inv_w = W > 0.0f ? 1.0 / (double)W : 0.0;
 
   // items of at most `chunk` rows: long enough to amortise a subgrid's
@@ -876,10 +937,11 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
         !device_array(&gs.v1, n) || !device_array(&gs.start, nkeys + 1) ||
         !device_array(&gs.cnt, nkeys + 1) || !device_array(&gs.islot, nkeys + 1) ||
         !device_array(&gs.several, nkeys + 1) || !device_array(&gs.mslot, nkeys + 1) ||
-        !device_array(&gs.off, ns) || !device_array(&gs.pick, ns + 1))
+        !device_array(&gs.off, ns) || !device_array(&gs.placed, 2 * (size_t)ns) || !device_array(&gs.pick, ns + 1))
       return give_up();
     GVM_HIP_TRY(hipMemcpyAsync(gs.off, off.data(), sizeof(unsigned int) * ns,
                                hipMemcpyHostToDevice, st));
+    GVM_HIP_TRY(hipMemsetAsync(gs.placed, 0, sizeof(unsigned int) * 2 * ns, st));
     hipLaunchKernelGGL(plan_keys_kernel, dim3((unsigned)std::min<long>(1024, (vmax + 255) / 256), ns),
                        dim3(256), 0, st, ctx->slice_tab, s0, gs.off, N, gs.k0, gs.v0);
     GVM_CHECK_LAUNCH();
@@ -926,7 +988,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     if (!got) return give_up();
     hipLaunchKernelGGL(items_kernel, dim3(blocks_for(nkeys)), dim3(256), 0, st, gs.start, gs.islot,
                        gs.mslot, nkeys, g.chunk, row0, ntiles, s0, (unsigned int)nitems,
-                       (unsigned int)nmerges, part.first, part.second,
+                       (unsigned int)nmerges, gs.placed, gs.placed + ns, part.first, part.second,
                        g.tile_slot + (long)s0 * ntiles);
     GVM_CHECK_LAUNCH();
     GVM_HIP_TRY(hipStreamSynchronize(st));  // the group's scratch is freed
@@ -1020,8 +1082,8 @@ namespace {
 template <int NP>
 void launch_spread(gvm_ctx* ctx, long slot0, int nitems, int k0, float* part) {
   const GridPlan& g = ctx->gplan;
-  hipLaunchKernelGGL((spread_kernel<NP>), dim3((nitems + 3) / 4), dim3(256), 0, ctx->stream,
-                     g.items + slot0, nitems, g.rec, g.meta, g.rot, ctx->slice_tab, ctx->cmax,
+  hipLaunchKernelGGL((spread_kernel<NP>), dim3(nitems), dim3(64), 0, ctx->stream,
+                     g.items + slot0, slot0, g.rec, g.meta, g.rot, ctx->slice_tab, ctx->cmax,
                      g.inv_w, k0, g.planes, part);
 }
 
@@ -1030,10 +1092,10 @@ void launch_cols(gvm_ctx* ctx, int s0, int ns, const float* part, float2* H) {
   // four columns per block (64 KB of LDS at 2N = 2048, two blocks per CU), two
   // where four would need 256 KB
   constexpr int BC = N <= 2048 ? 4 : 2;
-  constexpr int T = N <= 128 ? 64 : N >= 1024 ? 512 : N / 2;
+  constexpr int T = N <= 128 ? 64 : N >= 2048 ? 1024 : N / 2;
   const GridPlan& g = ctx->gplan;
   const int nb = (N + BC) / BC;  // columns 0 .. N
-  hipLaunchKernelGGL((grid_cols_kernel<N, BC, T>), dim3((nb + 7) / 8 * 8, g.planes, ns), dim3(T), 0,
+  hipLaunchKernelGGL((grid_cols_kernel<N, BC, T>), dim3(nb, g.planes, ns), dim3(T), 0,
                      ctx->stream, (const float2*)part,
                      g.tile_slot + (long)s0 * (N / 8 + 1) * (N / 4), (int)g.slice_slot[s0],
                      g.planes, g.tw2, row_pitch(N), H);
@@ -1041,7 +1103,7 @@ void launch_cols(gvm_ctx* ctx, int s0, int ns, const float* part, float2* H) {
 
 template <int N, int B>
 void launch_rows(gvm_ctx* ctx, const RowsArgs& a) {
-  constexpr int T = N / 4 < 64 ? 64 : N / 4 > 512 ? 512 : N / 4;
+  constexpr int T = N / 4 < 64 ? 64 : N / 4;
   hipLaunchKernelGGL((grid_rows_kernel<N, B, T>), dim3(N, a.nsl), dim3(T), 0, ctx->stream, a);
 }
 
