@@ -238,17 +238,29 @@ __device__ __forceinline__ void degrid_block(const float2* __restrict__ grids, i
       o[u] = ok ? ldg(vo + v) : make_float2(0.f, 0.f);
       w[u] = ok ? ldg(weight + v) : 0.0f;
     }
+    // two neighbouring cells per load: a scattered load costs by its lanes, not by
+    // its bytes
+    typedef float cells_t __attribute__((ext_vector_type(4), aligned(8)));
     float2 t11[2], t12[2], t21[2], t22[2];
 #pragma unroll
     for (int u = 0; u < 2; u++) {
       t11[u] = t12[u] = t21[u] = t22[u] = make_float2(0.f, 0.f);
       if (c[u] >= 0) {
         const int i1 = c[u] & 0xffff, j1 = c[u] >> 16;
-        const int i2 = (i1 + 1) & mask, j2 = (j1 + 1) & mask;
-        t11[u] = grid[(long)N * j1 + i1];
-        t12[u] = grid[(long)N * j2 + i1];
-        t21[u] = grid[(long)N * j1 + i2];
-        t22[u] = grid[(long)N * j2 + i2];
+        const int j2 = (j1 + 1) & mask;
+        const bool wrap = i1 == mask;
+        const float2* g1 = grid + (long)N * j1;
+        const float2* g2 = grid + (long)N * j2;
+        const cells_t a = *(const cells_t*)(g1 + i1 - (wrap ? 1 : 0));
+        const cells_t b = *(const cells_t*)(g2 + i1 - (wrap ? 1 : 0));
+        t11[u] = wrap ? make_float2(a.z, a.w) : make_float2(a.x, a.y);
+        t12[u] = wrap ? make_float2(b.z, b.w) : make_float2(b.x, b.y);
+        t21[u] = make_float2(a.z, a.w);
+        t22[u] = make_float2(b.z, b.w);
+        if (wrap) {
+          t21[u] = g1[0];
+          t22[u] = g2[0];
+        }
       }
     }
 #pragma unroll
