@@ -43,6 +43,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <utility>
 #include <vector>
 
@@ -772,10 +773,22 @@ std::vector<double> kernel_correction(int N) {
         v * (kP1 + v * (kP2 + v * (kP3 + v * (kP4 + v * (kP5 + v * (double)kP6)))));
     val[q] = half * w[q] * std::exp2(-p);
   }
+  // cos(o t) by the recurrence in o
+  double c0[Q], c1[Q], t2[Q];
+  for (int q = 0; q < Q; q++) {
+    c0[q] = 1.0;
+    c1[q] = std::cos(kPi * pos[q] / N);
+    t2[q] = 2.0 * c1[q];
+  }
   std::vector<double> c(N);
   for (int o = 0; o <= N / 2; o++) {
     double s = 0.0;
-    for (int q = 0; q < Q; q++) s += val[q] * std::cos(kPi * o * pos[q] / N);
+    for (int q = 0; q < Q; q++) {
+      s += val[q] * c0[q];
+      const double next = t2[q] * c1[q] - c0[q];
+      c0[q] = c1[q];
+      c1[q] = next;
+    }
     if (o < N / 2) c[N / 2 + o] = 1.0 / s;
     c[N / 2 - o] = 1.0 / s;
   }
@@ -796,46 +809,11 @@ int row_pitch(int N) { return N + 8; }
 }  // namespace
 
 void free_grid_plan(GridPlan& g) {
-  (void)hipFree(g.rec);
-  (void)hipFree(g.meta);
-  (void)hipFree(g.rot);
-  (void)hipFree(g.items);
-  (void)hipFree(g.merges);
-  (void)hipFree(g.tile_slot);
-  (void)hipFree(g.tw2);
-  (void)hipFree(g.corr);
-  (void)hipFree(g.wcoef);
+  (void)hipFree(g.tables);
+  (void)hipFree(g.lists);
   (void)hipFree(g.ws);
   g = GridPlan{};
 }
-
-namespace {
-
-// Scratch of the plan's set-up, freed when it ends.
-struct PlanScratch {
-  unsigned int *k0 = nullptr, *k1 = nullptr, *v0 = nullptr, *v1 = nullptr, *start = nullptr,
-               *cnt = nullptr, *islot = nullptr, *several = nullptr, *mslot = nullptr,
-               *off = nullptr, *small = nullptr, *placed = nullptr;
-  uint2* pick = nullptr;
-  void* tmp = nullptr;
-  size_t tmp_bytes = 0;
-  ~PlanScratch() {
-    for (void* p : {(void*)k0, (void*)k1, (void*)v0, (void*)v1, (void*)start, (void*)cnt,
-                    (void*)islot, (void*)several, (void*)mslot, (void*)off, (void*)small, (void*)placed,
-                    (void*)pick, tmp})
-      (void)hipFree(p);
-  }
-  bool temp(size_t bytes) {
-    if (bytes <= tmp_bytes) return true;
-    (void)hipFree(tmp);
-    tmp_bytes = 0;
-    if (!device_array((char**)&tmp, bytes)) return false;
-    tmp_bytes = bytes;
-    return true;
-  }
-};
-
-}  // namespace
 
 // Sorts every slice's visibilities by tile and lays out the work items and
 // the workspace.  *ok = false (and GVM_OK) when this form does not apply: too
@@ -859,22 +837,28 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     return GVM_OK;
   };
 
-  PlanScratch sc;
-  if (!device_array(&sc.small, 1)) return give_up();
-  // W and the planes it needs
+  // W and the planes it needs (scratch from the context's set-up workspace and a
+  // few allocations for what the plan keeps: one for every array, and as many
+  // hipFree's, took more of a small observation's first pass than the sort)
   const unsigned int zero = 0u;
-  GVM_HIP_TRY(hipMemcpyAsync(sc.small, &zero, sizeof zero, hipMemcpyHostToDevice, st));
   long vmax = 0, total = 0;
   for (const Slice& s : ctx->slices) {
     vmax = std::max(vmax, s.nvis);
     total += s.nvis;
   }
-  hipLaunchKernelGGL(wmax_kernel, dim3((unsigned)std::min<long>(256, (vmax + 255) / 256), nsl),
-                     dim3(256), 0, st, ctx->slice_tab, sc.small);
-  GVM_CHECK_LAUNCH();
   unsigned int wbits = 0;
-  GVM_HIP_TRY(hipMemcpyAsync(&wbits, sc.small, sizeof wbits, hipMemcpyDeviceToHost, st));
-  GVM_HIP_TRY(hipStreamSynchronize(st));
+  {
+    Scratch sc(ctx);
+    sc.add(sizeof(unsigned int));
+    if (sc.reserve("adjoint plan")) return give_up();
+    unsigned int* wmax = sc.take<unsigned int>(1);
+    GVM_HIP_TRY(hipMemcpyAsync(wmax, &zero, sizeof zero, hipMemcpyHostToDevice, st));
+    hipLaunchKernelGGL(wmax_kernel, dim3((unsigned)std::min<long>(256, (vmax + 255) / 256), nsl),
+                       dim3(256), 0, st, ctx->slice_tab, wmax);
+    GVM_CHECK_LAUNCH();
+    GVM_HIP_TRY(hipMemcpyAsync(&wbits, wmax, sizeof wbits, hipMemcpyDeviceToHost, st));
+    GVM_HIP_TRY(hipStreamSynchronize(st));
+  }
   if (wbits >= 0x7f800000u) return give_up();  // an infinite or NaN w
   float W;
   static_assert(sizeof W == sizeof wbits, "float bits");
@@ -899,20 +883,59 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   g.chunk = (int)std::min(512L, std::max(64L, (total / 4096 + 63) / 64 * 64));
   const int shift_x = N / 2 - (int)ctx->g.x0_phs, shift_y = N / 2 - (int)ctx->g.y0_phs;
   const bool shifted = shift_x != 0 || shift_y != 0;
-  if (!device_array(&g.rec, (size_t)total) || !device_array(&g.meta, (size_t)total) ||
-      !device_array(&g.tile_slot, (size_t)nsl * ntiles) ||
-      (shifted && !device_array(&g.rot, (size_t)total)))
-    return give_up();
+  std::vector<float2> tw2(2 * (size_t)N);
+  for (int k = 0; k < 2 * N; k++) {
+    const double t = (double)k / (2 * N);
+    tw2[k] = make_float2((float)std::cos(2.0 * kPi * t), (float)std::sin(2.0 * kPi * t));
+  }
+  const std::vector<double> corr = kernel_correction(N);
+  // J_0, then 2 (+-) J_k (the planes hold c T_k for even k, -i c T_k for odd):
+  // J_k(zeta) = zeta^k / (2^k k!) sum_m (-1)^m (zeta / 2)^2m k! / (m! (m + k)!)
+  std::vector<double> wc((size_t)K * g.terms);
+  double lead = 1.0;
+  for (int k = 0; k < K; k++) {
+    if (k > 0) lead *= 0.5 / k;
+    const int odd = (k & 1) ? ((k + 1) >> 1) & 1 : (k >> 1) & 1;
+    double c = k == 0 ? 1.0 : odd ? -2.0 * lead : 2.0 * lead;
+    for (int m = 0; m < g.terms; m++) {
+      wc[(size_t)k * g.terms + m] = c;
+      c *= -0.25 / ((m + 1.0) * (m + 1.0 + k));
+    }
+  }
+  // one allocation for the tables and the rows; the tables first, in one upload
+  auto place = [](size_t& at, size_t bytes) {
+    const size_t p = at;
+    at += Scratch::round(bytes);
+    return p;
+  };
+  size_t at = 0;
+  const size_t p_tw2 = place(at, sizeof(float2) * tw2.size());
+  const size_t p_corr = place(at, sizeof(double) * corr.size());
+  const size_t p_wcoef = place(at, sizeof(double) * wc.size());
+  std::vector<char> up(at);
+  std::memcpy(up.data() + p_tw2, tw2.data(), sizeof(float2) * tw2.size());
+  std::memcpy(up.data() + p_corr, corr.data(), sizeof(double) * corr.size());
+  std::memcpy(up.data() + p_wcoef, wc.data(), sizeof(double) * wc.size());
+  const size_t p_slot = place(at, sizeof(int) * (size_t)nsl * ntiles);
+  const size_t p_rec = place(at, sizeof(float4) * (size_t)total);
+  const size_t p_meta = place(at, sizeof(uint2) * (size_t)total);
+  const size_t p_rot = place(at, shifted ? sizeof(float2) * (size_t)total : 0);
+  if (!device_array(&g.tables, at)) return give_up();
+  GVM_HIP_TRY(hipMemcpy(g.tables, up.data(), up.size(), hipMemcpyHostToDevice));
+  g.tw2 = (float2*)(g.tables + p_tw2);
+  g.corr = (double*)(g.tables + p_corr);
+  g.wcoef = (double*)(g.tables + p_wcoef);
+  g.tile_slot = (int*)(g.tables + p_slot);
+  g.rec = (float4*)(g.tables + p_rec);
+  g.meta = (uint2*)(g.tables + p_meta);
+  g.rot = shifted ? (float2*)(g.tables + p_rot) : nullptr;
 
-  std::vector<std::pair<long4*, int2*>> parts;  // a group's items and merges
+  std::vector<char*> parts;  // a group's items, then its merges
   std::vector<std::pair<long, long>> counts;
   struct PartsFree {
-    decltype(parts)& v;
+    std::vector<char*>& v;
     ~PartsFree() {
-      for (auto& p : v) {
-        (void)hipFree(p.first);
-        (void)hipFree(p.second);
-      }
+      for (char* p : v) (void)hipFree(p);
     }
   } parts_free{parts};
   g.slice_slot.assign(nsl + 1, 0);
@@ -926,31 +949,50 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
       n += ctx->slices[s1++].nvis;
     const int ns = s1 - s0;
     const long nkeys = (long)ns * ntiles;
-    PlanScratch gs;
     std::vector<unsigned int> off(ns);
     unsigned int first = 0;
     for (int s = 0; s < ns; s++) {
       off[s] = first;
       first += (unsigned int)ctx->slices[s0 + s].nvis;
     }
-    if (!device_array(&gs.k0, n) || !device_array(&gs.k1, n) || !device_array(&gs.v0, n) ||
-        !device_array(&gs.v1, n) || !device_array(&gs.start, nkeys + 1) ||
-        !device_array(&gs.cnt, nkeys + 1) || !device_array(&gs.islot, nkeys + 1) ||
-        !device_array(&gs.several, nkeys + 1) || !device_array(&gs.mslot, nkeys + 1) ||
-        !device_array(&gs.off, ns) || !device_array(&gs.placed, 2 * (size_t)ns) || !device_array(&gs.pick, ns + 1))
-      return give_up();
+    int bits = 1;
+    while (bits < 32 && (nkeys >> bits) != 0) bits++;
+    size_t bytes = 0, scan_bytes = 0;
+    {
+      rocprim::double_buffer<unsigned int> none(nullptr, nullptr);
+      GVM_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, none, none, (size_t)n, 0u,
+                                            (unsigned)bits, st));
+      unsigned int* u = nullptr;
+      GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, scan_bytes, u, u, 0u, (size_t)nkeys + 1,
+                                          rocprim::plus<unsigned int>(), st));
+    }
+    const size_t tmp_bytes = std::max(bytes, scan_bytes);
+    Scratch sc(ctx);
+    const size_t rows_b = sizeof(unsigned int) * (size_t)n, keys_b = sizeof(unsigned int) * (nkeys + 1);
+    for (size_t b : {rows_b, rows_b, rows_b, rows_b, keys_b, keys_b, keys_b, keys_b, keys_b,
+                     sizeof(unsigned int) * ns, sizeof(unsigned int) * 2 * ns,
+                     sizeof(uint2) * (ns + 1), tmp_bytes})
+      sc.add(b);
+    if (sc.reserve("adjoint plan")) return give_up();
+    struct {
+      unsigned int *k0, *k1, *v0, *v1, *start, *cnt, *islot, *several, *mslot, *off, *placed;
+      uint2* pick;
+      char* tmp;
+    } gs;
+    for (unsigned int** p : {&gs.k0, &gs.k1, &gs.v0, &gs.v1}) *p = sc.take<unsigned int>(n);
+    for (unsigned int** p : {&gs.start, &gs.cnt, &gs.islot, &gs.several, &gs.mslot})
+      *p = sc.take<unsigned int>(nkeys + 1);
+    gs.off = sc.take<unsigned int>(ns);
+    gs.placed = sc.take<unsigned int>(2 * ns);
+    gs.pick = sc.take<uint2>(ns + 1);
+    gs.tmp = sc.take<char>(tmp_bytes);
     GVM_HIP_TRY(hipMemcpyAsync(gs.off, off.data(), sizeof(unsigned int) * ns,
                                hipMemcpyHostToDevice, st));
     GVM_HIP_TRY(hipMemsetAsync(gs.placed, 0, sizeof(unsigned int) * 2 * ns, st));
     hipLaunchKernelGGL(plan_keys_kernel, dim3((unsigned)std::min<long>(1024, (vmax + 255) / 256), ns),
                        dim3(256), 0, st, ctx->slice_tab, s0, gs.off, N, gs.k0, gs.v0);
     GVM_CHECK_LAUNCH();
-    int bits = 1;
-    while (bits < 32 && (nkeys >> bits) != 0) bits++;
     rocprim::double_buffer<unsigned int> kb(gs.k0, gs.k1), vb(gs.v0, gs.v1);
-    size_t bytes = 0;
-    GVM_HIP_TRY(rocprim::radix_sort_pairs(nullptr, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits, st));
-    if (!gs.temp(bytes)) return give_up();
     GVM_HIP_TRY(rocprim::radix_sort_pairs(gs.tmp, bytes, kb, vb, (size_t)n, 0u, (unsigned)bits, st));
     hipLaunchKernelGGL(plan_records_kernel, dim3(blocks_for(n)), dim3(256), 0, st, ctx->slice_tab,
                        s0, gs.off, N, n, kb.current(), vb.current(), shift_x, shift_y,
@@ -962,13 +1004,11 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     hipLaunchKernelGGL(item_counts_kernel, dim3(blocks_for(nkeys + 1)), dim3(256), 0, st, gs.start,
                        nkeys, g.chunk, gs.cnt, gs.several);
     GVM_CHECK_LAUNCH();
-    GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, bytes, gs.cnt, gs.islot, (unsigned int)nitems,
+    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, scan_bytes, gs.cnt, gs.islot, (unsigned int)nitems,
                                         (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
-    if (!gs.temp(bytes)) return give_up();
-    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, bytes, gs.cnt, gs.islot, (unsigned int)nitems,
-                                        (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
-    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, bytes, gs.several, gs.mslot, (unsigned int)nmerges,
-                                        (size_t)nkeys + 1, rocprim::plus<unsigned int>(), st));
+    GVM_HIP_TRY(rocprim::exclusive_scan(gs.tmp, scan_bytes, gs.several, gs.mslot,
+                                        (unsigned int)nmerges, (size_t)nkeys + 1,
+                                        rocprim::plus<unsigned int>(), st));
     hipLaunchKernelGGL(pick_kernel, dim3(1), dim3(256), 0, st, gs.islot, gs.mslot, ntiles, ns,
                        gs.pick);
     GVM_CHECK_LAUNCH();
@@ -981,14 +1021,15 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
       g.slice_merge[s0 + s] = (long)pick[s].y;
     }
     const long ni = (long)pick[ns].x - nitems, nm = (long)pick[ns].y - nmerges;
-    std::pair<long4*, int2*> part{nullptr, nullptr};
-    const bool got = device_array(&part.first, (size_t)ni) && device_array(&part.second, (size_t)nm);
+    char* part = nullptr;
+    if (!device_array(&part, sizeof(long4) * (size_t)ni + sizeof(int2) * (size_t)nm)) return give_up();
     parts.push_back(part);
     counts.push_back({ni, nm});
-    if (!got) return give_up();
+    long4* items = (long4*)part;
+    int2* merges = (int2*)(items + ni);
     hipLaunchKernelGGL(items_kernel, dim3(blocks_for(nkeys)), dim3(256), 0, st, gs.start, gs.islot,
                        gs.mslot, nkeys, g.chunk, row0, ntiles, s0, (unsigned int)nitems,
-                       (unsigned int)nmerges, gs.placed, gs.placed + ns, part.first, part.second,
+                       (unsigned int)nmerges, gs.placed, gs.placed + ns, items, merges,
                        g.tile_slot + (long)s0 * ntiles);
     GVM_CHECK_LAUNCH();
     GVM_HIP_TRY(hipStreamSynchronize(st));  // the group's scratch is freed
@@ -999,23 +1040,24 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     s0 = s1;
   }
   if (parts.size() == 1) {
-    g.items = parts[0].first;
-    g.merges = parts[0].second;
+    g.lists = parts[0];
     parts.clear();
   } else {
-    if (!device_array(&g.items, (size_t)nitems) || !device_array(&g.merges, (size_t)nmerges))
+    if (!device_array(&g.lists, sizeof(long4) * (size_t)nitems + sizeof(int2) * (size_t)nmerges))
       return give_up();
-    long o = 0, om = 0;
+    char* o = g.lists;
+    char* om = g.lists + sizeof(long4) * (size_t)nitems;
     for (size_t k = 0; k < parts.size(); k++) {
-      GVM_HIP_TRY(hipMemcpyAsync(g.items + o, parts[k].first, sizeof(long4) * counts[k].first,
-                                 hipMemcpyDeviceToDevice, st));
-      GVM_HIP_TRY(hipMemcpyAsync(g.merges + om, parts[k].second, sizeof(int2) * counts[k].second,
-                                 hipMemcpyDeviceToDevice, st));
-      o += counts[k].first;
-      om += counts[k].second;
+      const size_t bi = sizeof(long4) * counts[k].first, bm = sizeof(int2) * counts[k].second;
+      GVM_HIP_TRY(hipMemcpyAsync(o, parts[k], bi, hipMemcpyDeviceToDevice, st));
+      GVM_HIP_TRY(hipMemcpyAsync(om, parts[k] + bi, bm, hipMemcpyDeviceToDevice, st));
+      o += bi;
+      om += bm;
     }
     GVM_HIP_TRY(hipStreamSynchronize(st));
   }
+  g.items = (long4*)g.lists;
+  g.merges = (int2*)(g.items + nitems);
 
   // batches of slices that share the workspace
   const size_t per_item = sizeof(float) * kSub * (size_t)K;
@@ -1046,32 +1088,6 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   const size_t bytes = g.part_bytes + per_slice * need_slices;
   if (bytes > budget) return give_up();
   if (!device_array((char**)&g.ws, bytes)) return give_up();
-
-  std::vector<float2> tw2(2 * (size_t)N);
-  for (int k = 0; k < 2 * N; k++) {
-    const double t = (double)k / (2 * N);
-    tw2[k] = make_float2((float)std::cos(2.0 * kPi * t), (float)std::sin(2.0 * kPi * t));
-  }
-  const std::vector<double> corr = kernel_correction(N);
-  // J_0, then 2 (+-) J_k (the planes hold c T_k for even k, -i c T_k for odd):
-  // J_k(zeta) = zeta^k / (2^k k!) sum_m (-1)^m (zeta / 2)^2m k! / (m! (m + k)!)
-  std::vector<double> wc((size_t)K * g.terms);
-  double lead = 1.0;
-  for (int k = 0; k < K; k++) {
-    if (k > 0) lead *= 0.5 / k;
-    const int odd = (k & 1) ? ((k + 1) >> 1) & 1 : (k >> 1) & 1;
-    double c = k == 0 ? 1.0 : odd ? -2.0 * lead : 2.0 * lead;
-    for (int m = 0; m < g.terms; m++) {
-      wc[(size_t)k * g.terms + m] = c;
-      c *= -0.25 / ((m + 1.0) * (m + 1.0 + k));
-    }
-  }
-  if (!device_array(&g.tw2, tw2.size()) || !device_array(&g.corr, corr.size()) ||
-      !device_array(&g.wcoef, wc.size()))
-    return give_up();
-  GVM_HIP_TRY(hipMemcpy(g.wcoef, wc.data(), sizeof(double) * wc.size(), hipMemcpyHostToDevice));
-  GVM_HIP_TRY(hipMemcpy(g.tw2, tw2.data(), sizeof(float2) * tw2.size(), hipMemcpyHostToDevice));
-  GVM_HIP_TRY(hipMemcpy(g.corr, corr.data(), sizeof(double) * corr.size(), hipMemcpyHostToDevice));
   g.usable = true;
   *ok = true;
   return GVM_OK;

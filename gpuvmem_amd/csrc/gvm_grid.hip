@@ -41,47 +41,6 @@ int blocks_for(long n) {
   return (int)std::max(1L, std::min<long>((n + kThreads - 1) / kThreads, 65536));
 }
 
-// Scratch of one call, cut from the context's set-up workspace: sizes are
-// added up first, then reserve() and take() in the same order.
-constexpr size_t kKeepScratch = 1UL << 30;  // a larger workspace is given back
-
-struct Scratch {
-  gvm_ctx* ctx;
-  size_t need = 0, at = 0;
-  explicit Scratch(gvm_ctx* c) : ctx(c) {}
-  Scratch(const Scratch&) = delete;
-  Scratch& operator=(const Scratch&) = delete;
-  ~Scratch() {
-    if (ctx->setup_bytes > kKeepScratch) {
-      (void)hipFree(ctx->setup_ws);
-      ctx->setup_ws = nullptr;
-      ctx->setup_bytes = 0;
-    }
-  }
-  static size_t round(size_t bytes) { return (bytes + 255) / 256 * 256; }
-  void add(size_t bytes) { need += round(bytes); }
-  gvm_status reserve(const char* what) {
-    if (need <= ctx->setup_bytes) return GVM_OK;
-    (void)hipFree(ctx->setup_ws);
-    ctx->setup_ws = nullptr;
-    ctx->setup_bytes = 0;
-    if (hipMalloc((void**)&ctx->setup_ws, need) != hipSuccess) {
-      (void)hipGetLastError();
-      ctx->setup_ws = nullptr;
-      set_error(std::string(what) + ": out of device memory");
-      return GVM_ERR_OOM;
-    }
-    ctx->setup_bytes = need;
-    return GVM_OK;
-  }
-  template <class T>
-  T* take(size_t count) {
-    T* p = (T*)(ctx->setup_ws + at);
-    at += round(sizeof(T) * count);
-    return p;
-  }
-};
-
 // Number of bits a radix sort needs for keys in [0, sentinel].
 int key_bits(uint32_t sentinel) {
   int b = 1;
