@@ -705,7 +705,8 @@ gvm_status rebuild_splits(gvm_ctx* ctx) {
   return GVM_OK;
 }
 
-gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize) {
+gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
+                   bool set) {
   const gvm_geometry& g = ctx->g;
   const int N = g.N;
   const long n = (long)N * N;
@@ -721,6 +722,11 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
     gvm_status st = split_work(ctx);
     if (st) return st;
     ctx->epoch++;
+  }
+  // (the gridded form's last kernel writes every value itself)
+  if (set && (!ctx->adj_gridded || nsl == 0)) {
+    gvm_status st = gvm_vec_zero(ctx, result, n * g.image_count);
+    if (st) return st;
   }
   if (mode != GVM_ADJOINT_DIRECT && !ctx->adj_gridded) {
     long vmax = 0;
@@ -741,7 +747,7 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
     GVM_HIP_TRY(hipEventRecord(ctx->tev[2 * pair], ctx->stream));
   }
   if (ctx->adj_gridded) {
-    gvm_status st = adjoint_grid(ctx, I, result, flag_opt, normalize);
+    gvm_status st = adjoint_grid(ctx, I, result, flag_opt, normalize, set);
     if (st) return st;
   } else if (mode == GVM_ADJOINT_DIRECT) {
     const double dxr = g.deltax * 3.14159265358979323846 / 180.0;

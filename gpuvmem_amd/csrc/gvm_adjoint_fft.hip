@@ -581,6 +581,7 @@ struct RowsArgs {
   float noise_cut, fg_scale, threshold;
   const float* gcf;
   int normalize, flag_opt;
+  int set;            // images of a result to be written whole, 0 to add to it
   double wz;          // 2 pi W
   double dx, dy;      // radians per pixel
   int x0, y0;         // phase centre
@@ -626,7 +627,19 @@ __global__ __launch_bounds__(T, 4) void grid_rows_kernel(RowsArgs a) {
       some |= on[u][e];
     }
   }
-  if (!__syncthreads_or(some)) return;
+  some = __syncthreads_or(some);
+  if (a.set && !a.each)  // zero outside the mask, and the other images
+    for (int m = 0; m < a.set; m++) {
+#pragma unroll
+      for (int u = 0; u < PP; u++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          const int cp = threadIdx.x + u * T;
+          if (cp < N / 2 && (m != (a.flag_opt & 1) || !on[u][e]))
+            a.result[m * n + (long)i * N + 2 * cp + e] = 0.0f;
+        }
+    }
+  if (!some) return;
   double zeta[PP][2];
 #pragma unroll
   for (int u = 0; u < PP; u++)
@@ -718,7 +731,7 @@ __global__ __launch_bounds__(T, 4) void grid_rows_kernel(RowsArgs a) {
       float sc = a.fg_scale * sd.pb[k];
       if (a.gcf) sc = sc * a.gcf[k];
       const float d = (float)(-(gv * inv_scale) * (double)sc * inv_nvis);
-      out[k] = a.each ? d : chain_rule(out[k], d, sd.nudiv, a.I[k], a.I[n + k], a);
+      out[k] = a.each ? d : chain_rule(a.set ? 0.0f : out[k], d, sd.nudiv, a.I[k], a.I[n + k], a);
     }
 }
 
@@ -727,10 +740,13 @@ __global__ __launch_bounds__(T, 4) void grid_rows_kernel(RowsArgs a) {
 __global__ __launch_bounds__(256) void chain_kernel(RowsArgs a, int N) {
   const long n = (long)N * N;
   for (long k = blockIdx.x * 256L + threadIdx.x; k < n; k += (long)gridDim.x * 256) {
-    if (!(a.noise[k] < a.noise_cut)) continue;
+    const bool on = a.noise[k] < a.noise_cut;
+    for (int m = 0; m < a.set; m++)
+      if (!on || m != (a.flag_opt & 1)) a.result[m * n + k] = 0.0f;
+    if (!on) continue;
     const float i0 = a.I[k], alpha = a.I[n + k];
     float* out = a.result + (a.flag_opt & 1) * n + k;
-    float r = *out;
+    float r = a.set ? 0.0f : *out;
     for (int s = 0; s < a.nsl; s++)
       r = chain_rule(r, a.each[(long)s * n + k], a.tab[a.s0 + s].nudiv, i0, alpha, a);
     *out = r;
@@ -1125,7 +1141,7 @@ void launch_rows(gvm_ctx* ctx, const RowsArgs& a) {
 
 template <int N>
 gvm_status run_batch(gvm_ctx* ctx, int s0, int s1, const float* I, float* result, int flag_opt,
-                     int normalize) {
+                     int normalize, bool set) {
   const GridPlan& g = ctx->gplan;
   const int K = g.planes;
   const long slot0 = g.slice_slot[s0];
@@ -1174,6 +1190,7 @@ gvm_status run_batch(gvm_ctx* ctx, int s0, int s1, const float* I, float* result
   a.gcf = ctx->gcf;
   a.normalize = normalize;
   a.flag_opt = flag_opt;
+  a.set = set ? ctx->g.image_count : 0;
   a.wz = g.wz;
   a.dx = ctx->g.deltax * kPi / 180.0;
   a.dy = ctx->g.deltay * kPi / 180.0;
@@ -1202,19 +1219,20 @@ gvm_status run_batch(gvm_ctx* ctx, int s0, int s1, const float* I, float* result
 
 }  // namespace
 
-gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize) {
+gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
+                        bool set) {
   const GridPlan& g = ctx->gplan;
   for (size_t b = 0; b + 1 < g.batch0.size(); b++) {
     const int s0 = g.batch0[b], s1 = g.batch0[b + 1];
     gvm_status st = GVM_ERR_ARG;
     switch (ctx->g.N) {
-      case 64: st = run_batch<64>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 128: st = run_batch<128>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 256: st = run_batch<256>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 512: st = run_batch<512>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 1024: st = run_batch<1024>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 2048: st = run_batch<2048>(ctx, s0, s1, I, result, flag_opt, normalize); break;
-      case 4096: st = run_batch<4096>(ctx, s0, s1, I, result, flag_opt, normalize); break;
+      case 64: st = run_batch<64>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 128: st = run_batch<128>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 256: st = run_batch<256>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 512: st = run_batch<512>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 1024: st = run_batch<1024>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 2048: st = run_batch<2048>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
+      case 4096: st = run_batch<4096>(ctx, s0, s1, I, result, flag_opt, normalize, set && b == 0); break;
     }
     if (st) return st;
   }

@@ -739,15 +739,25 @@ extern "C" gvm_status gvm_epoch(const gvm_ctx* ctx, long* epoch) {
   return GVM_OK;
 }
 
-extern "C" gvm_status gvm_dchi2(gvm_ctx* ctx, const float* I_dev, float* result_dev,
-                                int flag_opt, int normalize) {
+static gvm_status dchi2(gvm_ctx* ctx, const float* I_dev, float* result_dev, int flag_opt,
+                        int normalize, bool set) {
   GVM_REQUIRE(ctx && I_dev && result_dev, "gvm_dchi2: null argument");
   GVM_REQUIRE(flag_opt >= 0, "gvm_dchi2: negative flag_opt");
   if (!ctx->have_residuals) {
     set_error("gvm_dchi2: no residuals (call gvm_chi2 first)");
     return GVM_ERR_STATE;
   }
-  return adjoint(ctx, I_dev, result_dev, flag_opt, normalize);
+  return adjoint(ctx, I_dev, result_dev, flag_opt, normalize, set);
+}
+
+extern "C" gvm_status gvm_dchi2(gvm_ctx* ctx, const float* I_dev, float* result_dev,
+                                int flag_opt, int normalize) {
+  return dchi2(ctx, I_dev, result_dev, flag_opt, normalize, false);
+}
+
+extern "C" gvm_status gvm_dchi2_set(gvm_ctx* ctx, const float* I_dev, float* result_dev,
+                                    int flag_opt, int normalize) {
+  return dchi2(ctx, I_dev, result_dev, flag_opt, normalize, true);
 }
 
 extern "C" gvm_status gvm_timing_reset(gvm_ctx* ctx) {

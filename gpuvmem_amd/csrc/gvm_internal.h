@@ -228,12 +228,13 @@ gvm_status timing_fold(gvm_ctx* ctx, int n);
 // Launchers implemented in the .hip files.
 gvm_status forward_chi2(gvm_ctx* ctx, float* I, int flag_opt, int normalize,
                         double* out);
-gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt,
-                   int normalize);
+gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
+                   bool set = false);
 // The gridded form of the adjoint: its plan (*ok = false when it does not
 // apply) and its launches; free_grid_plan frees and clears a plan.
 gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok);
-gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize);
+gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
+                        bool set);
 void free_grid_plan(GridPlan& g);
 // Rebuilds the adjoint's range table and workspace for the current form.
 gvm_status rebuild_splits(gvm_ctx* ctx);

@@ -4,6 +4,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <typeinfo>
 
 #include "gvm/factory.h"
 #include "gvm/framework.h"
@@ -259,8 +260,12 @@ void ObjectiveFunction::gradientSequence(float* p, float* xi, int iter) {
     // AddToDPhi sequence and the copy to xi in one kernel
     for (Fi* fi : fis) fi->setIteration(iter);
     Chi2* chi2 = static_cast<Chi2*>(fis[0]);
-    chi2->restartDGi();
-    chi2->calcGi(p, xi);
+    if (typeid(*chi2) == typeid(Chi2)) {
+      chi2->restartAndCalcGi(p);
+    } else {
+      chi2->restartDGi();
+      chi2->calcGi(p, xi);
+    }
     std::vector<gvm_prior_term> terms(fis.size() - 1);
     for (size_t k = 1; k < fis.size(); k++) fis[k]->priorTerm(&terms[k - 1], true);
     check(gvm_dphi_assemble(gvm::ctx(), p, chi2->getResult(), dphi, xi, terms.data(),
@@ -388,6 +393,11 @@ bool Chi2::enqueueValue(float* p, int slot) {
 void Chi2::calcGi(float* p, float* xi) {
   check(gvm_dchi2(gvm::ctx(), p, result_dchi2, globals().flag_opt, normalize ? 1 : 0),
         "gvm_dchi2");
+}
+
+void Chi2::restartAndCalcGi(float* p) {
+  check(gvm_dchi2_set(gvm::ctx(), p, result_dchi2, globals().flag_opt, normalize ? 1 : 0),
+        "gvm_dchi2_set");
 }
 
 void Chi2::restartDGi() {

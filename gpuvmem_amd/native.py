@@ -172,6 +172,7 @@ HIP_API = {
     "gvm_laplacian_value_enqueue": [_P, _P, _I, _I],
     "gvm_values_read": [_P, _I, _DP],
     "gvm_dchi2": [_P, _P, _P, _I, _I],
+    "gvm_dchi2_set": [_P, _P, _P, _I, _I],
     "gvm_get_residuals": [_P, _I, _P],
     "gvm_entropy_value": [_P, _P, _I, _F, _F, _DP],
     "gvm_entropy_grad": [_P, _P, _P, _I, _F, _F, _F],

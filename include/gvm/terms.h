@@ -21,6 +21,8 @@ class Chi2 : public Fi {
   void configure(int penalizatorIndex, int imageIndex, int imageToAdd, bool normalize) override;
   void setFgScale(float fg_scale) override { this->fg_scale = fg_scale; }
   float getFgScale() override { return this->fg_scale; }
+  // restartDGi and calcGi in one device call
+  void restartAndCalcGi(float* p);
   // the device gradient buffer calcGi accumulates into
   float* getResult() const { return result_dchi2; }
 

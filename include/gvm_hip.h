@@ -275,6 +275,10 @@ gvm_status gvm_epoch(const gvm_ctx* ctx, long* epoch);
  * cleared first (Chi2::restartDGi does that). */
 gvm_status gvm_dchi2(gvm_ctx* ctx, const float* I_dev, float* result_dev,
                      int flag_opt, int normalize);
+/* The same into a result that need not be cleared: restartDGi and calcGi in one
+ * call, every value of result_dev written. */
+gvm_status gvm_dchi2_set(gvm_ctx* ctx, const float* I_dev, float* result_dev,
+                         int flag_opt, int normalize);
 
 /* Residuals V_r of one slice from the last gvm_chi2 (host float[2*nvis]);
  * replaces the Vr readback of MFS::writeResiduals (src/mfs.cu:1115-1155). */

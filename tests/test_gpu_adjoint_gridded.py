@@ -16,7 +16,8 @@ import numpy as np
 import pytest
 
 import oracle
-from gpuvmem_amd.device import Context
+from gpuvmem_amd import native
+from gpuvmem_amd.device import Context, DeviceBuffer
 from gpuvmem_amd.problem import small_problem
 
 pytestmark = pytest.mark.gpu
@@ -179,3 +180,36 @@ def test_rows_that_are_not_numbers(bad):
     g = r.download(np.float32, (2, p.N, p.M))[0]
     ctx.close()
     assert on.any() and np.all(np.isnan(g[on])) and np.all(g[~on] == 0)
+
+
+@pytest.mark.parametrize("mode", ["bf16x3", "direct"])
+@pytest.mark.parametrize("flag,nsl", [(0, 1), (1, 1), (0, 3), (1, 3), (0, 0)])
+def test_a_result_that_is_set(mode, flag, nsl):
+    """gvm_dchi2_set into any memory gives what gvm_dchi2 adds to a cleared one."""
+    print(f"case: set {mode} flag {flag} slices {nsl}", flush=True)
+    p = small_problem(npix=64, n_antennas=6, seed=31)
+    rng = np.random.default_rng(nsl)
+    img = p.initial_image()
+    img[0] += (rng.random((p.N, p.M)) * 20.0).astype(np.float32)
+    img[1] = rng.uniform(-1.0, 2.0, (p.N, p.M)).astype(np.float32)
+    ctx = Context(p, adjoint=mode, add_data=False)
+    for s in range(nsl):
+        cells = np.stack([rng.uniform(0, 40, 400), rng.uniform(-31, 31, 400)], 1)
+        ctx.add(p.freq * (1.0 + 0.1 * s), *_rows(p, cells, w=rng.uniform(-1e4, 1e4, 400))[1:])
+    d = ctx.image(img)
+    if nsl == 0:  # (a context may refuse to evaluate nothing: then there is no gradient either)
+        try:
+            ctx.chi2(d, flag_opt=flag)
+        except native.GvmError:
+            ctx.close()
+            return
+    else:
+        ctx.chi2(d, flag_opt=flag)
+    out = []
+    for fn, fill in ((ctx.lib.gvm_dchi2, 0.0), (ctx.lib.gvm_dchi2_set, np.nan)):
+        r = DeviceBuffer.from_array(np.full(2 * p.M * p.N, fill, np.float32))
+        native.check(fn(ctx.ctx, d.ptr, r.ptr, flag, 1), "dchi2")
+        ctx.sync()
+        out.append(r.download(np.float32))
+    ctx.close()
+    assert np.array_equal(out[0], out[1])
