@@ -8,17 +8,22 @@ components; objective chi2 + Entropy (lambda 0.01, G 0.001) + TSV
 ObjectiveFunction::calcFunction + one calcGradient (the pair of
 src/frprmn.cu:130-135) at a fixed image, all inputs resident in HBM.
 
-Prints one JSON line.  The roofline figure is for the dominant kernel, the
-DChi2 adjoint GEMM: algorithmic work 4 flop per (pixel, visibility) over the
-pixels it computes (its 128 x 64 sub-tiles that hold a pixel on the mask; the
-reference's DChi2 computes the pixels on the mask) per launch, over its
-average duration (HIP events on the context's stream).  The cpu_baseline leg
+Prints one JSON line.  The roofline figure is for the dominant part, the DChi2
+adjoint, over its average duration (HIP events on the context's stream).  By
+gridding and FFT (the default wherever it applies): the bytes it cannot do
+without, 32 per visibility (the sorted record and the residual) and 16 per
+pixel, against the HBM peak.  As a GEMM: 4 flop per (pixel, visibility) over
+the pixels it computes (its 128 x 64 sub-tiles that hold a pixel on the mask;
+the reference's DChi2 computes the pixels on the mask), against the MFMA peak.
+The cpu_baseline leg
 times the FP64 oracle on the host cores on a bounded sample (full-size
 forward chi2 + the separable FP64 gradient over a slice of the
 visibilities, extrapolated linearly in the visibility count).  The
 time_to_image object times L-BFGS to a common objective with the plain FP32
 and the split-precision adjoint, and the split form once more from the
-learned warm start of the committed network (gpuvmem_amd/data/).
+learned warm start of the committed network (gpuvmem_amd/data/).  (Where both
+forms run by gridding and FFT, as here, the first two legs differ by the
+evaluation graphs alone.)
 
 Other modes, each printing its own JSON line: --workload 0/2/3 (other
 workloads), --time-to-image ITERS (split precision against plain FP32 at
@@ -44,6 +49,7 @@ sys.path.insert(0, str(ROOT))
 # the learned warm start of the 1024^2 workload (trained by bench.py --warm-start
 # --ws-workload 1 --ws-save-model)
 WARM_MODEL = ROOT / "gpuvmem_amd" / "data" / "warm_start_1024sq.npz"
+PEAK_HBM_TBS = 8.0
 PEAK_TFLOPS = {"f16x3": 2500.0, "bf16x3": 2500.0, "f32": 157.3, "direct": 157.3}
 DTYPE = {
     "f16x3": "fp16 hi/lo x3 MFMA adjoint (fp32 accumulate, fp64 combine); fp32 forward",
@@ -51,6 +57,8 @@ DTYPE = {
     "f32": "fp32 MFMA adjoint; fp32 forward",
     "direct": "fp32 VALU direct-sum adjoint; fp32 forward",
 }
+DTYPE_GRIDDED = ("fp32 gridding (MFMA) and FFT adjoint (fp64 plane weights and merges); fp32 "
+                 "forward")
 
 
 def bench_image(p) -> np.ndarray:
@@ -427,7 +435,7 @@ def bench_unet_step(steps: int, warmup: int, levels: int = 6, base: int = 32, ba
            "config": {"levels": levels, "base_channels": base, "batch": batch,
                       "image": [npix, npix], "parameters": net.nparams,
                       "weights": "bf16 (fp32 master)",
-                      "convolutions": "implicit GEMM on v_mfma_f32_32x32x2_f32"}}
+                      "convolutions": "plane tiles on v_mfma_f32_32x32x2_f32"}}
     net.close()
     ctx.close()
     return out
@@ -1033,13 +1041,42 @@ def main() -> int:
 
     nvt = p.nvis_total
     nsl = len(p.all_slices())
-    traffic, traffic_src = profiled_traffic(args.adjoint, nvt, ctx.split_vis())
-    # the adjoint computes the sub-tiles that hold a pixel on the mask: the work
-    # of a launch is 4 flop per (computed pixel, visibility)
-    px = ctx.adjoint_computed_pixels()
-    flops = 4.0 * px * nvt
-    achieved = flops / (adj_ms * 1e-3) / 1e12
-    peak = PEAK_TFLOPS[args.adjoint]
+    gridded = ctx.adjoint_gridded()
+    traffic, traffic_src = ((None, None) if gridded else
+                            profiled_traffic(args.adjoint, nvt, ctx.split_vis()))
+    if gridded:
+        need = 32.0 * nvt + 16.0 * p.M * p.N
+        roofline = {
+            "bound": "hbm",
+            "achieved": need / (adj_ms * 1e-3) / 1e12,
+            "peak": PEAK_HBM_TBS,
+            "unit": "TB/s",
+            "frac": need / (adj_ms * 1e-3) / 1e12 / PEAK_HBM_TBS,
+            "kernel": "gridded adjoint (spread, merge, columns, rows)",
+            "kernel_ms": adj_ms,
+            "algorithmic_bytes_per_launch": need,
+        }
+    else:
+        # the GEMM computes the sub-tiles that hold a pixel on the mask: the work
+        # of a launch is 4 flop per (computed pixel, visibility)
+        px = ctx.adjoint_computed_pixels()
+        flops = 4.0 * px * nvt
+        achieved = flops / (adj_ms * 1e-3) / 1e12
+        roofline = {
+            "bound": "mfma",
+            "achieved": achieved,
+            "peak": PEAK_TFLOPS[args.adjoint],
+            "unit": "TFLOP/s",
+            "frac": achieved / PEAK_TFLOPS[args.adjoint],
+            "kernel": f"adjoint_gemm_kernel ({args.adjoint})",
+            "kernel_ms": adj_ms,
+            "algorithmic_flop_per_launch": flops,
+            "computed_pixels": px,
+            "image_pixels": p.M * p.N,
+            "full_image_flop_per_launch": 4.0 * p.M * p.N * nvt,
+        }
+    roofline.update(traffic=traffic, traffic_source=traffic_src,
+                    traffic_unit="bytes/launch (HBM, rocprofv3 FETCH_SIZE+WRITE_SIZE)")
     line = {
         "metric": ("obj+grad evals/s (1024^2, 1.76M vis)" if args.workload == 1 else
                    f"obj+grad evals/s ({p.M}^2, {nsl} slices, {nvt} vis)"),
@@ -1052,7 +1089,7 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": DTYPE[args.adjoint],
+        "dtype": DTYPE_GRIDDED if gridded else DTYPE[args.adjoint],
         "data": ("synthetic (seeded generator: 50-antenna array, 200 Gaussian components, 1 mJy "
                  "noise)" if args.workload == 1 else "synthetic (seeded generator)"),
         "config": {
@@ -1067,22 +1104,7 @@ def main() -> int:
             "split_vis": ctx.split_vis(),
             "autotune": tune,
         },
-        "roofline": {
-            "bound": "mfma",
-            "achieved": achieved,
-            "peak": peak,
-            "unit": "TFLOP/s",
-            "frac": achieved / peak,
-            "traffic": traffic,
-            "traffic_unit": "bytes/launch (HBM, rocprofv3 FETCH_SIZE+WRITE_SIZE)",
-            "traffic_source": traffic_src,
-            "kernel": f"adjoint_gemm_kernel ({args.adjoint})",
-            "kernel_ms": adj_ms,
-            "algorithmic_flop_per_launch": flops,
-            "computed_pixels": px,
-            "image_pixels": p.M * p.N,
-            "full_image_flop_per_launch": 4.0 * p.M * p.N * nvt,
-        },
+        "roofline": roofline,
     }
     line["value_evaluation_us"] = value_latency(obj, d_img, ctx)
     if args.calibrate_copy_mib > 0:

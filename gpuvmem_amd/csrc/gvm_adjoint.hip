@@ -829,6 +829,12 @@ extern "C" gvm_status gvm_set_fft_mode(gvm_ctx* ctx, int mode) {
   return GVM_OK;
 }
 
+extern "C" gvm_status gvm_adjoint_gridded(const gvm_ctx* ctx, int* gridded) {
+  GVM_REQUIRE(ctx && gridded, "gvm_adjoint_gridded: null argument");
+  *gridded = ctx->adj_gridded ? 1 : 0;
+  return GVM_OK;
+}
+
 extern "C" gvm_status gvm_adjoint_computed_pixels(const gvm_ctx* ctx, long* pixels) {
   GVM_REQUIRE(ctx && pixels, "gvm_adjoint_computed_pixels: null argument");
   *pixels = ctx->adjoint_mode == GVM_ADJOINT_DIRECT ? ctx->adj_px_direct : ctx->adj_px_gemm;

@@ -234,196 +234,255 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
 }
 
 // ---- weight gradient ----
+constexpr int kWgradPixels = 8192;  // pixels of an FP32 partial
+constexpr int kWgradChunk = 128;    // pixels staged at a time
+
 struct WgradArgs {
   const float* in;    // [B][Ci][H][W]
   const float* out;   // forward output (ReLU mask), or NULL
   const float* dout;  // [B][Co][H][W]
-  float* part;        // [partial][Co][Ci][K][K]
-  double* bpart;      // [partial][Co]
+  float* part;        // [range][Co][Ci][K][K]
+  double* bpart;      // [range][Co]
   int B, Ci, Co, H, W;
-  int tiles_x, tiles_y, ntiles, per;  // tiles of pixels; tiles per block
+  unsigned int rw;    // about 2^32 / W
 };
 
-constexpr int kWgradW = 16;  // pixel columns of a tile
-
-// A wave owns 32 output x 32 input channels of every tap (nine 32 x 32 blocks)
-// and adds tiles of SH x 16 pixels: K = pixels, A = g[co][q], B = in[ci][q + tap]
-// read from the staged planes.  WM x WN waves cover channels, WK waves take
-// different tiles and leave a partial each; the partials are summed in FP64 in a
-// fixed order.  Channel pitches are twice an odd number, so that the 32 channels
-// and the two pixels of an MFMA operand fall on 64 different banks.  The blocks of
-// the first input channels also leave the bias gradient's partials (FP64).
-template <int KS, int WM, int WN, int WK, int SH>
-__global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
-  constexpr int KK = KS * KS, P = KS / 2, PW = kWgradW + KS - 1, PH = SH + KS - 1;
-  constexpr int Q = SH * kWgradW, GP = Q + 1, IP = PH * PW | 1;
-  static_assert(WM * WN * WK == 4, "four waves");
-  // A thread keeps its pixel and takes every CG-th (CI-th) channel of it: a load's
-  // address is the tile's plus a constant.
-  constexpr int CG = 256 / Q, CI = 256 / (PH * PW);
-  constexpr int NG1 = WM * 32 / CG, NI1 = (WN * 32 + CI - 1) / CI, NG = NG1 * WK, NIN = NI1 * WK;
-  static_assert(CG * Q == 256 && NG1 * CG == WM * 32, "whole channels per thread");
-  __shared__ float lg[WK][WM * 32 * GP];
-  __shared__ float li[WK][WN * 32 * IP];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
-  const int wk = wave / (WM * WN), wm = wave % WM, wn = wave / WM % WN;
-  const int HW = a.H * a.W;
-  const int co0 = blockIdx.y * WM * 32, ci0 = blockIdx.x * WN * 32;
-  const int first = blockIdx.z * a.per, last = min(a.ntiles, first + a.per);
-  const int gq = t % Q, gc = t / Q, ir = t % (PH * PW), ic = t / (PH * PW);
-  float rg[NG], rm[NG], ri[NIN];
-  // this thread's first addresses in the tiles being loaded (one per WK), and
-  // whether its pixel lies inside; the loads go between the MFMAs of the tiles
-  // before.  An address out of range reads element 0 and becomes zero when stored.
-  long ig[WK], ii[WK];
-  bool og[WK], oi[WK];
-  auto origins = [&](int tile0) {
-#pragma unroll
-    for (int k = 0; k < WK; k++) {
-      const int tile = min(tile0 + k, a.ntiles - 1);
-      const int tx = tile % a.tiles_x * kWgradW, ty = tile / a.tiles_x % a.tiles_y * SH;
-      const long tb = tile / a.tiles_x / a.tiles_y;
-      const int gx = tx + gq % kWgradW, gy = ty + gq / kWgradW;
-      const int ix = tx + ir % PW - P, iy = ty + ir / PW - P;
-      og[k] = tile0 + k < last && gx < a.W && gy < a.H;
-      oi[k] = tile0 + k < last && ic < CI && ix >= 0 && ix < a.W && iy >= 0 && iy < a.H;
-      ig[k] = (tb * a.Co + co0 + gc) * HW + gy * a.W + gx;
-      ii[k] = (tb * a.Ci + ci0 + ic) * HW + iy * a.W + ix;
-    }
-  };
-  auto load_g = [&](int j) {
-    const int k = j / NG1, c = j % NG1 * CG;
-    const long i = og[k] && co0 + gc + c < a.Co ? ig[k] + (long)c * HW : 0;
-    rg[j] = a.dout[i];
-    if (a.out) rm[j] = a.out[i];
-  };
-  auto load_in = [&](int j) {
-    const int k = j / NI1, c = j % NI1 * CI;
-    ri[j] = a.in[oi[k] && ci0 + ic + c < a.Ci ? ii[k] + (long)c * HW : 0];
-  };
-  auto store = [&]() {
-#pragma unroll
-    for (int j = 0; j < NG; j++) {
-      const int k = j / NG1, c = gc + j % NG1 * CG;
-      lg[k][c * GP + gq] = og[k] && co0 + c < a.Co && (!a.out || rm[j] > 0.0f) ? rg[j] : 0.0f;
-    }
-#pragma unroll
-    for (int j = 0; j < NIN; j++) {
-      const int k = j / NI1, c = ic + j % NI1 * CI;
-      if (ic < CI && c < WN * 32)
-        li[k][c * IP + ir] = oi[k] && ci0 + c < a.Ci ? ri[j] : 0.0f;
-    }
-  };
-  f32x16_t acc[KK];
-#pragma unroll
-  for (int k = 0; k < KK; k++)
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[k][e] = 0.0f;
-  // bias: thread t sums part of the g values of channel t / TPC
-  constexpr int TPC = 256 / (WM * 32);
-  double bsum = 0.0;
-  const float* pa = &lg[wk][(wm * 32 + lr) * GP + lh];
-  const float* pb = &li[wk][(wn * 32 + lr) * IP + lh];
-  if (first < last) {
-    origins(first);
-#pragma unroll
-    for (int j = 0; j < NG; j++) load_g(j);
-#pragma unroll
-    for (int j = 0; j < NIN; j++) load_in(j);
+// Linear pixel index of a batch as (image, pixel of its plane), advanced by chunks.
+struct PixelPos {
+  int q, b, p;
+  __device__ __forceinline__ void start(int q0, int HW) {
+    q = q0;
+    b = q0 > 0 ? q0 / HW : 0;
+    p = q0 - b * HW;  // (-1 before the first)
   }
-  for (int tile = first; tile < last; tile += WK) {
+  __device__ __forceinline__ void next(int HW) {
+    q += kWgradChunk;
+    p += kWgradChunk;
+    while (p >= HW) {
+      p -= HW;
+      b++;
+    }
+  }
+};
+
+// A wave owns one tap's 32 output x 32 input channels over a range of 8192 pixels
+// (a FP32 partial; FP64 after that): K = pixels in their linear order (b, y, x), A =
+// g[co][q], B = in[ci][q + tap].  That is an im2col GEMM's order, so the bits do not
+// depend on how taps and channels are spread over waves; one tap per wave makes more
+// waves of every layer of a network (9 x 128 for 2^20 pixels of 32 x 32 channels, and
+// for each level down) than the chip has matrix units.  A block's waves share the row
+// ky = blockIdx.x % KS of taps: for them the input is one linear run of pixels, (ky -
+// K/2) W away and one to either side, staged without regard to the image's edges; a
+// wave clears the operands of pixels whose tap lies outside with a mask of the
+// chunk's 128 pixels.
+// KS waves multiply and eight load: address arithmetic between the MFMAs of three
+// waves took four times their time (2^20 pixels of 32 x 32 channels: 595 us, with
+// three loaders 490, with eight 326; the MFMAs alone 125).  A wave's sum is one chain
+// of dependent MFMAs, which take 50 ns each: 205 us is the least for a range.  LDS is double buffered, one barrier per chunk;
+// values are loaded two chunks ahead.  Odd pitches keep 32 channels on 32 banks.  The
+// loaders of the first taps also sum the bias gradient's partials (FP64).
+constexpr int kWgradLoaders = 8;
+
+// I: a byte offset into the tensors, 32 bits where they are below 4 GiB (one
+// addition per load instead of three).
+template <int KS, class I>
+__global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(WgradArgs a) {
+  constexpr int KK = KS * KS, P = KS / 2, NL = kWgradLoaders, NCH = 32 / NL;
+  constexpr int GP = kWgradChunk + 1, IP = (kWgradChunk + KS - 1) | 1;
+  __shared__ float lg[2][32 * GP];
+  __shared__ float li[2][32 * IP];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int HW = a.H * a.W, npix = a.B * HW;
+  const int ky = blockIdx.x % KS, ci0 = blockIdx.x / KS * 32, co0 = blockIdx.y * 32;
+  const int kbeg = blockIdx.z * kWgradPixels, kend = min(npix, kbeg + kWgradPixels);
+  const int chunks = (kend - kbeg + kWgradChunk - 1) / kWgradChunk;
+  // this lane's pixels of the chunk
+  PixelPos gp[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) gp[h].start(kbeg + lane + 64 * h, HW);
+  if (wave >= KS) {
+    // ---- loaders: channels w, w + NL, ... of both operands ----
+    const int w = wave - KS, te = w * 64 + lane;
+    // the staged run starts P before the chunk; its last KS - 1 values by thread
+    PixelPos ip[2], tail;
+#pragma unroll
+    for (int h = 0; h < 2; h++) ip[h].start(kbeg + lane + 64 * h - P, HW);
+    tail.start(kbeg + kWgradChunk - P + te % 2, HW);
+    float rg[2][NCH], rm[2][NCH], ri[2][NCH], re = 0.0f;
+    bool og[2];
+    double bs[NCH];
+#pragma unroll
+    for (int j = 0; j < NCH; j++) bs[j] = 0.0;
+    // how many of this wave's channels exist; a pixel out of range reads as that of
+    // element 0, a channel out of range as the last one, and both become zero when
+    // they are stored
+    const int ng = max(0, (a.Co - co0 - w + NL - 1) / NL);
+    const int ni = max(0, (a.Ci - ci0 - w + NL - 1) / NL);
+    const I plane = (I)HW * 4u, step = plane * NL, gi = plane * a.Co, ii = plane * a.Ci;
+    const I g0 = plane * (co0 + (ng ? w : 0)), i0 = plane * (ci0 + (ni ? w : 0));
+    const float* mask = a.out ? a.out : a.dout;
+    const int tc = te / 2;
+    const bool end = KS > 1 && te < 64, ot = end && ci0 + tc < a.Ci;
+    const I t0 = plane * (ci0 + (ot ? tc : 0));
+    auto at = [](const float* p, I k) { return *(const float*)((const char*)p + k); };
+    auto load = [&]() {
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        og[h] = gp[h].q < kend;
+        I k = og[h] ? gi * gp[h].b + (I)gp[h].p * 4u + g0 : 0;
+#pragma unroll
+        for (int j = 0; j < NCH; j++) {
+          rg[h][j] = at(a.dout, k);
+          rm[h][j] = at(mask, k);
+          k += j + 1 < ng ? step : 0;
+        }
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int p = ip[h].p + (ky - P) * a.W;
+        I k = ip[h].q < npix && p >= 0 && p < HW ? ii * ip[h].b + (I)p * 4u + i0 : 0;
+#pragma unroll
+        for (int j = 0; j < NCH; j++) {
+          ri[h][j] = at(a.in, k);
+          k += j + 1 < ni ? step : 0;
+        }
+      }
+      if (end) {
+        const int p = tail.p + (ky - P) * a.W;
+        re = at(a.in, tail.q < npix && p >= 0 && p < HW ? ii * tail.b + (I)p * 4u + t0 : 0);
+        tail.next(HW);
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        gp[h].next(HW);
+        ip[h].next(HW);
+      }
+    };
+    const bool all = !a.out;
+    auto store = [&](int buf) {
+      float* dg = &lg[buf][w * GP + lane];
+      float* di = &li[buf][w * IP + lane];
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int j = 0; j < NCH; j++) {
+          rg[h][j] = og[h] && j < ng && (all || rm[h][j] > 0.0f) ? rg[h][j] : 0.0f;
+          dg[j * NL * GP + 64 * h] = rg[h][j];
+          di[j * NL * IP + 64 * h] = j < ni ? ri[h][j] : 0.0f;
+        }
+      if (end) li[buf][tc * IP + kWgradChunk + te % 2] = ot ? re : 0.0f;
+      if (blockIdx.x == 0)
+#pragma unroll
+        for (int j = 0; j < NCH; j++) bs[j] += (double)rg[0][j] + (double)rg[1][j];
+    };
+    load();
+    store(0);
+    load();
     __syncthreads();
-    store();
-    __syncthreads();
+    for (int k = 1; k <= chunks; k++) {
+      if (k < chunks) {
+        store(k & 1);
+        load();
+      }
+      __syncthreads();
+    }
     if (blockIdx.x == 0) {
 #pragma unroll
-      for (int k = 0; k < WK; k++)
-        for (int q = t % TPC; q < Q; q += TPC) bsum += (double)lg[k][t / TPC * GP + q];
-    }
-    origins(tile + WK);  // (past the end: nothing is loaded)
-    constexpr int STEPS = Q / 2, LG = (NG + STEPS - 1) / STEPS, LI = (NIN + STEPS - 1) / STEPS;
-    // between two MFMAs: a value of the step after, and loads of the tiles after
-    float va[2], vb[2][KK];
-    auto read = [&](int s, int k) {
-      const int q = 2 * s;
-      if (k == 0) va[s & 1] = pa[q];
-      vb[s & 1][k] = pb[(q / kWgradW + k / KS) * PW + q % kWgradW + k % KS];
-    };
+      for (int j = 0; j < NCH; j++) {
+        const int c = w + j * NL;
+        double v = bs[j];
 #pragma unroll
-    for (int k = 0; k < KK; k++) read(0, k);
-#pragma unroll
-    for (int s = 0; s < STEPS; s++)
-#pragma unroll
-      for (int k = 0; k < KK; k++) {
-        __builtin_amdgcn_sched_barrier(0);
-        acc[k] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[s & 1], vb[s & 1][k], acc[k], 0, 0, 0);
-        if (s + 1 < STEPS) read(s + 1, k);
-#pragma unroll
-        for (int q = k; q < LG + LI; q += KK) {
-          if (q < LG && s * LG + q < NG) load_g(s * LG + q);
-          if (q >= LG && s * LI + q - LG < NIN) load_in(s * LI + q - LG);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+        if (lane == 0 && co0 + c < a.Co)
+          a.bpart[(long)blockIdx.z * a.Co + co0 + c] = v;
       }
+    }
+    return;
   }
-  float* dst = a.part + (long)(blockIdx.z * WK + wk) * a.Co * a.Ci * KK;
-  const int ci = ci0 + wn * 32 + lr;
+  // ---- the waves that multiply ----
+  const int lr = lane & 31, lh = lane >> 5;
+  const int kx = wave;
+  f32x16_t acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+  __syncthreads();
+  for (int k = 0; k < chunks; k++) {
+    // the chunk's pixels whose tap lies inside, as this half wave's bits
+    unsigned int bits[4];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      int y = (int)__umulhi((unsigned int)gp[h].p, a.rw), x = gp[h].p - y * a.W;
+      if (x < 0) {
+        y--;
+        x += a.W;
+      } else if (x >= a.W) {
+        y++;
+        x -= a.W;
+      }
+      x += kx - P;
+      y += ky - P;
+      const unsigned long long m =
+          __ballot(gp[h].q < kend && x >= 0 && x < a.W && y >= 0 && y < a.H) >> lh;
+      bits[2 * h] = (unsigned int)m;
+      bits[2 * h + 1] = (unsigned int)(m >> 32);
+      gp[h].next(HW);
+    }
+    const float* pa = &lg[k & 1][lr * GP + lh];
+    const float* pb = &li[k & 1][lr * IP + kx + lh];
+    // operands four steps ahead
+    constexpr int STEPS = kWgradChunk / 2, AHEAD = 4;
+    float va[AHEAD], vb[AHEAD];
+#pragma unroll
+    for (int s = 0; s < AHEAD; s++) {
+      va[s] = pa[2 * s];
+      vb[s] = pb[2 * s];
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+      // all ones where the pixel's bit is set
+      const int on = __builtin_amdgcn_sbfe((int)bits[s / 16], 2 * s % 32, 1);
+      const float x = __int_as_float(__float_as_int(vb[s % AHEAD]) & on);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(va[s % AHEAD], x, acc, 0, 0, 0);
+      if (s + AHEAD < STEPS) {
+        va[s % AHEAD] = pa[2 * (s + AHEAD)];
+        vb[s % AHEAD] = pb[2 * (s + AHEAD)];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+  }
+  float* dst = a.part + (long)blockIdx.z * a.Co * a.Ci * KK;
+  const int ci = ci0 + lr;
 #pragma unroll
   for (int e = 0; e < 16; e++) {
-    const int co = co0 + wm * 32 + 8 * (e >> 2) + 4 * lh + (e & 3);
-    if (co >= a.Co || ci >= a.Ci) continue;
-#pragma unroll
-    for (int k = 0; k < KK; k++) dst[((long)co * a.Ci + ci) * KK + k] = acc[k][e];
-  }
-  if (blockIdx.x == 0) {
-#pragma unroll
-    for (int o = TPC / 2; o > 0; o >>= 1) bsum += __shfl_down(bsum, o, TPC);
-    const int co = co0 + t / TPC;
-    if (t % TPC == 0 && co < a.Co) a.bpart[(long)blockIdx.z * a.Co + co] = bsum;
+    const int co = co0 + 8 * (e >> 2) + 4 * lh + (e & 3);
+    if (co < a.Co && ci < a.Ci) dst[((long)co * a.Ci + ci) * KK + ky * KS + kx] = acc[e];
   }
 }
 
 // dw = the FP64 sum of the weight-grad partials, dbias that of the bias partials,
-// in a fixed order: SEG threads take a run of an element's partials each, and their
-// sums are added in order.  (One thread per element leaves most of the chip idle
-// where there are many partials of few weights: 9216 weights of 2048 partials took
-// 152 us.)
-template <int SEG>
+// in the ranges' order.
 __global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restrict__ part, int npart,
                                                           long n, float* __restrict__ dw,
-                                                          const double* __restrict__ bpart,
-                                                          int nbpart, int Co,
+                                                          const double* __restrict__ bpart, int Co,
                                                           float* __restrict__ dbias) {
-  constexpr int E = kT / SEG;  // elements of a block
-  __shared__ double seg[SEG][E];
-  const int e = threadIdx.x % E, sg = threadIdx.x / E;
-  const long i = (long)blockIdx.x * E + e;
+  const long i = blockIdx.x * (long)kT + threadIdx.x;
   double s = 0.0;
   if (i < n) {
-    const int per = (npart + SEG - 1) / SEG, last = min(npart, (sg + 1) * per);
-    int r = sg * per;
-    for (; r + 8 <= last; r += 8) {
-      float v[8];
+    int r = 0;
+    for (; r + 16 <= npart; r += 16) {
+      float v[16];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = part[(long)(r + u) * n + i];
+      for (int u = 0; u < 16; u++) v[u] = part[(long)(r + u) * n + i];
 #pragma unroll
-      for (int u = 0; u < 8; u++) s += (double)v[u];
+      for (int u = 0; u < 16; u++) s += (double)v[u];
     }
-    for (; r < last; r++) s += (double)part[(long)r * n + i];
-  } else if (i < n + Co) {
-    const int per = (nbpart + SEG - 1) / SEG, last = min(nbpart, (sg + 1) * per);
-    for (int r = sg * per; r < last; r++) s += bpart[(long)r * Co + (i - n)];
-  }
-  if constexpr (SEG > 1) {
-    seg[sg][e] = s;
-    __syncthreads();
-    if (sg) return;
-    for (int q = 1; q < SEG; q++) s += seg[q][e];
-  }
-  if (i < n)
+    for (; r < npart; r++) s += (double)part[(long)r * n + i];
     dw[i] = (float)s;
-  else if (i < n + Co)
+  } else if (i < n + Co) {
+    for (int r = 0; r < npart; r++) s += bpart[(long)r * Co + (i - n)];
     dbias[i - n] = (float)s;
+  }
 }
 
 // Pooling, upsampling and channel copies move memory and nothing else.  A block
@@ -687,46 +746,14 @@ gvm_status conv_fwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   return launched("gvm_nn_conv_fwd");
 }
 
-// The weight gradient's launch: how many waves cover channels, and how many
-// partials a sum over the pixels is cut into.
-struct WgradPlan {
-  int wm, wn, wk, sh, tiles_x, tiles_y, ntiles, per, nsplit;
-};
-
-WgradPlan wgrad_plan(int B, int Ci, int Co, int H, int W) {
-  WgradPlan p{};
-  const int nco = (Co + 31) / 32, nci = (Ci + 31) / 32;
-  p.wm = nco % 2 == 0 || nco > 4 ? 2 : 1;
-  p.wn = nci % 2 == 0 || nci > 4 ? 2 : 1;
-  p.wk = 4 / (p.wm * p.wn);
-  p.sh = p.wk == 1 ? 4 : 2;
-  p.tiles_x = (W + kWgradW - 1) / kWgradW;
-  p.tiles_y = (H + p.sh - 1) / p.sh;
-  p.ntiles = B * p.tiles_x * p.tiles_y;
-  // about two rounds of one block per CU, partials of at most 8192 pixels (the FP32 sums
-  // stay short), at least four rounds of tiles per block
-  const long blocks = (long)((Co + 32 * p.wm - 1) / (32 * p.wm)) * ((Ci + 32 * p.wn - 1) / (32 * p.wn));
-  const long most = std::max(1L, (long)p.ntiles / (4 * p.wk));
-  const long fill = std::min(most, std::max(1L, 512 / blocks));
-  const long pixels = ((long)p.ntiles * p.sh * kWgradW + 8192L * p.wk - 1) / (8192L * p.wk);
-  const long want = std::max(fill, pixels);
-  p.per = (int)(((p.ntiles + want - 1) / want + p.wk - 1) / p.wk * p.wk);
-  p.nsplit = (p.ntiles + p.per - 1) / p.per;
-  return p;
-}
-
 template <int KS>
-void launch_wgrad(gvm_ctx* ctx, const WgradPlan& p, const WgradArgs& a) {
-  const dim3 grid((unsigned)((a.Ci + 32 * p.wn - 1) / (32 * p.wn)),
-                  (unsigned)((a.Co + 32 * p.wm - 1) / (32 * p.wm)), (unsigned)p.nsplit);
-  if (p.wm == 2 && p.wn == 2)
-    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 2, 2, 1, 4>), grid, dim3(256), 0, ctx->stream, a);
-  else if (p.wm == 2)
-    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 2, 1, 2, 2>), grid, dim3(256), 0, ctx->stream, a);
-  else if (p.wn == 2)
-    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 1, 2, 2, 2>), grid, dim3(256), 0, ctx->stream, a);
+void launch_wgrad(gvm_ctx* ctx, const WgradArgs& a, int ranges) {
+  const dim3 grid((unsigned)((a.Ci + 31) / 32 * KS), (unsigned)((a.Co + 31) / 32), (unsigned)ranges);
+  const dim3 block(64 * (KS + kWgradLoaders));
+  if ((long)a.B * std::max(a.Ci, a.Co) * a.H * a.W < (1L << 30))
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, unsigned int>), grid, block, 0, ctx->stream, a);
   else
-    hipLaunchKernelGGL((conv_wgrad_kernel<KS, 1, 1, 4, 2>), grid, dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL((conv_wgrad_kernel<KS, unsigned long>), grid, block, 0, ctx->stream, a);
 }
 
 template <class WT>
@@ -751,11 +778,10 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   }
   // weight and bias gradients: partials in the context's network workspace (the
   // bias's first, in FP64), then their FP64 sums
-  const WgradPlan p = wgrad_plan(B, Ci, Co, H, W);
+  const int ranges = (int)(((long)B * H * W + kWgradPixels - 1) / kWgradPixels);
   const long nw = (long)Co * Ci * K * K;
-  const int npart = p.nsplit * p.wk;
-  const size_t bias_elems = 2 * (size_t)p.nsplit * Co;
-  const size_t need = bias_elems + (size_t)npart * nw;
+  const size_t bias_elems = 2 * (size_t)ranges * Co;
+  const size_t need = bias_elems + (size_t)ranges * nw;
   if (need > ctx->nn_part_elems) {
     GVM_REQUIRE(!ctx->capturing, "gvm_nn_conv_bwd: the workspace would grow under capture");
     GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -765,18 +791,14 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     GVM_HIP_TRY(hipMalloc((void**)&ctx->nn_part, sizeof(float) * need));
     ctx->nn_part_elems = need;
   }
-  const WgradArgs a{in,  mask, dout, ctx->nn_part + bias_elems, (double*)ctx->nn_part, B, Ci, Co, H,
-                    W,   p.tiles_x, p.tiles_y, p.ntiles, p.per};
+  const WgradArgs a{in, mask, dout, ctx->nn_part + bias_elems, (double*)ctx->nn_part, B, Ci, Co, H,
+                    W,  (unsigned int)std::min(0xffffffffUL, ((1UL << 32) + W - 1) / W)};
   if (K == 3)
-    launch_wgrad<3>(ctx, p, a);
+    launch_wgrad<3>(ctx, a, ranges);
   else
-    launch_wgrad<1>(ctx, p, a);
-  if (npart >= 32)
-    hipLaunchKernelGGL(wgrad_reduce_kernel<8>, dim3((unsigned)((nw + Co + kT / 8 - 1) / (kT / 8))),
-                       dim3(kT), 0, ctx->stream, a.part, npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
-  else
-    hipLaunchKernelGGL(wgrad_reduce_kernel<1>, dim3((unsigned)((nw + Co + kT - 1) / kT)), dim3(kT), 0,
-                       ctx->stream, a.part, npart, nw, dw, a.bpart, p.nsplit, Co, dbias);
+    launch_wgrad<1>(ctx, a, ranges);
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((nw + Co + kT - 1) / kT)), dim3(kT), 0,
+                     ctx->stream, a.part, ranges, nw, dw, a.bpart, Co, dbias);
   return launched("gvm_nn_conv_bwd");
 }
 

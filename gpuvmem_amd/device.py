@@ -198,10 +198,17 @@ class Context:
         native.check(self.lib.gvm_get_split_vis(self.ctx, C.byref(v)), "gvm_get_split_vis")
         return v.value
 
+    def adjoint_gridded(self) -> bool:
+        """gvm_adjoint_gridded: whether the last gradient ran by gridding and
+        FFT."""
+        v = C.c_int()
+        native.check(self.lib.gvm_adjoint_gridded(self.ctx, C.byref(v)), "gvm_adjoint_gridded")
+        return bool(v.value)
+
     def adjoint_computed_pixels(self) -> int:
         """gvm_adjoint_computed_pixels: the pixels whose sums the adjoint of
-        the current form computes (the work of one launch is 4 x this x the
-        visibilities)."""
+        the current form computes as a GEMM or as the direct sum (then the work
+        of one launch is 4 x this x the visibilities)."""
         v = C.c_long()
         native.check(self.lib.gvm_adjoint_computed_pixels(self.ctx, C.byref(v)),
                      "gvm_adjoint_computed_pixels")

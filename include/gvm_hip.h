@@ -207,8 +207,11 @@ gvm_status gvm_num_slices(const gvm_ctx* ctx, int* n);
 /* Copy of the geometry the context was created with. */
 gvm_status gvm_get_geometry(const gvm_ctx* ctx, gvm_geometry* out);
 
-/* Adjoint form used by gvm_dchi2 (GVM_ADJOINT_*; default GVM_ADJOINT_BF16X3: on
- * MI355X it is the faster split form and the more accurate one at 1024^2). */
+/* Adjoint form used by gvm_dchi2 (GVM_ADJOINT_*; default GVM_ADJOINT_BF16X3).
+ * F32, F16X3 and BF16X3 all run by gridding and FFT where that applies (sums of a
+ * few 1e-7, below each of theirs); the form then only matters for the GEMM that
+ * takes over: few visibilities on images of 2048^2 and more, or w terms that need
+ * more than 32 planes.  DIRECT always is the direct sum. */
 gvm_status gvm_set_adjoint(gvm_ctx* ctx, int mode);
 
 /* ---- objective: chi2 ----------------------------------------------------- */
@@ -484,8 +487,8 @@ gvm_status gvm_timing_adjoint_ms(gvm_ctx* ctx, double* avg_ms, long* count);
 
 /* ---- adjoint K tile: the visibility-range length ------------------------ */
 /* No counterpart in the reference.  It has no effect while the adjoint runs by
- * gridding and FFT.  Each workgroup of the split-precision adjoint accumulates one 256 x 256 output tile over a range of about
- * `split_vis` visibilities in FP32 (the ranges are summed in FP64): shorter
+ * gridding and FFT.  Each workgroup of the split-precision adjoint accumulates
+ * one 256 x 256 output tile over a range of about `split_vis` visibilities in FP32 (the ranges are summed in FP64): shorter
  * ranges keep the FP32 accumulation short, longer ones write fewer partial
  * tiles.  Default 6144, and 3072 for images of 2048^2 and larger (where
  * ranges of 6144 bring the gradient's relative error near 1e-5); allowed
@@ -499,11 +502,14 @@ gvm_status gvm_set_fft_mode(gvm_ctx* ctx, int mode);
 gvm_status gvm_get_split_vis(const gvm_ctx* ctx, long* split_vis);
 /* No counterpart in the reference (whose DChi2 computes the pixels on the
  * mask, noise < noise_cut): the pixels whose sums the adjoint of the current
- * form computes when it runs as a GEMM or as the direct sum.  The split-precision GEMM computes the 128 x 64 sub-tiles of
- * its workgroup tiles that hold a pixel on the mask and skips the others; the
+ * form computes when it runs as a GEMM or as the direct sum.  The
+ * split-precision GEMM computes the 128 x 64 sub-tiles of its workgroup tiles that hold a pixel on the mask and skips the others; the
  * direct form, its blocks of 256 consecutive pixels that hold one.  The work
  * of one adjoint launch is 4 x pixels x visibilities flop. */
 gvm_status gvm_adjoint_computed_pixels(const gvm_ctx* ctx, long* pixels);
+/* 1 when the last gvm_dchi2 ran by gridding and FFT, 0 when it ran as a GEMM or
+ * as the direct sum (for measurement). */
+gvm_status gvm_adjoint_gridded(const gvm_ctx* ctx, int* gridded);
 /* Autotuner: times the adjoint of the current residuals (a gvm_chi2 must
  * have run) for each candidate range length (NULL: 1536, 2048, 3072, 4096,
  * 6144, 8192, up to 3072 for images of 2048^2 and larger), with HIP events,
