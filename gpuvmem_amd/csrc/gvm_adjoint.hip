@@ -671,10 +671,14 @@ gvm_status build_splits(gvm_ctx* ctx, int mode, int ntiles, long n) {
 
 // Fewer rows than this over all slices: the GEMM is the faster one.  The
 // gridded form's time is that of its FFTs, the GEMM's falls with the rows:
-// one evaluation at 2048^2 takes 226 / 163 us (gridded / GEMM) at 30 rows, 248
-// / 270 at 840, 264 / 307 at 5,700; at 4096^2 881 / 631, 1005 / 820, 1160 / 1332;
-// at 1024^2 and below the gridded form is faster from 30 rows on (73 / 80).
-static long min_gridded_rows(int N) { return N < 2048 ? 0 : (long)N * N / 8192; }
+// one evaluation at 2048^2 takes 210 / 161 us (gridded / GEMM) at 30 rows, 234
+// / 267 at 840, 249 / 306 at 5,700; at 4096^2 904 / 628, 1001 / 822, 1101 / 1331;
+// at 1024^2, where launches decide (the GEMM has one less), 81 / 75, 86 / 77,
+// 88 / 140.  Below that the two are alike up to about 1,000 rows, and the gridded
+// form is the more accurate one (1e-7 against 1e-6).
+static long min_gridded_rows(int N) {
+  return N < 1024 ? 0 : N == 1024 ? 1024 : (long)N * N / 8192;
+}
 
 // Decides how the adjoint of the current form runs and sizes its workspace:
 // the GEMM forms by gridding and FFT (gvm_adjoint_fft.hip) where that applies,

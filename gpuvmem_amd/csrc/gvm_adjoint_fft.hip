@@ -272,9 +272,10 @@ __global__ void pick_kernel(const unsigned int* __restrict__ islot,
 // leaves it in LDS; then four rows per step, lane l evaluates the kernel of
 // row l / 16 at grid row and column l % 16, and the planes' products go to
 // v_mfma_f32_16x16x4_f32 (A: ky, B: kx c T_k; real and imaginary parts).
-// Per step and wave 2 NP MFMAs of 32 cycles against about 50 VALU
-// instructions: at NP = 4 the MFMA pipe bounds it, 64 cycles per visibility,
-// 54 us of the chip for 1.76 M visibilities at 2 GHz.
+// Per step and wave 2 NP MFMAs of 32 cycles against about 50 VALU instructions,
+// which take as long at NP = 4: the next step's operands are formed between this
+// step's MFMAs (in turn: 128 us for 1.76 M visibilities, so: 117; the MFMAs alone
+// would take 46).  A block is one wave (four held a CU until the longest was done).
 template <int NP>
 __global__ __launch_bounds__(64) void spread_kernel(
     const long4* __restrict__ items, long slot0, const float4* __restrict__ rec,
@@ -479,7 +480,8 @@ __device__ __forceinline__ float2 folded_cell(const float2* __restrict__ part,
 // columns (a divisor of four, so they share their two tile columns) of one
 // plane per block.  The tiles' slots are staged in LDS and two columns are
 // loaded at a time, so that a thread keeps sixteen loads in flight: a gather
-// through slots in memory waited twice per cell and took 97 us at 1024^2.
+// through slots in memory waited twice per cell and took 97 us at 1024^2, staged
+// 45, and 42 since blocks without rows leave at the edges too.
 template <int N, int BC, int T>
 __global__ __launch_bounds__(T) void grid_cols_kernel(const float2* __restrict__ part,
                                                       const int* __restrict__ tile_slot, int slot0,
@@ -607,7 +609,7 @@ __device__ __forceinline__ float chain_rule(float r, float d, float nudiv, float
 // inputs X and N - X need the same two values.  A plane's weight at a pixel is
 // zeta^k times a power series in zeta^2; the series' coefficients are read from
 // LDS, once for all of a thread's pixels (from memory, per pixel, they were two
-// thirds of the kernel's loads and took 310 us at 2048^2 with 6 planes).
+// thirds of the kernel's loads: 310 us at 2048^2 with 6 planes, now 185).
 template <int N, int B, int T>
 __global__ __launch_bounds__(T, 4) void grid_rows_kernel(RowsArgs a) {
   __shared__ float2 lds[B * N];

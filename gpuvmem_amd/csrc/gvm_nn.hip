@@ -42,8 +42,11 @@ __device__ __forceinline__ float wload(const unsigned short* w, long i) {
 // kernel that keeps its index arithmetic out of the loop runs at its rate (154
 // TFLOP/s measured): pixels are tiled in the image's plane, a tile with its halo
 // is staged in LDS once per chunk of channels and read at nine shifts, and the
-// addresses of a thread's loads are computed once per block.  (An im2col loop
-// that formed every element's coordinates as it loaded it ran at 26 TFLOP/s.)
+// addresses of a thread's loads are computed once per block.  Weights are read
+// along memory (lanes a row apart read 64 lines per load: 326 against 235 us for 512
+// channels at 32 x 32 x 4) and no load sits in a branch of its own.  Forward and
+// input gradient run at 90-110 TFLOP/s.  (An im2col loop that formed every
+// element's coordinates as it loaded it ran at 26.)
 // ---------------------------------------------------------------------------
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 enum { CONV_FWD = 0, CONV_BWD_DATA = 1 };
@@ -716,7 +719,10 @@ void launch_tile(gvm_ctx* ctx, ConvArgs<WT> a) {
 }
 
 // The tile: 8 x 32 pixels and 64 channels (32 where there are no more) when that
-// fills the chip, else 8 x 8 pixels and 64 channels.
+// gives every CU two blocks, else 8 x 8 pixels and 64 channels.  The wide tile reads
+// each weight for four times the pixels: layers of 19 GFLOP take 170-183 us with it
+// (64 channels at 256 x 256 x 4) and 207-220 with the narrow one (256 channels at 64 x
+// 64 x 4, 512 at 32 x 32 x 4), where it would have 256 and 128 blocks for 256 CUs.
 template <int MODE, int KS, class WT>
 void conv_tile(gvm_ctx* ctx, const ConvArgs<WT>& a) {
   constexpr int CK = KS == 3 ? 8 : 32;
