@@ -492,7 +492,21 @@ __global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restric
 // takes part of one plane (blockIdx.y: the planes, a grid-stride loop), so that an
 // index is split once, in 32 bits, and a thread moves V values with a wide access.
 // (One value per thread and three 64-bit divisions: upsampling to 1024 x 1024 x 32
-// took 129 us, 1.3 TB/s.)
+// took 129 us, 1.3 TB/s.)  Planes of fewer units than a block has threads are taken
+// `group` at a time: one by one, 65,536 planes of 4 x 4 took 30 us, most threads idle.
+template <class I, class F>
+__device__ __forceinline__ void for_planes(long planes, int group, I n, F f) {
+  if (group == 1) {
+    for (long p = blockIdx.y; p < planes; p += gridDim.y)
+      for (I o = blockIdx.x * (I)kT + threadIdx.x; o < n; o += (I)gridDim.x * kT) f(p, o);
+    return;
+  }
+  // group * n <= kT: one pass of the block
+  const int q = threadIdx.x / (int)n, o = threadIdx.x - q * (int)n;
+  if (q >= group) return;
+  for (long p = (long)blockIdx.y * group + q; p < planes; p += (long)gridDim.y * group) f(p, (I)o);
+}
+
 template <int V>
 struct Vec;
 template <>
@@ -511,27 +525,27 @@ struct Vec<4> {
 // V pixels of two rows of `in` averaged by pairs: V / 2 pixels (V = 2: one).
 template <int V, class I>
 __global__ __launch_bounds__(kT) void pool_fwd_kernel(const float* __restrict__ in,
-                                                      float* __restrict__ out, long nbc, I H, I W) {
+                                                      float* __restrict__ out, long nbc, int group,
+                                                      I H, I W) {
   typedef typename Vec<V>::type vin;
   typedef typename Vec<V / 2>::type vout;
-  const I h = H / 2, w = W / 2, wv = W / V, n = h * wv;
-  for (long c = blockIdx.y; c < nbc; c += gridDim.y)
-    for (I o = blockIdx.x * (I)kT + threadIdx.x; o < n; o += (I)gridDim.x * kT) {
-      const I y = o / wv, x = o - y * wv;
-      const float* s = in + c * ((long)H * W) + (long)(2 * y) * W + x * V;
-      vin r[2];
-      // V = 2: W is even, but a row may start at any 4 bytes
-      __builtin_memcpy(&r[0], V == 4 ? __builtin_assume_aligned(s, 16) : s, sizeof(vin));
-      __builtin_memcpy(&r[1], V == 4 ? __builtin_assume_aligned(s + W, 16) : s + W, sizeof(vin));
-      vout v;
-      if constexpr (V == 4) {
-        v[0] = 0.25f * ((r[0][0] + r[0][1]) + (r[1][0] + r[1][1]));
-        v[1] = 0.25f * ((r[0][2] + r[0][3]) + (r[1][2] + r[1][3]));
-      } else {
-        v = 0.25f * ((r[0][0] + r[0][1]) + (r[1][0] + r[1][1]));
-      }
-      *(vout*)(out + c * ((long)h * w) + (long)y * w + x * (V / 2)) = v;
+  const I h = H / 2, w = W / 2, wv = W / V;
+  for_planes(nbc, group, h * wv, [&](long c, I o) {
+    const I y = o / wv, x = o - y * wv;
+    const float* s = in + c * ((long)H * W) + (long)(2 * y) * W + x * V;
+    vin r[2];
+    // V = 2: W is even, but a row may start at any 4 bytes
+    __builtin_memcpy(&r[0], V == 4 ? __builtin_assume_aligned(s, 16) : s, sizeof(vin));
+    __builtin_memcpy(&r[1], V == 4 ? __builtin_assume_aligned(s + W, 16) : s + W, sizeof(vin));
+    vout v;
+    if constexpr (V == 4) {
+      v[0] = 0.25f * ((r[0][0] + r[0][1]) + (r[1][0] + r[1][1]));
+      v[1] = 0.25f * ((r[0][2] + r[0][3]) + (r[1][2] + r[1][3]));
+    } else {
+      v = 0.25f * ((r[0][0] + r[0][1]) + (r[1][0] + r[1][1]));
     }
+    *(vout*)(out + c * ((long)h * w) + (long)y * w + x * (V / 2)) = v;
+  });
 }
 
 // out[b][c0 + c][Y][X] = scale in[b][c][Y/2][X/2]: V / 2 pixels to V pixels of two
@@ -539,66 +553,62 @@ __global__ __launch_bounds__(kT) void pool_fwd_kernel(const float* __restrict__ 
 template <int V, class I>
 __global__ __launch_bounds__(kT) void up_kernel(const float* __restrict__ in,
                                                 float* __restrict__ out, int B, int C, int Cd,
-                                                int c0, I H, I W, float scale) {
+                                                int c0, int group, I H, I W, float scale) {
   typedef typename Vec<V / 2>::type vin;
   typedef typename Vec<V>::type vout;
-  const I W2 = 2 * W, wv = W2 / V, n = H * wv;
-  for (long p = blockIdx.y; p < (long)B * C; p += gridDim.y) {
+  const I W2 = 2 * W, wv = W2 / V;
+  for_planes((long)B * C, group, H * wv, [&](long p, I o) {
     const long b = p / C, c = p - b * C;
-    for (I o = blockIdx.x * (I)kT + threadIdx.x; o < n; o += (I)gridDim.x * kT) {
-      const I y = o / wv, x = o - y * wv;
-      const vin r = scale * *(const vin*)(in + p * ((long)H * W) + (long)y * W + x * (V / 2));
-      vout v;
-      if constexpr (V == 4)
-        v = vout{r[0], r[0], r[1], r[1]};
-      else
-        v = vout{r, r};
-      float* d = out + (b * Cd + c0 + c) * (4 * (long)H * W) + (long)(2 * y) * W2 + x * V;
-      __builtin_memcpy(V == 4 ? __builtin_assume_aligned(d, 16) : d, &v, sizeof(vout));
-      __builtin_memcpy(V == 4 ? __builtin_assume_aligned(d + W2, 16) : d + W2, &v, sizeof(vout));
-    }
-  }
+    const I y = o / wv, x = o - y * wv;
+    const vin r = scale * *(const vin*)(in + p * ((long)H * W) + (long)y * W + x * (V / 2));
+    vout v;
+    if constexpr (V == 4)
+      v = vout{r[0], r[0], r[1], r[1]};
+    else
+      v = vout{r, r};
+    float* d = out + (b * Cd + c0 + c) * (4 * (long)H * W) + (long)(2 * y) * W2 + x * V;
+    __builtin_memcpy(V == 4 ? __builtin_assume_aligned(d, 16) : d, &v, sizeof(vout));
+    __builtin_memcpy(V == 4 ? __builtin_assume_aligned(d + W2, 16) : d + W2, &v, sizeof(vout));
+  });
 }
 
 // din[b][c][y][x] = sum of the four dout[b][c0 + c][2y + dy][2x + dx]
 template <int V, class I>
 __global__ __launch_bounds__(kT) void up_bwd_kernel(const float* __restrict__ dout,
                                                     float* __restrict__ din, int B, int C, int Cd,
-                                                    int c0, I H, I W) {
+                                                    int c0, int group, I H, I W) {
   typedef typename Vec<V>::type vin;
   typedef typename Vec<V / 2>::type vout;
-  const I W2 = 2 * W, wv = W2 / V, n = H * wv;
-  for (long p = blockIdx.y; p < (long)B * C; p += gridDim.y) {
+  const I W2 = 2 * W, wv = W2 / V;
+  for_planes((long)B * C, group, H * wv, [&](long p, I o) {
     const long b = p / C, c = p - b * C;
-    for (I o = blockIdx.x * (I)kT + threadIdx.x; o < n; o += (I)gridDim.x * kT) {
-      const I y = o / wv, x = o - y * wv;
-      const float* s = dout + (b * Cd + c0 + c) * (4 * (long)H * W) + (long)(2 * y) * W2 + x * V;
-      vin r[2];
-      __builtin_memcpy(&r[0], V == 4 ? __builtin_assume_aligned(s, 16) : s, sizeof(vin));
-      __builtin_memcpy(&r[1], V == 4 ? __builtin_assume_aligned(s + W2, 16) : s + W2, sizeof(vin));
-      vout v;
-      if constexpr (V == 4) {
-        v[0] = (r[0][0] + r[0][1]) + (r[1][0] + r[1][1]);
-        v[1] = (r[0][2] + r[0][3]) + (r[1][2] + r[1][3]);
-      } else {
-        v = (r[0][0] + r[0][1]) + (r[1][0] + r[1][1]);
-      }
-      *(vout*)(din + p * ((long)H * W) + (long)y * W + x * (V / 2)) = v;
+    const I y = o / wv, x = o - y * wv;
+    const float* s = dout + (b * Cd + c0 + c) * (4 * (long)H * W) + (long)(2 * y) * W2 + x * V;
+    vin r[2];
+    __builtin_memcpy(&r[0], V == 4 ? __builtin_assume_aligned(s, 16) : s, sizeof(vin));
+    __builtin_memcpy(&r[1], V == 4 ? __builtin_assume_aligned(s + W2, 16) : s + W2, sizeof(vin));
+    vout v;
+    if constexpr (V == 4) {
+      v[0] = (r[0][0] + r[0][1]) + (r[1][0] + r[1][1]);
+      v[1] = (r[0][2] + r[0][3]) + (r[1][2] + r[1][3]);
+    } else {
+      v = (r[0][0] + r[0][1]) + (r[1][0] + r[1][1]);
     }
-  }
+    *(vout*)(din + p * ((long)H * W) + (long)y * W + x * (V / 2)) = v;
+  });
 }
 
 template <int V, class I>
 __global__ __launch_bounds__(kT) void copy_channels_kernel(const float* __restrict__ src,
                                                            float* __restrict__ dst, int B, int C,
-                                                           int Cs, int s0, int Cd, int d0, I HW) {
+                                                           int Cs, int s0, int Cd, int d0,
+                                                           int group, I HW) {
   typedef typename Vec<V>::type vec;
-  for (long p = blockIdx.y; p < (long)B * C; p += gridDim.y) {
+  for_planes((long)B * C, group, (I)(HW / V), [&](long p, I o) {
     const long b = p / C, c = p - b * C;
-    const vec* s = (const vec*)(src + (b * Cs + s0 + c) * (long)HW);
-    vec* d = (vec*)(dst + (b * Cd + d0 + c) * (long)HW);
-    for (I o = blockIdx.x * (I)kT + threadIdx.x; o < HW / V; o += (I)gridDim.x * kT) d[o] = s[o];
-  }
+    ((vec*)(dst + (b * Cd + d0 + c) * (long)HW))[o] =
+        ((const vec*)(src + (b * Cs + s0 + c) * (long)HW))[o];
+  });
 }
 
 __global__ __launch_bounds__(kT) void add_kernel(const float* __restrict__ src,
@@ -690,10 +700,14 @@ namespace {
 
 bool aligned(const void* p, size_t n) { return (uintptr_t)p % n == 0; }
 
+// Planes of n units that a block takes at a time.
+int plane_group(long n) { return (int)std::max(1L, kT / n); }
+
 // Blocks for n units of each of `planes` planes.
 dim3 plane_grid(long n, long planes) {
+  const int group = plane_group(n);
   return dim3((unsigned)std::max(1L, std::min(65535L, (n + kT - 1) / kT)),
-              (unsigned)std::min(65535L, planes));
+              (unsigned)std::min(65535L, (planes + group - 1) / group));
 }
 
 // The variant of a plane kernel: four values a thread where rows and pointers allow
@@ -849,8 +863,9 @@ extern "C" gvm_status gvm_nn_pool_fwd(gvm_ctx* ctx, const float* in, float* out,
   plane_launch(H * (long)W, W % 4 == 0 && aligned(in, 16) && aligned(out, 8), [&](auto v, auto i) {
     constexpr int V = v.value;
     typedef decltype(i) I;
-    hipLaunchKernelGGL((pool_fwd_kernel<V, I>), plane_grid((long)H / 2 * (W / V), (long)B * C),
-                       dim3(kT), 0, ctx->stream, in, out, (long)B * C, (I)H, (I)W);
+    const long n = (long)H / 2 * (W / V);
+    hipLaunchKernelGGL((pool_fwd_kernel<V, I>), plane_grid(n, (long)B * C), dim3(kT), 0,
+                       ctx->stream, in, out, (long)B * C, plane_group(n), (I)H, (I)W);
   });
   return launched("gvm_nn_pool_fwd");
 }
@@ -863,9 +878,10 @@ extern "C" gvm_status gvm_nn_pool_bwd(gvm_ctx* ctx, const float* dout, float* di
                [&](auto v, auto i) {
                  constexpr int V = v.value;
                  typedef decltype(i) I;
-                 hipLaunchKernelGGL((up_kernel<V, I>),
-                                    plane_grid((long)H / 2 * (W / V), (long)B * C), dim3(kT), 0,
-                                    ctx->stream, dout, din, B, C, C, 0, (I)(H / 2), (I)(W / 2), 0.25f);
+                 const long n = (long)H / 2 * (W / V);
+                 hipLaunchKernelGGL((up_kernel<V, I>), plane_grid(n, (long)B * C), dim3(kT), 0,
+                                    ctx->stream, dout, din, B, C, C, 0, plane_group(n),
+                                    (I)(H / 2), (I)(W / 2), 0.25f);
                });
   return launched("gvm_nn_pool_bwd");
 }
@@ -878,9 +894,10 @@ extern "C" gvm_status gvm_nn_up_fwd(gvm_ctx* ctx, const float* in, float* out, i
                [&](auto v, auto i) {
                  constexpr int V = v.value;
                  typedef decltype(i) I;
-                 hipLaunchKernelGGL((up_kernel<V, I>),
-                                    plane_grid((long)H * (2L * W / V), (long)B * C), dim3(kT), 0,
-                                    ctx->stream, in, out, B, C, Cd, c0, (I)H, (I)W, 1.0f);
+                 const long n = (long)H * (2L * W / V);
+                 hipLaunchKernelGGL((up_kernel<V, I>), plane_grid(n, (long)B * C), dim3(kT), 0,
+                                    ctx->stream, in, out, B, C, Cd, c0, plane_group(n), (I)H, (I)W,
+                                    1.0f);
                });
   return launched("gvm_nn_up_fwd");
 }
@@ -893,9 +910,10 @@ extern "C" gvm_status gvm_nn_up_bwd(gvm_ctx* ctx, const float* dout, float* din,
                [&](auto v, auto i) {
                  constexpr int V = v.value;
                  typedef decltype(i) I;
-                 hipLaunchKernelGGL((up_bwd_kernel<V, I>),
-                                    plane_grid((long)H * (2L * W / V), (long)B * C), dim3(kT), 0,
-                                    ctx->stream, dout, din, B, C, Cd, c0, (I)H, (I)W);
+                 const long n = (long)H * (2L * W / V);
+                 hipLaunchKernelGGL((up_bwd_kernel<V, I>), plane_grid(n, (long)B * C), dim3(kT), 0,
+                                    ctx->stream, dout, din, B, C, Cd, c0, plane_group(n), (I)H,
+                                    (I)W);
                });
   return launched("gvm_nn_up_bwd");
 }
@@ -907,12 +925,13 @@ extern "C" gvm_status gvm_nn_copy_channels(gvm_ctx* ctx, const float* src, float
               "gvm_nn_copy_channels: bad sizes");
   const bool wide = HW % 4 == 0 && aligned(src, 16) && aligned(dst, 16);
   const dim3 grid = plane_grid(wide ? HW / 4 : HW, (long)B * C);
+  const int group = plane_group(wide ? HW / 4 : HW);
   if (wide)
     hipLaunchKernelGGL((copy_channels_kernel<4, int>), grid, dim3(kT), 0, ctx->stream, src, dst, B,
-                       C, Cs, s0, Cd, d0, HW);
+                       C, Cs, s0, Cd, d0, group, HW);
   else
     hipLaunchKernelGGL((copy_channels_kernel<1, long>), grid, dim3(kT), 0, ctx->stream, src, dst, B,
-                       C, Cs, s0, Cd, d0, (long)HW);
+                       C, Cs, s0, Cd, d0, group, (long)HW);
   return launched("gvm_nn_copy_channels");
 }
 

@@ -119,3 +119,34 @@ def test_plane_kernels_at_every_alignment(ctx, H, W, shift):
                           atol=16 * EPS * float(x.abs().max()))
     got = run(lib.gvm_nn_copy_channels, (B, Cd, H, W), B, 2, Cc, 1, Cd, 2, H * W)
     assert torch.equal(got[:, 2:4], x[:, 1:]) and not got[:, :2].any() and not got[:, 4].any()
+
+
+@pytest.mark.parametrize("B,C,H,W,shift", [(300, 7, 2, 2, 0), (41, 5, 4, 4, 0), (9, 13, 6, 10, 1),
+                                           (1, 1, 2, 2, 0), (700, 100, 2, 4, 0)])
+def test_planes_smaller_than_a_block(ctx, B, C, H, W, shift):
+    """Several planes per block, whose count they do not divide."""
+    print(f"case: {B} x {C} planes {H}x{W}", flush=True)
+    lib = ctx.lib
+    x = torch.randn(B, C, H, W, generator=torch.Generator().manual_seed(B))
+    src = DeviceBuffer.from_array(np.concatenate([np.zeros(shift, np.float32), x.numpy().ravel()]))
+
+    def run(fn, shape, *args):
+        n = int(np.prod(shape))
+        buf = ctx.zeros(shift + n + 4)
+        native.check(fn(ctx.ctx, src.ptr + 4 * shift, buf.ptr + 4 * shift, *args), "plane")
+        ctx.sync()
+        a = buf.download(np.float32)
+        assert not a[:shift].any() and not a[shift + n:].any()
+        return torch.from_numpy(a[shift:shift + n].reshape(shape).copy())
+
+    up = x.repeat_interleave(2, 2).repeat_interleave(2, 3)
+    four = 4 * EPS * float(x.abs().max())
+    assert torch.equal(run(lib.gvm_nn_up_fwd, (B, C, 2 * H, 2 * W), B, C, C, 0, H, W), up)
+    assert torch.equal(run(lib.gvm_nn_pool_bwd, (B, C, 2 * H, 2 * W), B, C, 2 * H, 2 * W), 0.25 * up)
+    mean = F.avg_pool2d(x, 2)
+    got = run(lib.gvm_nn_pool_fwd, mean.shape, B, C, H, W)
+    assert torch.allclose(got, mean, rtol=0, atol=four)
+    got = run(lib.gvm_nn_up_bwd, mean.shape, B, C, C, 0, H // 2, W // 2)
+    assert torch.allclose(got, 4.0 * mean, rtol=0, atol=4 * four)
+    got = run(lib.gvm_nn_copy_channels, (B, C + 2, H, W), B, C, C, 0, C + 2, 1, H * W)
+    assert torch.equal(got[:, 1:-1], x) and not got[:, 0].any() and not got[:, -1].any()
