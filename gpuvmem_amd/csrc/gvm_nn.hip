@@ -236,6 +236,81 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs<WT> a) {
   }
 }
 
+// The same product for shapes whose tiles would be mostly padding: an im2col GEMM
+// of 64 outputs x 64 consecutive pixels (of any rows and images) per block, each wave
+// a 32 x 32 block of it.  K advances in chunks of 16 that are staged k-major, every
+// value's coordinates formed as it is loaded (26 TFLOP/s; a tile kernel's 90-110 need
+// tiles that are full).  K's order is the tile kernel's, so are the bits.
+template <int MODE, int KS, class WT>
+__global__ __launch_bounds__(256) void conv_im2col_kernel(ConvArgs<WT> a) {
+  constexpr int KK = KS * KS, P = KS / 2, CK = 16, T = 64;
+  __shared__ float As[CK][T + 4];
+  __shared__ float Bs[CK][T + 4];
+  const int HW = a.H * a.W, npix = a.B * HW, Kd = a.C * KK;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
+  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  auto weight = [&](int m, int k) {
+    if (m >= a.M || k >= Kd) return 0.0f;
+    if constexpr (MODE == CONV_FWD) return wload(a.w, (long)m * Kd + k);  // w[m][c][tap]
+    const int c = k / KK, tap = k - c * KK;  // w[c][m][tap]
+    return wload(a.w, ((long)c * a.M + m) * KK + tap);
+  };
+  auto value = [&](int k, int q) {
+    if (k >= Kd || q >= npix) return 0.0f;
+    const int c = k / KK, tap = k - c * KK, b = q / HW, p = q - b * HW;
+    const int dy = tap / KS - P, dx = tap % KS - P;
+    const int y = p / a.W + (MODE == CONV_FWD ? dy : -dy);
+    const int x = p % a.W + (MODE == CONV_FWD ? dx : -dx);
+    if (y < 0 || y >= a.H || x < 0 || x >= a.W) return 0.0f;
+    const long i = ((long)b * a.C + c) * HW + (long)y * a.W + x;
+    if (MODE == CONV_BWD_DATA && a.mask && !(a.mask[i] > 0.0f)) return 0.0f;
+    return a.in[i];
+  };
+  float ra[4], rb[4];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int e = t + 256 * j;
+      ra[j] = weight(m0 + e / CK, k0 + e % CK);
+      rb[j] = value(k0 + e / T, n0 + e % T);
+    }
+  };
+  f32x16_t acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+  load(0);
+  for (int k0 = 0; k0 < Kd; k0 += CK) {
+    __syncthreads();  // the chunk before has been read
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int e = t + 256 * j;
+      As[e % CK][e / CK] = ra[j];
+      Bs[e / T][e % T] = rb[j];
+    }
+    __syncthreads();
+    if (k0 + CK < Kd) load(k0 + CK);
+#pragma unroll
+    for (int s = 0; s < CK / 2; s++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[2 * s + lh][wm + lr], Bs[2 * s + lh][wn + lr],
+                                                 acc, 0, 0, 0);
+  }
+  const int n = n0 + wn + lr;
+  if (n >= npix) return;
+  const int b = n / HW, p = n - b * HW;
+#pragma unroll
+  for (int e = 0; e < 16; e++) {
+    const int co = m0 + wm + 8 * (e >> 2) + 4 * lh + (e & 3);
+    if (co >= a.M) continue;
+    float v = acc[e];
+    if constexpr (MODE == CONV_FWD) {
+      v = v + a.bias[co];
+      if (a.relu) v = fmaxf(v, 0.0f);
+    }
+    a.dst[((long)b * a.M + co) * HW + p] = v;
+  }
+}
+
 // ---- weight gradient ----
 constexpr int kWgradPixels = 8192;  // pixels of an FP32 partial
 constexpr int kWgradChunk = 128;    // pixels staged at a time
@@ -732,21 +807,68 @@ void launch_tile(gvm_ctx* ctx, ConvArgs<WT> a) {
                      ctx->stream, a);
 }
 
-// The tile: 8 x 32 pixels and 64 channels (32 where there are no more) when that
-// gives every CU two blocks, else 8 x 8 pixels and 64 channels.  The wide tile reads
-// each weight for four times the pixels: layers of 19 GFLOP take 170-183 us with it
-// (64 channels at 256 x 256 x 4) and 207-220 with the narrow one (256 channels at 64 x
+// What a launch would take, in microseconds: a start, a chain of chunks, and the chip's
+// share of every block's chunks (fits to 1,280 shapes of 1 to 128 channels and 1 to
+// 1024 x 1024 pixels; within 15 % for two shapes of three).
+struct ConvCost {
+  double start, chain, block, extra;
+  double us(long blocks, long chunks) const {
+    return start + chain * chunks + block * blocks * (chunks + extra);
+  }
+};
+
+// 3 x 3: the tile is 8 x 32 pixels and 64 channels (32 where there are no more) when
+// that gives every CU two blocks, else 8 x 8 pixels and 64 channels.  The wide tile
+// reads each weight for four times the pixels: layers of 19 GFLOP take 170-183 us with
+// it (64 channels at 256 x 256 x 4) and 207-220 with the narrow one (256 channels at 64 x
 // 64 x 4, 512 at 32 x 32 x 4), where it would have 256 and 128 blocks for 256 CUs.
+// Images much smaller or narrower than a tile leave it mostly empty, and one input
+// channel leaves a chunk of eight so: there the im2col kernel is the faster one (us, tiles /
+// im2col: 128 channels, 2,048 images of 4 x 4: 1283 / 175; 64 channels, 4 images of 4096 x
+// 1: 347 / 43; 1 to 64 channels at 1024 x 1024: 176 / 113; but 16 channels at 1024 x
+// 1024: 112 / 314).
+// 1 x 1: the tile kernel has nothing to share between taps.  It is ahead with full
+// tiles for every CU, 32 output channels or fewer and 16 input channels or more (16 to
+// 16 channels at 1024 x 1024: 76 / 81 us, 64 to 1: 94 / 119), and behind elsewhere (64 to
+// 64 channels at 1024 x 1024: 213 / 194, 1 to 16: 76 / 60, 32 to 16 at 64 x 64: 8.7 / 5.7,
+// 65,536 images of one pixel: 2263 / 21).  More outputs than 32 on 8 x 8 tiles of which
+// no CU gets a second are a shorter chain (64 to 128 channels, 32 images of 7 x 7: 7.3 / 9.2).
 template <int MODE, int KS, class WT>
-void conv_tile(gvm_ctx* ctx, const ConvArgs<WT>& a) {
-  constexpr int CK = KS == 3 ? 8 : 32;
-  const long wide = (long)((a.W + 31) / 32) * ((a.H + 7) / 8) * a.B;
-  if (a.M <= 32)
-    launch_tile<MODE, KS, 32, 8, 32, CK, WT>(ctx, a);
-  else if (wide * ((a.M + 63) / 64) >= 512)
-    launch_tile<MODE, KS, 64, 8, 32, CK, WT>(ctx, a);
-  else
-    launch_tile<MODE, KS, 64, 8, 8, CK, WT>(ctx, a);
+void conv_launch(gvm_ctx* ctx, const ConvArgs<WT>& a) {
+  auto blocks = [&](long th, long tw, long mt) {
+    return (a.W + tw - 1) / tw * ((a.H + th - 1) / th) * a.B * ((a.M + mt - 1) / mt);
+  };
+  const long npix = (long)a.B * a.H * a.W;
+  const dim3 cols((unsigned)((npix + 63) / 64), (unsigned)((a.M + 63) / 64));
+  const long tiles = blocks(8, 32, 32);
+  const bool fits = cols.x < (1u << 24);  // 2^32 threads are the limit of a launch
+  auto im2col = [&]() {
+    hipLaunchKernelGGL((conv_im2col_kernel<MODE, KS, WT>), cols, dim3(256), 0, ctx->stream, a);
+  };
+  if constexpr (KS == 1) {
+    const bool full = tiles >= ctx->cu_count && 2 * 256 * tiles <= 3 * npix;
+    if (a.M > 32 && a.C >= 16 && blocks(8, 8, 64) <= ctx->cu_count)
+      launch_tile<MODE, 1, 64, 8, 8, 32, WT>(ctx, a);
+    else if (fits && (a.M > 32 || a.C < 16 || !full))
+      im2col();
+    else
+      launch_tile<MODE, 1, 32, 8, 32, 32, WT>(ctx, a);
+  } else {
+    const long wide = blocks(8, 32, 64), chunks = (a.C + 7) / 8;
+    const double tile_us = a.M <= 32     ? ConvCost{5.2, 2.6, 0.0069, 0.75}.us(tiles, chunks)
+                           : wide >= 512 ? ConvCost{5.0, 0.15, 0.018, 1.1}.us(wide, chunks)
+                                         : ConvCost{4.8, 1.75, 0.0036, 1.4}.us(blocks(8, 8, 64), chunks);
+    const double im2col_us = ConvCost{3.6, 1.0, 0.00143, 2.7}.us(
+        (long)cols.x * cols.y, ((long)a.C * 9 + 15) / 16);
+    if (fits && (a.C == 1 || im2col_us < tile_us))
+      im2col();
+    else if (a.M <= 32)
+      launch_tile<MODE, 3, 32, 8, 32, 8, WT>(ctx, a);
+    else if (wide >= 512)
+      launch_tile<MODE, 3, 64, 8, 32, 8, WT>(ctx, a);
+    else
+      launch_tile<MODE, 3, 64, 8, 8, 8, WT>(ctx, a);
+  }
 }
 
 template <class WT>
@@ -760,9 +882,9 @@ gvm_status conv_fwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
               "gvm_nn_conv_fwd: sizes beyond the kernels' 32-bit indices");
   const ConvArgs<WT> a{in, nullptr, w, bias, out, B, Co, Ci, H, W, relu, 0, 0};
   if (K == 3)
-    conv_tile<CONV_FWD, 3>(ctx, a);
+    conv_launch<CONV_FWD, 3>(ctx, a);
   else
-    conv_tile<CONV_FWD, 1>(ctx, a);
+    conv_launch<CONV_FWD, 1>(ctx, a);
   return launched("gvm_nn_conv_fwd");
 }
 
@@ -792,9 +914,9 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   if (din) {
     const ConvArgs<WT> a{dout, mask, w, nullptr, din, B, Ci, Co, H, W, 0, 0, 0};
     if (K == 3)
-      conv_tile<CONV_BWD_DATA, 3>(ctx, a);
+      conv_launch<CONV_BWD_DATA, 3>(ctx, a);
     else
-      conv_tile<CONV_BWD_DATA, 1>(ctx, a);
+      conv_launch<CONV_BWD_DATA, 1>(ctx, a);
   }
   // weight and bias gradients: partials in the context's network workspace (the
   // bias's first, in FP64), then their FP64 sums

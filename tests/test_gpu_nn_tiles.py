@@ -121,6 +121,61 @@ def test_plane_kernels_at_every_alignment(ctx, H, W, shift):
     assert torch.equal(got[:, 2:4], x[:, 1:]) and not got[:, :2].any() and not got[:, 4].any()
 
 
+def _conv(ctx, x, w, b, relu, split=None):
+    """Forward on the device of x viewed as images of `split` pixels (1 x 1 layers)."""
+    B, Ci, H, W = x.shape
+    Co, _, K, _ = w.shape
+    H, W = split or (H, W)
+    out = ctx.zeros(B * Co * H * W)
+    bufs = [_dev(t) for t in (x, w, b)]
+    native.check(ctx.lib.gvm_nn_conv_fwd(ctx.ctx, *(t.ptr for t in bufs), out.ptr, B, Ci, Co, H, W,
+                                         K, int(relu)), "fwd")
+    ctx.sync()
+    return out.download(np.float32).reshape(B, Co, *x.shape[2:])
+
+
+@pytest.mark.parametrize("B,Ci,Co,H,W,K,relu,bf16", [
+    (5, 12, 20, 3, 2, 3, True, False),      # images much smaller than a tile
+    (3, 2, 70, 40, 1, 3, True, True),       # and narrower
+    (2, 17, 33, 1, 300, 1, True, False),
+    (130, 40, 66, 1, 1, 1, False, False),
+    (1, 1, 66, 67, 65, 3, True, False),     # one input channel; one output for its gradient
+    (2, 16, 65, 126, 510, 3, True, True),   # 8 x 32 tiles of 64 channels, forward
+    (2, 65, 16, 126, 510, 3, True, False),  # and for the input gradient
+    (2, 20, 30, 125, 260, 1, True, False),  # 1 x 1: full tiles
+    (1, 30, 90, 15, 17, 1, False, True),    # 8 x 8 tiles
+    (2, 8, 30, 33, 70, 1, True, False),
+])
+def test_convolutions_of_small_and_narrow_images(ctx, B, Ci, Co, H, W, K, relu, bf16):
+    test_convolutions_at_the_edges_of_tiles(ctx, B, Ci, Co, H, W, K, relu, bf16)
+
+
+@pytest.mark.parametrize("M,C,K", [(64, 32, 3), (33, 20, 3), (20, 18, 1)])
+def test_an_image_does_not_depend_on_its_batch(ctx, M, C, K):
+    """The kernel is chosen by the sizes of the whole call; K's order is the same in
+    all, so an image gives the same bits alone as among 2,048 (or its pixels as a
+    line)."""
+    g = torch.Generator().manual_seed(M)
+    w, b = torch.randn(M, C, K, K, generator=g) * 0.3, torch.randn(M, generator=g)
+    if K == 1:
+        x = torch.randn(1, C, 256, 256, generator=g)
+        assert np.array_equal(_conv(ctx, x, w, b, True), _conv(ctx, x, w, b, True, (65536, 1)))
+        return
+    x = torch.randn(2048, C, 4, 4, generator=g)
+    all_of_them = _conv(ctx, x, w, b, True)
+    for i in (0, 700, 2047):
+        assert np.array_equal(_conv(ctx, x[i:i + 1], w, b, True)[0], all_of_them[i])
+
+
+def test_sixteen_million_images_of_one_pixel(ctx):
+    """A block per image would be a launch of 2^32 threads, which is refused."""
+    n = 1 << 24
+    x = torch.arange(n, dtype=torch.float32).reshape(n, 1, 1, 1) - 1000.0
+    w, b = torch.full((1, 1, 1, 1), 0.5), torch.ones(1)
+    y = _conv(ctx, x, w, b, True)
+    assert np.array_equal(y, (0.5 * x.numpy() + 1.0).clip(min=0.0))
+
+
 @pytest.mark.parametrize("B,C,H,W,shift", [(300, 7, 2, 2, 0), (41, 5, 4, 4, 0), (9, 13, 6, 10, 1),
                                            (1, 1, 2, 2, 0), (700, 100, 2, 4, 0)])
 def test_planes_smaller_than_a_block(ctx, B, C, H, W, shift):
