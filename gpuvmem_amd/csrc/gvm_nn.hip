@@ -323,6 +323,7 @@ struct WgradArgs {
   double* bpart;      // [range][Co]
   int B, Ci, Co, H, W;
   unsigned int rw;    // about 2^32 / W
+  int step_b, step_p; // kWgradChunk pixels as whole images and pixels of the next
 };
 
 // Linear pixel index of a batch as (image, pixel of its plane), advanced by chunks.
@@ -333,10 +334,13 @@ struct PixelPos {
     b = q0 > 0 ? q0 / HW : 0;
     p = q0 - b * HW;  // (-1 before the first)
   }
-  __device__ __forceinline__ void next(int HW) {
+  // (a chunk may hold many images: a loop over them took 156 us for 1,000 x 1,000
+  // channels of one pixel)
+  __device__ __forceinline__ void next(int HW, int step_b, int step_p) {
     q += kWgradChunk;
-    p += kWgradChunk;
-    while (p >= HW) {
+    b += step_b;
+    p += step_p;
+    if (p >= HW) {
       p -= HW;
       b++;
     }
@@ -428,12 +432,12 @@ __global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(W
       if (end) {
         const int p = tail.p + (ky - P) * a.W;
         re = at(a.in, tail.q < npix && p >= 0 && p < HW ? ii * tail.b + (I)p * 4u + t0 : 0);
-        tail.next(HW);
+        tail.next(HW, a.step_b, a.step_p);
       }
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        gp[h].next(HW);
-        ip[h].next(HW);
+        gp[h].next(HW, a.step_b, a.step_p);
+        ip[h].next(HW, a.step_b, a.step_p);
       }
     };
     const bool all = !a.out;
@@ -503,7 +507,7 @@ __global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(W
           __ballot(gp[h].q < kend && x >= 0 && x < a.W && y >= 0 && y < a.H) >> lh;
       bits[2 * h] = (unsigned int)m;
       bits[2 * h + 1] = (unsigned int)(m >> 32);
-      gp[h].next(HW);
+      gp[h].next(HW, a.step_b, a.step_p);
     }
     const float* pa = &lg[k & 1][lr * GP + lh];
     const float* pb = &li[k & 1][lr * IP + kx + lh];
@@ -535,6 +539,66 @@ __global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(W
   for (int e = 0; e < 16; e++) {
     const int co = co0 + 8 * (e >> 2) + 4 * lh + (e & 3);
     if (co < a.Co && ci < a.Ci) dst[((long)co * a.Ci + ci) * KK + ky * KS + kx] = acc[e];
+  }
+}
+
+// At most NP pixels, 16 or 32 (the deepest levels of a network on a small image,
+// layers of one pixel): the kernel above would stage mostly padding for few MFMAs (us, it
+// / this one: 512 x 512 channels of 4 x 4 pixels 27 / 6.6, of 5 x 4 27.1 / 9.6, 200,000 x
+// 8 of one pixel 124 / 11.8).  A block forms 64 outputs x 64 (input channel, tap) pairs, K =
+// the pixels, all of them staged at once; the sums are complete, and have the kernel's
+// order.
+template <int KS, int NP>
+__global__ __launch_bounds__(256) void conv_wgrad_few_kernel(WgradArgs a, float* __restrict__ dw,
+                                                             float* __restrict__ dbias) {
+  constexpr int KK = KS * KS, P = KS / 2, T = 64;
+  __shared__ float As[NP][T + 4];
+  __shared__ float Bs[NP][T + 4];
+  const int HW = a.H * a.W, npix = a.B * HW, N = a.Ci * KK;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 31, lh = lane >> 5;
+  const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+#pragma unroll
+  for (int j = 0; j < NP * T / 256; j++) {
+    const int e = t + 256 * j, q = e % NP, m = m0 + e / NP, n = n0 + e / NP;
+    const int b = q / HW, p = q - b * HW;
+    float g = 0.0f, v = 0.0f;
+    if (q < npix && m < a.Co) {
+      const long i = ((long)b * a.Co + m) * HW + p;
+      g = !a.out || a.out[i] > 0.0f ? a.dout[i] : 0.0f;
+    }
+    if (q < npix && n < N) {
+      const int c = n / KK, tap = n - c * KK;
+      const int y = p / a.W + tap / KS - P, x = p % a.W + tap % KS - P;
+      if (y >= 0 && y < a.H && x >= 0 && x < a.W)
+        v = a.in[((long)b * a.Ci + c) * HW + y * a.W + x];
+    }
+    As[q][e / NP] = g;
+    Bs[q][e / NP] = v;
+  }
+  __syncthreads();
+  f32x16_t acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NP / 2; s++)
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[2 * s + lh][wm + lr], Bs[2 * s + lh][wn + lr],
+                                               acc, 0, 0, 0);
+  const int n = n0 + wn + lr;
+#pragma unroll
+  for (int e = 0; e < 16; e++) {
+    const int m = m0 + wm + 8 * (e >> 2) + 4 * lh + (e & 3);
+    if (m < a.Co && n < N) dw[(long)m * N + n] = acc[e];
+  }
+  if (blockIdx.x == 0 && t < T && m0 + t < a.Co) {
+    double s[NP];
+#pragma unroll
+    for (int q = 0; q < NP; q++) s[q] = (double)As[q][t];
+#pragma unroll
+    for (int h = NP / 2; h > 0; h >>= 1)
+#pragma unroll
+      for (int q = 0; q < h; q++) s[q] += s[q + h];
+    dbias[m0 + t] = (float)s[0];
   }
 }
 
@@ -898,6 +962,17 @@ void launch_wgrad(gvm_ctx* ctx, const WgradArgs& a, int ranges) {
     hipLaunchKernelGGL((conv_wgrad_kernel<KS, unsigned long>), grid, block, 0, ctx->stream, a);
 }
 
+template <int KS>
+void launch_wgrad_few(gvm_ctx* ctx, const WgradArgs& a, float* dw, float* dbias) {
+  const dim3 grid((unsigned)((a.Ci * KS * KS + 63) / 64), (unsigned)((a.Co + 63) / 64));
+  if (a.B * a.H * a.W <= 16)
+    hipLaunchKernelGGL((conv_wgrad_few_kernel<KS, 16>), grid, dim3(256), 0, ctx->stream, a, dw,
+                       dbias);
+  else
+    hipLaunchKernelGGL((conv_wgrad_few_kernel<KS, 32>), grid, dim3(256), 0, ctx->stream, a, dw,
+                       dbias);
+}
+
 template <class WT>
 gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const float* out,
                            const float* dout, float* din, float* dw, float* dbias, int B, int Ci,
@@ -918,6 +993,14 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     else
       conv_launch<CONV_BWD_DATA, 1>(ctx, a);
   }
+  if ((long)B * H * W <= 32) {
+    const WgradArgs a{in, mask, dout, nullptr, nullptr, B, Ci, Co, H, W, 0, 0, 0};
+    if (K == 3)
+      launch_wgrad_few<3>(ctx, a, dw, dbias);
+    else
+      launch_wgrad_few<1>(ctx, a, dw, dbias);
+    return launched("gvm_nn_conv_bwd");
+  }
   // weight and bias gradients: partials in the context's network workspace (the
   // bias's first, in FP64), then their FP64 sums
   const int ranges = (int)(((long)B * H * W + kWgradPixels - 1) / kWgradPixels);
@@ -934,7 +1017,8 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     ctx->nn_part_elems = need;
   }
   const WgradArgs a{in, mask, dout, ctx->nn_part + bias_elems, (double*)ctx->nn_part, B, Ci, Co, H,
-                    W,  (unsigned int)std::min(0xffffffffUL, ((1UL << 32) + W - 1) / W)};
+                    W,  (unsigned int)std::min(0xffffffffUL, ((1UL << 32) + W - 1) / W),
+                    kWgradChunk / (H * W), kWgradChunk % (H * W)};
   if (K == 3)
     launch_wgrad<3>(ctx, a, ranges);
   else

@@ -145,6 +145,12 @@ def _conv(ctx, x, w, b, relu, split=None):
     (2, 20, 30, 125, 260, 1, True, False),  # 1 x 1: full tiles
     (1, 30, 90, 15, 17, 1, False, True),    # 8 x 8 tiles
     (2, 8, 30, 33, 70, 1, True, False),
+    (1, 70, 65, 4, 4, 3, True, False),      # 16 pixels: the whole weight gradient at once
+    (3, 9, 80, 5, 1, 3, True, True),
+    (1, 130, 3, 1, 1, 1, False, False),
+    (1, 7, 5, 17, 1, 3, True, False),       # and one more
+    (2, 65, 70, 4, 4, 3, True, False),      # 32
+    (1, 65, 70, 11, 3, 3, True, False),     # 33: in ranges
 ])
 def test_convolutions_of_small_and_narrow_images(ctx, B, Ci, Co, H, W, K, relu, bf16):
     test_convolutions_at_the_edges_of_tiles(ctx, B, Ci, Co, H, W, K, relu, bf16)
