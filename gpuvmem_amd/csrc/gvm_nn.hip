@@ -608,22 +608,23 @@ __global__ __launch_bounds__(kT) void wgrad_reduce_kernel(const float* __restric
                                                           long n, float* __restrict__ dw,
                                                           const double* __restrict__ bpart, int Co,
                                                           float* __restrict__ dbias) {
-  const long i = blockIdx.x * (long)kT + threadIdx.x;
-  double s = 0.0;
-  if (i < n) {
-    int r = 0;
-    for (; r + 16 <= npart; r += 16) {
-      float v[16];
+  for (long i = blockIdx.x * (long)kT + threadIdx.x; i < n + Co; i += (long)gridDim.x * kT) {
+    double s = 0.0;
+    if (i < n) {
+      int r = 0;
+      for (; r + 16 <= npart; r += 16) {
+        float v[16];
 #pragma unroll
-      for (int u = 0; u < 16; u++) v[u] = part[(long)(r + u) * n + i];
+        for (int u = 0; u < 16; u++) v[u] = part[(long)(r + u) * n + i];
 #pragma unroll
-      for (int u = 0; u < 16; u++) s += (double)v[u];
+        for (int u = 0; u < 16; u++) s += (double)v[u];
+      }
+      for (; r < npart; r++) s += (double)part[(long)r * n + i];
+      dw[i] = (float)s;
+    } else {
+      for (int r = 0; r < npart; r++) s += bpart[(long)r * Co + (i - n)];
+      dbias[i - n] = (float)s;
     }
-    for (; r < npart; r++) s += (double)part[(long)r * n + i];
-    dw[i] = (float)s;
-  } else if (i < n + Co) {
-    for (int r = 0; r < npart; r++) s += bpart[(long)r * Co + (i - n)];
-    dbias[i - n] = (float)s;
   }
 }
 
@@ -862,13 +863,19 @@ void plane_launch(long plane, bool wide, F f) {
     f(std::integral_constant<int, 2>(), 0);
 }
 
+// A launch of 2^32 threads or more wraps around without an error.
+constexpr long kMaxBlocks = (1L << 32) / 256 - 1;
+
 template <int MODE, int KS, int MT, int TH, int TW, int CK, class WT>
-void launch_tile(gvm_ctx* ctx, ConvArgs<WT> a) {
+gvm_status launch_tile(gvm_ctx* ctx, ConvArgs<WT> a) {
   a.tiles_x = (a.W + TW - 1) / TW;
   a.tiles_y = (a.H + TH - 1) / TH;
-  const dim3 grid((unsigned)((long)a.tiles_x * a.tiles_y * a.B), (unsigned)((a.M + MT - 1) / MT));
+  const long tiles = (long)a.tiles_x * a.tiles_y * a.B;
+  GVM_REQUIRE(tiles <= kMaxBlocks, "gvm_nn_conv: too large and narrow an image");
+  const dim3 grid((unsigned)tiles, (unsigned)((a.M + MT - 1) / MT));
   hipLaunchKernelGGL((conv_tile_kernel<MODE, KS, MT, TH, TW, CK, WT>), grid, dim3(256), 0,
                      ctx->stream, a);
+  return GVM_OK;
 }
 
 // What a launch would take, in microseconds: a start, a chain of chunks, and the chip's
@@ -898,25 +905,26 @@ struct ConvCost {
 // 65,536 images of one pixel: 2263 / 21).  More outputs than 32 on 8 x 8 tiles of which
 // no CU gets a second are a shorter chain (64 to 128 channels, 32 images of 7 x 7: 7.3 / 9.2).
 template <int MODE, int KS, class WT>
-void conv_launch(gvm_ctx* ctx, const ConvArgs<WT>& a) {
+gvm_status conv_launch_part(gvm_ctx* ctx, const ConvArgs<WT>& a) {
   auto blocks = [&](long th, long tw, long mt) {
     return (a.W + tw - 1) / tw * ((a.H + th - 1) / th) * a.B * ((a.M + mt - 1) / mt);
   };
   const long npix = (long)a.B * a.H * a.W;
   const dim3 cols((unsigned)((npix + 63) / 64), (unsigned)((a.M + 63) / 64));
   const long tiles = blocks(8, 32, 32);
-  const bool fits = cols.x < (1u << 24);  // 2^32 threads are the limit of a launch
+  const bool fits = (long)cols.x <= kMaxBlocks;
   auto im2col = [&]() {
     hipLaunchKernelGGL((conv_im2col_kernel<MODE, KS, WT>), cols, dim3(256), 0, ctx->stream, a);
+    return GVM_OK;
   };
   if constexpr (KS == 1) {
     const bool full = tiles >= ctx->cu_count && 2 * 256 * tiles <= 3 * npix;
     if (a.M > 32 && a.C >= 16 && blocks(8, 8, 64) <= ctx->cu_count)
-      launch_tile<MODE, 1, 64, 8, 8, 32, WT>(ctx, a);
+      return launch_tile<MODE, 1, 64, 8, 8, 32, WT>(ctx, a);
     else if (fits && (a.M > 32 || a.C < 16 || !full))
-      im2col();
+      return im2col();
     else
-      launch_tile<MODE, 1, 32, 8, 32, 32, WT>(ctx, a);
+      return launch_tile<MODE, 1, 32, 8, 32, 32, WT>(ctx, a);
   } else {
     const long wide = blocks(8, 32, 64), chunks = (a.C + 7) / 8;
     const double tile_us = a.M <= 32     ? ConvCost{5.2, 2.6, 0.0069, 0.75}.us(tiles, chunks)
@@ -925,14 +933,30 @@ void conv_launch(gvm_ctx* ctx, const ConvArgs<WT>& a) {
     const double im2col_us = ConvCost{3.6, 1.0, 0.00143, 2.7}.us(
         (long)cols.x * cols.y, ((long)a.C * 9 + 15) / 16);
     if (fits && (a.C == 1 || im2col_us < tile_us))
-      im2col();
+      return im2col();
     else if (a.M <= 32)
-      launch_tile<MODE, 3, 32, 8, 32, 8, WT>(ctx, a);
+      return launch_tile<MODE, 3, 32, 8, 32, 8, WT>(ctx, a);
     else if (wide >= 512)
-      launch_tile<MODE, 3, 64, 8, 32, 8, WT>(ctx, a);
+      return launch_tile<MODE, 3, 64, 8, 32, 8, WT>(ctx, a);
     else
-      launch_tile<MODE, 3, 64, 8, 8, 8, WT>(ctx, a);
+      return launch_tile<MODE, 3, 64, 8, 8, 8, WT>(ctx, a);
   }
+}
+
+// At most 2^29 pixels of whole images at a time: every kernel chosen above then has
+// room for them in one launch.
+template <int MODE, int KS, class WT>
+gvm_status conv_launch(gvm_ctx* ctx, ConvArgs<WT> a) {
+  const long hw = (long)a.H * a.W, B = a.B, per = std::max(1L, (1L << 29) / hw);
+  for (long b = 0; b < B; b += per) {
+    a.B = (int)std::min(per, B - b);
+    const gvm_status st = conv_launch_part<MODE, KS>(ctx, a);
+    if (st) return st;
+    a.in += a.B * a.C * hw;
+    if (a.mask) a.mask += a.B * a.C * hw;
+    a.dst += a.B * a.M * hw;
+  }
+  return GVM_OK;
 }
 
 template <class WT>
@@ -945,11 +969,8 @@ gvm_status conv_fwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
                   (long)Co * K * K < (1L << 24),
               "gvm_nn_conv_fwd: sizes beyond the kernels' 32-bit indices");
   const ConvArgs<WT> a{in, nullptr, w, bias, out, B, Co, Ci, H, W, relu, 0, 0};
-  if (K == 3)
-    conv_launch<CONV_FWD, 3>(ctx, a);
-  else
-    conv_launch<CONV_FWD, 1>(ctx, a);
-  return launched("gvm_nn_conv_fwd");
+  const gvm_status st = K == 3 ? conv_launch<CONV_FWD, 3>(ctx, a) : conv_launch<CONV_FWD, 1>(ctx, a);
+  return st ? st : launched("gvm_nn_conv_fwd");
 }
 
 template <int KS>
@@ -988,10 +1009,9 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
   const float* mask = relu ? out : nullptr;
   if (din) {
     const ConvArgs<WT> a{dout, mask, w, nullptr, din, B, Ci, Co, H, W, 0, 0, 0};
-    if (K == 3)
-      conv_launch<CONV_BWD_DATA, 3>(ctx, a);
-    else
-      conv_launch<CONV_BWD_DATA, 1>(ctx, a);
+    const gvm_status st =
+        K == 3 ? conv_launch<CONV_BWD_DATA, 3>(ctx, a) : conv_launch<CONV_BWD_DATA, 1>(ctx, a);
+    if (st) return st;
   }
   if ((long)B * H * W <= 32) {
     const WgradArgs a{in, mask, dout, nullptr, nullptr, B, Ci, Co, H, W, 0, 0, 0};
@@ -1023,7 +1043,7 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
     launch_wgrad<3>(ctx, a, ranges);
   else
     launch_wgrad<1>(ctx, a, ranges);
-  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3((unsigned)((nw + Co + kT - 1) / kT)), dim3(kT), 0,
+  hipLaunchKernelGGL(wgrad_reduce_kernel, dim3(nblocks(nw + Co)), dim3(kT), 0,
                      ctx->stream, a.part, ranges, nw, dw, a.bpart, Co, dbias);
   return launched("gvm_nn_conv_bwd");
 }

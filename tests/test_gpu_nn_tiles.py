@@ -211,3 +211,42 @@ def test_planes_smaller_than_a_block(ctx, B, C, H, W, shift):
     assert torch.allclose(got, 4.0 * mean, rtol=0, atol=4 * four)
     got = run(lib.gvm_nn_copy_channels, (B, C + 2, H, W), B, C, C, 0, C + 2, 1, H * W)
     assert torch.equal(got[:, 1:-1], x) and not got[:, 0].any() and not got[:, -1].any()
+
+
+def test_more_weights_than_threads_of_a_launch(ctx):
+    """21,846 x 21,846 channels of 3 x 3 taps are more than 2^32 weights: their
+    gradient's sums are taken by a loop, not by a thread each."""
+    Ci = Co = 21846
+    B, H, W, n = 33, 1, 1, 21846 * 21846 * 9
+    assert n > 1 << 32
+    print(f"case: {n} weights", flush=True)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((B, Ci)).astype(np.float32)
+    dy = rng.standard_normal((B, Co)).astype(np.float32)
+    dx, ddy, dw, db = (DeviceBuffer.from_array(x), DeviceBuffer.from_array(dy), DeviceBuffer(4 * n),
+                       ctx.zeros(Co))
+    native.check(ctx.lib.gvm_nn_conv_bwd(ctx.ctx, dx.ptr, dx.ptr, None, ddy.ptr, None, dw.ptr, db.ptr,
+                                         B, Ci, Co, H, W, 3, 0), "bwd")
+    ctx.sync()
+    row = np.empty((Ci, 3, 3), np.float32)
+    for co in (0, 9999, Co - 1):
+        native.check(ctx.lib.gvm_memcpy_d2h(row.ctypes.data, dw.ptr + 4 * co * Ci * 9, row.nbytes), "copy")
+        ref = dy[:, co].astype(np.float64) @ x.astype(np.float64)
+        size = np.abs(dy[:, co]).astype(np.float64) @ np.abs(x)
+        assert np.all(np.abs(row[:, 1, 1] - ref) <= (B + 2) * EPS * size)
+        row[:, 1, 1] = 0.0
+        assert not row.any()
+    assert np.allclose(db.download(np.float32), dy.sum(0, dtype=np.float64), rtol=1e-5, atol=1e-5)
+
+
+def test_a_thousand_million_pixels(ctx):
+    """Images are taken in parts that a launch has room for."""
+    n = (1 << 30) + 77
+    print(f"case: {n} images of one pixel", flush=True)
+    x = torch.arange(n, dtype=torch.int32, device="cuda").remainder_(4096).float()
+    y, w, b = torch.full_like(x, -1.0), _dev(torch.full((1,), 0.5)), _dev(torch.ones(1))
+    torch.cuda.synchronize()
+    native.check(ctx.lib.gvm_nn_conv_fwd(ctx.ctx, x.data_ptr(), w.ptr, b.ptr, y.data_ptr(), n, 1, 1,
+                                         1, 1, 1, 1), "fwd")
+    ctx.sync()
+    assert torch.equal(y, x.mul_(0.5).add_(1.0))
