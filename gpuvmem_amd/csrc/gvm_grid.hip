@@ -13,10 +13,11 @@
 // scheduling.
 //
 // Gridder: rows are sorted by 8 x 8 tile of cells, once for every tile that
-// their taps reach (at most four tiles for kernels up to 9 x 9), and a wave
-// owns a tile, one cell per lane.  Sorting every (row, tap) pair instead, 173 M
+// their taps reach (at most four tiles for kernels up to 9 x 9), and a block
+// owns a tile.  Sorting every (row, tap) pair instead, 173 M
 // pairs for 1.76 M rows and 7 x 7 taps, took 12 ms and 5 GB of scratch memory
-// allocated and freed on each call, 107 - 137 ms in all.
+// allocated and freed on each call, 107 - 137 ms in all; it is kept for single taps and
+// for few rows on a large grid, where it is the faster one (use_entries).
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/iterator/transform_iterator.hpp>
@@ -189,6 +190,18 @@ __global__ __launch_bounds__(kThreads) void tile_first_kernel(const uint32_t* __
 typedef short short2_t __attribute__((ext_vector_type(2)));
 typedef short short8_t __attribute__((ext_vector_type(8)));
 
+// A cell's value and weight from its sums (src/functions.cu:1527-1559)
+__device__ __forceinline__ void cell_value(float ws, float aux, float re, float im, float2* vo,
+                                           float* w) {
+#pragma clang fp contract(off)
+  *w = 0.f;
+  *vo = make_float2(0.f, 0.f);
+  if (aux != 0.0f && ws != 0.0f) {
+    *w = ws * ws / aux;
+    *vo = make_float2(re / ws, im / ws);
+  }
+}
+
 template <bool LDS_TAPS>
 __global__ __launch_bounds__(kThreads) void grid_tiles_kernel(
     const uint32_t* __restrict__ ids, const uint32_t* __restrict__ start, GridGeom g,
@@ -288,14 +301,155 @@ __global__ __launch_bounds__(kThreads) void grid_tiles_kernel(
               im = __shfl(acc, (lane & 15) + 48, 64);
   if (lane >= 16) return;
   const int cx = c0 + cell.x, cy = r0 + cell.y;
-  float weff = 0.f;
-  float2 out = make_float2(0.f, 0.f);
-  if (aux != 0.0f && ws != 0.0f) {
-    weff = ws * ws / aux;
-    out = make_float2(re / ws, im / ws);
+  cell_value(ws, aux, re, im, cell_vo + (long)g.N * cy + cx, cell_w + (long)g.N * cy + cx);
+}
+
+// The same sums from (row, tap) entries sorted by cell, for single taps and for few rows
+// on a large grid: nothing here goes over the grid's cells or a tile's rows.  Entry
+// e is tap e % taps of row e / taps (rows and twins as above); a stable sort keeps a
+// cell's entries in row order.
+__global__ __launch_bounds__(kThreads) void entry_keys_kernel(const double* __restrict__ uvw,
+                                                              long nvis, GridGeom g,
+                                                              uint32_t* __restrict__ keys,
+                                                              uint32_t* __restrict__ ids) {
+#pragma clang fp contract(off)
+  const uint32_t taps = (uint32_t)(g.wx * g.wy), n = (uint32_t)(2 * nvis) * taps;
+  for (uint32_t e = blockIdx.x * kThreads + threadIdx.x; e < n; e += gridDim.x * kThreads) {
+    const uint32_t z = e / taps, t = e - z * taps;
+    const bool twin = z >= nvis;
+    const long vi = twin ? z - nvis : z;
+    double u = uvw[3 * vi], v = uvw[3 * vi + 1];
+    if (twin) {
+      u = -u;
+      v = -v;
+    }
+    u = u / g.lambda;
+    v = v / g.lambda;
+    const double jf = u / g.deltau + g.cj + 0.5;
+    const double kf = v / g.deltav + g.ck + 0.5;
+    uint32_t key = (uint32_t)((long)g.M * g.N);
+    if (fabs(jf) < 1073741824.0 && fabs(kf) < 1073741824.0) {
+      const int j = (int)jf - g.supx + (int)(t % (uint32_t)g.wx);
+      const int k = (int)kf - g.supy + (int)(t / (uint32_t)g.wx);
+      if (k >= 0 && k < g.M && j >= 0 && j < g.N) key = (uint32_t)((long)g.N * k + j);
+    }
+    keys[e] = key;
+    ids[e] = e;
   }
-  cell_vo[(long)g.N * cy + cx] = out;
-  cell_w[(long)g.N * cy + cx] = weff;
+}
+
+// The cell that starts at sorted entry p: its value and weight at index p, weight 0 where
+// none starts.  64 entries' products at a time are formed by a wave's lanes and left in
+// LDS; lanes 0 to 3 add one sum each, four entries a read: 16 ns an entry (one lane
+// adding all four sums: 26).  A thread adds a short run itself.
+__global__ __launch_bounds__(kThreads) void entry_cells_kernel(
+    const uint32_t* __restrict__ keys, const uint32_t* __restrict__ ids, long n, long nvis,
+    GridGeom g, const float* __restrict__ taps, const float* __restrict__ weight,
+    const float2* __restrict__ vo, float2* __restrict__ cell_vo, float* __restrict__ cell_w) {
+#pragma clang fp contract(off)
+  constexpr int kShort = 16;
+  __shared__ __align__(16) float prod[kThreads / 64][4][64 + 4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t off = (uint32_t)((long)g.M * g.N), nt = (uint32_t)(g.wx * g.wy);
+  auto products = [&](uint32_t id, float* q) {
+    const uint32_t z = id / nt, t = id - z * nt;
+    const long vi = z >= nvis ? z - nvis : z;
+    const float w = weight[vi];
+    float2 v = vo[vi];
+    if (z >= nvis) v.y = -v.y;
+    const float k = taps[g.kn * (t / (uint32_t)g.wx) + t % (uint32_t)g.wx];
+    q[0] = w * k;
+    q[1] = w * (k * k);
+    q[2] = w * v.x * k;
+    q[3] = w * v.y * k;
+  };
+  for (long i0 = (long)blockIdx.x * kThreads + threadIdx.x - lane; i0 < n;
+       i0 += (long)gridDim.x * kThreads) {
+    const long i = i0 + lane;
+    const uint32_t key = i < n ? keys[i] : off;
+    const bool head = key != off && (i == 0 || keys[i - 1] != key);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    bool more = head;
+    if (head) {
+      uint32_t id[kShort];
+      int cnt = 1;
+#pragma unroll
+      for (int u = 0; u < kShort; u++) {
+        const long p = min(i + u, n - 1);
+        id[u] = ids[p];
+        cnt = u == cnt && i + u < n && keys[p] == key ? u + 1 : cnt;
+      }
+      more = cnt == kShort;
+#pragma unroll
+      for (int u = 0; u < kShort; u += 4) {
+        if (u >= cnt) break;
+        float q[4][4];
+#pragma unroll
+        for (int h = 0; h < 4; h++) products(id[u + h], q[h]);  // (past the run's end: not added)
+#pragma unroll
+        for (int h = 0; h < 4; h++)
+#pragma unroll
+          for (int c = 0; c < 4; c++) s[c] = u + h < cnt ? s[c] + q[h][c] : s[c];
+      }
+    }
+    for (unsigned long long m = __ballot(more); m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t lk = (uint32_t)__builtin_amdgcn_readlane((int)key, l);
+      // sum c continues in lane c
+      float t = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const float from = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[c]), l));
+        t = lane == c ? from : t;
+      }
+      // products are a gather behind their ids: a round's are formed while the round
+      // before is added, its ids read a round before that
+      long p = i0 + l + kShort + lane;
+      auto entry = [&](long p, uint32_t* id) {
+        *id = ids[min(p, n - 1)];
+        return __popcll(__ballot(p < n && keys[min(p, n - 1)] == lk));  // a run is contiguous
+      };
+      uint32_t id, id1;
+      float q[4];
+      int cnt = entry(p, &id), cnt1 = entry(p + 64, &id1);
+      products(id, q);  // (of other runs' entries, too: not added)
+      while (cnt > 0) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int c = 0; c < 4; c++) prod[wave][c][lane] = q[c];
+        __builtin_amdgcn_wave_barrier();
+        p += 64;
+        uint32_t id2;
+        const int cnt2 = entry(p + 64, &id2);
+        if (cnt1 > 0) products(id1, q);
+        const float* mine = prod[wave][lane & 3];
+        if (cnt == 64) {
+#pragma unroll
+          for (int j = 0; j < 64; j += 4) {
+            const float4 v = *(const float4*)(mine + j);
+            t = t + v.x;
+            t = t + v.y;
+            t = t + v.z;
+            t = t + v.w;
+          }
+        } else {
+          for (int j = 0; j < cnt; j++) t = t + mine[j];
+        }
+        if (cnt < 64) break;
+        cnt = cnt1;
+        cnt1 = cnt2;
+        id1 = id2;
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const float sum = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), c));
+        if (lane == l) s[c] = sum;
+      }
+    }
+    if (i >= n) continue;
+    cell_w[i] = 0.f;
+    if (head) cell_value(s[0], s[1], s[2], s[3], cell_vo + i, cell_w + i);
+  }
 }
 
 struct IsKept {
@@ -304,19 +458,20 @@ struct IsKept {
 
 // Kept cells (weight > 0) to rows at the cell centre, in row-major cell order
 // (src/functions.cu:1527-1539, 1587-1607): uvw in metres, w = 0.
+// keys: the cells' indices (sorted entries), or none (every cell in turn).
 __global__ __launch_bounds__(kThreads) void grid_emit_kernel(
-    const int* __restrict__ pos, GridGeom g, const float2* __restrict__ cell_vo,
-    const float* __restrict__ cell_w, long capacity, double* __restrict__ uvw_out,
-    float2* __restrict__ vo_out, float* __restrict__ w_out) {
+    const int* __restrict__ pos, GridGeom g, const uint32_t* __restrict__ keys, long n,
+    const float2* __restrict__ cell_vo, const float* __restrict__ cell_w, long capacity,
+    double* __restrict__ uvw_out, float2* __restrict__ vo_out, float* __restrict__ w_out) {
 #pragma clang fp contract(off)
-  const long n = (long)g.M * g.N;
   for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < n;
        r += (long)gridDim.x * blockDim.x) {
     const float w = cell_w[r];
     if (!(w > 0.0f)) continue;
     const long o = pos[r];
     if (o >= capacity) continue;
-    const int gj = (int)(r % g.N), gk = (int)(r / g.N);
+    const long cell = keys ? (long)keys[r] : r;
+    const int gj = (int)(cell % g.N), gk = (int)(cell / g.N);
     const double ul = ((double)gj - g.cj) * g.deltau;
     const double vl = ((double)gk - g.ck) * g.deltav;
     uvw_out[3 * o] = ul * g.lambda;
@@ -325,6 +480,25 @@ __global__ __launch_bounds__(kThreads) void grid_emit_kernel(
     vo_out[o] = cell_vo[r];
     w_out[o] = w;
   }
+}
+
+// The form by its estimated time in microseconds.  Entries: their sort and sums.  Tiles:
+// passes over the cells, the sort, and the chain of the rows that reach a tile (0.06
+// for each of an even share: the fullest tiles, whose 40 ns a row decide, have more.
+// Single taps hit cells as unevenly as rows lie, and their entries are no more than the
+// rows: 0.15, and no allowance on the entries' side).  Both sides in us, entries / tiles:
+// 300,000 rows on 64 x 64 with one tap 237 / 589, all in one cell 4,850 / 11,800; 1.7 M rows
+// there with 3 x 3 taps 1,840 / 4,410; 100 rows on 4096 x 4096 with 7 x 7 taps 107 / 268;
+// but 10,000 rows on 64 x 64 with 7 x 7 taps 276 / 189, 1.7 M on 512 x 512 with 3 x 3 taps
+// 2,050 / 661.  At most 2^26 entries (2.4 GB of scratch).
+bool use_entries(const GridGeom& g, long nvis) {
+  const double rows = 2.0 * nvis, cells = (double)g.M * g.N, taps = (double)g.wx * g.wy;
+  const double reached = (1.0 + (g.wx - 1) / 8.0) * (1.0 + (g.wy - 1) / 8.0);
+  const double share = rows * reached / ((double)g.ntx * g.nty);
+  const double entry_us = taps == 1.0 ? 10.0 + 7.5e-5 * rows : 25.0 + 8.5e-5 * rows * taps;
+  const double tile_us =
+      1.1e-5 * cells + 6e-5 * rows * g.tx * g.ty + (taps == 1.0 ? 0.15 : 0.06) * share;
+  return entry_us < tile_us && rows * taps <= 67108864.0;
 }
 
 // ---- weighting schemes -----------------------------------------------------
@@ -586,8 +760,11 @@ extern "C" gvm_status gvm_grid_visibilities_dev(gvm_ctx* ctx, const gvm_ckernel*
   GVM_REQUIRE(nvis >= 0 && nvis <= (((1L << 31) - 1) / (2L * nx * ny)),
               "gvm_grid_visibilities_dev: rows x taps exceed 2^31 entries");
   if (nvis == 0) return GVM_OK;
-  const long n = 2 * nvis * g.tx * g.ty, cells = (long)geo.M * geo.N;
-  const int ntiles = g.ntx * g.nty, bits = key_bits((uint32_t)ntiles);
+  const long cells = (long)geo.M * geo.N, entries = 2 * nvis * g.wx * g.wy;
+  const bool by_entry = use_entries(g, nvis);
+  const long n = by_entry ? entries : 2 * nvis * g.tx * g.ty;
+  const long slots = by_entry ? entries : cells;  // where a cell's sums may be
+  const int ntiles = g.ntx * g.nty, bits = key_bits((uint32_t)(by_entry ? cells : ntiles));
   GVM_HIP_TRY(hipSetDevice(ctx->device));
 
   gvm_status st;
@@ -598,56 +775,67 @@ extern "C" gvm_status gvm_grid_visibilities_dev(gvm_ctx* ctx, const gvm_ckernel*
   size_t scan_bytes = 0;
   const auto kept = [](const float* w) { return rocprim::make_transform_iterator(w, IsKept()); };
   GVM_HIP_TRY(rocprim::exclusive_scan(nullptr, scan_bytes, kept(nullptr), (int*)nullptr, 0,
-                                      (size_t)cells, rocprim::plus<int>()));
+                                      (size_t)slots, rocprim::plus<int>()));
   const size_t ntaps = (size_t)kernel->m * kernel->n;
   sc.add(sizeof(float) * ntaps);
-  sc.add(sizeof(float4) * 2 * nvis);
-  sc.add(sizeof(uint32_t) * (ntiles + 1));
+  if (!by_entry) {
+    sc.add(sizeof(float4) * 2 * nvis);
+    sc.add(sizeof(uint32_t) * (ntiles + 1));
+  }
   sc.add(scan_bytes);
-  sc.add(sizeof(int) * cells);
-  sc.add(sizeof(float2) * cells);
-  sc.add(sizeof(float) * cells);
+  sc.add(sizeof(int) * slots);
+  sc.add(sizeof(float2) * slots);
+  sc.add(sizeof(float) * slots);
   if ((st = sc.reserve(what))) return st;
   ps.take(sc);
   float* taps_d = sc.take<float>(ntaps);
-  float4* rec = sc.take<float4>(2 * nvis);
-  uint32_t* start = sc.take<uint32_t>(ntiles + 1);
+  float4* rec = by_entry ? nullptr : sc.take<float4>(2 * nvis);
+  uint32_t* start = by_entry ? nullptr : sc.take<uint32_t>(ntiles + 1);
   char* stmp = sc.take<char>(scan_bytes);
-  int* pos = sc.take<int>(cells);
-  float2* cvo = sc.take<float2>(cells);
-  float* cw = sc.take<float>(cells);
+  int* pos = sc.take<int>(slots);
+  float2* cvo = sc.take<float2>(slots);
+  float* cw = sc.take<float>(slots);
   GVM_HIP_TRY(hipMemcpy(taps_d, kernel->taps, sizeof(float) * ntaps, hipMemcpyHostToDevice));
   const float2* vo = reinterpret_cast<const float2*>(vo_dev);
-  hipLaunchKernelGGL(grid_keys_kernel, dim3(blocks_for(nvis)), dim3(kThreads), 0, nullptr,
-                     uvw_m_dev, weight_dev, vo, nvis, g, rec, ps.k[0], ps.v[0]);
-  if ((st = launch_ok(what)) || (st = ps.sort((size_t)n, bits, what))) return st;
-  hipLaunchKernelGGL(tile_first_kernel, dim3(blocks_for(ntiles + 1)), dim3(kThreads), 0, nullptr,
-                     ps.keys(), n, ntiles, start);
-  if ((st = launch_ok(what))) return st;
-  const dim3 tiles(ntiles);
-  if (g.wx * g.wy <= kLdsTaps)
-    hipLaunchKernelGGL((grid_tiles_kernel<true>), tiles, dim3(kThreads), 0, nullptr, ps.ids(), start,
-                       g, taps_d, rec, cvo, cw);
-  else
-    hipLaunchKernelGGL((grid_tiles_kernel<false>), tiles, dim3(kThreads), 0, nullptr, ps.ids(),
-                       start, g, taps_d, rec, cvo, cw);
-  if ((st = launch_ok(what))) return st;
+  if (by_entry) {
+    hipLaunchKernelGGL(entry_keys_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, nullptr,
+                       uvw_m_dev, nvis, g, ps.k[0], ps.v[0]);
+    if ((st = launch_ok(what)) || (st = ps.sort((size_t)n, bits, what))) return st;
+    hipLaunchKernelGGL(entry_cells_kernel, dim3(blocks_for(n)), dim3(kThreads), 0, nullptr,
+                       ps.keys(), ps.ids(), n, nvis, g, taps_d, weight_dev, vo, cvo, cw);
+    if ((st = launch_ok(what))) return st;
+  } else {
+    hipLaunchKernelGGL(grid_keys_kernel, dim3(blocks_for(nvis)), dim3(kThreads), 0, nullptr,
+                       uvw_m_dev, weight_dev, vo, nvis, g, rec, ps.k[0], ps.v[0]);
+    if ((st = launch_ok(what)) || (st = ps.sort((size_t)n, bits, what))) return st;
+    hipLaunchKernelGGL(tile_first_kernel, dim3(blocks_for(ntiles + 1)), dim3(kThreads), 0, nullptr,
+                       ps.keys(), n, ntiles, start);
+    if ((st = launch_ok(what))) return st;
+    const dim3 tiles(ntiles);
+    if (g.wx * g.wy <= kLdsTaps)
+      hipLaunchKernelGGL((grid_tiles_kernel<true>), tiles, dim3(kThreads), 0, nullptr, ps.ids(),
+                         start, g, taps_d, rec, cvo, cw);
+    else
+      hipLaunchKernelGGL((grid_tiles_kernel<false>), tiles, dim3(kThreads), 0, nullptr, ps.ids(),
+                         start, g, taps_d, rec, cvo, cw);
+    if ((st = launch_ok(what))) return st;
+  }
   // output row of each kept cell
-  GVM_HIP_TRY(rocprim::exclusive_scan(stmp, scan_bytes, kept(cw), pos, 0, (size_t)cells,
+  GVM_HIP_TRY(rocprim::exclusive_scan(stmp, scan_bytes, kept(cw), pos, 0, (size_t)slots,
                                       rocprim::plus<int>()));
   int last = 0;
   float last_w = 0.f;
-  GVM_HIP_TRY(hipMemcpy(&last, pos + cells - 1, sizeof(int), hipMemcpyDeviceToHost));
-  GVM_HIP_TRY(hipMemcpy(&last_w, cw + cells - 1, sizeof(float), hipMemcpyDeviceToHost));
+  GVM_HIP_TRY(hipMemcpy(&last, pos + slots - 1, sizeof(int), hipMemcpyDeviceToHost));
+  GVM_HIP_TRY(hipMemcpy(&last_w, cw + slots - 1, sizeof(float), hipMemcpyDeviceToHost));
   const long count = (long)last + IsKept()(last_w);
   if (count > capacity) {
     set_error("gvm_grid_visibilities_dev: " + std::to_string(count) +
               " gridded rows exceed the output capacity " + std::to_string(capacity));
     return GVM_ERR_ARG;
   }
-  hipLaunchKernelGGL(grid_emit_kernel, dim3(blocks_for(cells)), dim3(kThreads), 0, nullptr, pos, g,
-                     cvo, cw, capacity, uvw_out_dev, reinterpret_cast<float2*>(vo_out_dev),
-                     weight_out_dev);
+  hipLaunchKernelGGL(grid_emit_kernel, dim3(blocks_for(slots)), dim3(kThreads), 0, nullptr, pos, g,
+                     by_entry ? ps.keys() : nullptr, slots, cvo, cw, capacity, uvw_out_dev,
+                     reinterpret_cast<float2*>(vo_out_dev), weight_out_dev);
   if ((st = launch_ok(what))) return st;
   GVM_HIP_TRY(hipDeviceSynchronize());
   *nout = count;

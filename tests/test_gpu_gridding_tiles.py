@@ -70,6 +70,35 @@ def test_crowded_cells(rows, centre):
     _grid_both(p, k, *_rows(p, rows, rows, centre))
 
 
+@pytest.mark.parametrize("npix,m,n,rows,support", [
+    (64, 1, 1, 5000, None), (64, 1, 1, 60000, None),    # single taps
+    (64, 2, 2, 300000, None),                           # crowded cells of a small grid
+    (2048, 1, 1, 1, None), (2048, 7, 9, 100, None), (1024, 3, 2, 33, None),  # few rows
+    (2048, 5, 6, 120, (6, 2)), (2048, 33, 35, 3, None),
+])
+def test_sums_by_entry(npix, m, n, rows, support):
+    p = small_problem(npix=npix, n_antennas=5, seed=2, dump_seconds=3600.0)
+    k = GriddingKernel.from_taps(np.random.default_rng(m * n).uniform(0.1, 1.0, (m, n))
+                                 .astype(np.float32))
+    if support:
+        k.support_x, k.support_y = support
+    print(f"case: gridder by entry {npix}^2 {m} x {n} taps {rows} rows", flush=True)
+    _grid_both(p, k, *_rows(p, rows, rows + m))
+
+
+@pytest.mark.parametrize("runs", [(1, 2, 3, 5000), (15, 16, 17, 32, 4000), (79, 80, 81, 144, 6000),
+                                  (63, 64, 65, 128, 200, 1, 6000)])
+def test_runs_of_entries(runs):
+    """Cells of the given row counts, rows interleaved, one tap."""
+    p = small_problem(npix=64, n_antennas=5, seed=2)
+    parts = [_rows(p, n, 10 + i, centre=(3 * i + 1, 2 * i - 9)) for i, n in enumerate(runs)]
+    uvw, vo, w = (np.concatenate([q[c] for q in parts]) for c in range(3))
+    order = np.random.default_rng(len(uvw)).permutation(len(uvw))
+    k = GriddingKernel.from_taps(np.full((1, 1), 0.7, np.float32))
+    print(f"case: runs {runs}", flush=True)
+    assert _grid_both(p, k, uvw[order], vo[order], w[order]) > 0
+
+
 @pytest.mark.parametrize("scheme", ["uniform", "briggs"])
 @pytest.mark.parametrize("runs", [(1,), (15, 16, 17, 1), (63, 64, 65, 79, 80, 81), (4000, 2, 9)])
 def test_weighting_runs(scheme, runs):
