@@ -688,7 +688,9 @@ static gvm_status split_work(gvm_ctx* ctx) {
   ctx->adj_gridded = false;
   long rows = 0;
   for (const Slice& s : ctx->slices) rows += s.nvis;
-  if (mode != GVM_ADJOINT_DIRECT && rows >= min_gridded_rows(N)) {
+  if (mode != GVM_ADJOINT_DIRECT &&
+      (ctx->gridding == GVM_GRIDDING_ALWAYS ||
+       (ctx->gridding == GVM_GRIDDING_AUTO && rows >= min_gridded_rows(N)))) {
     bool ok = false;
     gvm_status st = build_grid_plan(ctx, &ok);
     if (st) return st;

@@ -502,6 +502,20 @@ extern "C" gvm_status gvm_set_adjoint(gvm_ctx* ctx, int mode) {
   return GVM_OK;
 }
 
+extern "C" gvm_status gvm_set_gridding(gvm_ctx* ctx, int when) {
+  GVM_REQUIRE(ctx, "gvm_set_gridding: null context");
+  GVM_REQUIRE(when == GVM_GRIDDING_NEVER || when == GVM_GRIDDING_AUTO ||
+                  when == GVM_GRIDDING_ALWAYS,
+              "gvm_set_gridding: unknown choice");
+  GVM_REQUIRE(!ctx->capturing, "gvm_set_gridding: capturing");
+  if (ctx->gridding != when) {
+    ctx->gridding = when;
+    ctx->split_mode = -1;  // decided by the next gvm_dchi2
+    ctx->epoch++;
+  }
+  return GVM_OK;
+}
+
 extern "C" gvm_status gvm_add_visibilities(gvm_ctx* ctx, float freq, long nvis,
                                            const double* uvw, const float* vo,
                                            const float* weight, int* slice_out) {

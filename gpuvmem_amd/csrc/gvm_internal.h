@@ -144,6 +144,7 @@ struct gvm_ctx {
   double mask_fmax = 0.0;       // max |sqrt(1 - r^2) - 1| over the pixels on the mask
   gvm::GridPlan gplan;
   int adjoint_mode = GVM_ADJOINT_BF16X3;
+  int gridding = GVM_GRIDDING_AUTO;
   long split_vis = 6144;        // target visibilities per adjoint range (K tile), default_split_vis
   int fft_mode = 0;             // FFT batching: 0 automatic, 1 wide, 2 narrow
   std::vector<gvm::Slice> slices;

@@ -112,6 +112,11 @@ class Context:
     def set_adjoint(self, mode: str) -> None:
         native.check(self.lib.gvm_set_adjoint(self.ctx, native.ADJOINT_MODES[mode]), "gvm_set_adjoint")
 
+    def set_gridding(self, when: str) -> None:
+        """gvm_set_gridding: "never" (the GEMM that the form names), "auto" or
+        "always" (wherever gridding applies)."""
+        native.check(self.lib.gvm_set_gridding(self.ctx, native.GRIDDING[when]), "gvm_set_gridding")
+
     def image(self, img: np.ndarray) -> DeviceBuffer:
         assert img.dtype == np.float32 and img.size == 2 * self.n
         return DeviceBuffer.from_array(img)

@@ -18,6 +18,7 @@ GVM_NOALLOC_DOT_MAX_N = 1 << 37
 GVM_BEAM_AIRYDISK = 0
 GVM_BEAM_GAUSSIAN = 1
 ADJOINT_MODES = {"f32": 0, "f16x3": 1, "bf16x3": 2, "direct": 3}
+GRIDDING = {"never": 0, "auto": 1, "always": 2}
 WEIGHTING_SCHEMES = {"natural": 0, "uniform": 1, "briggs": 2, "radial": 3}
 
 
@@ -162,6 +163,7 @@ HIP_API = {
     "gvm_get_split_vis": [_P, C.POINTER(_L)],
     "gvm_adjoint_computed_pixels": [_P, C.POINTER(_L)],
     "gvm_adjoint_gridded": [_P, C.POINTER(_I)],
+    "gvm_set_gridding": [_P, _I],
     "gvm_autotune_adjoint": [_P, _P, _I, C.POINTER(_L), _DP, _IP],
     "gvm_weighting_apply_dev": [_P, _I, _F, C.POINTER(UVTaper), _I, _P, _P, _P, _P],
     "gvm_setup_beam_noise_dev": [_I, _P, _P, _P, _P, _D, _DP, _DP, _DP, _DP, _DP, _DP],

@@ -213,6 +213,12 @@ gvm_status gvm_get_geometry(const gvm_ctx* ctx, gvm_geometry* out);
  * takes over: few visibilities on images of 2048^2 and more, or w terms that need
  * more than 32 planes.  DIRECT always is the direct sum. */
 gvm_status gvm_set_adjoint(gvm_ctx* ctx, int mode);
+/* No counterpart in the reference.  Whether the forms F32, F16X3 and BF16X3 run by
+ * gridding and FFT (default GVM_GRIDDING_AUTO). */
+#define GVM_GRIDDING_NEVER 0 /* always the GEMM that the form names            */
+#define GVM_GRIDDING_AUTO 1  /* where it applies and the GEMM is not the faster */
+#define GVM_GRIDDING_ALWAYS 2 /* wherever it applies                            */
+gvm_status gvm_set_gridding(gvm_ctx* ctx, int when);
 
 /* ---- objective: chi2 ----------------------------------------------------- */
 
