@@ -955,8 +955,12 @@ extern "C" gvm_status gvm_autotune_adjoint(gvm_ctx* ctx, const long* candidates,
     set_error("gvm_autotune_adjoint: scratch allocation failed");
     return GVM_ERR_OOM;
   }
-  // the tuning launches are not part of the adjoint timing
+  // the tuning launches are not part of the adjoint timing; the range length is the
+  // GEMM's, so it is the GEMM that is timed (gridding would give every candidate the
+  // same time, and a length picked by noise to the GEMM that takes over some day)
   ctx->timing_paused = true;
+  const int gridding = ctx->gridding;
+  ctx->gridding = GVM_GRIDDING_NEVER;
   long best = candidates[0];
   double best_ms = 1e300;
   gvm_status st = GVM_OK;
@@ -982,6 +986,8 @@ extern "C" gvm_status gvm_autotune_adjoint(gvm_ctx* ctx, const long* candidates,
     }
   }
   ctx->timing_paused = false;
+  ctx->gridding = gridding;
+  ctx->split_mode = -1;
   if (st) {
     cleanup();
     if (st == GVM_ERR_HIP) set_error("gvm_autotune_adjoint: timing failed");
@@ -989,7 +995,6 @@ extern "C" gvm_status gvm_autotune_adjoint(gvm_ctx* ctx, const long* candidates,
   }
   cleanup();
   ctx->split_vis = best;
-  ctx->split_mode = -1;
   ctx->epoch++;
   tune_store(key, best);
   *chosen = best;

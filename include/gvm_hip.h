@@ -517,7 +517,7 @@ gvm_status gvm_adjoint_computed_pixels(const gvm_ctx* ctx, long* pixels);
  * as the direct sum (for measurement). */
 gvm_status gvm_adjoint_gridded(const gvm_ctx* ctx, int* gridded);
 /* Autotuner: times the adjoint of the current residuals (a gvm_chi2 must
- * have run) for each candidate range length (NULL: 1536, 2048, 3072, 4096,
+ * have run), as the GEMM also where gridding takes its place, for each candidate range length (NULL: 1536, 2048, 3072, 4096,
  * 6144, 8192, up to 3072 for images of 2048^2 and larger), with HIP events,
  * and keeps the fastest.  The choice is cached
  * per shape (M, total visibilities, slices, adjoint form, CU count) for the

@@ -140,3 +140,27 @@ def test_the_choice():
     with pytest.raises(native.GvmError):
         native.check(ctx.lib.gvm_set_gridding(ctx.ctx, 3), "gvm_set_gridding")
     ctx.close()
+
+
+def test_the_autotuner_times_the_gemm(tmp_path, monkeypatch):
+    """While the gradients run by gridding, range lengths are still the GEMM's: its
+    times are what is compared and kept, and the gradient is what it was before."""
+    monkeypatch.setenv("GVM_TUNE_CACHE", str(tmp_path / "tune.txt"))
+    p = small_problem(npix=512, n_antennas=8, seed=77)
+    p.noise = np.full_like(p.noise, 0.5 * p.noise_cut)
+    ctx = Context(p, add_data=False)
+    for s in _slices(p, (150000, 49983), seed=3):
+        ctx.add(*s)
+    d = ctx.image(_image(p, 4))
+    ctx.chi2(d)
+    before = _gradient(ctx, d)
+    ctx.reset_timing()
+    for _ in range(5):
+        _gradient(ctx, d)
+    gridded_ms = ctx.adjoint_time_ms()[0]
+    r = ctx.autotune([512, 1536, 6144])
+    print(f"gridded {gridded_ms:.3f} ms, GEMM by range length {r}", flush=True)
+    # 2e11 products of three 16-bit MFMA products: 0.5 ms at the matrix units' peak
+    assert not r["cached"] and min(r["ms"].values()) > 0.5 > gridded_ms
+    assert np.array_equal(_gradient(ctx, d), before) and ctx.adjoint_gridded()
+    ctx.close()
