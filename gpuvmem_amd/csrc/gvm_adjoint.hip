@@ -583,6 +583,15 @@ __global__ void adjoint_epilogue_kernel(const float* __restrict__ part,
 
 namespace {
 
+// Ranges of a slice of nv rows when they are kept near kvis rows.
+long slice_ranges(const gvm_ctx* ctx, long nv, long kvis, int ntiles) {
+  const long nsl = (long)ctx->slices.size();
+  const long fill = (4L * std::max(ctx->cu_count, 64) + ntiles - 1) / ntiles;
+  const long k = (nv + kvis - 1) / kvis;
+  // small observations: more, shorter ranges so the GPU fills
+  return std::max(1L, std::max(k, std::min((fill + nsl - 1) / nsl, std::max(1L, nv / 512))));
+}
+
 // Splits the visibilities of every slice into ranges for the GEMM
 // workgroups.  Each range accumulates in FP32 MFMA accumulators and the
 // ranges are combined in FP64, so ranges are kept near ctx->split_vis
@@ -609,17 +618,12 @@ gvm_status build_splits(gvm_ctx* ctx, int mode, int ntiles, long n) {
     GVM_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
     const long avail = (long)(free_b + sizeof(float) * ctx->adj_part_elems) / 2;
     const long budget = std::max<long>(8, std::min(kMaxWorkspace, avail) / (long)(sizeof(float) * n));
-    const long fill = (4L * std::max(ctx->cu_count, 64) + ntiles - 1) / ntiles;
     long kvis = kSplitVis;
     std::vector<long> ns(nsl);
     for (;;) {
       long total = 0;
       for (int s = 0; s < nsl; s++) {
-        const long nv = ctx->slices[s].nvis;
-        long k = (nv + kvis - 1) / kvis;
-        // small observations: more, shorter ranges so the GPU fills
-        k = std::max(k, std::min((fill + nsl - 1) / nsl, std::max(1L, nv / 512)));
-        ns[s] = std::max(1L, k);
+        ns[s] = slice_ranges(ctx, ctx->slices[s].nvis, kvis, ntiles);
         total += ns[s];
       }
       if (((total + 7) / 8) * 8 <= budget || kvis >= (1L << 30)) break;
@@ -669,15 +673,42 @@ gvm_status build_splits(gvm_ctx* ctx, int mode, int ntiles, long n) {
 
 }  // namespace
 
-// Fewer rows than this over all slices: the GEMM is the faster one.  The
-// gridded form's time is that of its FFTs, the GEMM's falls with the rows:
-// one evaluation at 2048^2 takes 210 / 161 us (gridded / GEMM) at 30 rows, 234
-// / 267 at 840, 249 / 306 at 5,700; at 4096^2 904 / 628, 1001 / 822, 1101 / 1331;
-// at 1024^2, where launches decide (the GEMM has one less), 81 / 75, 86 / 77,
-// 88 / 140.  Below that the two are alike up to about 1,000 rows, and the gridded
-// form is the more accurate one (1e-7 against 1e-6).
+// Fewer rows than this over all slices: the GEMM, unless clearly the slower.  The gridded form's time is
+// that of its FFTs, the GEMM's falls with the rows: one evaluation at 2048^2 takes
+// 210 / 161 us (gridded / GEMM) at 30 rows, 234 / 267 at 840, 249 / 306 at 5,700; at
+// 4096^2 904 / 628, 1001 / 822, 1101 / 1331; at 1024^2 81 / 75 at 30, 88 / 140 at 5,700.
+// Smaller images are gridded at any number of rows unless the GEMM is much faster.
 static long min_gridded_rows(int N) {
   return N < 1024 ? 0 : N == 1024 ? 1024 : (long)N * N / 8192;
+}
+
+// The GEMM's time over the gridded form's.  Both
+// times in microseconds, fitted to 290 observations of 1 to 64 slices of 10 to 5,000 rows,
+// 64^2 to 2048^2 pixels and 1 to 31 planes (within 35 % for nine of ten).  Gridded: a
+// set of transforms per slice and plane, rows and subgrids per plane.  GEMM: a partial image
+// per range, and the chain of a range's rows in every block that a CU takes.  Many
+// slices of few rows, or many planes for few rows, are the GEMM's: 64 slices of 100 rows at
+// 2048^2 with 6 planes take 16.8 ms gridded and 1.5 as a GEMM, one of 10 rows at 1024^2 with
+// 31 planes 0.24 and 0.04; 1,000 rows there with one plane are not (0.05 and 0.15).
+static double gemm_over_gridded(const gvm_ctx* ctx, int ntiles) {
+  const double n = (double)ctx->g.N * ctx->g.N, mpx = 1e-6 * n, K = ctx->gplan.planes;
+  const double nsl = (double)ctx->slices.size();
+  double rows = 0.0, subgrids = 0.0;
+  long ranges = 0, longest = 0;
+  for (const Slice& s : ctx->slices) {
+    rows += (double)s.nvis;
+    subgrids += std::min((double)s.nvis, 0.6 * n / 64.0);
+    const long r = slice_ranges(ctx, s.nvis, ctx->split_vis, ntiles);
+    ranges += r;
+    longest = std::max(longest, ((s.nvis + r - 1) / r + kKV - 1) / kKV * kKV);
+  }
+  const double gridded_us = 27.0 + 1.6 * K + mpx * nsl * (11.0 + 7.5 * K) + 3.1e-5 * rows * K +
+                            8e-4 * subgrids * K;
+  const double blocks = (double)ntiles * ranges * ctx->adj_px_gemm / n;
+  const double row_us = ctx->adjoint_mode == GVM_ADJOINT_F32 ? 0.47 : 0.127;
+  const double gemm_us = 11.0 + 3.5 * mpx * ((ranges + 7) / 8 * 8) + 1.06 * nsl +
+                         row_us * longest * std::max(1.0, blocks / ctx->cu_count);
+  return gemm_us / gridded_us;
 }
 
 // Decides how the adjoint of the current form runs and sizes its workspace:
@@ -685,23 +716,27 @@ static long min_gridded_rows(int N) {
 // else in ranges of visibilities; the direct form one range per slice.
 static gvm_status split_work(gvm_ctx* ctx) {
   const int N = ctx->g.N, mode = ctx->adjoint_mode;
+  const int tiles_x = (N + kTile - 1) / kTile, ntiles = tiles_x * tiles_x;
   ctx->adj_gridded = false;
   long rows = 0;
   for (const Slice& s : ctx->slices) rows += s.nvis;
-  if (mode != GVM_ADJOINT_DIRECT &&
-      (ctx->gridding == GVM_GRIDDING_ALWAYS ||
-       (ctx->gridding == GVM_GRIDDING_AUTO && rows >= min_gridded_rows(N)))) {
+  if (mode != GVM_ADJOINT_DIRECT && ctx->gridding != GVM_GRIDDING_NEVER) {
     bool ok = false;
-    gvm_status st = build_grid_plan(ctx, &ok);
+    gvm_status st = probe_grid_plan(ctx, &ok);
     if (st) return st;
+    // with rows enough the gridded form keeps a call up to four times the GEMM's time: it
+    // is the more accurate one (2e-7 of FP64, the 16-bit GEMMs up to 4e-6); with few it
+    // has to be ahead by more than the estimate is off
+    if (ok && ctx->gridding == GVM_GRIDDING_AUTO)
+      ok = gemm_over_gridded(ctx, ntiles) > (rows < min_gridded_rows(N) ? 1.5 : 0.25);
+    if (ok && (st = build_grid_plan(ctx, &ok))) return st;
     if (ok) {
       ctx->adj_gridded = true;
       ctx->split_mode = mode;
       return GVM_OK;
     }
   }
-  const int tiles_x = (N + kTile - 1) / kTile;
-  return build_splits(ctx, mode, tiles_x * tiles_x, (long)N * N);
+  return build_splits(ctx, mode, ntiles, (long)N * N);
 }
 
 gvm_status rebuild_splits(gvm_ctx* ctx) {

@@ -826,49 +826,41 @@ int row_pitch(int N) { return N + 8; }
 
 }  // namespace
 
-void free_grid_plan(GridPlan& g) {
+// Frees what build_grid_plan made; the planes stay known.
+static void release_grid_plan(GridPlan& g) {
   (void)hipFree(g.tables);
   (void)hipFree(g.lists);
   (void)hipFree(g.ws);
+  g.tables = g.lists = g.ws = nullptr;
+  g.built = g.usable = false;
+}
+
+void free_grid_plan(GridPlan& g) {
+  release_grid_plan(g);
   g = GridPlan{};
 }
 
-// Sorts every slice's visibilities by tile and lays out the work items and
-// the workspace.  *ok = false (and GVM_OK) when this form does not apply: too
-// many w planes, or not enough memory; the GEMM form then takes the call.
-gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
+// W and the planes it needs.  *ok = false when they are too many, or there is an
+// infinite or NaN w; the GEMM form then takes the call.
+gvm_status probe_grid_plan(gvm_ctx* ctx, bool* ok) {
   *ok = false;
   GridPlan& g = ctx->gplan;
-  if (g.built) {
-    *ok = g.usable;
+  if (g.probed) {
+    *ok = g.applies;
     return GVM_OK;
   }
-  GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  free_grid_plan(g);
-  g.built = true;
-  const int N = ctx->g.N, nsl = (int)ctx->slices.size();
-  const unsigned int ntiles = (unsigned int)(N / 8 + 1) * (N / 4);
   hipStream_t st = ctx->stream;
-  auto give_up = [&]() {
-    free_grid_plan(g);
-    g.built = true;
-    return GVM_OK;
-  };
-
-  // W and the planes it needs (scratch from the context's set-up workspace and a
-  // few allocations for what the plan keeps: one for every array, and as many
-  // hipFree's, took more of a small observation's first pass than the sort)
+  GVM_HIP_TRY(hipStreamSynchronize(st));
+  free_grid_plan(g);
+  const int nsl = (int)ctx->slices.size();
   const unsigned int zero = 0u;
-  long vmax = 0, total = 0;
-  for (const Slice& s : ctx->slices) {
-    vmax = std::max(vmax, s.nvis);
-    total += s.nvis;
-  }
+  long vmax = 0;
+  for (const Slice& s : ctx->slices) vmax = std::max(vmax, s.nvis);
   unsigned int wbits = 0;
   {
     Scratch sc(ctx);
     sc.add(sizeof(unsigned int));
-    if (sc.reserve("adjoint plan")) return give_up();
+    if (sc.reserve("adjoint plan")) return GVM_OK;
     unsigned int* wmax = sc.take<unsigned int>(1);
     GVM_HIP_TRY(hipMemcpyAsync(wmax, &zero, sizeof zero, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(wmax_kernel, dim3((unsigned)std::min<long>(256, (vmax + 255) / 256), nsl),
@@ -877,7 +869,8 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     GVM_HIP_TRY(hipMemcpyAsync(&wbits, wmax, sizeof wbits, hipMemcpyDeviceToHost, st));
     GVM_HIP_TRY(hipStreamSynchronize(st));
   }
-  if (wbits >= 0x7f800000u) return give_up();  // an infinite or NaN w
+  g.probed = true;
+  if (wbits >= 0x7f800000u) return GVM_OK;  // an infinite or NaN w
   float W;
   static_assert(sizeof W == sizeof wbits, "float bits");
   __builtin_memcpy(&W, &wbits, sizeof W);
@@ -885,7 +878,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   int K = 1;
   for (double e = zmax; e > kPlaneTol; e *= 0.5 * zmax / K) {  // 2 (zmax / 2)^K / K!
     K++;
-    if (K > kMaxPlanes) return give_up();
+    if (K > kMaxPlanes) return GVM_OK;
   }
   g.planes = K;
   g.wz = 2.0 * kPi * (double)W;
@@ -893,8 +886,39 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   g.terms = 2;
   for (double t = 0.25 * zmax * zmax; t > 1e-11; g.terms++)
     t *= 0.25 * zmax * zmax / ((double)g.terms * g.terms);
-  if (g.terms > kMaxTerms) return give_up();
+  if (g.terms > kMaxTerms) return GVM_OK;
   g.inv_w = W > 0.0f ? 1.0 / (double)W : 0.0;
+  g.applies = *ok = true;
+  return GVM_OK;
+}
+
+// Sorts every slice's visibilities by tile and lays out the work items and
+// the workspace, for the planes of probe_grid_plan.  *ok = false (and GVM_OK) when there
+// is not enough memory; the GEMM form then takes the call.
+// (Scratch from the context's set-up workspace and a few allocations for what the plan
+// keeps: one for every array, and as many hipFree's, took more of a small observation's
+// first pass than the sort.)
+gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
+  *ok = false;
+  GridPlan& g = ctx->gplan;
+  if (g.built) {
+    *ok = g.usable;
+    return GVM_OK;
+  }
+  g.built = true;
+  const int N = ctx->g.N, nsl = (int)ctx->slices.size(), K = g.planes;
+  const unsigned int ntiles = (unsigned int)(N / 8 + 1) * (N / 4);
+  hipStream_t st = ctx->stream;
+  auto give_up = [&]() {
+    release_grid_plan(g);
+    g.built = true;
+    return GVM_OK;
+  };
+  long vmax = 0, total = 0;
+  for (const Slice& s : ctx->slices) {
+    vmax = std::max(vmax, s.nvis);
+    total += s.nvis;
+  }
 
   // items of at most `chunk` rows: long enough to amortise a subgrid's
   // stores, short enough that a small observation fills the chip

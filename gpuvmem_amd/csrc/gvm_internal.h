@@ -72,8 +72,10 @@ struct SliceDev {
 // sorted by grid tile, the work items, and the workspace.  Built by the first
 // gvm_dchi2 after the slices changed.
 struct GridPlan {
-  bool built = false;   // decided for the current slices
-  bool usable = false;  // this form applies to them
+  bool probed = false;   // the planes are known for the current slices
+  bool applies = false;  // this form can take them (w planes and terms)
+  bool built = false;    // the rest below, or found not to fit
+  bool usable = false;   // built, and it fits
   int planes = 0;       // w planes
   int terms = 0;        // terms of the plane weights' series
   int chunk = 0;        // rows per work item at most
@@ -231,8 +233,10 @@ gvm_status forward_chi2(gvm_ctx* ctx, float* I, int flag_opt, int normalize,
                         double* out);
 gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
                    bool set = false);
-// The gridded form of the adjoint: its plan (*ok = false when it does not
-// apply) and its launches; free_grid_plan frees and clears a plan.
+// The gridded form of the adjoint: how many planes it needs (*ok = false when it does
+// not apply), its plan (*ok = false when there is no memory for it) and its launches;
+// free_grid_plan frees and clears a plan.
+gvm_status probe_grid_plan(gvm_ctx* ctx, bool* ok);
 gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok);
 gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
                         bool set);

@@ -48,9 +48,8 @@ typedef int gvm_status;
 
 /* Adjoint (DChi2) evaluation forms.  The first three evaluate the sums by
  * gridding and FFT in FP32 (FP32 MFMA spreading, FP64 combination) where that
- * applies, with the same result for each; where it does not (few rows on a
- * large image, w terms of more than about two turns, no memory for its
- * workspace) they are a GEMM with the operands named here. */
+ * applies, with the same result for each; where it does not (gvm_set_adjoint says
+ * when) they are a GEMM with the operands named here. */
 #define GVM_ADJOINT_F32 0      /* separable complex GEMM, FP32 MFMA            */
 #define GVM_ADJOINT_F16X3 1    /* FP16 hi/lo split, 3 MFMA products, FP32 acc  */
 #define GVM_ADJOINT_BF16X3 2   /* BF16 hi/lo split, 3 MFMA products, FP32 acc  */
@@ -209,9 +208,13 @@ gvm_status gvm_get_geometry(const gvm_ctx* ctx, gvm_geometry* out);
 
 /* Adjoint form used by gvm_dchi2 (GVM_ADJOINT_*; default GVM_ADJOINT_BF16X3).
  * F32, F16X3 and BF16X3 all run by gridding and FFT where that applies (sums of a
- * few 1e-7, below each of theirs); the form then only matters for the GEMM that
- * takes over: few visibilities on images of 2048^2 and more, or w terms that need
- * more than 32 planes.  DIRECT always is the direct sum. */
+ * few 1e-7, below each of theirs); the form then only matters for the GEMM that takes
+ * over: for w terms that need more than 32 planes (about two turns at the farthest
+ * pixel) or are not finite; without memory for the plan; where few rows are shared by so
+ * many slices and planes that it is more than four times faster by estimate; and on
+ * images of 1024^2 with fewer than 1,024 rows, or larger ones with fewer than one
+ * row to 8,192 pixels, wherever it is not clearly the slower.  gvm_set_gridding chooses
+ * otherwise.  DIRECT always is the direct sum. */
 gvm_status gvm_set_adjoint(gvm_ctx* ctx, int mode);
 /* No counterpart in the reference.  Whether the forms F32, F16X3 and BF16X3 run by
  * gridding and FFT (default GVM_GRIDDING_AUTO). */

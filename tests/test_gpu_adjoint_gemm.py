@@ -164,3 +164,33 @@ def test_the_autotuner_times_the_gemm(tmp_path, monkeypatch):
     assert not r["cached"] and min(r["ms"].values()) > 0.5 > gridded_ms
     assert np.array_equal(_gradient(ctx, d), before) and ctx.adjoint_gridded()
     ctx.close()
+
+
+@pytest.mark.parametrize("npix,nsl,rows,turns,gridded", [
+    (256, 64, 10, 0.3, False),   # many slices of few rows, 12 planes
+    (64, 1, 10, 2.0, False),     # few rows, 30 planes
+    (64, 1, 6000, 2.0, True),
+    (256, 2, 10, 0.02, True),
+    (256, 64, 10, 0.0, True),    # one plane
+    (1024, 1, 30, 0.3, False),   # below the line of few rows: the faster form
+    (1024, 1, 1000, 0.0, True),
+])
+def test_few_rows_on_many_transforms(npix, nsl, rows, turns, gridded):
+    """The form is chosen by slices and planes as well as by rows."""
+    print(f"case: {npix}^2 {nsl} slices of {rows} rows, {turns} turns", flush=True)
+    p = small_problem(npix=npix, n_antennas=6, seed=4)
+    p.noise = np.full_like(p.noise, 0.5 * p.noise_cut)
+    slices = [(f, uvw * [1.0, 1.0, 2.0 * turns], vo, w)
+              for f, uvw, vo, w in _slices(p, (rows,) * nsl, seed=npix)]
+    ctx = Context(p, add_data=False)
+    for s in slices:
+        ctx.add(*s)
+    d = ctx.image(_image(p, 5))
+    ctx.chi2(d)
+    g = _gradient(ctx, d)[0]
+    assert ctx.adjoint_gridded() == gridded
+    other = {True: "never", False: "always"}[gridded]
+    ctx.set_gridding(other)
+    assert _rel(g, _gradient(ctx, d)[0].astype(np.float64)) < TOL
+    assert ctx.adjoint_gridded() != gridded
+    ctx.close()
