@@ -868,6 +868,7 @@ gvm_status probe_grid_plan(gvm_ctx* ctx, bool* ok) {
     GVM_CHECK_LAUNCH();
     GVM_HIP_TRY(hipMemcpyAsync(&wbits, wmax, sizeof wbits, hipMemcpyDeviceToHost, st));
     GVM_HIP_TRY(hipStreamSynchronize(st));
+    sc.idle();
   }
   g.probed = true;
   if (wbits >= 0x7f800000u) return GVM_OK;  // an infinite or NaN w
@@ -1075,6 +1076,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
                        g.tile_slot + (long)s0 * ntiles);
     GVM_CHECK_LAUNCH();
     GVM_HIP_TRY(hipStreamSynchronize(st));  // the group's scratch is freed
+    sc.idle();
     nitems += ni;
     nmerges += nm;
     if (nitems > 0x7fffffffL) return give_up();

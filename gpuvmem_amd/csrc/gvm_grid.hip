@@ -838,6 +838,7 @@ extern "C" gvm_status gvm_grid_visibilities_dev(gvm_ctx* ctx, const gvm_ckernel*
                      reinterpret_cast<float2*>(vo_out_dev), weight_out_dev);
   if ((st = launch_ok(what))) return st;
   GVM_HIP_TRY(hipDeviceSynchronize());
+  sc.idle();
   *nout = count;
   return GVM_OK;
 }
@@ -1023,5 +1024,6 @@ extern "C" gvm_status gvm_weighting_apply_dev(gvm_ctx* ctx, int scheme, float ro
     if ((st = launch_ok(what))) return st;
   }
   GVM_HIP_TRY(hipDeviceSynchronize());
+  sc.idle();
   return GVM_OK;
 }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -155,7 +156,9 @@ struct gvm_ctx {
   // epoch changes whenever recorded device pointers or launches go stale
   bool capturing = false;
   long epoch = 0;
-  // set-up workspace: scratch of the gridder and the weighting schemes
+  // set-up workspace: scratch of the gridder, the weighting schemes and the adjoint's plan
+  // (on the null stream and on the context's, from any thread: one Scratch at a time)
+  std::mutex setup_mutex;
   char* setup_ws = nullptr;
   size_t setup_bytes = 0;
   // network workspace: the weight-gradient partials of a convolution
@@ -175,16 +178,21 @@ struct gvm_ctx {
 namespace gvm {
 
 // Scratch of one call, cut from the context's set-up workspace: sizes are
-// added up first, then reserve() and take() in the same order.
+// added up first, then reserve() and take() in the same order.  Other threads' calls
+// wait for its end, and its end for the device, unless the call has (idle()): whoever
+// comes next may use another stream.
 constexpr size_t kKeepScratch = 1UL << 30;  // a larger workspace is given back
 
 struct Scratch {
   gvm_ctx* ctx;
+  std::unique_lock<std::mutex> lock;
   size_t need = 0, at = 0;
-  explicit Scratch(gvm_ctx* c) : ctx(c) {}
+  explicit Scratch(gvm_ctx* c) : ctx(c), lock(c->setup_mutex) {}
   Scratch(const Scratch&) = delete;
   Scratch& operator=(const Scratch&) = delete;
+  void idle() { at = 0; }  // the device has finished with what was taken
   ~Scratch() {
+    if (at > 0) (void)hipDeviceSynchronize();
     if (ctx->setup_bytes > kKeepScratch) {
       (void)hipFree(ctx->setup_ws);
       ctx->setup_ws = nullptr;

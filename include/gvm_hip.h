@@ -142,7 +142,9 @@ typedef struct {
  * uvw_m_dev / vo_dev / weight_dev: the raw rows on the device (metres,
  * before the Hermitian flip; 3, 2 and 1 values per row); the outputs hold
  * `capacity` rows (M*N always suffices); *nout receives the count.
- * Synchronises the device. */
+ * Synchronises the device.  Scratch memory is the context's: this call, the weighting
+ * schemes and the first gradient on new visibilities wait for each other when several
+ * threads make them on one context.  Up to 1 GiB of it is kept until gvm_destroy. */
 gvm_status gvm_grid_visibilities_dev(gvm_ctx* ctx, const gvm_ckernel* kernel, float freq,
                                      long nvis, const double* uvw_m_dev, const float* vo_dev,
                                      const float* weight_dev, double* uvw_out_dev,
