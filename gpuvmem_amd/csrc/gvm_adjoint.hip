@@ -729,12 +729,24 @@ static gvm_status split_work(gvm_ctx* ctx) {
     // has to be ahead by more than the estimate is off
     if (ok && ctx->gridding == GVM_GRIDDING_AUTO)
       ok = gemm_over_gridded(ctx, ntiles) > (rows < min_gridded_rows(N) ? 1.5 : 0.25);
+    // the memory of the form that does not run is given back unless it is small (then a
+    // caller may go back and forth between the forms)
+    if (ok && sizeof(float) * ctx->adj_part_elems > kKeepScratch) {
+      GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
+      GVM_HIP_TRY(hipFree(ctx->adj_part));
+      ctx->adj_part = nullptr;
+      ctx->adj_part_elems = 0;
+    }
     if (ok && (st = build_grid_plan(ctx, &ok))) return st;
     if (ok) {
       ctx->adj_gridded = true;
       ctx->split_mode = mode;
       return GVM_OK;
     }
+  }
+  if (ctx->gplan.bytes > kKeepScratch) {
+    GVM_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    release_grid_plan(ctx->gplan);
   }
   return build_splits(ctx, mode, ntiles, (long)N * N);
 }

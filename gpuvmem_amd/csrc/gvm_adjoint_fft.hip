@@ -826,12 +826,12 @@ int row_pitch(int N) { return N + 8; }
 
 }  // namespace
 
-// Frees what build_grid_plan made; the planes stay known.
-static void release_grid_plan(GridPlan& g) {
+void release_grid_plan(GridPlan& g) {
   (void)hipFree(g.tables);
   (void)hipFree(g.lists);
   (void)hipFree(g.ws);
   g.tables = g.lists = g.ws = nullptr;
+  g.bytes = 0;
   g.built = g.usable = false;
 }
 
@@ -964,6 +964,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   const size_t p_meta = place(at, sizeof(uint2) * (size_t)total);
   const size_t p_rot = place(at, shifted ? sizeof(float2) * (size_t)total : 0);
   if (!device_array(&g.tables, at)) return give_up();
+  g.bytes = at;
   GVM_HIP_TRY(hipMemcpy(g.tables, up.data(), up.size(), hipMemcpyHostToDevice));
   g.tw2 = (float2*)(g.tables + p_tw2);
   g.corr = (double*)(g.tables + p_corr);
@@ -1100,6 +1101,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
     }
     GVM_HIP_TRY(hipStreamSynchronize(st));
   }
+  g.bytes += sizeof(long4) * (size_t)nitems + sizeof(int2) * (size_t)nmerges;
   g.items = (long4*)g.lists;
   g.merges = (int2*)(g.items + nitems);
 
@@ -1108,7 +1110,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   const size_t per_slice = sizeof(float2) * (size_t)K * N * row_pitch(N);
   size_t free_b = 0, total_b = 0;
   GVM_HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-  const size_t budget = std::min<size_t>(32UL << 30, (free_b + sizeof(float) * ctx->adj_part_elems) / 2);
+  const size_t budget = std::min<size_t>(32UL << 30, free_b / 2);
   g.batch0.clear();
   size_t need_part = 0, need_slices = 0;
   for (int s = 0; s < nsl;) {
@@ -1132,6 +1134,7 @@ gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok) {
   const size_t bytes = g.part_bytes + per_slice * need_slices;
   if (bytes > budget) return give_up();
   if (!device_array((char**)&g.ws, bytes)) return give_up();
+  g.bytes += bytes;
   g.usable = true;
   *ok = true;
   return GVM_OK;

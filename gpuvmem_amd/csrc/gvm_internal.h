@@ -95,6 +95,7 @@ struct GridPlan {
   char* lists = nullptr;     // holds items, merges
   char* ws = nullptr;        // subgrids, then the transformed columns
   size_t part_bytes = 0;     // of the subgrids
+  size_t bytes = 0;          // of tables, lists and ws
   std::vector<long> slice_slot;  // slice s owns items [slice_slot[s], slice_slot[s + 1])
   std::vector<long> slice_merge;  // and merges [slice_merge[s], slice_merge[s + 1])
   std::vector<int> batch0;       // slices that share the workspace: [batch0[b], batch0[b + 1])
@@ -243,11 +244,13 @@ gvm_status adjoint(gvm_ctx* ctx, const float* I, float* result, int flag_opt, in
                    bool set = false);
 // The gridded form of the adjoint: how many planes it needs (*ok = false when it does
 // not apply), its plan (*ok = false when there is no memory for it) and its launches;
-// free_grid_plan frees and clears a plan.
+// release_grid_plan frees what build_grid_plan made (the planes stay known),
+// free_grid_plan all.
 gvm_status probe_grid_plan(gvm_ctx* ctx, bool* ok);
 gvm_status build_grid_plan(gvm_ctx* ctx, bool* ok);
 gvm_status adjoint_grid(gvm_ctx* ctx, const float* I, float* result, int flag_opt, int normalize,
                         bool set);
+void release_grid_plan(GridPlan& g);
 void free_grid_plan(GridPlan& g);
 // Rebuilds the adjoint's range table and workspace for the current form.
 gvm_status rebuild_splits(gvm_ctx* ctx);

@@ -7,6 +7,7 @@ its sums are short, else against the gridded form, which its own tests hold to
 Tolerance: 1e-5 relative L2, the gradient's bar; 1.15e-5 against the gridded form."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from gpuvmem_amd import native
@@ -193,4 +194,29 @@ def test_few_rows_on_many_transforms(npix, nsl, rows, turns, gridded):
     ctx.set_gridding(other)
     assert _rel(g, _gradient(ctx, d)[0].astype(np.float64)) < TOL
     assert ctx.adjoint_gridded() != gridded
+    ctx.close()
+
+
+def test_the_form_that_does_not_run_keeps_little_memory():
+    """4096^2 with 60,000 rows: a plan of 1.9 GiB (8 planes) and a GEMM workspace of 1.5;
+    going from one to the other gives back what is over 1 GiB."""
+    p = small_problem(npix=4096, n_antennas=4, seed=6, dump_seconds=3600.0)
+    p.noise = np.full_like(p.noise, 0.5 * p.noise_cut)
+    slices = [(f, uvw * [1.0, 1.0, 0.2], vo, w) for f, uvw, vo, w in _slices(p, (60000,))]
+    ctx = Context(p, add_data=False)
+    ctx.add(*slices[0])
+    d = ctx.image(p.initial_image())
+    ctx.chi2(d)
+    r = ctx.zeros(2 * ctx.n)
+    ctx.sync()
+    base, used = torch.cuda.mem_get_info()[0], {}
+    for k, when in enumerate(("always", "never", "always", "never")):
+        ctx.set_gridding(when)
+        ctx.dchi2(d, r)
+        ctx.sync()
+        assert ctx.adjoint_gridded() == (when == "always")
+        used[k] = (base - torch.cuda.mem_get_info()[0]) / 2 ** 30
+    print(f"GiB in use: {used}", flush=True)
+    assert 1.5 < used[0] < 2.25 and 1.25 < used[1] < 1.75
+    assert abs(used[2] - used[0]) < 0.25 and abs(used[3] - used[1]) < 0.25
     ctx.close()
