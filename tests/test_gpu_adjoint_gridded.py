@@ -8,9 +8,10 @@ and too many planes for it (the GEMM takes the call), slices of very
 different length, and rows that are not numbers.
 
 Tolerance: the FP32 transform of (2N)^2 points rounds about 2 log2(2N) <= 26
-times per value at 6e-8 each, at random, times at most 3 for the kernel
-correction off the centre: 3 sqrt(26) 6e-8 = 9e-7, plus 1e-7 each for the
-kernel's evaluation, the spreading sums and the final float: 1.5e-6.  The
+times per value at 6e-8 each, at random, times 3 for the kernel correction off
+the centre (its rms over the image: it grows to 3.1 along each axis, 9.5 at a corner,
+and the corners have a test of their own): 3 sqrt(26) 6e-8 = 9e-7, plus 1e-7 each for
+the kernel's evaluation, the spreading sums and the final float: 1.5e-6.  The
 GEMM's cases keep the 1e-5 that its own tests use."""
 import numpy as np
 import pytest
@@ -213,3 +214,94 @@ def test_a_result_that_is_set(mode, flag, nsl):
         out.append(r.download(np.float32))
     ctx.close()
     assert np.array_equal(out[0], out[1])
+
+
+def test_the_largest_image():
+    """4096^2 has blocks of its own: two columns (8,192-point transforms), rows of
+    1,024 threads."""
+    n = 4096
+    p = _open_mask(small_problem(npix=n, n_antennas=4, seed=7, dump_seconds=600.0))
+    rng = np.random.default_rng(n)
+    cells = np.stack([rng.uniform(0, n, 3000), rng.uniform(-n + 1, n - 1, 3000)], 1)
+    edge = [0.0, 3.75, n / 2 - 0.25, n / 2, n / 2 + 2.25, n - 1e-4]
+    cells = np.concatenate([cells, [(a, b) for a in edge for b in [0.0, -2.0, n / 2, n - 1.5]]])
+    s = _rows(p, cells, w=rng.uniform(-1e5, 1e5, len(cells)))
+    _check(p, [s], seed=n, repeat=True, pixels=60)
+    ctx = Context(p, add_data=False)
+    ctx.add(*s)
+    d = ctx.image(p.initial_image())
+    ctx.chi2(d)
+    r = ctx.zeros(2 * n * n)
+    ctx.dchi2(d, r)
+    ctx.sync()
+    assert ctx.adjoint_gridded()
+    ctx.close()
+
+
+@pytest.mark.parametrize("npix,turns", [(64, 0.0), (256, 0.3), (1024, 0.02), (2048, 0.02)])
+def test_corner_pixels(npix, turns):
+    """The corners by themselves: the kernel's transform falls to 1 / 3.1 at an
+    edge and 1 / 9.5 at a corner, and rounding is multiplied by as much there.  sqrt(26)
+    6e-8 of the transforms times 9.5, plus 1e-7 each for the spreading sums, the final
+    float and the kernel's evaluation times its share at a corner: 2.9e-6 + 0.3e-6."""
+    p = _open_mask(small_problem(npix=npix, n_antennas=5, seed=npix))
+    p.antenna_diameter, p.pb_cutoff = 1.0, 1.0  # a beam that reaches the corners
+    rng = np.random.default_rng(npix + 1)
+    n, m = npix, 4000
+    x = n / 2 * abs(p.deltax) * np.pi / 180.0
+    f = 2 * x * x / (1 + np.sqrt(1 - 2 * x * x))
+    cells = np.stack([rng.uniform(0, 0.48 * n, m), rng.uniform(-0.48 * n, 0.48 * n, m)], 1)
+    s = _rows(p, cells, w=rng.uniform(-1, 1, m) * turns / f)
+    ctx = Context(p, add_data=False)
+    ctx.add(*s)
+    d = ctx.image(p.initial_image())
+    ctx.chi2(d)
+    vr = ctx.residuals(0, m).astype(np.float64)
+    e = np.r_[0:6, n - 6:n]
+    pix = np.array([(i, j) for i in e for j in e])
+    ref = _direct_sums(p, s, vr[:, 0] + 1j * vr[:, 1], pix)
+    got = {}
+    for when, form in (("always", "f32"), ("never", "f32"), ("never", "bf16x3")):
+        ctx.set_gridding(when)
+        ctx.set_adjoint(form)
+        r = ctx.zeros(2 * n * n)
+        ctx.dchi2(d, r)
+        ctx.sync()
+        g = r.download(np.float32, (2, n, n))[0]
+        got[when, form] = np.linalg.norm(g[pix[:, 0], pix[:, 1]] - ref) / np.linalg.norm(ref)
+    print(f"{n}^2 {turns} turns, corners: {got}", flush=True)
+    assert got["always", "f32"] < 3.2e-6
+    ctx.close()
+
+
+@pytest.mark.parametrize("flag", [0, 1])
+def test_a_result_that_is_set_over_several_batches(flag):
+    """Eleven slices at 1024^2 with 6 planes (51 MB of transforms each): ten share the
+    workspace, the last has it for itself and writes the result straight."""
+    p = small_problem(npix=1024, n_antennas=5, seed=12)
+    rng = np.random.default_rng(flag)
+    x = 512 * abs(p.deltax) * np.pi / 180.0
+    f = 2 * x * x / (1 + np.sqrt(1 - 2 * x * x))
+    img = p.initial_image()
+    img[0] += (rng.random((p.N, p.M)) * 20.0).astype(np.float32)
+    img[1] = rng.uniform(-1.0, 2.0, (p.N, p.M)).astype(np.float32)
+    ctx = Context(p, add_data=False)
+    ctx.set_gridding("always")
+    for k in range(11):
+        cells = np.stack([rng.uniform(0, 400, 100), rng.uniform(-400, 400, 100)], 1)
+        ctx.add(p.freq * (1.0 + 0.02 * k),
+                *_rows(p, cells, w=rng.uniform(-1, 1, 100) * 0.02 / f, seed=k)[1:])
+    d = ctx.image(img)
+    ctx.chi2(d, flag_opt=flag)
+    out = []
+    for fn, fill, when in ((ctx.lib.gvm_dchi2, 0.0, "always"), (ctx.lib.gvm_dchi2_set, np.nan, "always"),
+                           (ctx.lib.gvm_dchi2_set, np.nan, "never")):
+        ctx.set_gridding(when)
+        r = DeviceBuffer.from_array(np.full(2 * p.M * p.N, fill, np.float32))
+        native.check(fn(ctx.ctx, d.ptr, r.ptr, flag, 1), "dchi2")
+        ctx.sync()
+        assert ctx.adjoint_gridded() == (when == "always")
+        out.append(r.download(np.float32))
+    ctx.close()
+    assert np.array_equal(out[0], out[1])
+    assert np.linalg.norm(out[0] - out[2]) < 1.15e-5 * np.linalg.norm(out[2])
