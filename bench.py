@@ -20,16 +20,15 @@ times the FP64 oracle on the host cores on a bounded sample (full-size
 forward chi2 + the separable FP64 gradient over a slice of the
 visibilities, extrapolated linearly in the visibility count).  The
 time_to_image object times L-BFGS to a common objective with the plain FP32
-and the split-precision adjoint, and the split form once more from the
-learned warm start of the committed network (gpuvmem_amd/data/).  (Where both
-forms run by gridding and FFT, as here, the first two legs differ by the
-evaluation graphs alone.)
+GEMM adjoint and with the default one (bf16x3, by gridding and FFT at this size), and the
+default once more from the learned warm start of the committed network
+(gpuvmem_amd/data/).
 
 Other modes, each printing its own JSON line: --workload 0/2/3 (other
-workloads), --time-to-image ITERS (split precision against plain FP32 at
+workloads), --time-to-image ITERS (the default adjoint against the plain FP32 GEMM at
 equal objective, median over observations), --precision-study, --gridding,
---warm-start (the learned warm start; --ws-* options), --graphs and
---autotune (modifiers of the evals/s run).
+--warm-start (the learned warm start; --ws-* options), --graphs, --gemm (the GEMM
+that --adjoint names instead of gridding) and --autotune (modifiers of the evals/s run).
 """
 from __future__ import annotations
 
@@ -486,16 +485,29 @@ def _slice_problem(p, k):
     return q
 
 
+def form_context(p, form: str):
+    """A context whose adjoint runs as `form` and no other: "gridded", or the GEMM or
+    direct sum of that name ("mode/L": with visibility ranges of L)."""
+    from gpuvmem_amd.device import Context
+
+    mode, _, ranges = form.partition("/")
+    ctx = Context(p, adjoint="bf16x3" if mode == "gridded" else mode)
+    ctx.set_gridding("always" if mode == "gridded" else "never")
+    if ranges:
+        ctx.set_split_vis(int(ranges))
+    return ctx
+
+
 def time_to_image(p, iterations: int, forms=("f32", "bf16x3"), warm_model=None) -> dict:
     """L-BFGS (memory 10) from the default initial image with each adjoint
-    form, up to `iterations` iterations (the reference's optimiser may stop
+    form (f32: its GEMM; the others as they run by default, by gridding and FFT where
+    that applies), up to `iterations` iterations (the reference's optimiser may stop
     earlier when its line search makes no progress).  The target is the
     objective value every form reached (the largest of the final values),
     and each form is timed to its first iteration at or below it.  Each
     context does one untimed evaluation first (workspace allocation).  Every
-    form runs with the same settings: evaluation graphs replayed and the
-    adjoint range length autotuned, so the ratio measures the adjoint's
-    precision form alone.
+    form runs with the same settings: evaluation graphs replayed and a GEMM's
+    range length autotuned, so the ratio measures the adjoint's form alone.
 
     With `warm_model` (a network written by WarmStart.save), the last form
     runs once more from the learned warm start: the dirty image, the
@@ -511,13 +523,19 @@ def time_to_image(p, iterations: int, forms=("f32", "bf16x3"), warm_model=None) 
         name = mode + "_warm" if warm_leg else mode
         extras = mode != "direct"
         ctx = Context(p, adjoint=mode)
+        if mode == "f32":
+            ctx.set_gridding("never")
         obj = Objective(ctx, fw_config(terms, lambdas=(0.01, 1e-3)))
         obj.set_graphs(extras)
         warm = ctx.image(p.initial_image())
         xi = ctx.zeros(2 * p.M * p.N)
         obj.value(warm)
-        tune = ctx.autotune() if extras else None
         obj.gradient(warm, xi, 0)
+        gridded, tune = ctx.adjoint_gridded(), None
+        if extras and not gridded:
+            obj.value(warm)
+            tune = ctx.autotune()
+            obj.gradient(warm, xi, 0)
         rec = {}
         if warm_leg:
             from gpuvmem_amd import warmstart as W
@@ -552,7 +570,8 @@ def time_to_image(p, iterations: int, forms=("f32", "bf16x3"), warm_model=None) 
             "gradient_calls": res.gradient_calls,
             "graphs": extras,
             "graph_replays": obj.graph_launches(),
-            "split_vis": ctx.split_vis() if mode != "direct" else None,
+            "gridded": gridded,
+            "split_vis": None if mode == "direct" or gridded else ctx.split_vis(),
             "autotune": tune,
             **rec,
         }
@@ -582,9 +601,9 @@ def tti_observations(p, workload: int, iterations: int, n_obs: int, warm_model=N
     """time_to_image on n_obs observations (new sky and noise seeds, same
     array): the line search is chaotic, so where each form stops, and the
     ratio at the common objective, vary from one observation to the next.
-    Returns the median ratio of plain FP32 seconds to split-precision
-    seconds with the per-observation records, and with `warm_model` the
-    median ratio of plain FP32 seconds to split-precision seconds from the
+    Returns the median ratio of the plain FP32 GEMM's seconds to the default
+    form's with the per-observation records, and with `warm_model` the
+    median ratio of the plain FP32 GEMM's seconds to the default form's from the
     learned warm start, both to the value all runs reached."""
     obs = []
     for k in range(max(1, n_obs)):
@@ -608,11 +627,11 @@ def tti_observations(p, workload: int, iterations: int, n_obs: int, warm_model=N
     ratios = [o["ratio"] for o in obs if o["ratio"]]
     out = {
         "value": float(np.median(ratios)) if ratios else None,
-        "unit": "x (plain FP32 seconds / split-precision seconds, median over observations)",
+        "unit": "x (plain FP32 GEMM seconds / default form's seconds, median over observations)",
         "config": {"workload": f"{p.M}x{p.N} image, {p.nvis} visibilities, chi2+entropy+TSV, "
                                f"L-BFGS m=10, at most {iterations} iterations per form",
                    "observations": len(obs),
-                   "settings": "both forms: evaluation graphs, autotuned adjoint range length"},
+                   "settings": "both forms: evaluation graphs; GEMM: autotuned range length"},
         "median_per_iteration_ratio": float(np.median([o["per_iteration_ratio"] for o in obs])),
         "observations": obs,
     }
@@ -620,7 +639,7 @@ def tti_observations(p, workload: int, iterations: int, n_obs: int, warm_model=N
         ws = [o["forms"]["bf16x3_warm"] for o in obs]
         out["warm_start"] = {
             "value": float(np.median([o["ratio_warm"] for o in obs])),
-            "unit": "x (plain FP32 seconds / split-precision + graphs + learned warm start "
+            "unit": "x (plain FP32 GEMM seconds / default form + graphs + learned warm start "
                     "seconds, to the objective all runs reached; median over observations)",
             "median_ratio_split_same_target": float(np.median([o["ratio_split_all"]
                                                                for o in obs])),
@@ -646,11 +665,10 @@ def make_problem_of(workload: int, **overrides):
 def precision_study(p, pixels: int = 64, split_vis: int = 0) -> dict:
     """Each adjoint form against FP64: chi2 against the oracle's FP64
     forward pass, the gradient against FP64 direct sums on a pixel sample
-    inside the mask, and the split forms against the FP32 and direct forms
-    over the whole image."""
+    inside the mask, and the split GEMMs and the gridded form against the FP32 GEMM
+    and the direct sum over the whole image."""
     sys.path.insert(0, str(ROOT / "oracle"))
     import oracle
-    from gpuvmem_amd.device import Context
 
     img = bench_image(p)
     orc = oracle.Oracle(p, separable=True)
@@ -660,9 +678,9 @@ def precision_study(p, pixels: int = 64, split_vis: int = 0) -> dict:
     pix = inside[rng.choice(len(inside), pixels, replace=False)]
     gref = orc.dchi2_pixels(vr, pix)
     out, full = {}, {}
-    for mode in ("direct", "f32", "f16x3", "bf16x3"):
-        ctx = Context(p, adjoint=mode)
-        if split_vis and mode != "direct":
+    for mode in ("direct", "f32", "f16x3", "bf16x3", "gridded"):
+        ctx = form_context(p, mode)
+        if split_vis and mode not in ("direct", "gridded"):
             ctx.set_split_vis(split_vis)
         d = ctx.image(img)
         v = ctx.chi2(d)
@@ -682,7 +700,7 @@ def precision_study(p, pixels: int = 64, split_vis: int = 0) -> dict:
                      "grad_rel_l2_vs_fp64_pixels": float(np.linalg.norm(gs - gref) / np.linalg.norm(gref)),
                      "adjoint_ms": ms}
         print(f"# precision {mode}: {out[mode]}", file=sys.stderr, flush=True)
-    for mode in ("f32", "f16x3", "bf16x3"):
+    for mode in ("f32", "f16x3", "bf16x3", "gridded"):
         for base in ("direct", "f32"):
             if mode != base:
                 out[mode][f"grad_rel_l2_vs_{base}_image"] = float(
@@ -690,9 +708,10 @@ def precision_study(p, pixels: int = 64, split_vis: int = 0) -> dict:
     return {"pixels": pixels, "forms": out}
 
 
-def replay_image_study(p, iterations: int, forms=("bf16x3", "f16x3", "f32/6144")) -> dict:
+def replay_image_study(p, iterations: int,
+                       forms=("bf16x3", "f16x3", "f32/6144", "gridded")) -> dict:
     """The image after `iterations` CG-FRPRMN iterations (chi2 + entropy +
-    TSV from the default image) with the plain FP32 adjoint, its applied step
+    TSV from the default image) with the plain FP32 GEMM, its applied step
     lengths recorded, then the same path in each other form with those steps
     replayed: what separates the final images is then the adjoint's
     arithmetic, not the line search's branch decisions.  Reports each form's
@@ -702,16 +721,13 @@ def replay_image_study(p, iterations: int, forms=("bf16x3", "f16x3", "f32/6144")
     default ranges are 3072 visibilities, and the workspace limit keeps them
     from getting shorter), which shows how far the path carries a
     rounding-level difference in the gradient."""
-    from gpuvmem_amd.device import Context, Objective, fw_config
+    from gpuvmem_amd.device import Objective, fw_config
 
     terms = [("Chi2", -1, 0.0), ("Entropy", 0, 0.001), ("TotalSquaredVariation", 1, 0.0)]
     mask = p.noise < p.noise_cut
     runs = {}
     for mode in ("f32",) + tuple(forms):
-        form, _, rng = mode.partition("/")
-        ctx = Context(p, adjoint=form)
-        if rng:
-            ctx.set_split_vis(int(rng))
+        ctx = form_context(p, mode)
         obj = Objective(ctx, fw_config(terms, lambdas=(0.01, 1e-3)))
         if mode != "f32":
             obj.set_line_search_replay(runs["f32"]["steps"])
@@ -744,10 +760,7 @@ def replay_image_study(p, iterations: int, forms=("bf16x3", "f16x3", "f32/6144")
     gref = orc.dchi2_pixels(vr, pix)
     grads = {}
     for mode in ("f32",) + tuple(forms):
-        form, _, rng = mode.partition("/")
-        ctx = Context(p, adjoint=form)
-        if rng:
-            ctx.set_split_vis(int(rng))
+        ctx = form_context(p, mode)
         d = ctx.image(final)
         ctx.chi2(d)
         res = ctx.zeros(2 * p.M * p.N)
@@ -790,7 +803,7 @@ def replay_image_study(p, iterations: int, forms=("bf16x3", "f16x3", "f32/6144")
 
 
 def gradient_difference_study(p, iterations: int,
-                              forms=("f32", "f32/6144", "bf16x3", "f16x3")) -> dict:
+                              forms=("f32", "f32/6144", "bf16x3", "f16x3", "gridded")) -> dict:
     """How each form's gradient error changes between two consecutive
     images of an optimisation path, against the change of the gradient
     itself: the FP32 form's CG path (chi2 + entropy + TSV) gives image B after
@@ -799,13 +812,13 @@ def gradient_difference_study(p, iterations: int,
     below the others'), each form's error d = g_form - g is taken at A and
     B on the mask; Polak-Ribiere's gamma and L-BFGS's y see
     |d(B) - d(A)| / |g(B) - g(A)|."""
-    from gpuvmem_amd.device import Context, Objective, fw_config
+    from gpuvmem_amd.device import Objective, fw_config
 
     terms = [("Chi2", -1, 0.0), ("Entropy", 0, 0.001), ("TotalSquaredVariation", 1, 0.0)]
     mask = p.noise < p.noise_cut
     imgs, steps = {}, None
     for name, n in (("B", iterations), ("A", iterations - 1)):
-        ctx = Context(p, adjoint="f32")
+        ctx = form_context(p, "f32")
         obj = Objective(ctx, fw_config(terms, lambdas=(0.01, 1e-3)))
         if steps is not None:
             obj.set_line_search_replay(steps[:n])
@@ -818,10 +831,7 @@ def gradient_difference_study(p, iterations: int,
         ctx.close()
     grads = {}
     for mode in ("direct",) + tuple(forms):
-        form, _, rng = mode.partition("/")
-        ctx = Context(p, adjoint=form)
-        if rng:
-            ctx.set_split_vis(int(rng))
+        ctx = form_context(p, mode)
         for name, img in imgs.items():
             d = ctx.image(img)
             ctx.chi2(d)
@@ -870,24 +880,27 @@ def main() -> int:
     ap.add_argument("--no-tti", action="store_true",
                     help="default run: leave out the time-to-image and plain-FP32 legs")
     ap.add_argument("--time-to-image", type=int, default=0, metavar="ITERS",
-                    help="instead of evals/s: L-BFGS time-to-image of the split-precision "
-                         "adjoint against the plain FP32 one at equal objective value")
+                    help="instead of evals/s: L-BFGS time-to-image of the default adjoint "
+                         "against the plain FP32 GEMM at equal objective value")
     ap.add_argument("--study-iterations", type=int, default=0, metavar="ITERS",
                     help="precision study: also the image after ITERS CG-FRPRMN iterations, "
-                         "FP32 path replayed in the split forms")
+                         "the FP32 GEMM's path replayed in the other forms")
     ap.add_argument("--split-vis", type=int, default=0, metavar="L",
                     help="precision study: visibility range length of the GEMM forms "
                          "(default: the context's)")
     ap.add_argument("--diff-study", type=int, default=0, metavar="ITERS",
                     help="precision study: each form's gradient error between the last two "
                          "images of an ITERS-step FP32 CG path, against the gradient's change")
-    ap.add_argument("--study-forms", default="bf16x3,f16x3,f32/6144",
-                    help="precision study: the forms that replay the FP32 path (mode or mode/L)")
+    ap.add_argument("--study-forms", default="bf16x3,f16x3,f32/6144,gridded",
+                    help="precision study: the forms that replay the FP32 path (a GEMM or direct "
+                         "mode, mode/L, or gridded)")
     ap.add_argument("--precision-study", action="store_true",
                     help="instead of evals/s: each adjoint form against FP64 (use with "
                          "--workload 2: 2048^2, 4.35M vis)")
+    ap.add_argument("--gemm", action="store_true",
+                    help="the GEMM that --adjoint names instead of gridding and FFT")
     ap.add_argument("--autotune", action="store_true",
-                    help="pick the adjoint's range length by timing before the run")
+                    help="pick the GEMM's range length by timing before the run")
     ap.add_argument("--graphs", action="store_true",
                     help="replay captured HIP graphs of the value and gradient evaluations")
     ap.add_argument("--warm-start", action="store_true",
@@ -1001,6 +1014,8 @@ def main() -> int:
             "higher_is_better": True, "n_gpus": 1, "data": "synthetic", **r}), flush=True)
         return 0
     ctx = Context(p, adjoint=args.adjoint)
+    if args.gemm:
+        ctx.set_gridding("never")
     terms = [("Chi2", -1, 0.0), ("Entropy", 0, 0.001), ("TotalSquaredVariation", 1, 0.0)]
     obj = Objective(ctx, fw_config(terms, lambdas=(0.01, 1e-3)))
     obj.set_graphs(args.graphs)
@@ -1112,7 +1127,7 @@ def main() -> int:
     obj.close()
     ctx.close()
     if not args.no_tti and args.workload == 1 and args.adjoint != "f32":
-        # the plain FP32 form's evals/s on the same step, then time to image
+        # the plain FP32 GEMM's evals/s on the same step, then time to image
         line["plain_fp32"] = plain_fp32_step(p, args.steps, args.warmup, args.graphs)
         print(f"# plain FP32 step: {line['plain_fp32']}", file=sys.stderr, flush=True)
         tti = tti_observations(p, args.workload, args.tti_iterations, args.tti_observations,
@@ -1158,10 +1173,10 @@ def value_latency(obj, d_img, ctx, n: int = 200) -> dict:
 
 
 def plain_fp32_step(p, steps: int, warmup: int, graphs: bool) -> dict:
-    """The benchmark's step with the plain FP32 MFMA adjoint."""
-    from gpuvmem_amd.device import Context, Objective, fw_config
+    """The benchmark's step with the plain FP32 MFMA GEMM as the adjoint."""
+    from gpuvmem_amd.device import Objective, fw_config
 
-    ctx = Context(p, adjoint="f32")
+    ctx = form_context(p, "f32")
     terms = [("Chi2", -1, 0.0), ("Entropy", 0, 0.001), ("TotalSquaredVariation", 1, 0.0)]
     obj = Objective(ctx, fw_config(terms, lambdas=(0.01, 1e-3)))
     obj.set_graphs(graphs)
@@ -1200,7 +1215,7 @@ def compact_tti(r: dict) -> dict:
             rec[m] = {k: f[k] for k in ("seconds_to_target", "iterations_to_target",
                                         "seconds_to_target_all", "iterations_to_target_all",
                                         "iterations_run", "seconds_run", "final_objective",
-                                        "final_chi2", "split_vis", "prediction_used",
+                                        "final_chi2", "gridded", "split_vis", "prediction_used",
                                         "start_objective", "start_seconds",
                                         "image_rel_l2_vs_f32") if k in f}
         obs.append(rec)

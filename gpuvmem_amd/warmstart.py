@@ -330,7 +330,7 @@ def dirty_image(ctx: Context, p) -> np.ndarray:
 
 def solve(p, init: Optional[np.ndarray] = None, iterations: int = 400,
           optimizer: str = "CG-FRPRMN", graphs: Optional[bool] = None, adjoint: str = "bf16x3",
-          terms=None, lambdas=None):
+          terms=None, lambdas=None, gridding: str = "auto"):
     """The plain MEM optimisation (CG-FRPRMN, the workload's optimiser, or
     CG-LBFGS with memory 10), run to its own tolerance or `iterations`, from
     the default image or `init` (image 0), on the objective `terms` /
@@ -338,6 +338,7 @@ def solve(p, init: Optional[np.ndarray] = None, iterations: int = 400,
     of objective values with the starting value first, seconds to each entry,
     result)."""
     ctx = Context(p, adjoint=adjoint)
+    ctx.set_gridding(gridding)
     obj = Objective(ctx, fw_config(TERMS if terms is None else terms,
                                    lambdas=LAMBDAS if lambdas is None else lambdas))
     obj.set_graphs(GRAPHS if graphs is None else graphs)
@@ -517,8 +518,8 @@ def evaluate(ws: WarmStart, seeds, iterations: int = 400, optimizer: str = "CG-F
     held-out observations: iterations and seconds (dirty image and inference
     included for the warm start) to the objective value both reach, and the
     relative L2 error of both final images against the true sky inside the
-    mask.  With plain=True, also the plain FP32 form (FP32 adjoint, no
-    graphs, default image) to the value all three reach."""
+    mask.  With plain=True, also the plain FP32 form (FP32 GEMM as
+    the adjoint, no graphs, default image) to the value all three reach."""
     rows = []
     for s in seeds:
         p = observation(s, which)
@@ -542,7 +543,8 @@ def evaluate(ws: WarmStart, seeds, iterations: int = 400, optimizer: str = "CG-F
         extra = {}
         if plain:
             img_p, tr_p, sc_p, _ = solve(p, iterations=iterations, optimizer=optimizer,
-                                         graphs=False, adjoint="f32", **obj_kw)
+                                         graphs=False, adjoint="f32", gridding="never",
+                                         **obj_kw)
             t3 = max(target, tr_p[-1])
             cp, cw = time_to(tr_p, sc_p, t3), time_to(tr_w, sc_w, t3)
             extra = dict(f_plain=tr_p[-1], iters_plain=cp[0], seconds_plain=cp[1],
