@@ -482,23 +482,23 @@ __global__ __launch_bounds__(kThreads) void grid_emit_kernel(
   }
 }
 
-// The form by its estimated time in microseconds.  Entries: their sort and sums.  Tiles:
-// passes over the cells, the sort, and the chain of the rows that reach a tile (0.06
-// for each of an even share: the fullest tiles, whose 40 ns a row decide, have more.
-// Single taps hit cells as unevenly as rows lie, and their entries are no more than the
-// rows: 0.15, and no allowance on the entries' side).  Both sides in us, entries / tiles:
-// 300,000 rows on 64 x 64 with one tap 237 / 589, all in one cell 4,850 / 11,800; 1.7 M rows
-// there with 3 x 3 taps 1,840 / 4,410; 100 rows on 4096 x 4096 with 7 x 7 taps 107 / 268;
-// but 10,000 rows on 64 x 64 with 7 x 7 taps 276 / 189, 1.7 M on 512 x 512 with 3 x 3 taps
-// 2,050 / 661.  At most 2^26 entries (2.4 GB of scratch).
+// Single taps are summed by entry: as many entries as rows, no chain but a cell's own (us,
+// entries / tiles: 300,000 rows on 64 x 64 243 / 589, all in one cell 4,850 / 11,800; the
+// 1.76 M rows of the 1024 x 1024 workload 2,760 / 2,970 with the copy of their cells to the
+// host; but 1.7 M rows spread evenly over 1024 x 1024 371 / 298).  Else by the estimated time in
+// microseconds.  Entries: their sort and sums.  Tiles: passes over the cells, the sort, and
+// the chain of the rows that reach a tile (0.06 for each of an even share: the fullest
+// tiles, whose 40 ns a row decide, have more).  1.7 M rows on 64 x 64 with 3 x 3 taps take
+// 1,840 / 4,410, 100 rows on 4096 x 4096 with 7 x 7 taps 104 / 268; but 10,000 rows on 64 x
+// 64 with 7 x 7 taps 276 / 189, 1.7 M on 512 x 512 with 3 x 3 taps 2,050 / 661.  At most 2^26
+// entries (2.4 GB of scratch).
 bool use_entries(const GridGeom& g, long nvis) {
   const double rows = 2.0 * nvis, cells = (double)g.M * g.N, taps = (double)g.wx * g.wy;
   const double reached = (1.0 + (g.wx - 1) / 8.0) * (1.0 + (g.wy - 1) / 8.0);
   const double share = rows * reached / ((double)g.ntx * g.nty);
-  const double entry_us = taps == 1.0 ? 10.0 + 7.5e-5 * rows : 25.0 + 8.5e-5 * rows * taps;
-  const double tile_us =
-      1.1e-5 * cells + 6e-5 * rows * g.tx * g.ty + (taps == 1.0 ? 0.15 : 0.06) * share;
-  return entry_us < tile_us && rows * taps <= 67108864.0;
+  const double entry_us = 25.0 + 8.5e-5 * rows * taps;
+  const double tile_us = 1.1e-5 * cells + 6e-5 * rows * g.tx * g.ty + 0.06 * share;
+  return rows * taps <= 67108864.0 && (taps == 1.0 || entry_us < tile_us);
 }
 
 // ---- weighting schemes -----------------------------------------------------
