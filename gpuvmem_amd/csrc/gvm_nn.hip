@@ -14,6 +14,7 @@
 
 #include "gvm_internal.h"
 #include "gvm_nn.h"
+#include "gvm_nn_pixels.h"
 
 namespace gvm {
 namespace {
@@ -313,7 +314,6 @@ __global__ __launch_bounds__(256) void conv_im2col_kernel(ConvArgs<WT> a) {
 
 // ---- weight gradient ----
 constexpr int kWgradPixels = 8192;  // pixels of an FP32 partial
-constexpr int kWgradChunk = 128;    // pixels staged at a time
 
 struct WgradArgs {
   const float* in;    // [B][Ci][H][W]
@@ -324,27 +324,6 @@ struct WgradArgs {
   int B, Ci, Co, H, W;
   unsigned int rw;    // about 2^32 / W
   int step_b, step_p; // kWgradChunk pixels as whole images and pixels of the next
-};
-
-// Linear pixel index of a batch as (image, pixel of its plane), advanced by chunks.
-struct PixelPos {
-  int q, b, p;
-  __device__ __forceinline__ void start(int q0, int HW) {
-    q = q0;
-    b = q0 > 0 ? q0 / HW : 0;
-    p = q0 - b * HW;  // (-1 before the first)
-  }
-  // (a chunk may hold many images: a loop over them took 156 us for 1,000 x 1,000
-  // channels of one pixel)
-  __device__ __forceinline__ void next(int HW, int step_b, int step_p) {
-    q += kWgradChunk;
-    b += step_b;
-    p += step_p;
-    if (p >= HW) {
-      p -= HW;
-      b++;
-    }
-  }
 };
 
 // A wave owns one tap's 32 output x 32 input channels over a range of 8192 pixels
@@ -421,8 +400,8 @@ __global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(W
       }
 #pragma unroll
       for (int h = 0; h < 2; h++) {
-        const int p = ip[h].p + (ky - P) * a.W;
-        I k = ip[h].q < npix && p >= 0 && p < HW ? ii * ip[h].b + (I)p * 4u + i0 : 0;
+        const int p = ip[h].shifted((ky - P) * a.W, HW, npix);
+        I k = p >= 0 ? ii * ip[h].b + (I)p * 4u + i0 : 0;
 #pragma unroll
         for (int j = 0; j < NCH; j++) {
           ri[h][j] = at(a.in, k);
@@ -430,8 +409,8 @@ __global__ __launch_bounds__(64 * (KS + kWgradLoaders)) void conv_wgrad_kernel(W
         }
       }
       if (end) {
-        const int p = tail.p + (ky - P) * a.W;
-        re = at(a.in, tail.q < npix && p >= 0 && p < HW ? ii * tail.b + (I)p * 4u + t0 : 0);
+        const int p = tail.shifted((ky - P) * a.W, HW, npix);
+        re = at(a.in, p >= 0 ? ii * tail.b + (I)p * 4u + t0 : 0);
         tail.next(HW, a.step_b, a.step_p);
       }
 #pragma unroll
@@ -926,9 +905,9 @@ gvm_status conv_launch_part(gvm_ctx* ctx, const ConvArgs<WT>& a) {
     else
       return launch_tile<MODE, 1, 32, 8, 32, 32, WT>(ctx, a);
   } else {
-    const long wide = blocks(8, 32, 64), chunks = (a.C + 7) / 8;
+    const long wide = blocks(8, 32, 64), chunks = (a.C + 7) / 8, two_each = 2L * ctx->cu_count;
     const double tile_us = a.M <= 32     ? ConvCost{5.2, 2.6, 0.0069, 0.75}.us(tiles, chunks)
-                           : wide >= 512 ? ConvCost{5.0, 0.15, 0.018, 1.1}.us(wide, chunks)
+                           : wide >= two_each ? ConvCost{5.0, 0.15, 0.018, 1.1}.us(wide, chunks)
                                          : ConvCost{4.8, 1.75, 0.0036, 1.4}.us(blocks(8, 8, 64), chunks);
     const double im2col_us = ConvCost{3.6, 1.0, 0.00143, 2.7}.us(
         (long)cols.x * cols.y, ((long)a.C * 9 + 15) / 16);
@@ -936,7 +915,7 @@ gvm_status conv_launch_part(gvm_ctx* ctx, const ConvArgs<WT>& a) {
       return im2col();
     else if (a.M <= 32)
       return launch_tile<MODE, 3, 32, 8, 32, 8, WT>(ctx, a);
-    else if (wide >= 512)
+    else if (wide >= two_each)
       return launch_tile<MODE, 3, 64, 8, 32, 8, WT>(ctx, a);
     else
       return launch_tile<MODE, 3, 64, 8, 8, 8, WT>(ctx, a);
