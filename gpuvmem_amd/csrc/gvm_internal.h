@@ -85,7 +85,7 @@ struct GridPlan {
   float4* rec = nullptr;     // sorted rows: (dx, dy, w, weight)
   uint2* meta = nullptr;     // (row of its slice, cell within the tile and fold)
   float2* rot = nullptr;     // phase-centre rotation, or none
-  long4* items = nullptr;    // (first row, rows, slice, 0)
+  long4* items = nullptr;    // (first row, rows, slice, which item to take in this place)
   int2* merges = nullptr;    // tiles with several items: (first, count)
   int* tile_slot = nullptr;  // [slice][tile]: first item, or -1
   float2* tw2 = nullptr;     // e^{2 pi i k / 2N}
