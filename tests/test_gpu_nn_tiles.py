@@ -250,3 +250,12 @@ def test_a_thousand_million_pixels(ctx):
                                          1, 1, 1, 1), "fwd")
     ctx.sync()
     assert torch.equal(y, x.mul_(0.5).add_(1.0))
+
+
+def test_pixels_beyond_the_weight_gradients_indices(ctx):
+    """Refused before anything is launched: the last range would end past 2^31."""
+    z = ctx.zeros(4)
+    st = ctx.lib.gvm_nn_conv_bwd(ctx.ctx, z.ptr, z.ptr, None, z.ptr, None, z.ptr, z.ptr,
+                                 (1 << 31) - 100, 1, 1, 1, 1, 1, 0)
+    with pytest.raises(native.GvmError):
+        native.check(st, "bwd")
