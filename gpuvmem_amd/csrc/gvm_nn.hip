@@ -986,7 +986,7 @@ gvm_status conv_bwd_launch(gvm_ctx* ctx, const float* in, const WT* w, const flo
                   (long)Co * K * K < (1L << 24),
               "gvm_nn_conv_bwd: sizes beyond the kernels' 32-bit indices");
   // (the end of the last range, and two chunks past it, are 32-bit indices too)
-  GVM_REQUIRE((long)B * H * W <= (1L << 31) - 2 * kWgradPixels,
+  GVM_REQUIRE((long)B * H * W <= (1L << 31) - kWgradPixels,
               "gvm_nn_conv_bwd: pixels beyond the weight gradient's 32-bit indices");
   const float* mask = relu ? out : nullptr;
   if (din) {
